@@ -363,6 +363,17 @@ int tfhip_dequant_affine(const void *q, int bits, int64_t n, double scale,
                          double min, void *out, int to_int32);
 int tfhip_dequant_f16(const void *q, int64_t n, float *out);
 
+/* decodeWeights as a whole (io_utils.ts:119-292 for the numeric dtypes): uploads a weight buffer of
+ * `bytes` from host memory once and expands its `count` tensors with one launch, each into a new block
+ * of the library's pool (outs[i]; the caller frees them with tfhip_free). Tensor i has elems[i] elements
+ * from byte offsets[i] of the buffer on, any alignment; scale_min holds its scale and min at 2i and 2i+1
+ * (used by the affine kinds). kinds: 0 four-byte elements copied as they are (float32, int32), 1 one-byte
+ * elements copied (bool), 2 / 3 uint8 affine to float32 / int32, 4 / 5 uint16 affine to float32 / int32,
+ * 6 float16. The same values as tfhip_dequant_affine and tfhip_dequant_f16. The host buffer may be reused
+ * on return; on failure no block is left behind. */
+int tfhip_decode_weights(const void *host, size_t bytes, int64_t count, const int64_t *offsets,
+                         const int64_t *elems, const int *kinds, const double *scale_min, void **outs);
+
 /* ---- glue kernels of a MobileNetV2 graph -------------------------------------
  * tfhip_add: broadcasting Add (tfjs-backend-cpu/src/kernels/Add.ts:23-30,
  *   utils/binary_impl.ts:25-68). out has `rank` (<= 6) dims out_shape; a and b

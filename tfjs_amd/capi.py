@@ -70,6 +70,8 @@ SIGNATURES = {
     "tfhip_dequant_affine": [ctypes.c_void_p, ctypes.c_int, c_i64, ctypes.c_double, ctypes.c_double,
                              ctypes.c_void_p, ctypes.c_int],
     "tfhip_dequant_f16": [ctypes.c_void_p, c_i64, ctypes.c_void_p],
+    "tfhip_decode_weights": [ctypes.c_void_p, ctypes.c_size_t, c_i64, c_i64p, c_i64p, ctypes.POINTER(ctypes.c_int),
+                             ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)],
     "tfhip_add": [c_f32p, c_i64p, c_f32p, c_i64p, c_f32p, c_i64p, ctypes.c_int],
     "tfhip_mean_hw": [c_f32p, c_f32p, c_i64, c_i64, c_i64, c_i64],
     "tfhip_binary": [ctypes.c_int, c_f32p, c_i64p, c_f32p, c_i64p, c_f32p, c_i64p, ctypes.c_int],
@@ -121,6 +123,13 @@ class DeviceBuffer:
         ptr = ctypes.c_void_p()
         check(load_library().tfhip_alloc(max(1, self.nbytes), ctypes.byref(ptr)))
         self.ptr = ptr.value
+
+    @classmethod
+    def adopt(cls, ptr, nbytes):
+        """A block that an entry point of the library has allocated."""
+        buf = cls.__new__(cls)
+        buf.nbytes, buf.ptr = nbytes, ptr
+        return buf
 
     @classmethod
     def from_numpy(cls, array):

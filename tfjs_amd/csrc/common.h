@@ -7,6 +7,9 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <tuple>
+#include <utility>
+
 #include "../../include/tfjs_hip.h"
 
 namespace tfhip {
@@ -39,6 +42,9 @@ struct FixedWorkspace {
   ~FixedWorkspace();
 };
 bool workspace_is_fixed();
+// Host memory -> [d, d + bytes) of a live block, through the pinned staging ring, on the library's stream;
+// the host range may be reused on return.
+int stage_upload(char *d, const char *h, size_t bytes);
 // Records the number of K slices a GEMM launch was cut into (tfhip_workspace_info reports the last).
 void note_splits(int splits);
 size_t fixed_workspace_bytes();
@@ -143,8 +149,32 @@ bool capturing();
 
 // Launch bookkeeping for measurement: the label of the kernel an entry point
 // chose (as a profiler prints the symbol), and how many times each entry point
-// enqueues its kernel (see tfhip_set_launch_repeat).
-void note_kernel(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
+// enqueues its kernel (see tfhip_set_launch_repeat). The label is put together
+// when somebody asks for it: a launch only leaves the format (a string literal)
+// and its arguments (whole numbers and string literals) behind, because printing
+// them costs as much host time as a fifth of the launch.
+struct KernelLabel {
+  static constexpr int kMax = 8;
+  const char *fmt;
+  long long arg[kMax];
+  int (*print)(char *to, size_t len, const KernelLabel &label);
+};
+extern KernelLabel g_kernel_label;
+template <size_t... I, typename... A>
+int print_kernel_label(char *to, size_t len, const KernelLabel &l, std::index_sequence<I...>, std::tuple<A...> *) {
+  if constexpr (sizeof...(A) == 0) return snprintf(to, len, "%s", l.fmt);
+  else return snprintf(to, len, l.fmt, (A)l.arg[I]...);
+}
+template <typename... A>
+inline void note_kernel(const char *fmt, A... args) {
+  static_assert(sizeof...(A) <= KernelLabel::kMax, "arguments of a kernel label");
+  int i = 0;
+  ((g_kernel_label.arg[i++] = (long long)args), ...);
+  g_kernel_label.fmt = fmt;
+  g_kernel_label.print = [](char *to, size_t len, const KernelLabel &l) {
+    return print_kernel_label(to, len, l, std::index_sequence_for<A...>(), (std::tuple<A...> *)nullptr);
+  };
+}
 int launch_repeat();
 
 // Tuning overrides (tfhip_set_tuning, or TFHIP_<NAME> in the environment at

@@ -9,6 +9,8 @@ Each call uploads its operands, launches, downloads the result and frees its
 buffers; `device_*` variants keep data resident for benchmarking.
 """
 import ctypes
+import functools
+import math
 
 import numpy as np
 
@@ -66,6 +68,16 @@ def _opt(a):
     return None if a is None else _f32(a)
 
 
+@functools.lru_cache(maxsize=1024)
+def _stride_array(strides):
+    """The C array of a tuple of strides. The entry points only read them, and a program passes the same
+    few again and again: building one takes 0.8 us, a fifth of what a launch costs the host."""
+    return i64_array(strides)
+
+
+_NO_STRIDES = i64_array([0, 0, 0])
+
+
 def matmul_dims(a_shape, b_shape, transpose_a, transpose_b):
     """Shape bookkeeping of BatchMatMul.ts:36-74 (error text included)."""
     a_shape, b_shape = list(a_shape), list(b_shape)
@@ -89,11 +101,13 @@ def device_fused_matmul(a, b, out, batch_a, batch_b, m, n, k, transpose_a=False,
                         bias=None, bias_strides=None, activation="linear", prelu=None,
                         prelu_strides=None, leakyrelu_alpha=0.2):
     """Launch on DeviceBuffers already resident (no copies, no sync)."""
-    check(load_library().tfhip_fused_matmul(
-        a.ptr, b.ptr, out.ptr, batch_a, batch_b, m, n, k, int(bool(transpose_a)), int(bool(transpose_b)),
-        bias.ptr if bias is not None else None, i64_array(bias_strides or [0, 0, 0]),
+    status = load_library().tfhip_fused_matmul(
+        a.ptr, b.ptr, out.ptr, batch_a, batch_b, m, n, k, 1 if transpose_a else 0, 1 if transpose_b else 0,
+        bias.ptr if bias is not None else None, _stride_array(tuple(bias_strides)) if bias_strides else _NO_STRIDES,
         ACTIVATIONS[activation], prelu.ptr if prelu is not None else None,
-        i64_array(prelu_strides or [0, 0, 0]), float(leakyrelu_alpha)))
+        _stride_array(tuple(prelu_strides)) if prelu_strides else _NO_STRIDES, float(leakyrelu_alpha))
+    if status:
+        check(status)
 
 
 def fused_matmul(a, b, bias=None, activation="linear", prelu=None, leakyrelu_alpha=0.2,
@@ -396,75 +410,70 @@ DTYPE_VALUE_SIZE_MAP = {"float32": 4, "float16": 2, "int32": 4, "uint16": 2, "ui
                         "complex64": 8}
 
 
-def _decode_plan(specs):
-    """Validates the manifest entries as decodeWeight does
-    (tfjs-core/src/io/io_utils.ts:196-216, :248-250, :288-290) and returns
-    [(name, dtype, shape, size, byte offset, quantization or None)], total bytes."""
-    plan, offset = [], 0
-    for spec in specs:
-        name, dtype, shape = spec["name"], spec["dtype"], list(spec["shape"])
-        size = int(np.prod(shape, dtype=np.int64)) if shape else 1
-        if "quantization" in spec:
-            q = spec["quantization"]
-            qd = q["dtype"]
-            if qd in ("uint8", "uint16"):
-                if not ("min" in q and "scale" in q):
-                    raise ValueError("Weight %s with quantization %s doesn't have corresponding metadata "
-                                     "min and scale." % (name, qd))
-            elif qd == "float16":
-                if dtype != "float32":
-                    raise ValueError("Weight %s is quantized with %s which only supports weights of type "
-                                     "float32 not %s." % (name, qd, dtype))
-            else:
-                raise ValueError("Weight %s has unknown quantization dtype %s. Supported quantization "
-                                 "dtypes are: 'uint8', 'uint16', and 'float16'." % (name, qd))
-            if dtype not in ("float32", "int32"):
-                raise ValueError("Unsupported dtype in weight '%s': %s" % (name, dtype))
-            nbytes = size * DTYPE_VALUE_SIZE_MAP[qd]
-            plan.append((name, dtype, shape, size, offset, q))
+# kinds of tfhip_decode_weights by (quantization dtype or None, dtype of the weight)
+_DECODE_KINDS = {(None, "float32"): 0, (None, "int32"): 0, (None, "bool"): 1, ("uint8", "float32"): 2,
+                 ("uint8", "int32"): 3, ("uint16", "float32"): 4, ("uint16", "int32"): 5, ("float16", "float32"): 6}
+
+
+def _check_spec(name, dtype, q):
+    """Refuses a manifest entry as decodeWeight does (tfjs-core/src/io/io_utils.ts:196-216, :248-250, :288-290)."""
+    if q is not None:
+        qd = q["dtype"]
+        if qd in ("uint8", "uint16"):
+            if not ("min" in q and "scale" in q):
+                raise ValueError("Weight %s with quantization %s doesn't have corresponding metadata "
+                                 "min and scale." % (name, qd))
+        elif qd == "float16":
+            if dtype != "float32":
+                raise ValueError("Weight %s is quantized with %s which only supports weights of type "
+                                 "float32 not %s." % (name, qd, dtype))
         else:
-            if dtype not in ("float32", "int32", "bool"):
-                raise ValueError("Unsupported dtype in weight '%s': %s" % (name, dtype))
-            nbytes = size * DTYPE_VALUE_SIZE_MAP[dtype]
-            plan.append((name, dtype, shape, size, offset, None))
-        offset += nbytes
-    return plan, offset
+            raise ValueError("Weight %s has unknown quantization dtype %s. Supported quantization "
+                             "dtypes are: 'uint8', 'uint16', and 'float16'." % (name, qd))
+    raise ValueError("Unsupported dtype in weight '%s': %s" % (name, dtype))
+
+
+def _decode_plan(specs):
+    """Validates the manifest entries and returns [(name, shape, size, bytes of the decoded tensor)], the
+    arguments of tfhip_decode_weights and the bytes the manifest covers."""
+    plan, offset = [], 0
+    count = len(specs)
+    offsets, elems, kinds = (ctypes.c_int64 * count)(), (ctypes.c_int64 * count)(), (ctypes.c_int * count)()
+    scale_min = (ctypes.c_double * (2 * count))()
+    for i, spec in enumerate(specs):
+        name, dtype, shape = spec["name"], spec["dtype"], list(spec["shape"])
+        size = math.prod(shape)
+        q = spec.get("quantization")
+        qd = q["dtype"] if q is not None else None
+        kind = _DECODE_KINDS.get((qd, dtype))
+        if kind is None:
+            _check_spec(name, dtype, q)
+        if 2 <= kind <= 5:
+            if "scale" not in q or "min" not in q:
+                _check_spec(name, dtype, q)
+            scale_min[2 * i], scale_min[2 * i + 1] = q["scale"], q["min"]
+        offsets[i], elems[i], kinds[i] = offset, size, kind
+        plan.append((name, shape, size * (1 if kind == 1 else 4)))
+        offset += size * DTYPE_VALUE_SIZE_MAP[qd or dtype]
+    return plan, (count, offsets, elems, kinds, scale_min), offset
 
 
 def decode_weights_to_device(buffer, specs):
     """The dequantize-on-load path with everything staying on the GPU: the whole
-    weight buffer is uploaded once, each quantized entry is expanded by one
-    kernel reading at its byte offset inside that upload, plain entries are
-    copied from the host bytes. Returns {name: (DeviceBuffer, shape)} holding
+    weight buffer is uploaded once and one kernel expands every entry from its byte
+    offset inside that upload. Returns {name: (DeviceBuffer, shape)} holding
     float32 / int32 values (bool entries as bytes)."""
     init()
-    raw = np.frombuffer(bytes(buffer), dtype=np.uint8)
-    plan, total = _decode_plan(specs)
+    plan, args, total = _decode_plan(specs)
+    try:
+        raw = np.frombuffer(buffer, dtype=np.uint8)
+    except (TypeError, ValueError, BufferError):   # no contiguous bytes of its own
+        raw = np.frombuffer(bytes(buffer), dtype=np.uint8)
     if total > raw.size:
         raise ValueError("weight buffer holds %d bytes, the manifest needs %d" % (raw.size, total))
-    lib = load_library()
-    out = {}
-    dq = DeviceBuffer.from_numpy(raw) if any(q is not None for *_, q in plan) else None
-    try:
-        for name, dtype, shape, size, off, q in plan:
-            if q is None:
-                item = 1 if dtype == "bool" else 4
-                dst = DeviceBuffer(size * item)
-                dst.upload(raw[off:off + size * item])
-            else:
-                dst = DeviceBuffer(size * 4)
-                src = ctypes.c_void_p(dq.ptr + off)
-                if q["dtype"] == "float16":
-                    check(lib.tfhip_dequant_f16(src, size, dst.ptr))
-                else:
-                    check(lib.tfhip_dequant_affine(src, 8 if q["dtype"] == "uint8" else 16, size,
-                                                   float(q["scale"]), float(q["min"]), dst.ptr,
-                                                   int(dtype == "int32")))
-            out[name] = (dst, shape)
-    finally:
-        if dq is not None:
-            dq.free()
-    return out
+    outs = (ctypes.c_void_p * len(plan))()
+    check(load_library().tfhip_decode_weights(raw.ctypes.data, total, *args, outs))
+    return {name: (DeviceBuffer.adopt(ptr, nbytes), shape) for (name, shape, nbytes), ptr in zip(plan, outs)}
 
 
 def decode_weights(buffer, specs):
