@@ -1,12 +1,14 @@
 // FusedDepthwiseConv2D, NHWC float32.
 //
-// Bandwidth-bound (about 2 flops per byte), so no matrix cores. Three kernels:
+// Bandwidth-bound (about 2 flops per byte), so no matrix cores. Four kernels:
 //  * depthwise_3x3_cols: 3x3, stride 1 or 2, channel multiplier 1 (every
 //    MobileNet layer). Lanes lie along an output row in memory order, one float4
 //    of one column each, and walk down a chunk of rows with the input rows in a
 //    register ring; no LDS, no barriers.
 //  * depthwise_3x3_halo: the same shapes when a tensor is too large for 32-bit
 //    buffer offsets; stages an input halo tile of 32 channels in LDS.
+//  * depthwise_cols_sums: the same walk for 5x5 filters and for channel counts
+//    that are no multiple of four, with running sums instead of a row ring.
 //  * depthwise_generic: any filter, stride, dilation, channel multiplier.
 // Each output accumulates its taps in the reference's own order (filter row,
 // then filter column: tfjs-backend-cpu/src/kernels/DepthwiseConv2dNative.ts:62-95)
@@ -141,6 +143,7 @@ constexpr unsigned kDwNoOffset = 0xffffffffu;
 // instead, 21.6 and 13.6 us).
 constexpr long long kDwStreamBytes = 8LL << 20;
 typedef unsigned int dw_uint4 __attribute__((ext_vector_type(4)));
+typedef unsigned int dw_uint2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float4 dw_load4(__amdgpu_buffer_rsrc_t r, unsigned off) {
 #ifndef TFHIP_DW_LOAD_AUX
@@ -219,6 +222,7 @@ struct DwColsArgs {
   int chunks_h, rows;  // row chunks per image, output rows per chunk
   int xcd_run;         // > 0: workgroup ids are dealt to the XCDs in contiguous runs of this many
   unsigned x_bytes, y_bytes;
+  int streamed;        // the result is stored non-temporally (kDwStreamBytes)
 };
 
 template <int S, bool GENERAL, bool STREAM>
@@ -300,9 +304,175 @@ __global__ __launch_bounds__(kColsThreads) void depthwise_3x3_cols(DwParams p, E
   }
 }
 
+// ---- F x F, channel multiplier 1, dilation 1, stride S: the same walk with running sums ------
+// The 5x5 filters, and channel counts that are no multiple of four (a lane owns VEC = 2 or 1 channels of
+// one column instead of four). Keeping the five input rows of a window in registers, as the kernel above
+// keeps three, would take 120 of them beside the 100 of the filter; here an input row is used the moment it
+// has arrived - it adds filter row i - S o to every output row o of the lane's column that it belongs
+// to - and dropped, so the lane keeps ceil(F / S) sums instead of F rows. Each sum still takes its taps
+// from zero by filter row, then column, one fused multiply-add each: the bits of the general kernel.
+// That one fetches every tap's input and filter value per output element (50 loads, four 64-bit divisions):
+// [8,57,43,120] 5x5 stride 2, 12 MB, 22.9 us there and 5.6 here (2 us of bytes: the launch is bound by the latency
+// of its few loads per lane); [3,99,74,570] 3x3, 100 MB, 147 -> 20 us.
+template <int VEC>
+struct DwVec {
+  float v[VEC];
+};
+
+template <int VEC>
+__device__ __forceinline__ DwVec<VEC> dw_load(__amdgpu_buffer_rsrc_t r, unsigned off) {
+  DwVec<VEC> t;
+  if (VEC == 4) {
+    const float4 q = dw_load4(r, off);
+    t.v[0] = q.x; t.v[1 % VEC] = q.y; t.v[2 % VEC] = q.z; t.v[3 % VEC] = q.w;
+  } else if (VEC == 2) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+    t.v[0] = __uint_as_float(q[0]); t.v[1 % VEC] = __uint_as_float(q[1]);
+  } else {
+    t.v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+  }
+  return t;
+}
+
+template <int VEC, bool STREAM>
+__device__ __forceinline__ void dw_store(__amdgpu_buffer_rsrc_t r, unsigned off, const DwVec<VEC> &t) {
+  constexpr int kAux = STREAM ? 2 : 0;
+  if (VEC == 4) dw_store4<STREAM>(r, off, make_float4(t.v[0], t.v[1 % VEC], t.v[2 % VEC], t.v[3 % VEC]));
+  else if (VEC == 2) __builtin_amdgcn_raw_buffer_store_b64((dw_uint2){__float_as_uint(t.v[0]), __float_as_uint(t.v[1 % VEC])}, r, (int)off, 0, kAux);
+  else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(t.v[0]), r, (int)off, 0, kAux);
+}
+
+// c4_total and row_quads of the arguments count units of VEC channels.
+template <int F, int S, int VEC, bool GENERAL, bool STREAM>
+__global__ __launch_bounds__(kColsThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void depthwise_cols_sums(DwParams p, Epilogue e, DwColsArgs g) {
+  constexpr int NACC = (F + S - 1) / S;   // output rows in progress
+  const unsigned wg = g.xcd_run ? (blockIdx.x % 8) * (unsigned)g.xcd_run + blockIdx.x / 8 : blockIdx.x;
+  const int bx = (int)(wg % (unsigned)g.blocks_per_row);
+  const unsigned t = wg / (unsigned)g.blocks_per_row;
+  const int chunk = (int)(t % (unsigned)g.chunks_h), n = (int)(t / (unsigned)g.chunks_h);
+  const int f = bx * kColsThreads + (int)threadIdx.x;
+  if (f >= g.row_quads) return;
+  const int ow = f / g.c4_total, q = f - ow * g.c4_total;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)g.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.y, 0, (int)g.y_bytes, 0x00020000);
+  constexpr unsigned kUnit = 4u * VEC;
+  const unsigned pix = (unsigned)g.c4_total * kUnit;   // bytes per pixel
+  const unsigned x_row = (unsigned)p.in_w * pix, y_row = (unsigned)p.out_w * pix;
+  const unsigned x_img = (unsigned)n * (unsigned)p.in_h * x_row, y_img = (unsigned)n * (unsigned)p.out_h * y_row;
+  const int oh0 = chunk * g.rows;
+  const int rows = oh0 + g.rows <= p.out_h ? g.rows : p.out_h - oh0;
+  const int rows_in = (rows - 1) * S + F;
+  const int ih0 = oh0 * S - p.pad_top;
+  unsigned x_col[F];
+#pragma unroll
+  for (int wc = 0; wc < F; ++wc) {
+    const int iw = ow * S - p.pad_left + wc;
+    x_col[wc] = (iw >= 0 && iw < p.in_w) ? (unsigned)iw * pix + (unsigned)q * kUnit : kDwNoOffset;
+  }
+  const unsigned y_col = (unsigned)f * kUnit;
+  auto fetch = [&](DwVec<VEC> (&row)[F], int i) __attribute__((always_inline)) {
+    const int ih = ih0 + i;
+    const bool row_ok = ih >= 0 && ih < p.in_h && i < rows_in;
+    const unsigned row_off = x_img + (unsigned)ih * x_row;
+#pragma unroll
+    for (int wc = 0; wc < F; ++wc)
+      row[wc] = dw_load<VEC>(rx, (row_ok && x_col[wc] != kDwNoOffset) ? row_off + x_col[wc] : kDwNoOffset);
+  };
+  // the first window's rows, the filter and the bias: one round trip for all of them
+  DwVec<VEC> first[F - S][F], cur[S][F], nxt[S][F], w[F * F], bias = {};
+#pragma unroll
+  for (int i = 0; i < F - S; ++i) fetch(first[i], i);
+#pragma unroll
+  for (int j = 0; j < S; ++j) fetch(cur[j], F - S + j);
+#pragma unroll
+  for (int k = 0; k < F * F; ++k)
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) w[k].v[v] = p.w[((long long)k * g.c4_total + q) * VEC + v];
+  const int c = q * VEC;
+  if (!GENERAL && e.bias) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) bias.v[v] = e.bias[(long long)(c + v) * e.bias_s[3]];
+  }
+  DwVec<VEC> acc[NACC] = {};
+  // filter row wr of an output row in progress
+  auto add = [&](DwVec<VEC> &a, const DwVec<VEC> (&row)[F], int wr) __attribute__((always_inline)) {
+#pragma unroll
+    for (int wc = 0; wc < F; ++wc)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v)
+        a.v[v] = fmaf(row[wc].v[v], w[wr * F + wc].v[v], (wr == 0 && wc == 0) ? 0.f : a.v[v]);
+  };
+#pragma unroll
+  for (int i = 0; i < F - S; ++i)
+#pragma unroll
+    for (int d = 0; d * S <= i; ++d) add(acc[d % NACC], first[i], i - d * S);
+  for (int o0 = 0; o0 < rows; o0 += NACC) {
+#pragma unroll
+    for (int k = 0; k < NACC; ++k) {
+      const int o = o0 + k;
+      if (o < rows) {
+        // rows S o + F - S .. S o + F - 1 complete output row o and go into the ones after it
+#pragma unroll
+        for (int j = 0; j < S; ++j) fetch(nxt[j], S * (o + 1) + F - S + j);
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+#pragma unroll
+          for (int d = 0; d * S <= F - S + j; ++d) add(acc[(k + d) % NACC], cur[j], F - S + j - d * S);
+        const int oh = oh0 + o;
+        DwVec<VEC> &a = acc[k % NACC];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+          a.v[v] = GENERAL ? finish(e, a.v[v], 0, 0, c + v, n, oh, ow) : relu_family(a.v[v] + bias.v[v], e.activation);
+        const unsigned off = y_img + (unsigned)oh * y_row + y_col;
+        dw_store<VEC, STREAM>(ry, off, a);
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+#pragma unroll
+          for (int wc = 0; wc < F; ++wc) cur[j][wc] = nxt[j][wc];
+      }
+    }
+  }
+}
+
 int balanced_tile(int extent, int max_tile) {
   const int tiles = (extent + max_tile - 1) / max_tile;
   return (extent + tiles - 1) / tiles;
+}
+
+// Output rows per lane of the column kernels: chunks as long as `rows` read few rows twice; shorter ones, down to a
+// single row, until the launch has `per_cu` wavefronts for every compute unit. Fills the launch geometry; false when
+// it does not fit a grid.
+bool plan_cols(DwColsArgs &g, const DwParams &p, int vec, int rows, int per_cu) {
+  g.c4_total = p.in_c / vec;
+  g.row_quads = p.out_w * g.c4_total;
+  g.blocks_per_row = (g.row_quads + kColsThreads - 1) / kColsThreads;
+  if (tuning(kTuneDwRows) > 0) {
+    rows = tuning(kTuneDwRows);
+  } else {
+    const long long want = (long long)per_cu * num_cus();
+    while (rows > 1 && (long long)g.blocks_per_row * ((p.out_h + rows - 1) / rows) * p.batch < want) rows = (rows + 1) / 2;
+  }
+  rows = rows > p.out_h ? p.out_h : rows;
+  g.rows = balanced_tile(p.out_h, rows);
+  g.chunks_h = (p.out_h + g.rows - 1) / g.rows;
+  g.x_bytes = (unsigned)((long long)p.batch * p.in_h * p.in_w * p.in_c * 4);
+  g.y_bytes = (unsigned)((long long)p.batch * p.out_h * p.out_w * p.in_c * 4);
+  g.streamed = g.y_bytes >= kDwStreamBytes;
+  const long long wgs = (long long)g.blocks_per_row * g.chunks_h * p.batch;
+  g.xcd_run = wgs % 8 == 0 ? (int)(wgs / 8) : 0;
+  return wgs <= 0x7fffffffLL;
+}
+
+template <int F, int S, int VEC>
+int launch_cols_sums(const DwParams &p, const Epilogue &e, const DwColsArgs &g, bool general) {
+  const dim3 grid((unsigned)((long long)g.blocks_per_row * g.chunks_h * p.batch)), block(kColsThreads);
+  const bool streamed = !general && g.streamed;
+  note_kernel("depthwise_cols_sums<%d, %d, %d, %s, %s>", F, S, VEC, general ? "true" : "false", streamed ? "true" : "false");
+  if (general) TFHIP_LAUNCH((depthwise_cols_sums<F, S, VEC, true, false><<<grid, block, 0, stream()>>>(p, e, g)));
+  else if (streamed) TFHIP_LAUNCH((depthwise_cols_sums<F, S, VEC, false, true><<<grid, block, 0, stream()>>>(p, e, g)));
+  else TFHIP_LAUNCH((depthwise_cols_sums<F, S, VEC, false, false><<<grid, block, 0, stream()>>>(p, e, g)));
+  return kOk;
 }
 
 }  // namespace
@@ -378,6 +548,7 @@ extern "C" int tfhip_fused_depthwise_conv2d(
 
   const bool aligned16 = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(filter) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(y) % 16 == 0;
+  const bool aligned8 = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) % 8 == 0;
   // The 3x3 kernels read a zero for a tap outside the image and multiply it by the filter value; the
   // reference skips the tap (DepthwiseConv2dNative.ts:72-86), which differs under a value that is not
   // finite: such a filter, where a window can reach outside, takes the general kernel, which skips.
@@ -389,39 +560,22 @@ extern "C" int tfhip_fused_depthwise_conv2d(
     const int rc = scan_filter(filter, f_h * f_w * in_c * ch_mul, "tfhip_fused_depthwise_conv2d", &nonfinite);
     if (rc != kOk) return rc;
   }
-  const bool fast = f_h == 3 && f_w == 3 && ch_mul == 1 && dilation_h == 1 && dilation_w == 1 &&
-                    stride_h == stride_w && (stride_h == 1 || stride_h == 2) && in_c % 4 == 0 && aligned16 &&
-                    batch <= 65535 && !nonfinite;
+  // square 3x3 and 5x5 filters whose windows move by one or two pixels
+  const bool walk = f_h == f_w && (f_h == 3 || f_h == 5) && ch_mul == 1 && dilation_h == 1 && dilation_w == 1 &&
+                    stride_h == stride_w && (stride_h == 1 || stride_h == 2) && !nonfinite;
+  const bool quads = in_c % 4 == 0 && aligned16;
+  const bool fast = walk && f_h == 3 && quads && batch <= 65535;
   // the row pipeline addresses both tensors with 32-bit byte offsets
   const bool fits32 = batch * in_h * in_w * in_c * 4 <= 0xfffffff0LL && total * 4 <= 0xfffffff0LL;
   if (fast && fits32 && tuning(kTuneDwHalo) <= 0) {
     const int S = (int)stride_h;
     DwColsArgs g;
-    g.c4_total = (int)(in_c / 4);
-    g.row_quads = (int)out_w * g.c4_total;
-    g.blocks_per_row = (g.row_quads + kColsThreads - 1) / kColsThreads;
-    // Rows per chunk: a chunk of r output rows fetches (r - 1) S + 3 input rows, so longer chunks re-read
-    // fewer rows, and shorter ones make more wavefronts. 14 rows (8 at stride 2) measured best on
-    // [8,112,112,96] with operands from memory (stride 1: 18.7 us at 14 rows, 19.2 at 8, 20.5 at 4, 22.2 at 28;
-    // stride 2: 11.6 at 8, 13.5 at 14); smaller launches take shorter chunks until there are two
-    // wavefronts for every SIMD of the chip.
-    int rows = S == 1 ? 14 : 8;
-    if (tuning(kTuneDwRows) > 0) {
-      rows = tuning(kTuneDwRows);
-    } else {
-      const long long want = 8LL * num_cus();
-      while (rows > 1 && (long long)g.blocks_per_row * ((out_h + rows - 1) / rows) * batch < want) rows = (rows + 1) / 2;
-    }
-    rows = rows > out_h ? (int)out_h : rows;
-    g.rows = balanced_tile((int)out_h, rows);
-    g.chunks_h = ((int)out_h + g.rows - 1) / g.rows;
-    g.x_bytes = (unsigned)(batch * in_h * in_w * in_c * 4);
-    g.y_bytes = (unsigned)(total * 4);
-    const long long wgs = (long long)g.blocks_per_row * g.chunks_h * batch;
-    if (wgs <= 0x7fffffffLL) {
-      g.xcd_run = wgs % 8 == 0 ? (int)(wgs / 8) : 0;
+    // 14 output rows per lane (8 at stride 2) measured best on [8,112,112,96] with operands from memory
+    // (stride 1: 18.7 us at 14 rows, 19.2 at 8, 20.5 at 4, 22.2 at 28; stride 2: 11.6 at 8, 13.5 at 14)
+    if (plan_cols(g, p, 4, S == 1 ? 14 : 8, 8)) {
+      const long long wgs = (long long)g.blocks_per_row * g.chunks_h * batch;
       const bool general = !(e.addressing == kChannel && activation <= TFHIP_RELU6);
-      const bool streamed = !general && total * 4 >= kDwStreamBytes;
+      const bool streamed = !general && g.streamed;
       note_kernel("depthwise_3x3_cols<%d, %s, %s>", S, general ? "true" : "false", streamed ? "true" : "false");
       const dim3 grid((unsigned)wgs), block(kColsThreads);
       if (S == 1 && streamed)
@@ -437,6 +591,23 @@ extern "C" int tfhip_fused_depthwise_conv2d(
       else
         TFHIP_LAUNCH((depthwise_3x3_cols<2, true, false><<<grid, block, 0, stream()>>>(p, e, g)));
       return kOk;
+    }
+  }
+  if (walk && !fast && fits32) {
+    DwColsArgs g;
+    const int vec = quads ? 4 : (in_c % 2 == 0 && aligned8 ? 2 : 1);
+    // (a 5x5 lane of four channels is heavy on registers and a chunk of one row fetches five: two wavefronts per
+    // compute unit are enough there - [8,57,43,120] stride 2: 5.6 us at 704 workgroups, 6.4 at 1320, 8.1 at 2552)
+    if (plan_cols(g, p, vec, stride_h == 1 ? 14 : 8, f_h == 5 && vec == 4 ? 2 : 8)) {
+      const bool general = !(e.addressing == kChannel && activation <= TFHIP_RELU6);
+      const bool one = stride_h == 1;
+      if (f_h == 5) {
+        if (vec == 4) return one ? launch_cols_sums<5, 1, 4>(p, e, g, general) : launch_cols_sums<5, 2, 4>(p, e, g, general);
+        if (vec == 2) return one ? launch_cols_sums<5, 1, 2>(p, e, g, general) : launch_cols_sums<5, 2, 2>(p, e, g, general);
+        return one ? launch_cols_sums<5, 1, 1>(p, e, g, general) : launch_cols_sums<5, 2, 1>(p, e, g, general);
+      }
+      if (vec == 2) return one ? launch_cols_sums<3, 1, 2>(p, e, g, general) : launch_cols_sums<3, 2, 2>(p, e, g, general);
+      if (vec == 1) return one ? launch_cols_sums<3, 1, 1>(p, e, g, general) : launch_cols_sums<3, 2, 1>(p, e, g, general);
     }
   }
   if (fast) {
