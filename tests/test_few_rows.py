@@ -1,0 +1,105 @@
+"""Products of few rows against the oracle, at the edges of the kernel that takes them: row blocks of 16, strips of 16 and
+64 columns, k groups of 16 and their slices, extents that no float4 fits, operands at odd addresses, and the
+two forms of adding the slices (a counter per strip; in a recording, a launch of its own)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tfjs_amd import capi
+from tfjs_amd.capi import DeviceBuffer, check, i64_array
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from tfjs_amd import pyhost
+    pyhost.init()
+    return capi.load_library()
+
+
+def _last_kernel(lib):
+    name = ctypes.create_string_buffer(256)
+    lib.tfhip_last_kernel(name, 256)
+    return name.value.decode()
+
+
+class _Product:
+    """out = act(a b + bias) with every operand `shift` floats into its block."""
+
+    def __init__(self, lib, m, n, k, act, shift=0):
+        rng = np.random.default_rng(m * 31 + n * 7 + k)
+        self.lib, self.act, self.shift, self.shape = lib, act, shift, (m, n, k)
+        self.host = [rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n), (n,))]
+        self.bufs = [DeviceBuffer.from_numpy(np.concatenate([np.full(shift, np.nan, np.float32), x.reshape(-1)])) for x in self.host]
+        self.bufs.append(DeviceBuffer.from_numpy(np.full(shift + m * n, np.nan, np.float32)))
+
+    def launch(self):
+        m, n, k = self.shape
+        a, b, bias, out = (buf.ptr + 4 * self.shift for buf in self.bufs)
+        check(self.lib.tfhip_fused_matmul(a, b, out, 1, 1, m, n, k, 0, 0, bias, i64_array([0, 0, 1]),
+                                          capi.ACTIVATIONS[self.act], None, i64_array([0] * 3), 0.2))
+
+    def result(self):
+        m, n, _ = self.shape
+        return self.bufs[-1].download(np.float32, m * n, 4 * self.shift).reshape(m, n)
+
+    def free(self):
+        for buf in self.bufs:
+            buf.free()
+
+
+@pytest.mark.parametrize("m,n,k,act,shift", [
+    (1, 1, 1, "linear", 0), (16, 16, 16, "relu", 0), (17, 17, 17, "relu6", 1), (32, 1000, 1280, "linear", 0),
+    (33, 77, 513, "sigmoid", 0), (64, 65, 1030, "elu", 3), (64, 1024, 300, "leakyrelu", 0), (5, 4097, 2050, "relu", 0),
+    (23, 4100, 2049, "linear", 1), (64, 2051, 4099, "linear", 0), (1, 64, 4095, "elu", 0), (2, 40, 16 * 64 * 8 + 1, "linear", 2),
+])
+def test_against_the_oracle(lib, m, n, k, act, shift):
+    from oracle import pyoracle as orc
+    p = _Product(lib, m, n, k, act, shift)
+    try:
+        for _ in range(2):   # (the second launch finds the counters the first one left)
+            p.launch()
+            assert _last_kernel(lib).startswith("few_rows<")
+            got = p.result()
+            want = orc.fused_matmul(p.host[0], p.host[1], bias=p.host[2], activation=act, leakyrelu_alpha=0.2)
+            assert np.max(np.abs(got - want) / np.maximum(1.0, np.abs(want))) <= 1e-4
+    finally:
+        p.free()
+
+
+def test_a_recording_gives_the_same_bits(lib):
+    p = _Product(lib, 19, 200, 2000, "relu")
+    try:
+        p.launch()
+        want = p.result()
+        graph, nodes = ctypes.c_int(), ctypes.c_int()
+        check(lib.tfhip_capture_begin())
+        p.launch()
+        check(lib.tfhip_capture_end(ctypes.byref(graph), ctypes.byref(nodes)))
+        assert nodes.value == 2
+        for _ in range(3):
+            p.bufs[-1].upload(np.full(19 * 200, np.nan, np.float32))
+            check(lib.tfhip_graph_launch(graph.value))
+            np.testing.assert_array_equal(p.result().view(np.uint32), want.view(np.uint32))
+            p.launch()
+            np.testing.assert_array_equal(p.result().view(np.uint32), want.view(np.uint32))
+        check(lib.tfhip_graph_destroy(graph.value))
+    finally:
+        p.free()
+
+
+def test_what_lies_behind_a_row_stays_out_of_it(lib):
+    """A float4 at the end of a row of A reaches into the next row: its Inf and NaN must not."""
+    p = _Product(lib, 4, 20, 18, "linear")
+    try:
+        p.host[0][2] = np.nan
+        p.host[0][3] = np.inf
+        p.bufs[0].upload(p.host[0])
+        p.launch()
+        got = p.result()
+        np.testing.assert_allclose(got[:2], p.host[0][:2].astype(np.float64) @ p.host[1] + p.host[2], rtol=0, atol=1e-5)
+        assert np.isnan(got[2]).all() and not np.isfinite(got[3]).any()
+    finally:
+        p.free()

@@ -1,12 +1,14 @@
 // _FusedMatMul / BatchMatMul entry point: validates the operands, picks the
 // loaders the memory layout allows and a tile shape, and launches gemm_kernel.
 #include "gemm_host.h"
+#include "few_rows.h"
 #include "skinny_gemm.h"
 
 using namespace tfhip;
 
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
+  if (!transpose_a && !transpose_b && few_rows_applies(p, vec)) return launch_few_rows(p);
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());
     if (!transpose_a && !transpose_b) return launch_gemm_shape<kLoadKVec, kLoadXVec>(shape, p);
@@ -18,6 +20,66 @@ int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, 
 }
 
 namespace tfhip {
+namespace {
+
+constexpr int kFewRowsCounters = 256;
+static __device__ int few_rows_counters[kFewRowsCounters];   // one per strip that is cut, zero between launches
+
+template <int MB, int CB>
+int launch_few_rows_shape(FewRowsArgs &q) {
+  const int strips = (q.N + 16 * CB - 1) / (16 * CB);
+  // A wavefront wants about as many k groups as it fetches at once (64, 32 or 16 groups per workgroup); more
+  // workgroups than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
+  int splits = (q.groups + 64 / MB - 1) / (64 / MB);
+  if (splits > 256 / strips) splits = 256 / strips;
+  q.splits = 1;
+  q.groups_per_split = q.groups;
+  if (splits > 1) {
+    q.ws = static_cast<float *>(workspace((size_t)strips * splits * 256 * MB * CB * sizeof(float)));
+    if (q.ws) {
+      q.splits = splits;
+      q.groups_per_split = (q.groups + splits - 1) / splits;
+    }
+  }
+  note_splits(q.splits);
+  // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
+  // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
+  q.finish_apart = q.splits > 1 && capturing();
+  note_kernel("few_rows<%d, %d>", MB, CB);
+  const dim3 grid((unsigned)(strips * q.splits)), block(64 * kFewRowsWaves);
+  if (q.finish_apart) {
+    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)strips), block, 0, stream()>>>(q)));
+  } else {
+    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q)));
+  }
+  return kOk;
+}
+
+}  // namespace
+
+int launch_few_rows(const GemmParams &p) {
+  FewRowsArgs q = {};
+  q.a = p.a; q.b = p.b; q.c = p.c;
+  q.bias = p.epi.bias; q.bias_stride = p.epi.bias ? p.epi.bias_s[3] : 0;
+  q.prelu = p.epi.prelu; q.prelu_stride = p.epi.prelu ? p.epi.prelu_s[3] : 0;
+  q.residual = p.epi.residual;
+  q.leaky_alpha = p.epi.leaky_alpha;
+  q.activation = p.epi.activation;
+  q.M = p.M; q.N = p.N; q.K = p.K;
+  q.a_bytes = (unsigned)((long long)p.M * p.K * 4);
+  q.b_bytes = (unsigned)((long long)p.K * p.N * 4);
+  q.groups = (p.K + 15) / 16;
+  static int *counters = nullptr;
+  if (!counters) TFHIP_CHECK_HIP(hipGetSymbolAddress(reinterpret_cast<void **>(&counters), HIP_SYMBOL(few_rows_counters)));
+  q.counters = counters;
+  // Strips of 64 columns, whole cache lines, once B is tens of megabytes (1 x 4096 x 4096: 14.2 us, 15.5 with strips
+  // of 16), else of 16: as many workgroups as there are.
+  const bool wide = (long long)p.K * p.N >= (8LL << 20);
+  if (p.M <= 16) return wide ? launch_few_rows_shape<1, 4>(q) : launch_few_rows_shape<1, 1>(q);
+  if (p.M <= 32) return wide ? launch_few_rows_shape<2, 4>(q) : launch_few_rows_shape<2, 1>(q);
+  return wide ? launch_few_rows_shape<4, 2>(q) : launch_few_rows_shape<4, 1>(q);
+}
+
 namespace {
 
 // Scratch of tfhip_fused_matmul_noalloc: the split-K partial sums that
