@@ -424,9 +424,24 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
     if (rc == kOk && residual) rc = launch_add_residual(y, residual, M * out_c);
     return rc;
   }
-  if (vec) {
-    const int shape = choose_tile_shape(M, out_c, K, 1, num_cus());
-    return launch_gemm_shape<kLoadIm2colVec, kLoadXVec>(shape, p);
+  if (!nchw && p.a_bytes != 0 && p.b_bytes != 0) {
+    const bool filter_rows = dilation_w == 1;
+    g.seg_len = (int)(filter_rows ? f_w * in_c : in_c);
+    g.taps = (int)(filter_rows ? 1 : f_w);
+    g.units = (g.seg_len + 3) / 4;
+    g.unit_magic = g.units == 1 ? 0 : (int)(unsigned)(((1ULL << 32) + g.units - 1) / g.units);
+    g.row_len = (int)(in_w * in_c); g.image_len = (int)(in_h * in_w * in_c);
+    g.stride_wc = (int)(stride_w * in_c); g.pad_leftc = (int)(pad_left * in_c);
+    g.seg_row = (int)(dilation_h * in_w * in_c); g.seg_col = (int)(dilation_w * in_c);
+    const int64_t units = (filter_rows ? f_h : f_h * f_w) * (int64_t)g.units;
+    // (the magic number is exact while units * g.units < 2^32)
+    if (units * g.units < (int64_t(1) << 32) && in_h * in_w * in_c < lim && dilation_h * in_w * in_c < lim &&
+        (f_h - 1) * dilation_h * in_w * in_c + f_w * dilation_w * in_c < lim && stride_w * out_w * in_c < lim && pad_left * in_c < lim) {
+      p.K = (int)(4 * units);
+      const int shape = choose_tile_shape(M, out_c, p.K, 1, num_cus());
+      if (vec) return launch_gemm_shape<kLoadWindows, kLoadXVec>(shape, p);
+      return launch_gemm_shape<kLoadWindowsAny, kLoadFilter>(shape, p);
+    }
   }
   if (out_c <= 32) return launch_gemm<256, 32, 16, 4, 1, kLoadIm2colScalar, kLoadScalar>(p);
   return launch_gemm<64, 64, 16, 2, 2, kLoadIm2colScalar, kLoadScalar>(p);

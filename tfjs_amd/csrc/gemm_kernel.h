@@ -33,13 +33,18 @@
 //   enqueued right behind.
 // * Loaders (template parameter) decide how a tile is fetched:
 //     kLoadKVec   operand is k-contiguous in memory (A row-major, or B given
-//                 transposed): 16-byte loads along k, transposed into LDS
+//                 transposed): 16-byte loads along k. kLoadKAny: the same for
+//                 rows of any length and 4-byte alignment (a buffer load needs no
+//                 more); what a row's last 16 bytes hold of the next row is masked
 //     kLoadXVec   operand is x-contiguous (B row-major, or A given transposed):
-//                 16-byte loads along x, 16-byte LDS stores
+//                 16-byte loads along x, transposed into LDS; any row length and
+//                 alignment (the last ones of a row reach into columns nobody keeps)
 //     kLoadScalar any strides, element loads with bounds checks
-//     kLoadIm2colVec / kLoadIm2colScalar (A only): the rows of A are the
-//                 receptive fields of an NHWC (or, scalar only, any-stride)
-//                 image, gathered on the fly -- A is never materialised.
+//     kLoadWindows / kLoadWindowsAny / kLoadIm2colScalar (A only): the rows of A
+//                 are the receptive fields of an NHWC (any-stride, for the last
+//                 one) image, gathered on the fly -- A is never materialised. See
+//                 ConvGeom for how k runs; kLoadFilter is the B that goes with
+//                 kLoadWindowsAny, the row-major filter with k counted the same way.
 // * Workgroup ids are re-ordered so that the ids that land on one XCD (the
 //   hardware deals consecutive ids round-robin over 8 XCDs, each with its own
 //   L2) cover one contiguous band of tiles.
@@ -54,7 +59,10 @@
 
 namespace tfhip {
 
-enum LoadKind { kLoadKVec = 0, kLoadXVec = 1, kLoadScalar = 2, kLoadIm2colVec = 3, kLoadIm2colScalar = 4 };
+enum LoadKind {
+  kLoadKVec = 0, kLoadXVec = 1, kLoadScalar = 2, kLoadWindows = 3, kLoadIm2colScalar = 4, kLoadWindowsAny = 5, kLoadFilter = 6,
+  kLoadKAny = 7
+};
 
 struct ConvGeom {
   // input addressing: x[n*xs_n + ih*xs_h + iw*xs_w + c*xs_c]
@@ -63,6 +71,16 @@ struct ConvGeom {
   int f_w;            // k = (r * f_w + s) * in_c + c
   int stride_h, stride_w, dil_h, dil_w, pad_top, pad_left;
   int out_h, out_w;
+  // kLoadWindows*: a filter row (columns not dilated), else a filter tap, is a segment: `seg_len` floats that lie side
+  // by side in the image as in the filter, so one comparison with the image row's ends covers all its columns
+  // and channels. k runs over the segments in units of four (the last of a segment may be partly empty: k counts
+  // 4 * units per segment). Finding a unit costs one multiplication by `unit_magic` = 2^32 / units rounded up
+  // (0: one unit per segment); with two divisions per fetch instead, the address arithmetic took as long as
+  // the matrix instructions (8 x 56 x 56 x 64, 3 x 3: 31 us).
+  int seg_len, units, unit_magic, taps;   // taps: segments per filter row
+  int row_len, image_len;                 // floats
+  int stride_wc, pad_leftc;               // in floats of an image row
+  int seg_row, seg_col;                   // floats from one filter row to the next, from one tap to the next
 };
 
 struct GemmParams {
@@ -155,13 +173,23 @@ __device__ __forceinline__ void init_loader(LoaderState<VECS> &st, long long sx,
       st.row_off[i] = kNoOffset;
       continue;
     }
-    if (KIND == kLoadKVec) {
+    if (KIND == kLoadKVec || KIND == kLoadKAny) {
       const int x = x0 + f / (BK / 4);
       st.row_off[i] = x < X ? (unsigned)((long long)x * sx * 4) : kNoOffset;
-    } else if (KIND == kLoadXVec) {
+    } else if (KIND == kLoadXVec || KIND == kLoadFilter) {
       const int x = x0 + (f / BK) * 4;   // consecutive lanes: consecutive k
       st.row_off[i] = x < X ? (unsigned)(x * 4) : kNoOffset;
-    } else if (KIND == kLoadIm2colVec || KIND == kLoadIm2colScalar) {
+    } else if (KIND == kLoadWindows || KIND == kLoadWindowsAny) {
+      const int m = x0 + f / (BK / 4);
+      const int ow = m % g.out_w;
+      const int t2 = m / g.out_w;
+      const int oh = t2 % g.out_h, n = t2 / g.out_h;
+      const int ih = oh * g.stride_h - g.pad_top;
+      st.row_ih[i] = m < X ? ih : -(1 << 28);   // (a row that no image has)
+      st.row_iw[i] = ow * g.stride_wc - g.pad_leftc;
+      // (a window that begins before the image: exact modulo 2^32)
+      st.row_off[i] = 4u * ((unsigned)n * (unsigned)g.image_len + (unsigned)(ih * g.row_len) + (unsigned)st.row_iw[i]);
+    } else if (KIND == kLoadIm2colScalar) {
       const int m = x0 + f / (BK / 4);
       if (m < X) {
         const int ow = m % g.out_w;
@@ -201,18 +229,56 @@ __device__ __forceinline__ void load_tile(float4 (&reg)[VECS], const LoaderState
           (k < K && st.row_off[i] != kNoOffset) ? st.row_off[i] + (unsigned)((long long)k * sk * 4) : kNoOffset;
       reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
     }
-  } else if (KIND == kLoadIm2colVec) {
-    // in_c % 4 == 0: the four k values of a fetch share one filter tap (r, s)
+  } else if (KIND == kLoadKAny) {
     const int k = k0 + (tid % (BK / 4)) * 4;
-    const int tap = k / g.in_c, c = k - tap * g.in_c;
-    const int r = tap / g.f_w, s = tap - r * g.f_w;
-    const int dh = r * g.dil_h, dw = s * g.dil_w;
-    const bool k_ok = k < K;
 #pragma unroll
     for (int i = 0; i < VECS; ++i) {
-      const int ih = st.row_ih[i] + dh, iw = st.row_iw[i] + dw;
-      const bool ok = k_ok && st.row_off[i] != kNoOffset && ih >= 0 && ih < g.in_h && iw >= 0 && iw < g.in_w;
-      const unsigned off = ok ? st.row_off[i] + (unsigned)((ih * g.xs_h + iw * g.xs_w + c) * 4) : kNoOffset;
+      const unsigned off = (k < K && st.row_off[i] != kNoOffset) ? st.row_off[i] + (unsigned)(k * 4) : kNoOffset;
+      float4 v = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
+      v.y = k + 1 < K ? v.y : 0.f;
+      v.z = k + 2 < K ? v.z : 0.f;
+      v.w = k + 3 < K ? v.w : 0.f;
+      reg[i] = v;
+    }
+  } else if (KIND == kLoadWindows || KIND == kLoadWindowsAny) {
+    const int k = k0 + (tid % (BK / 4)) * 4;
+    const int q = k >> 2;
+    const int seg = g.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)g.unit_magic) : q;
+    const int in_seg = 4 * (q - seg * g.units);
+    int fr = seg, fs = 0;
+    if (g.taps > 1) {
+      fr = seg / g.taps;
+      fs = seg - fr * g.taps;
+    }
+    const int dh = fr * g.dil_h, dl = fs * g.seg_col + in_seg;
+    const unsigned at = 4u * (unsigned)(fr * g.seg_row + dl);
+#pragma unroll
+    for (int i = 0; i < VECS; ++i) {
+      const bool row_in = k < K && (unsigned)(st.row_ih[i] + dh) < (unsigned)g.in_h;
+      const int lin = st.row_iw[i] + dl;
+      if (KIND == kLoadWindows) {   // in_c % 4 == 0: a unit lies inside the image row or outside
+        const unsigned off = row_in && (unsigned)lin < (unsigned)g.row_len ? st.row_off[i] + at : kNoOffset;
+        reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
+      } else {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool in = row_in && in_seg + j < g.seg_len && (unsigned)(lin + j) < (unsigned)g.row_len;
+          v[j] = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(in ? st.row_off[i] + at + 4u * j : kNoOffset), 0, 0));
+        }
+        reg[i] = make_float4(v[0], v[1], v[2], v[3]);
+      }
+    }
+  } else if (KIND == kLoadFilter) {
+    const int k = k0 + tid % BK;   // (256 % BK == 0: the same for every i)
+    const int q = k >> 2;
+    const int seg = g.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)g.unit_magic) : q;
+    const int in_seg = k - 4 * seg * g.units;
+    const unsigned at = (unsigned)(seg * g.seg_len + in_seg) * (unsigned)sk * 4u;
+#pragma unroll
+    for (int i = 0; i < VECS; ++i) {
+      const unsigned off = k < K && in_seg < g.seg_len && st.row_off[i] != kNoOffset ? st.row_off[i] + at : kNoOffset;
       reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
     }
   } else if (KIND == kLoadScalar) {
@@ -260,7 +326,7 @@ __device__ __forceinline__ void store_tile(float *__restrict__ lds, const float4
     if (i < first || i >= last) continue;
     const int f = tid + i * 256;
     if ((BX * BK / 4) % 256 != 0 && f >= BX * BK / 4) continue;
-    if (KIND == kLoadXVec) {
+    if (KIND == kLoadXVec || KIND == kLoadFilter) {
       // four consecutive x at one k: transposed, element by element
       const int k = f % BK, xq = f / BK;
       float *d = lds + (xq * 4) * PITCH + k;
@@ -636,6 +702,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
           const float4 out4 = make_float4(out[0], out[1], out[2], out[3]);
           if (through) store_result4_through(rsrc_c, (unsigned)((base + col) * 4), out4);
           else store_result4(C + base + col, out4);
+        } else if (through && !conv_addr && !R && col + 4 <= p.N) {   // (a buffer store needs 4-byte alignment only)
+          store_result4_through(rsrc_c, (unsigned)((base + col) * 4), make_float4(out[0], out[1], out[2], out[3]));
         } else {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
