@@ -1,4 +1,4 @@
-"""Products of few rows against the oracle, at the edges of the kernel that takes them: row blocks of 16, strips of 16 and
+"""Small products against the oracle, at the edges of the kernel that takes them: row blocks of 16 and 32, strips of 16 and
 64 columns, k groups of 16 and their slices, extents that no float4 fits, operands at odd addresses, and the
 two forms of adding the slices (a counter per strip; in a recording, a launch of its own)."""
 import ctypes
@@ -52,8 +52,9 @@ class _Product:
 
 @pytest.mark.parametrize("m,n,k,act,shift", [
     (1, 1, 1, "linear", 0), (16, 16, 16, "relu", 0), (17, 17, 17, "relu6", 1), (32, 1000, 1280, "linear", 0),
-    (33, 77, 513, "sigmoid", 0), (64, 65, 1030, "elu", 3), (64, 1024, 300, "leakyrelu", 0), (5, 4097, 2050, "relu", 0),
-    (23, 4100, 2049, "linear", 1), (64, 2051, 4099, "linear", 0), (1, 64, 4095, "elu", 0), (2, 40, 16 * 64 * 8 + 1, "linear", 2),
+    (33, 77, 513, "sigmoid", 0), (64, 65, 1030, "elu", 3), (64, 1024, 320, "leakyrelu", 0), (5, 4097, 2050, "relu", 0),
+    (23, 4100, 2049, "linear", 1), (100, 1009, 1535, "linear", 0), (1, 64, 4095, "elu", 0), (2, 40, 16 * 64 * 8 + 1, "linear", 2),
+    (196, 96, 576, "relu", 0), (49, 163, 961, "linear", 1), (1009, 33, 321, "relu6", 0), (81, 16, 5000, "sigmoid", 0),
 ])
 def test_against_the_oracle(lib, m, n, k, act, shift):
     from oracle import pyoracle as orc

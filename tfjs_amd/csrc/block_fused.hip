@@ -16,8 +16,8 @@
 //              reads of E each, into D in LDS, laid out as the A operand of the
 //              projection (pixel-major, channel-contiguous)
 //     phase P  projection on the matrix cores: D times the slice of the projection's
-//              weights from LDS, accumulated in registers over the slices (k ascending
-//              as in a plain GEMM over all mid channels)
+//              weights from LDS, accumulated in registers: k ascending inside a slice, then the
+//              slices' sums in order
 //   P of slice i and X of slice i + 1 run back to back between the same two barriers
 //   (two barriers per slice); the weights of the next slice travel from memory to
 //   registers one phase ahead and to LDS at the end of phase D.
@@ -27,10 +27,11 @@
 // k-contiguous rows, what a lane's 16-byte fragment read wants), prepared once per
 // model by tfhip_transpose2d: staging a slice is then a plain 16-byte copy.
 //
-// The instruction order of every stage is that of the separate kernels (gemm_kernel:
-// k = 16 t + 4 g + j for the j-th instruction of k group t, bias-initialised, residual
-// added last; the depthwise kernels: taps from zero by row then column, bias,
-// activation), so the block has the bits of the three (four) separate launches.
+// The instruction order of the expansion and the depthwise stage is that of the separate
+// kernels (gemm_kernel: k = 16 t + 4 g + j for the j-th instruction of k group t,
+// bias-initialised; the depthwise kernels: taps from zero by row then column, bias,
+// activation). The projection's sums are cut at the slices, as the kernels for small
+// products cut theirs: the two differ by rounding only.
 #include "block_fused.h"
 #include "common.h"
 #include "epilogue.h"
@@ -293,15 +294,17 @@ __global__ __launch_bounds__(kThreads) void inverted_residual_block(BlockArgs g)
       if (!u_on[u]) continue;
       const float *arow = tileD + (16 * u_pmb[u] + r) * PITCH + 4 * grp;
       const float *brow = w3s + (16 * u_nb[u] + r) * PITCH + 4 * grp;
+      float4_t sum = {0.f, 0.f, 0.f, 0.f};   // of the slice: shorter chains of sums round less
 #pragma unroll
       for (int t = 0; t < NCB; ++t) {
         const float4 a = *reinterpret_cast<const float4 *>(arow + 16 * t);
         const float4 b = *reinterpret_cast<const float4 *>(brow + 16 * t);
-        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, acc[u], 0, 0, 0);
-        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, acc[u], 0, 0, 0);
-        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, acc[u], 0, 0, 0);
-        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, acc[u], 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, sum, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, sum, 0, 0, 0);
       }
+      acc[u] += sum;
     }
     // ---- phase X: expansion of the next slice
     if (slice + 1 < g.slices) expand();

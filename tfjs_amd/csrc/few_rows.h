@@ -1,17 +1,17 @@
-// Products of few rows: C[M x N] = A[M x K] * B[K x N] with M up to 64, row-major, any extents and any 4-byte
-// alignment (a dense layer on a handful of examples, the layers of an encoder on a short sentence).
+// Small products: C[M x N] = A[M x K] * B[K x N], row-major, any extents and any 4-byte alignment (a dense layer on a
+// handful of examples, an encoder on a short sentence, the late layers of a mobile network on one picture).
 //
-// Such a product is bound by fetching B once, and at the sizes that occur (a few megabytes) by latency: the launch,
-// one trip to memory, the sum. So there is no LDS stage and no k loop to speak of. A workgroup of eight wavefronts
-// takes a strip of 16 CB columns, its wavefronts take k groups of 16 in turn, and each has the fetches of U groups
+// Such a product is bound by latency: the launch, one trip to memory, the sum; with very few rows and a large B, by
+// fetching B once. So there is no LDS stage and no k loop to speak of. A workgroup of eight wavefronts takes 16 MB
+// rows of a strip of 16 CB columns, its wavefronts take k groups of 16 in turn, and each has the fetches of U groups
 // out before it waits for the first.
 //  * lane (g, r) (g = lane / 16, r = lane % 16) feeds k = 16 T + 4 g + j in the j-th of the four matrix instructions
 //    (v_mfma_f32_16x16x4_f32) of group T: of A a float4 of row r, of B columns CB r .. CB r + CB - 1 of row k, 16
 //    lanes side by side. Buffer loads need 4-byte alignment only, and what lies beyond an operand reads as zero, dword
 //    by dword.
 //  * the wavefronts' sums meet in LDS and are added in order.
-//  * where the strips leave compute units idle, `splits` workgroups share one and cut its k: each leaves its sums in
-//    scratch, the last to arrive (a counter per strip) adds them in the order of k and finishes. One launch instead of
+//  * where the tiles leave compute units idle, `splits` workgroups share one and cut its k: each leaves its sums in
+//    scratch, the last to arrive (a counter per tile) adds them in the order of k and finishes. One launch instead of
 //    two, and the bits do not depend on who is last.
 #pragma once
 
@@ -31,6 +31,7 @@ struct FewRowsArgs {
   int M, N, K;
   unsigned a_bytes, b_bytes;
   int groups;               // of 16 k
+  int row_tiles;            // of 16 MB rows
   int splits, groups_per_split;
   int finish_apart;         // another launch adds the slices
   int activation;
@@ -46,15 +47,16 @@ constexpr long long kFewRowsMaxBytes = 0x40000000LL;
 constexpr int kThrough = 16;   // sc1
 
 // Sum over the slices (or, of one, over the wavefronts' sums in `lds`), bias, activation, residual and store of the
-// outputs of a strip; `bias` and `alpha` belong to the thread's column.
+// outputs of a tile; `bias` and `alpha` belong to the thread's column.
 template <int MB, int CB>
-__device__ __forceinline__ void finish_strip(const FewRowsArgs &p, int strip, float bias, float alpha, const float *lds) {
+__device__ __forceinline__ void finish_tile(const FewRowsArgs &p, int tile, float bias, float alpha, const float *lds) {
   constexpr int W = kFewRowsWaves, kCols = 16 * CB, kOut = 256 * MB * CB;
   static_assert((64 * W) % kCols == 0, "a thread keeps its column");
   const __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)uniform_pointer(p.ws + (long long)strip * p.splits * kOut), 0, p.splits * kOut * 4, 0x00020000);
+      (void *)uniform_pointer(p.ws + (long long)tile * p.splits * kOut), 0, p.splits * kOut * 4, 0x00020000);
+  const int strip = tile / p.row_tiles, m0 = (tile - strip * p.row_tiles) * 16 * MB;
   const int col = strip * kCols + (int)threadIdx.x % kCols;
-  const int live = min(kOut, p.M * kCols);   // elements of the strip that exist (its rows come first)
+  const int live = min(kOut, (p.M - m0) * kCols);   // elements of the tile that exist (its rows come first)
 #pragma unroll 1
   for (int i = threadIdx.x; i < live; i += 64 * W) {
     float v = 0.f;
@@ -75,7 +77,7 @@ __device__ __forceinline__ void finish_strip(const FewRowsArgs &p, int strip, fl
     }
     if (col >= p.N) continue;
     v = activate(v + bias, p.activation, alpha, p.leaky_alpha);
-    const long long at = (long long)(i / kCols) * p.N + col;
+    const long long at = (long long)(m0 + i / kCols) * p.N + col;
     p.c[at] = p.residual ? v + p.residual[at] : v;
   }
 }
@@ -93,7 +95,9 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
     const int per_xcd = gridDim.x / 8;
     if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   }
-  const int strip = id / p.splits, split = id - strip * p.splits;
+  // the slices of a tile side by side, then the row tiles of a strip
+  const int tile = id / p.splits, split = id - tile * p.splits;
+  const int strip = tile / p.row_tiles, m0 = (tile - strip * p.row_tiles) * kRows;
   const int n0 = strip * kCols;
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)p.a, 0, (int)p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)p.b, 0, (int)p.b_bytes, 0x00020000);
@@ -102,7 +106,7 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
 
   unsigned a_row[MB];
 #pragma unroll
-  for (int m = 0; m < MB; ++m) a_row[m] = 16 * m + r < p.M ? 4u * (unsigned)(16 * m + r) * (unsigned)p.K : kOutsideRow;
+  for (int m = 0; m < MB; ++m) a_row[m] = m0 + 16 * m + r < p.M ? 4u * (unsigned)(m0 + 16 * m + r) * (unsigned)p.K : kOutsideRow;
   const int col = n0 + CB * r;
   const unsigned b_col = col < p.N ? 4u * (unsigned)col : kOutsideRow;
   const unsigned pitch = 4u * (unsigned)p.N;
@@ -189,46 +193,52 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   // ---- k slices
   if (p.splits > 1) {
     const __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)uniform_pointer(p.ws + (long long)strip * p.splits * kOut), 0, p.splits * kOut * 4, 0x00020000);
+        (void *)uniform_pointer(p.ws + (long long)tile * p.splits * kOut), 0, p.splits * kOut * 4, 0x00020000);
 #pragma unroll 1
-    for (int i = tid; i < min(kOut, p.M * kCols); i += 64 * W)
+    for (int i = tid; i < min(kOut, (p.M - m0) * kCols); i += 64 * W)
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(wave_sum(i)), rsrc_ws, 4 * (split * kOut + i), 0, kThrough);
     if (p.finish_apart) return;
     __builtin_amdgcn_s_waitcnt(0);   // the stores are in memory
     __syncthreads();
     int *last = reinterpret_cast<int *>(lds);
     if (tid == 0) {
-      const int before = __hip_atomic_fetch_add(p.counters + strip, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (before == p.splits - 1) __hip_atomic_store(p.counters + strip, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int before = __hip_atomic_fetch_add(p.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (before == p.splits - 1) __hip_atomic_store(p.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       *last = before == p.splits - 1;
     }
     __syncthreads();
     if (!*last) return;
   }
-  finish_strip<MB, CB>(p, strip, bias, alpha, lds);
+  finish_tile<MB, CB>(p, tile, bias, alpha, lds);
 }
 
-// The sums of the slices of one strip each, where few_rows leaves them (FewRowsArgs::finish_apart).
+// The sums of the slices of one tile each, where few_rows leaves them (FewRowsArgs::finish_apart).
 template <int MB, int CB>
 __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows_finish(FewRowsArgs p) {
-  const int col = blockIdx.x * (16 * CB) + (int)threadIdx.x % (16 * CB);
+  const int col = (int)(blockIdx.x / p.row_tiles) * (16 * CB) + (int)threadIdx.x % (16 * CB);
   const float bias = p.bias && col < p.N ? p.bias[(long long)col * p.bias_stride] : 0.f;
   const float alpha = p.activation == TFHIP_PRELU && col < p.N ? p.prelu[(long long)col * p.prelu_stride] : 0.f;
-  finish_strip<MB, CB>(p, blockIdx.x, bias, alpha, nullptr);
+  finish_tile<MB, CB>(p, blockIdx.x, bias, alpha, nullptr);
 }
 
-// Whether this kernel takes the product of two row-major operands; `vec`: the tiled kernel could fetch both as float4.
-// Up to 32 rows it always wins over the tiled kernel (us, 1 x 1280 x 1000: 8.0 with its finishing launch, here 6.1;
-// 23 x 768 x 768: 8.0 and 6.1; 1 x 513 x 77, on its element loads: 10.7 and 4.8). With four row blocks the
-// matrix instructions take as long as the fetches and every strip reads all of A: it wins where no float4 fits
-// (64 x 4095 x 64: 26.0 and 8.8) or the columns are few (64 x 1280 x 1000: 11.1 and 8.8; but 64 x 768 x 3072: 8.1
-// and 10.0).
-inline bool few_rows_applies(const GemmParams &p, bool vec) {
-  return p.batch == 1 && p.M <= 64 && p.K > 0 && p.epi.channel_operands && p.epi.addressing != kConv &&
-         (p.M <= 32 || p.N <= 1024 || !vec) && (long long)p.M * p.K * 4 <= kFewRowsMaxBytes &&
-         (long long)p.K * p.N * 4 <= kFewRowsMaxBytes && tuning(kTuneTile) < 0 && tuning(kTuneSplitK) < 0;
+// Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
+// tiled kernel. Up to 32 rows always. Beyond, as long as every workgroup has a compute unit of its own: the fetches of
+// a whole k range are then out at once, where the tiled kernel goes round its pipeline once per 32 k (us, tiled and
+// here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7, 128 x 1024 x 1024 with two
+// row blocks 9.1 and 7.5). A short k has nothing to gain (784 x 192 x 32: 4.5 and 5.1), nor has a long one with two
+// row blocks, whose wavefronts fetch half as many groups at once (128 x 3072 x 768: 14.1 and 15.5).
+inline int few_rows_blocks(const GemmParams &p) {
+  if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
+      tuning(kTuneSplitK) >= 0 || (long long)p.M * p.K * 4 > kFewRowsMaxBytes || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
+    return 0;
+  const long long strips = (p.N + 15) / 16, cus = num_cus();
+  if (p.M <= 16) return 1;
+  if (p.M > 32 && p.K < 320) return 0;
+  if ((p.M + 15) / 16 * strips <= cus) return 1;
+  if (p.M <= 32 || ((p.M + 31) / 32 * strips <= cus && p.K <= 1536)) return 2;
+  return 0;
 }
 
-int launch_few_rows(const GemmParams &p);
+int launch_few_rows(const GemmParams &p, int row_blocks);
 
 }  // namespace tfhip

@@ -31,7 +31,10 @@ static int launch_ragged_gemm(GemmParams &p, bool transpose_b) {
 
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
-  if (!transpose_a && !transpose_b && few_rows_applies(p, vec)) return launch_few_rows(p);
+  if (!transpose_a && !transpose_b) {
+    const int row_blocks = few_rows_blocks(p);
+    if (row_blocks) return launch_few_rows(p, row_blocks);
+  }
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());
     if (!transpose_a && !transpose_b) return launch_gemm_shape<kLoadKVec, kLoadXVec>(shape, p);
@@ -47,19 +50,20 @@ namespace tfhip {
 namespace {
 
 constexpr int kFewRowsCounters = 256;
-static __device__ int few_rows_counters[kFewRowsCounters];   // one per strip that is cut, zero between launches
+static __device__ int few_rows_counters[kFewRowsCounters];   // one per tile that is cut, zero between launches
 
 template <int MB, int CB>
 int launch_few_rows_shape(FewRowsArgs &q) {
-  const int strips = (q.N + 16 * CB - 1) / (16 * CB);
-  // A wavefront wants about as many k groups as it fetches at once (64, 32 or 16 groups per workgroup); more
-  // workgroups than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
+  q.row_tiles = (q.M + 16 * MB - 1) / (16 * MB);
+  const long long tiles = (long long)((q.N + 16 * CB - 1) / (16 * CB)) * q.row_tiles;
+  // A wavefront wants about as many k groups as it fetches at once (64 or 32 groups per workgroup); more workgroups
+  // than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
   int splits = (q.groups + 64 / MB - 1) / (64 / MB);
-  if (splits > 256 / strips) splits = 256 / strips;
+  if (splits > kFewRowsCounters / tiles) splits = (int)(kFewRowsCounters / tiles);
   q.splits = 1;
   q.groups_per_split = q.groups;
   if (splits > 1) {
-    q.ws = static_cast<float *>(workspace((size_t)strips * splits * 256 * MB * CB * sizeof(float)));
+    q.ws = static_cast<float *>(workspace((size_t)tiles * splits * 256 * MB * CB * sizeof(float)));
     if (q.ws) {
       q.splits = splits;
       q.groups_per_split = (q.groups + splits - 1) / splits;
@@ -70,9 +74,9 @@ int launch_few_rows_shape(FewRowsArgs &q) {
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
   q.finish_apart = q.splits > 1 && capturing();
   note_kernel("few_rows<%d, %d>", MB, CB);
-  const dim3 grid((unsigned)(strips * q.splits)), block(64 * kFewRowsWaves);
+  const dim3 grid((unsigned)(tiles * q.splits)), block(64 * kFewRowsWaves);
   if (q.finish_apart) {
-    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)strips), block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)tiles), block, 0, stream()>>>(q)));
   } else {
     TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q)));
   }
@@ -81,7 +85,7 @@ int launch_few_rows_shape(FewRowsArgs &q) {
 
 }  // namespace
 
-int launch_few_rows(const GemmParams &p) {
+int launch_few_rows(const GemmParams &p, int row_blocks) {
   FewRowsArgs q = {};
   q.a = p.a; q.b = p.b; q.c = p.c;
   q.bias = p.epi.bias; q.bias_stride = p.epi.bias ? p.epi.bias_s[3] : 0;
@@ -99,9 +103,8 @@ int launch_few_rows(const GemmParams &p) {
   // Strips of 64 columns, whole cache lines, once B is tens of megabytes (1 x 4096 x 4096: 14.2 us, 15.5 with strips
   // of 16), else of 16: as many workgroups as there are.
   const bool wide = (long long)p.K * p.N >= (8LL << 20);
-  if (p.M <= 16) return wide ? launch_few_rows_shape<1, 4>(q) : launch_few_rows_shape<1, 1>(q);
-  if (p.M <= 32) return wide ? launch_few_rows_shape<2, 4>(q) : launch_few_rows_shape<2, 1>(q);
-  return wide ? launch_few_rows_shape<4, 2>(q) : launch_few_rows_shape<4, 1>(q);
+  if (row_blocks == 1) return wide ? launch_few_rows_shape<1, 4>(q) : launch_few_rows_shape<1, 1>(q);
+  return wide ? launch_few_rows_shape<2, 4>(q) : launch_few_rows_shape<2, 1>(q);
 }
 
 namespace {
