@@ -488,13 +488,13 @@ bool plan_expand_dw_stream(ExpandDwStreamArgs &g) {
   {
     const long long cus = num_cus();
     double best = 0;
-    for (int cand = g.out_h < 4 ? g.out_h : 4; cand <= g.out_h; ++cand) {
+    for (int cand = 1; cand <= g.out_h; ++cand) {
       const long long chunks = (g.out_h + cand - 1) / cand;
       const long long groups = ((long long)g.batch * chunks * g.strips * cgroups + 3) / 4;
       const long long per_cu = (groups + cus - 1) / cus;
       const double steps = cand + (g.stride == 1 ? 2.0 : 0.5) + 1.5;
       const double price = (double)per_cu * steps * (per_cu < 2 ? 1.25 : 1.0);
-      if (cand == (g.out_h < 4 ? g.out_h : 4) || price <= best) {
+      if (cand == 1 || price <= best) {
         best = price;
         rows = cand;
       }

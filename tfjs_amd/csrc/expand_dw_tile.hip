@@ -277,6 +277,7 @@ int launch_tile(const ExpandDwTileArgs &g, size_t lds_bytes) {
 template <int S, int KF, bool HALF>
 int launch_tile_ncb(const ExpandDwTileArgs &g, size_t lds_bytes) {
   switch (g.cs / 16) {
+    case 1: return launch_tile<S, KF, HALF, 1>(g, lds_bytes);
     case 2: return launch_tile<S, KF, HALF, 2>(g, lds_bytes);
     case 3: return launch_tile<S, KF, HALF, 3>(g, lds_bytes);
     default: return launch_tile<S, KF, HALF, 4>(g, lds_bytes);
@@ -315,7 +316,7 @@ bool plan_expand_dw_tile(ExpandDwTileArgs &g, size_t *lds_bytes) {
   if (g.out_h <= 0 || g.out_w <= 0) return false;
   const int forced_cs = tuning(kTuneTileSlice);
   int cs = 0;
-  if (forced_cs == 32 || forced_cs == 48 || forced_cs == 64) {
+  if (forced_cs == 16 || forced_cs == 32 || forced_cs == 48 || forced_cs == 64) {
     if (g.c % forced_cs != 0) return false;
     cs = forced_cs;
   } else if (g.out_h * g.stride <= 8 && g.c % 64 == 0) {
@@ -327,7 +328,7 @@ bool plan_expand_dw_tile(ExpandDwTileArgs &g, size_t *lds_bytes) {
   g.cs = cs;
   g.slices = g.c / cs;
   g.ecols = (g.out_w - 1) * g.stride + 3;
-  const size_t w_floats = (size_t)cs * (g.cin + 4);
+  size_t w_floats = (size_t)cs * (g.cin + 4);
   auto rows_for = [&](int chunks) { return (g.out_h + chunks - 1) / chunks; };
   auto bytes_for = [&](int rows) { return ((size_t)((rows - 1) * g.stride + 3) * g.ecols * (cs + 4) + w_floats) * sizeof(float); };
   const size_t lds_limit = 156 * 1024;
@@ -344,6 +345,40 @@ bool plan_expand_dw_tile(ExpandDwTileArgs &g, size_t *lds_bytes) {
     while ((long long)g.batch * g.slices * chunks < want && rows_for(chunks + 1) >= min_rows) ++chunks;
   }
   g.rows = rows_for(chunks);
+  // A launch that leaves compute units idle with this tiling (a few images) is bound by what one workgroup
+  // does from end to end: the tiling with the cheapest workgroup is then the better one, down to slices of 16
+  // channels and single rows. Priced in us, from sweeps of MobileNetV2's blocks at batches 1 to 16: a wave's
+  // matrix instructions (14 ns each), the staging of the weights (0.18 per 256 fetches), a quarter per
+  // round of depthwise items, and all of it once more for every further workgroup on the same unit. (At batch 1:
+  // 14x14, 64 -> 384 in 16 workgroups of 48 channels and seven rows 7.1 us, in 168 of 32 and one row 4.1;
+  // 7x7, 160 -> 960: 8.5 and 5.3.)
+  if (forced_cs < 0 && forced_chunks < 0 && (long long)g.batch * g.slices * chunks <= num_cus()) {
+    double best = 0;
+    const int base_cs = g.cs, base_rows = g.rows;
+    auto consider = [&](int slice, int rows) {
+      const int n_chunks = (g.out_h + rows - 1) / rows;
+      const long long groups = (long long)g.batch * n_chunks * (g.c / slice);
+      const int pixels = ((rows - 1) * g.stride + 3) * (g.ecols - 2);
+      const int blocks = (pixels + 15) / 16, quads = slice / 4;
+      const double each = (double)((blocks + 3) / 4) * (slice / 16) * (g.cin / 4.0) * 0.014 +
+                          (double)((quads * g.cin + 255) / 256) * 0.18 +
+                          (double)((rows * g.out_w + 256 / quads - 1) / (256 / quads)) * 0.25;
+      const double price = (double)((groups + num_cus() - 1) / num_cus()) * each;
+      if (best == 0 || price < best * 0.97) {
+        best = price;
+        g.cs = slice;
+        g.rows = rows;
+      }
+    };
+    consider(base_cs, base_rows);
+    for (int slice = 64; slice >= 16; slice -= 16) {
+      if (g.c % slice != 0) continue;
+      for (int rows = base_rows; rows >= 1; --rows) consider(slice, rows);
+    }
+    g.slices = g.c / g.cs;
+    cs = g.cs;
+    w_floats = (size_t)cs * (g.cin + 4);
+  }
   g.chunks_h = (g.out_h + g.rows - 1) / g.rows;
   g.erows = (g.rows - 1) * g.stride + 3;
   const long long image_bytes = (long long)g.out_h * g.out_w * g.c * 4;
