@@ -209,7 +209,7 @@ __device__ __forceinline__ void init_loader(LoaderState<VECS> &st, long long sx,
 
 // Issues this thread's share of the loads of the BX x BK tile at (x0, k0).
 template <int BX, int BK, int KIND, int VECS>
-__device__ __forceinline__ void load_tile(float4 (&reg)[VECS], const LoaderState<VECS> &st,
+__device__ __forceinline__ void load_tile(float4 (&reg)[VECS], int (&fix)[VECS], const LoaderState<VECS> &st,
                                           __amdgpu_buffer_rsrc_t rsrc, const float *__restrict__ base, long long sx,
                                           long long sk, int X, int K, int x0, int k0, int tid, const ConvGeom &g) {
   if (KIND == kLoadKVec) {
@@ -234,11 +234,8 @@ __device__ __forceinline__ void load_tile(float4 (&reg)[VECS], const LoaderState
 #pragma unroll
     for (int i = 0; i < VECS; ++i) {
       const unsigned off = (k < K && st.row_off[i] != kNoOffset) ? st.row_off[i] + (unsigned)(k * 4) : kNoOffset;
-      float4 v = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
-      v.y = k + 1 < K ? v.y : 0.f;
-      v.z = k + 2 < K ? v.z : 0.f;
-      v.w = k + 3 < K ? v.w : 0.f;
-      reg[i] = v;
+      reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
+      fix[i] = K - k;
     }
   } else if (KIND == kLoadWindows || KIND == kLoadWindowsAny) {
     const int k = k0 + (tid % (BK / 4)) * 4;
@@ -260,14 +257,13 @@ __device__ __forceinline__ void load_tile(float4 (&reg)[VECS], const LoaderState
         const unsigned off = row_in && (unsigned)lin < (unsigned)g.row_len ? st.row_off[i] + at : kNoOffset;
         reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
       } else {
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bool in = row_in && in_seg + j < g.seg_len && (unsigned)(lin + j) < (unsigned)g.row_len;
-          v[j] = __uint_as_float(
-              __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(in ? st.row_off[i] + at + 4u * j : kNoOffset), 0, 0));
-        }
-        reg[i] = make_float4(v[0], v[1], v[2], v[3]);
+        // a unit may begin before the image row, or end behind it or its segment: fetched from the row's first float
+        // on in the one case, what does not belong goes when the unit is stored
+        const int before = lin < 0 ? -lin : 0;
+        const unsigned off = row_in && before < 4 && lin < g.row_len ? st.row_off[i] + at + 4u * (unsigned)before : kNoOffset;
+        reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
+        const int real = min(g.row_len - lin, g.seg_len - in_seg);
+        fix[i] = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
       }
     }
   } else if (KIND == kLoadFilter) {
@@ -316,10 +312,24 @@ __device__ __forceinline__ void load_tile(float4 (&reg)[VECS], const LoaderState
   }
 }
 
+// What load_tile left to be done once the fetch has arrived (done there, it would wait for it at once): of four floats
+// the first fix & 0xffff count, the rest are zero; behind fix >> 16 zeros if the unit begins before the image row.
+template <int KIND>
+__device__ __forceinline__ float4 fix_up(float4 v, int fix) {
+  int real = fix;
+  if (KIND == kLoadWindowsAny) {
+    const int before = fix >> 16;
+    real = (int)(short)fix;
+    if (before & 1) v = make_float4(0.f, v.x, v.y, v.z);
+    if (before & 2) v = make_float4(0.f, 0.f, v.x, v.y);
+  }
+  return make_float4(real > 0 ? v.x : 0.f, real > 1 ? v.y : 0.f, real > 2 ? v.z : 0.f, real > 3 ? v.w : 0.f);
+}
+
 // Writes vectors [first, last) of the registers fetched by load_tile into an
 // x-major LDS tile [BX][PITCH].
 template <int BX, int BK, int PITCH, int KIND, int VECS>
-__device__ __forceinline__ void store_tile(float *__restrict__ lds, const float4 (&reg)[VECS], int tid,
+__device__ __forceinline__ void store_tile(float *__restrict__ lds, const float4 (&reg)[VECS], const int (&fix)[VECS], int tid,
                                            int first = 0, int last = VECS) {
 #pragma unroll
   for (int i = 0; i < VECS; ++i) {
@@ -337,7 +347,8 @@ __device__ __forceinline__ void store_tile(float *__restrict__ lds, const float4
     } else {
       // four consecutive k of one row
       const int row = f / (BK / 4), kq = f % (BK / 4);
-      *reinterpret_cast<float4 *>(lds + row * PITCH + kq * 4) = reg[i];
+      *reinterpret_cast<float4 *>(lds + row * PITCH + kq * 4) =
+          KIND == kLoadKAny || KIND == kLoadWindowsAny ? fix_up<KIND>(reg[i], fix[i]) : reg[i];
     }
   }
 }
@@ -455,6 +466,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
   //    every wave finished before it reached the barrier inside tile t-2.
   constexpr int D = T::PREFETCH;
   float4 ra[D][T::A_VECS], rb[D][T::B_VECS];
+  int fix_a[D][T::A_VECS], fix_b[D][T::B_VECS];
   const int k_tiles = KG > 1 ? group_k_tiles : (k_end - k_begin + BK - 1) / BK;
 
   // Every fetch is unconditional: a tile past K reads as zeros through the buffer
@@ -463,9 +475,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
   // conditional load makes it assume the shortest queue and wait for all).
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    load_tile<BM, BK, A_KIND, T::A_VECS>(ra[d], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0, k_begin + d * BK, tid,
+    load_tile<BM, BK, A_KIND, T::A_VECS>(ra[d], fix_a[d], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0, k_begin + d * BK, tid,
                                          p.conv);
-    load_tile<BN, BK, B_KIND, T::B_VECS>(rb[d], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0, k_begin + d * BK, tid,
+    load_tile<BN, BK, B_KIND, T::B_VECS>(rb[d], fix_b[d], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0, k_begin + d * BK, tid,
                                          p.conv);
   }
   // The accumulators start from the bias (lane l of a 16x16 block ends up with
@@ -490,11 +502,11 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
       for (int i = 0; i < T::TM; ++i) acc[i][j] = b4;
     }
   }
-  store_tile<BM, BK, T::PITCH, A_KIND, T::A_VECS>(lds_a, ra[0], tid);
-  store_tile<BN, BK, T::PITCH, B_KIND, T::B_VECS>(lds_b, rb[0], tid);
-  load_tile<BM, BK, A_KIND, T::A_VECS>(ra[0], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0, k_begin + D * BK, tid,
+  store_tile<BM, BK, T::PITCH, A_KIND, T::A_VECS>(lds_a, ra[0], fix_a[0], tid);
+  store_tile<BN, BK, T::PITCH, B_KIND, T::B_VECS>(lds_b, rb[0], fix_b[0], tid);
+  load_tile<BM, BK, A_KIND, T::A_VECS>(ra[0], fix_a[0], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0, k_begin + D * BK, tid,
                                        p.conv);
-  load_tile<BN, BK, B_KIND, T::B_VECS>(rb[0], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0, k_begin + D * BK, tid,
+  load_tile<BN, BK, B_KIND, T::B_VECS>(rb[0], fix_b[0], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0, k_begin + D * BK, tid,
                                        p.conv);
   lds_barrier();
 
@@ -562,15 +574,15 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
 #pragma unroll
         for (int piece = group * kPerGroup; piece < (group + 1) * kPerGroup && piece < kPieces; ++piece) {
           if (piece < T::A_VECS) {
-            store_tile<BM, BK, T::PITCH, A_KIND, T::A_VECS>(lds_a + nb * T::A_BUF, ra[slot], tid, piece, piece + 1);
+            store_tile<BM, BK, T::PITCH, A_KIND, T::A_VECS>(lds_a + nb * T::A_BUF, ra[slot], fix_a[slot], tid, piece, piece + 1);
           } else if (piece < kStores) {
-            store_tile<BN, BK, T::PITCH, B_KIND, T::B_VECS>(lds_b + nb * T::B_BUF, rb[slot], tid, piece - T::A_VECS,
+            store_tile<BN, BK, T::PITCH, B_KIND, T::B_VECS>(lds_b + nb * T::B_BUF, rb[slot], fix_b[slot], tid, piece - T::A_VECS,
                                                             piece - T::A_VECS + 1);
           } else if (piece == kStores) {
-            load_tile<BM, BK, A_KIND, T::A_VECS>(ra[slot], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0,
+            load_tile<BM, BK, A_KIND, T::A_VECS>(ra[slot], fix_a[slot], sa, rsrc_a, A, p.a_sx, p.a_sk, p.M, k_end, m0,
                                                  k_begin + (kt + 1 + D) * BK, tid, p.conv);
           } else {
-            load_tile<BN, BK, B_KIND, T::B_VECS>(rb[slot], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0,
+            load_tile<BN, BK, B_KIND, T::B_VECS>(rb[slot], fix_b[slot], sb, rsrc_b, B, p.b_sx, p.b_sk, p.N, k_end, n0,
                                                  k_begin + (kt + 1 + D) * BK, tid, p.conv);
           }
         }
