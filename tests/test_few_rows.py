@@ -104,3 +104,25 @@ def test_what_lies_behind_a_row_stays_out_of_it(lib):
         assert np.isnan(got[2]).all() and not np.isfinite(got[3]).any()
     finally:
         p.free()
+
+
+@pytest.mark.parametrize("xs,fs,stride,dil,pad,act", [
+    ((2, 9, 11, 64), (3, 3, 64, 17), 1, 1, "same", "relu6"),          # whole units
+    ((1, 20, 13, 45), (3, 3, 45, 33), 2, 1, "same", "leakyrelu"),      # units that straddle the image's edges and segments
+    ((3, 7, 6, 11), (7, 5, 11, 8), 1, 1, "same", "linear"),            # windows wider than the image allows
+    ((1, 12, 9, 203), (2, 2, 203, 30), 1, 2, "valid", "relu"),         # dilated: a segment per tap
+    ((2, 10, 10, 64), (3, 3, 64, 200), (1, 2), (2, 1), [[0, 0], [3, 1], [0, 2], [0, 0]], "sigmoid"),
+    ((1, 5, 5, 1023), (3, 3, 1023, 16), 1, 1, "same", "elu"),          # a k range cut into slices
+])
+def test_windows_of_an_image(lib, xs, fs, stride, dil, pad, act):
+    from oracle import pyoracle as orc
+    from tfjs_amd import pyhost as hip
+    rng = np.random.default_rng(sum(xs) + sum(fs))
+    x = rng.uniform(-1, 1, xs).astype(np.float32)
+    w = rng.normal(0, 0.2, fs).astype(np.float32)
+    kw = dict(strides=stride, dilations=dil, pad=pad, bias=rng.uniform(-1, 1, (fs[3],)).astype(np.float32), activation=act,
+              leakyrelu_alpha=0.1)
+    got = hip.fused_conv2d(x, w, **kw)
+    assert _last_kernel(lib).startswith("few_rows<")
+    want = orc.fused_conv2d(x, w, **kw)
+    assert np.max(np.abs(got - want) / np.maximum(1.0, np.abs(want))) <= 1e-4

@@ -8,6 +8,7 @@
 // A is gathered from the image inside the tile loader; nothing is unfolded in
 // memory. A 1x1 filter with stride 1 and no padding is an ordinary GEMM on the
 // image itself and takes the plain loaders.
+#include "few_rows.h"
 #include "gemm_host.h"
 
 using namespace tfhip;
@@ -438,6 +439,8 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
     if (units * g.units < (int64_t(1) << 32) && in_h * in_w * in_c < lim && dilation_h * in_w * in_c < lim &&
         (f_h - 1) * dilation_h * in_w * in_c + f_w * dilation_w * in_c < lim && stride_w * out_w * in_c < lim && pad_left * in_c < lim) {
       p.K = (int)(4 * units);
+      const int row_blocks = few_rows_blocks(p, true);
+      if (row_blocks) return launch_few_rows(p, row_blocks, vec ? kLoadWindows : kLoadWindowsAny);
       const int shape = choose_tile_shape(M, out_c, p.K, 1, num_cus());
       if (vec) return launch_gemm_shape<kLoadWindows, kLoadXVec>(shape, p);
       return launch_gemm_shape<kLoadWindowsAny, kLoadFilter>(shape, p);

@@ -9,6 +9,8 @@
 //    (v_mfma_f32_16x16x4_f32) of group T: of A a float4 of row r, of B columns CB r .. CB r + CB - 1 of row k, 16
 //    lanes side by side. Buffer loads need 4-byte alignment only, and what lies beyond an operand reads as zero, dword
 //    by dword.
+//  * A can be the windows of an NHWC image (KIND kLoadWindows, kLoadWindowsAny: a float4 is a unit of four k of a
+//    segment, see ConvGeom): the small convolutions of a network's later stages.
 //  * the wavefronts' sums meet in LDS and are added in order.
 //  * where the tiles leave compute units idle, `splits` workgroups share one and cut its k: each leaves its sums in
 //    scratch, the last to arrive (a counter per tile) adds them in the order of k and finishes. One launch instead of
@@ -34,6 +36,7 @@ struct FewRowsArgs {
   int row_tiles;            // of 16 MB rows
   int splits, groups_per_split;
   int finish_apart;         // another launch adds the slices
+  ConvGeom conv;            // A gathered from an image (k counted as there)
   int activation;
 };
 
@@ -82,8 +85,9 @@ __device__ __forceinline__ void finish_tile(const FewRowsArgs &p, int tile, floa
   }
 }
 
-template <int MB, int CB>
+template <int MB, int CB, int KIND>
 __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
+  constexpr bool kWindows = KIND != kLoadKAny;
   constexpr int W = kFewRowsWaves;
   constexpr int U = MB + CB <= 2 ? 8 : (MB + CB <= 4 ? 4 : 2);
   constexpr int kCols = 16 * CB, kRows = 16 * MB, kOut = kCols * kRows;
@@ -105,8 +109,22 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   const int end = min(p.groups, (split + 1) * p.groups_per_split);
 
   unsigned a_row[MB];
+  int row_ih[MB], row_lin[MB];   // windows: image row and position in it of the first element
 #pragma unroll
-  for (int m = 0; m < MB; ++m) a_row[m] = m0 + 16 * m + r < p.M ? 4u * (unsigned)(m0 + 16 * m + r) * (unsigned)p.K : kOutsideRow;
+  for (int m = 0; m < MB; ++m) {
+    const int row = m0 + 16 * m + r;
+    if (kWindows) {
+      const ConvGeom &c = p.conv;
+      const int ow = row % c.out_w, t2 = row / c.out_w;
+      const int oh = t2 % c.out_h, n = t2 / c.out_h;
+      const int ih = oh * c.stride_h - c.pad_top;
+      row_ih[m] = row < p.M ? ih : -(1 << 28);   // (a row that no image has)
+      row_lin[m] = ow * c.stride_wc - c.pad_leftc;
+      a_row[m] = 4u * ((unsigned)n * (unsigned)c.image_len + (unsigned)(ih * c.row_len) + (unsigned)row_lin[m]);
+    } else {
+      a_row[m] = row < p.M ? 4u * (unsigned)row * (unsigned)p.K : kOutsideRow;
+    }
+  }
   const int col = n0 + CB * r;
   const unsigned b_col = col < p.N ? 4u * (unsigned)col : kOutsideRow;
   const unsigned pitch = 4u * (unsigned)p.N;
@@ -114,26 +132,51 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   struct Chunk {
     uint4_t a[U][MB];
     unsigned b[U][4][CB];
+    int fix[U][MB];   // windows: what fix_up is to do
   };
   auto issue = [&](Chunk &c, int first) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = first + u * W, k = 16 * t + 4 * g;
-      const unsigned ka = t < end && k < p.K ? 4u * (unsigned)k : kOutside;
+      const bool on = t < end && k < p.K;
+      int row = k, live_rows = 4;   // of B, and how many of the four there are
+      if (kWindows) {
+        const ConvGeom &cg = p.conv;
+        const int q = k >> 2;
+        const int seg = cg.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)cg.unit_magic) : q;
+        const int in_seg = 4 * (q - seg * cg.units);
+        int fr = seg, fs = 0;
+        if (cg.taps > 1) {
+          fr = seg / cg.taps;
+          fs = seg - fr * cg.taps;
+        }
+        const int dh = fr * cg.dil_h, dl = fs * cg.seg_col + in_seg;
+        const unsigned at = 4u * (unsigned)(fr * cg.seg_row + dl);
+        row = seg * cg.seg_len + in_seg;
+        live_rows = cg.seg_len - in_seg;
 #pragma unroll
-      for (int m = 0; m < MB; ++m) c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(a_row[m] + ka), 0, 0);
-      const unsigned kb = t < end ? (unsigned)k * pitch + b_col : kOutside;
+        for (int m = 0; m < MB; ++m) {
+          const bool row_in = on && (unsigned)(row_ih[m] + dh) < (unsigned)cg.in_h;
+          const int lin = row_lin[m] + dl;
+          const int before = KIND == kLoadWindowsAny && lin < 0 ? -lin : 0;
+          const bool in = row_in && (KIND == kLoadWindowsAny ? before < 4 && lin < cg.row_len : (unsigned)lin < (unsigned)cg.row_len);
+          c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(in ? a_row[m] + at + 4u * (unsigned)before : kNoOffset), 0, 0);
+          const int real = min(cg.row_len - lin, live_rows);
+          c.fix[u][m] = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
+        }
+      } else {
+        const unsigned ka = on ? 4u * (unsigned)k : kOutside;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {   // (rows beyond K lie beyond the descriptor)
-        const int at = (int)(kb + (unsigned)j * pitch);
+        for (int m = 0; m < MB; ++m) c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(a_row[m] + ka), 0, 0);
+      }
+      const unsigned kb = on ? (unsigned)row * pitch + b_col : kOutside;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {   // (rows beyond the last lie beyond the descriptor)
+        const int at = (int)(KIND == kLoadWindowsAny && j >= live_rows ? kOutside : kb + (unsigned)j * pitch);
         if constexpr (CB == 4) {
           const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, at, 0, 0);
 #pragma unroll
           for (int q = 0; q < 4; ++q) c.b[u][j][q % CB] = v[q];
-        } else if constexpr (CB == 2) {
-          const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc_b, at, 0, 0);
-          c.b[u][j][0] = v[0];
-          c.b[u][j][CB - 1] = v[1];
         } else {
           c.b[u][j][0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, at, 0, 0);
         }
@@ -148,17 +191,22 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   auto multiply = [&](const Chunk &c, int first) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      if (first + u * W >= end) break;   // (the same for the whole wavefront)
       const int k = 16 * (first + u * W) + 4 * g;
+      float a4[MB][4];
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        // (the last float4 of a row may reach into the next one)
+        const float4 v = fix_up<KIND>(as_float4(c.a[u][m]), kWindows ? c.fix[u][m] : p.K - k);
+        a4[m][0] = v.x; a4[m][1] = v.y; a4[m][2] = v.z; a4[m][3] = v.w;
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-          // (the last float4 of a row may reach into the next one)
-          const float av = k + j < p.K ? __uint_as_float(c.a[u][m][j]) : 0.f;
+        for (int m = 0; m < MB; ++m)
 #pragma unroll
           for (int q = 0; q < CB; ++q)
-            acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, __uint_as_float(c.b[u][j][q]), acc[m][q], 0, 0, 0);
-        }
+            acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[m][j], __uint_as_float(c.b[u][j][q]), acc[m][q], 0, 0, 0);
     }
   };
 
@@ -225,20 +273,24 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows_finish(FewRowsArg
 // tiled kernel. Up to 32 rows always. Beyond, as long as every workgroup has a compute unit of its own: the fetches of
 // a whole k range are then out at once, where the tiled kernel goes round its pipeline once per 32 k (us, tiled and
 // here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7, 128 x 1024 x 1024 with two
-// row blocks 9.1 and 7.5). A short k has nothing to gain (784 x 192 x 32: 4.5 and 5.1), nor has a long one with two
-// row blocks, whose wavefronts fetch half as many groups at once (128 x 3072 x 768: 14.1 and 15.5).
-inline int few_rows_blocks(const GemmParams &p) {
+// row blocks 9.1 and 7.5; windows, [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1, [1,20,20,64] 3x3 -> 16 7.9 and 5.9). A
+// short k has nothing to gain (784 x 192 x 32: 4.5 and 5.1; windows of 240 floats 5.2 and 6.1), nor has a
+// long one with two row blocks, whose wavefronts fetch half as many groups at once (128 x 3072 x 768: 14.1 and 15.5).
+inline int few_rows_blocks(const GemmParams &p, bool windows) {
+  if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
   if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
-      tuning(kTuneSplitK) >= 0 || (long long)p.M * p.K * 4 > kFewRowsMaxBytes || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
+      tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
     return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();
   if (p.M <= 16) return 1;
-  if (p.M > 32 && p.K < 320) return 0;
+  if (p.M > 32 && p.K < 320 && !windows) return 0;
+  if (p.M <= 32 && p.K > 2048) return 2;   // half the fetches of B, and slices enough to fill the chip
   if ((p.M + 15) / 16 * strips <= cus) return 1;
   if (p.M <= 32 || ((p.M + 31) / 32 * strips <= cus && p.K <= 1536)) return 2;
   return 0;
 }
 
-int launch_few_rows(const GemmParams &p, int row_blocks);
+// `kind`: kLoadKAny (row-major A), kLoadWindows or kLoadWindowsAny.
+int launch_few_rows(const GemmParams &p, int row_blocks, int kind);
 
 }  // namespace tfhip

@@ -32,8 +32,8 @@ static int launch_ragged_gemm(GemmParams &p, bool transpose_b) {
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
   if (!transpose_a && !transpose_b) {
-    const int row_blocks = few_rows_blocks(p);
-    if (row_blocks) return launch_few_rows(p, row_blocks);
+    const int row_blocks = few_rows_blocks(p, false);
+    if (row_blocks) return launch_few_rows(p, row_blocks, kLoadKAny);
   }
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());
@@ -52,7 +52,7 @@ namespace {
 constexpr int kFewRowsCounters = 256;
 static __device__ int few_rows_counters[kFewRowsCounters];   // one per tile that is cut, zero between launches
 
-template <int MB, int CB>
+template <int MB, int CB, int KIND>
 int launch_few_rows_shape(FewRowsArgs &q) {
   q.row_tiles = (q.M + 16 * MB - 1) / (16 * MB);
   const long long tiles = (long long)((q.N + 16 * CB - 1) / (16 * CB)) * q.row_tiles;
@@ -73,19 +73,19 @@ int launch_few_rows_shape(FewRowsArgs &q) {
   // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
   q.finish_apart = q.splits > 1 && capturing();
-  note_kernel("few_rows<%d, %d>", MB, CB);
+  note_kernel("few_rows<%d, %d, %d>", MB, CB, KIND);
   const dim3 grid((unsigned)(tiles * q.splits)), block(64 * kFewRowsWaves);
   if (q.finish_apart) {
-    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)tiles), block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)tiles), block, 0, stream()>>>(q)));
   } else {
-    TFHIP_LAUNCH((few_rows<MB, CB><<<grid, block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q)));
   }
   return kOk;
 }
 
 }  // namespace
 
-int launch_few_rows(const GemmParams &p, int row_blocks) {
+int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   FewRowsArgs q = {};
   q.a = p.a; q.b = p.b; q.c = p.c;
   q.bias = p.epi.bias; q.bias_stride = p.epi.bias ? p.epi.bias_s[3] : 0;
@@ -94,8 +94,9 @@ int launch_few_rows(const GemmParams &p, int row_blocks) {
   q.leaky_alpha = p.epi.leaky_alpha;
   q.activation = p.epi.activation;
   q.M = p.M; q.N = p.N; q.K = p.K;
-  q.a_bytes = (unsigned)((long long)p.M * p.K * 4);
-  q.b_bytes = (unsigned)((long long)p.K * p.N * 4);
+  q.conv = p.conv;
+  q.a_bytes = kind == kLoadKAny ? (unsigned)((long long)p.M * p.K * 4) : p.a_bytes;
+  q.b_bytes = kind == kLoadKAny ? (unsigned)((long long)p.K * p.N * 4) : p.b_bytes;
   q.groups = (p.K + 15) / 16;
   static int *counters = nullptr;
   if (!counters) TFHIP_CHECK_HIP(hipGetSymbolAddress(reinterpret_cast<void **>(&counters), HIP_SYMBOL(few_rows_counters)));
@@ -103,8 +104,10 @@ int launch_few_rows(const GemmParams &p, int row_blocks) {
   // Strips of 64 columns, whole cache lines, once B is tens of megabytes (1 x 4096 x 4096: 14.2 us, 15.5 with strips
   // of 16), else of 16: as many workgroups as there are.
   const bool wide = (long long)p.K * p.N >= (8LL << 20);
-  if (row_blocks == 1) return wide ? launch_few_rows_shape<1, 4>(q) : launch_few_rows_shape<1, 1>(q);
-  return wide ? launch_few_rows_shape<2, 4>(q) : launch_few_rows_shape<2, 1>(q);
+  if (kind == kLoadWindows) return row_blocks == 1 ? launch_few_rows_shape<1, 1, kLoadWindows>(q) : launch_few_rows_shape<2, 1, kLoadWindows>(q);
+  if (kind == kLoadWindowsAny) return row_blocks == 1 ? launch_few_rows_shape<1, 1, kLoadWindowsAny>(q) : launch_few_rows_shape<2, 1, kLoadWindowsAny>(q);
+  if (row_blocks == 1) return wide ? launch_few_rows_shape<1, 4, kLoadKAny>(q) : launch_few_rows_shape<1, 1, kLoadKAny>(q);
+  return wide ? launch_few_rows_shape<2, 4, kLoadKAny>(q) : launch_few_rows_shape<2, 1, kLoadKAny>(q);
 }
 
 namespace {

@@ -55,10 +55,11 @@ inline int choose_tile_shape(long long M, long long N, long long K, long long ba
   // One 64 x 48 tile on (nearly) every compute unit and a long k: that tile with two groups of
   // wavefronts sharing it (choose_k_groups) beats the 32 x 32 tile the estimate below prefers
   // (1024 x 768 x 3072: 43.9 against 47.0 us back to back, 45.4 against 55.2 us with operands from
-  // memory; 1024 x 768 x 768: 15.5 against 15.7, 16.9 against 18.1).
+  // memory; 1024 x 768 x 768: 15.5 against 15.7, 16.9 against 18.1). With a quarter of the units idle it loses
+  // (208 x 2304 x 768, 192 tiles: 16.3 against 12.0; 728 x 768 x 3072: 50.8 against 42.0 on 128 x 96).
   {
     const long long tiles = ((M + 63) / 64) * ((N + 47) / 48) * batch;
-    if (tiles <= cus && tiles * 4 >= 3LL * cus && K >= 768) return 10;
+    if (tiles <= cus && tiles * 8 >= 7LL * cus && K >= 768) return 10;
   }
   int best = 0;
   double best_us = 0;
