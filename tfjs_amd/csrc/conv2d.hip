@@ -411,8 +411,11 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
     p.a_sx = in_c; p.a_sk = 1;
     return launch_plain_gemm(p, false, false, vec);
   }
+  // (With more taps than the matrix-core form holds, the lane-per-pixel form is for a workgroup of pixels at most: a
+  // lane then walks K taps on its own, where the implicit GEMM gathers whole filter rows: 2 x 60 x 60 x 3, 7x7 -> 8:
+  // 26.1 and 6.8 us, 8 x 112 x 112 x 3, 7x7/2 -> 64: 39.2 and 15.1.)
   if (!nchw && in_c <= 4 && out_c % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
-      p.epi.channel_operands && activation <= TFHIP_RELU6) {
+      p.epi.channel_operands && activation <= TFHIP_RELU6 && (K <= kMaxTaps || M <= 256)) {
     const bool few_taps = K <= kMaxTaps && M < lim - 256 && p.a_bytes != 0;
     // 32 channels per wavefront when there are pixels enough to fill the chip that
     // way, else 16 (twice the wavefronts)

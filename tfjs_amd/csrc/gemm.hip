@@ -6,29 +6,6 @@
 
 using namespace tfhip;
 
-// Rows no float4 fits, on the tiles that small and middling products take (a large one is rarely ragged): the
-// loaders that need 4-byte alignment only.
-static int launch_ragged_gemm(GemmParams &p, bool transpose_b) {
-  static const int shapes[] = {9, 11, 12};
-  int best = shapes[0];
-  double best_us = 0;
-  for (const int s : shapes) {
-    const double us = estimate_us(kTileShapes[s], p.M, p.N, p.K, p.batch, num_cus());
-    if (s == shapes[0] || us < best_us) {
-      best_us = us;
-      best = s;
-    }
-  }
-  if (transpose_b) {
-    if (best == 9) return launch_gemm<64, 64, 32, 2, 2, kLoadKAny, kLoadKAny>(p);
-    if (best == 11) return launch_gemm<32, 64, 32, 2, 2, kLoadKAny, kLoadKAny>(p);
-    return launch_gemm<32, 32, 32, 2, 2, kLoadKAny, kLoadKAny>(p);
-  }
-  if (best == 9) return launch_gemm<64, 64, 32, 2, 2, kLoadKAny, kLoadXVec>(p);
-  if (best == 11) return launch_gemm<32, 64, 32, 2, 2, kLoadKAny, kLoadXVec>(p);
-  return launch_gemm<32, 32, 32, 2, 2, kLoadKAny, kLoadXVec>(p);
-}
-
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
   if (!transpose_a && !transpose_b) {

@@ -225,6 +225,9 @@ inline int launch_gemm_shape(int shape, GemmParams &p) {
 // with float4 loads.
 int launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec);
 
+// The same for a row-major A (and a B of either kind) that cannot (gemm_ragged.hip).
+int launch_ragged_gemm(GemmParams &p, bool transpose_b);
+
 // Fills the bias / prelu part of an Epilogue from caller strides over `rank`
 // output dims (3: batch,row,col; 4: n,h,w,c) after validating them. Sets
 // kChannel addressing when every operand varies along the last axis only.
