@@ -126,3 +126,16 @@ def test_windows_of_an_image(lib, xs, fs, stride, dil, pad, act):
     assert _last_kernel(lib).startswith("few_rows<")
     want = orc.fused_conv2d(x, w, **kw)
     assert np.max(np.abs(got - want) / np.maximum(1.0, np.abs(want))) <= 1e-4
+
+
+def test_a_cut_product_after_shutdown_and_init(lib):
+    from tfjs_amd import pyhost
+    bits = []
+    for _ in range(2):
+        p = _Product(lib, 1, 64, 4095, "linear")
+        p.launch()
+        bits.append(p.result().view(np.uint32))
+        p.free()
+        pyhost.shutdown()
+        pyhost.init(0)
+    np.testing.assert_array_equal(bits[0], bits[1])

@@ -48,7 +48,7 @@ int stage_upload(char *d, const char *h, size_t bytes);
 // Records the number of K slices a GEMM launch was cut into (tfhip_workspace_info reports the last).
 void note_splits(int splits);
 size_t fixed_workspace_bytes();
-// Resolves the device address of gemm.hip's static scratch array for `device`
+// Resolves the addresses of gemm.hip's static device arrays (scratch, counters) on `device`
 // (which must be current). Called by tfhip_init.
 int setup_static_scratch(int device);
 

@@ -26,8 +26,28 @@ int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, 
 namespace tfhip {
 namespace {
 
+// Device memory that belongs to the library for as long as the process lasts. Every GPU the library runs on holds a
+// copy of each array, at an address of its own; in host code the names are only stand-ins for the symbols. The
+// addresses are resolved once per device by setup_static_scratch (with that device current), and a launch takes those of
+// the device that tfhip_init was last given.
 constexpr int kFewRowsCounters = 256;
 static __device__ int few_rows_counters[kFewRowsCounters];   // one per tile that is cut, zero between launches
+// The split-K partial sums of tfhip_fused_matmul_noalloc, which tfhip_fused_matmul keeps in the library's growing workspace.
+static __device__ __align__(256) float scratch[TFHIP_NOALLOC_SCRATCH_BYTES / sizeof(float)];
+
+constexpr int kMaxDevices = 64;
+struct DeviceArrays {
+  float *scratch;
+  int *few_rows_counters;
+};
+DeviceArrays g_device_arrays[kMaxDevices] = {};
+
+int resolve(const void *symbol, const char *name, int device, void **ptr) {
+  const hipError_t e = hipGetSymbolAddress(ptr, symbol);
+  if (e == hipSuccess && *ptr != nullptr) return kOk;
+  (void)hipGetLastError();
+  return fail(kHipError, "tfhip_init: hipGetSymbolAddress(%s) on device %d failed: %s", name, device, hipGetErrorString(e));
+}
 
 template <int MB, int CB, int KIND>
 int launch_few_rows_shape(FewRowsArgs &q) {
@@ -75,9 +95,7 @@ int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   q.a_bytes = kind == kLoadKAny ? (unsigned)((long long)p.M * p.K * 4) : p.a_bytes;
   q.b_bytes = kind == kLoadKAny ? (unsigned)((long long)p.K * p.N * 4) : p.b_bytes;
   q.groups = (p.K + 15) / 16;
-  static int *counters = nullptr;
-  if (!counters) TFHIP_CHECK_HIP(hipGetSymbolAddress(reinterpret_cast<void **>(&counters), HIP_SYMBOL(few_rows_counters)));
-  q.counters = counters;
+  q.counters = g_device_arrays[device_index()].few_rows_counters;
   // Strips of 64 columns, whole cache lines, once B is tens of megabytes (1 x 4096 x 4096: 14.2 us, 15.5 with strips
   // of 16), else of 16: as many workgroups as there are.
   const bool wide = (long long)p.K * p.N >= (8LL << 20);
@@ -87,35 +105,16 @@ int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   return wide ? launch_few_rows_shape<2, 4, kLoadKAny>(q) : launch_few_rows_shape<2, 1, kLoadKAny>(q);
 }
 
-namespace {
-
-// Scratch of tfhip_fused_matmul_noalloc: the split-K partial sums that
-// tfhip_fused_matmul keeps in the library's growing workspace. Every GPU the
-// library runs on holds its own copy of the array, at its own address, until
-// the process ends; in host code the name below is only a stand-in for the
-// symbol, and the per-device address is resolved once by setup_static_scratch
-// (with that device current) and used from then on.
-static __device__ __align__(256) float scratch[TFHIP_NOALLOC_SCRATCH_BYTES / sizeof(float)];
-
-constexpr int kMaxDevices = 64;
-float *g_scratch_ptr[kMaxDevices] = {};
-
-}  // namespace
-
 int setup_static_scratch(int device) {
   if (device < 0 || device >= kMaxDevices)
-    return fail(kBadArgument, "tfhip_init: device %d is beyond the %d devices the static scratch table covers", device,
+    return fail(kBadArgument, "tfhip_init: device %d is beyond the %d devices the table of device arrays covers", device,
                 kMaxDevices);
-  if (g_scratch_ptr[device] != nullptr) return kOk;
-  void *ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-  if (e != hipSuccess || ptr == nullptr) {
-    (void)hipGetLastError();
-    return fail(kHipError, "tfhip_init: hipGetSymbolAddress(scratch) on device %d failed: %s", device,
-                hipGetErrorString(e));
-  }
-  g_scratch_ptr[device] = static_cast<float *>(ptr);
-  return kOk;
+  DeviceArrays &d = g_device_arrays[device];
+  int rc = kOk;
+  if (d.scratch == nullptr) rc = resolve(HIP_SYMBOL(scratch), "scratch", device, reinterpret_cast<void **>(&d.scratch));
+  if (rc == kOk && d.few_rows_counters == nullptr)
+    rc = resolve(HIP_SYMBOL(few_rows_counters), "few_rows_counters", device, reinterpret_cast<void **>(&d.few_rows_counters));
+  return rc;
 }
 
 }  // namespace tfhip
@@ -140,7 +139,7 @@ extern "C" int tfhip_fused_matmul_noalloc(const float *a, const float *b, float 
                                           int activation, const float *prelu_weights,
                                           const int64_t prelu_strides[3], double leakyrelu_alpha) {
   TFHIP_REQUIRE_INIT();
-  float *ptr = g_scratch_ptr[device_index()];
+  float *ptr = g_device_arrays[device_index()].scratch;
   if (ptr == nullptr)
     return fail(kHipError, "tfhip_fused_matmul_noalloc: the static scratch array was not resolved on device %d",
                 device_index());
