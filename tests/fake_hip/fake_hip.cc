@@ -69,6 +69,7 @@ bool inside_locked(const void *p, size_t bytes, Block *b = nullptr) {
 
 void *take(size_t bytes, int device) {
   void *p = aligned_alloc(256, (bytes + 255) & ~size_t(255));
+  memset(p, 0, bytes);
   std::lock_guard<std::recursive_mutex> lock(m);
   blocks[(uintptr_t)p] = {bytes, device};
   return p;

@@ -21,3 +21,59 @@ for device in (0, 1, 0):
     check(lib.tfhip_shutdown())
 assert errors()[0] == 0, errors()
 """)
+
+
+MODEL = """
+import tempfile
+from tfjs_amd import workloads
+folder = tempfile.mkdtemp()
+workloads.write_model(folder, workloads.mobilenet_v2_weights(seed=1), np.uint8)
+model = workloads.DeviceMobileNetV2(folder, 1)
+model.set_input(np.zeros((1, 224, 224, 3), np.float32))
+filters = [op["w2"] for op, _ in model.plan if op["kind"] == "pwdw"]
+
+def write(name, value):
+    buf, shape = model.weights[name]
+    buf.upload(np.full(shape, value, np.float32))
+
+def predict():
+    '''Whether the call was a replay; it leaves no block behind that it did not find.'''
+    live, logits = pyhost.memory_info()["live"], model._logits is not None
+    model.predict()
+    assert pyhost.memory_info()["live"] == live + (model._logits is not None) - logits
+    return model._graph is not None
+
+def refused(message):
+    live, logits = pyhost.memory_info()["live"], model._logits is not None
+    try:
+        model.predict()
+    except capi.HipBackendError as e:
+        assert message in str(e), e
+        assert pyhost.memory_info()["live"] == live - logits
+        return True
+    return False
+"""
+
+
+def test_predict_launches_where_a_recording_is_refused():
+    """A filter written between two calls has to be searched for Inf / NaN again, which a recording cannot do:
+    the call launches, a later one records."""
+    fake_hip_util.run(MODEL + """
+assert not predict()
+write(filters[0], 0.5)
+assert not predict()
+assert predict() and predict()
+live = pyhost.memory_info()["live"]
+model.close()
+assert pyhost.memory_info()["live"] == 0
+model = workloads.DeviceMobileNetV2(folder, 1)
+write(filters[3], np.nan)
+assert refused("Inf or NaN") and refused("Inf or NaN")
+write(filters[3], 1.0)
+assert not predict()
+write(filters[3], np.inf)
+assert refused("Inf or NaN")        # (the recording first, then the launches)
+write(filters[3], 0.25)
+assert not predict() and predict()
+assert errors()[0] == 0, errors()
+""")

@@ -15,6 +15,7 @@ import os
 import numpy as np
 
 from . import quantization
+from .capi import HipBackendError
 
 # (expansion t, output channels c, repeats n, first stride s)
 MOBILENET_V2_BLOCKS = [(1, 16, 1, 1), (6, 24, 2, 2), (6, 32, 3, 2), (6, 64, 4, 2), (6, 96, 3, 1), (6, 160, 3, 2),
@@ -467,12 +468,21 @@ class DeviceMobileNetV2:
     def forward(self, before=None, after=None):
         """Enqueues one inference; returns the DeviceBuffer holding the logits.
         before(i, op) / after(i, op) are called around the launch of op i."""
-        lib, check, DeviceBuffer = self._lib, self._check, self._DeviceBuffer
         t = {"input": self.input}
+        try:
+            return self._enqueue(t, before, after)
+        except BaseException:   # a refused call: the activations go back
+            del t["input"]
+            for buf in t.values():
+                buf.free()
+            raise
+
+    def _enqueue(self, t, before, after):
+        lib, check, DeviceBuffer = self._lib, self._check, self._DeviceBuffer
         for i, (op, geom) in enumerate(self.plan):
             k = op["kind"]
             n_out = self.size[op["out"]]
-            out = DeviceBuffer(n_out * 4)
+            out = t[op["out"]] = DeviceBuffer(n_out * 4)
             if before:
                 before(i, op)
             if k == "conv" and "residual" in op:
@@ -513,7 +523,6 @@ class DeviceMobileNetV2:
                                              self._i64([0, 0, 1]), 0, None, self._i64([0, 0, 0]), 0.2))
             if after:
                 after(i, op)
-            t[op["out"]] = out
             for s in (op["src"] if isinstance(op["src"], tuple) else (op["src"],)):
                 if self.last_use.get(s) == i and s != "input":
                     t.pop(s).free()
@@ -532,21 +541,32 @@ class DeviceMobileNetV2:
         if self._graph is not None:
             self._check(self._lib.tfhip_graph_launch(self._graph))
             return self._logits.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
-        self._ran = True
         out = self.forward()
-        logits = out.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
-        out.free()
-        return logits
+        self._ran = True
+        try:
+            return out.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
+        finally:
+            out.free()
 
     def _record(self):
+        """Records the launches of an inference. Where one of them is refused while a recording is open (a filter
+        that has been written since the last call must be searched for Inf / NaN, which needs a wait), nothing is
+        recorded: this call launches, and the next one tries again."""
         graph, nodes = ctypes.c_int(), ctypes.c_int()
-        self._check(self._lib.tfhip_capture_begin())
+        if self._lib.tfhip_capture_begin() != 0:
+            return
         try:
             logits = self.forward()
-        except Exception:
+        except BaseException as e:
             self._lib.tfhip_capture_end(None, ctypes.byref(nodes))
+            if isinstance(e, HipBackendError):
+                return
             raise
-        self._check(self._lib.tfhip_capture_end(ctypes.byref(graph), ctypes.byref(nodes)))
+        try:
+            self._check(self._lib.tfhip_capture_end(ctypes.byref(graph), ctypes.byref(nodes)))
+        except HipBackendError:
+            logits.free()
+            return
         self._graph, self._logits = graph.value, logits
 
     def close(self):
