@@ -115,7 +115,10 @@ int tfhip_event_elapsed(int start_slot, int end_slot, float *ms);
  *    result from where the recorded result was. Blocks that were live at
  *    tfhip_capture_end and that a recorded kernel names must still be live at
  *    every tfhip_graph_launch, which checks this and fails without launching
- *    otherwise.
+ *    otherwise. So it does where a filter that was finite when a kernel was
+ *    recorded that multiplies padding by it has been given an Inf or a NaN
+ *    through this library (record again, or run the calls: they take or refuse
+ *    such a filter as they always do).
  *  - tfhip_capture_end(NULL, &nodes) discards the recording.
  * nodes: kernels in the graph. */
 int tfhip_capture_begin(void);

@@ -77,3 +77,29 @@ write(filters[3], 0.25)
 assert not predict() and predict()
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_a_replay_rests_on_what_its_filters_hold():
+    """A kernel that multiplies padding by its filter is not replayed once that holds an Inf or a NaN, and is again
+    when it is finite; predict() gives such a recording up and does what its launches do."""
+    fake_hip_util.run(MODEL + """
+assert not predict() and predict() and predict()
+before = fake.fake_hip_launches()
+write(filters[0], 0.5)              # finite: searched once, then replayed as before
+assert predict()
+searched = fake.fake_hip_launches()
+assert predict()
+assert fake.fake_hip_launches() - searched == searched - before - 2
+graph = model._graph
+check(lib.tfhip_graph_launch(graph))
+write(filters[5], np.inf)
+for _ in range(2):
+    assert lib.tfhip_graph_launch(graph) != 0 and b"Inf or NaN" in lib.tfhip_last_error()
+write(filters[5], 2.0)
+check(lib.tfhip_graph_launch(graph))
+write(filters[5], np.nan)
+assert refused("tfhip_fused_pointwise_depthwise") and refused("tfhip_fused_pointwise_depthwise")
+write(filters[5], 2.0)
+assert not predict() and predict()
+assert errors()[0] == 0, errors()
+""")

@@ -1,0 +1,70 @@
+"""DeviceMobileNetV2.predict replays a recording: every answer is the one that its launches give, whatever was written
+between two calls."""
+import numpy as np
+import pytest
+
+from tfjs_amd import pyhost, workloads
+from tfjs_amd.capi import HipBackendError
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def model(tmp_path):
+    pyhost.init()
+    workloads.write_model(str(tmp_path), workloads.mobilenet_v2_weights(seed=3), np.uint8)
+    m = workloads.DeviceMobileNetV2(str(tmp_path), 2)
+    m.set_input(workloads.mobilenet_v2_input(2))
+    yield m
+    m.close()
+
+
+def _launched(model):
+    out = model.forward()
+    logits = out.download(np.float32, 2000).reshape(2, 1000)
+    out.free()
+    return logits
+
+
+def _replayed(model):
+    """The logits of a replay: the bits of the launches (slices of k are added in the same order)."""
+    got = model.predict()
+    assert model._graph is not None
+    np.testing.assert_array_equal(got.view(np.uint32), _launched(model).view(np.uint32))
+    return got
+
+
+def test_replays_see_new_pictures_and_new_weights(model):
+    model.predict()
+    first = _replayed(model)
+    rng = np.random.default_rng(0)
+    for _ in range(3):
+        model.set_input(rng.uniform(-1, 1, (2, 224, 224, 3)))
+        assert not np.array_equal(_replayed(model), first)
+    # a filter that is searched for Inf / NaN, one that is not, a bias
+    pair = next(op for op, _ in model.plan if op["kind"] == "pwdw")
+    for name in (pair["w2"], pair["w"], pair["b2"]):
+        before = _replayed(model)
+        buf, shape = model.weights[name]
+        old = buf.download(np.float32, int(np.prod(shape)))
+        buf.upload(old * np.float32(0.5) + np.float32(0.01))
+        assert not np.array_equal(_replayed(model), before)
+        buf.upload(old)
+        np.testing.assert_array_equal(_replayed(model), before)
+
+
+def test_an_infinite_filter_is_not_replayed(model):
+    model.predict()
+    want = _replayed(model)
+    buf, shape = model.weights[next(op["w2"] for op, _ in model.plan if op["kind"] == "pwdw")]
+    old = buf.download(np.float32, int(np.prod(shape)))
+    for bad in (np.inf, np.nan):
+        broken = old.copy()
+        broken[7] = bad
+        buf.upload(broken)
+        for call in (model.predict, model.forward, model.predict):
+            with pytest.raises(HipBackendError, match="Inf or NaN"):
+                call()
+        buf.upload(old)
+        assert np.array_equal(model.predict(), want) and model._graph is None
+        np.testing.assert_array_equal(_replayed(model), want)

@@ -23,6 +23,14 @@ namespace {
 constexpr size_t kSlotBytes = size_t(4) << 20;
 constexpr int kSlots = 16;
 
+// What a search of a filter for Inf / NaN found.
+struct FilterScan {
+  uintptr_t ptr;
+  size_t elems;
+  uint64_t generation;
+  bool nonfinite;
+};
+
 struct RecordedGraph {
   hipGraphExec_t exec = nullptr;
   size_t nodes = 0;
@@ -34,6 +42,8 @@ struct RecordedGraph {
   };
   std::vector<Ref> refs;   // blocks a recorded kernel names and that were live when the recording ended
   std::vector<uintptr_t> writes;   // of those, the blocks a recorded call writes: a replay changes their contents
+  std::vector<FilterScan> scans;   // filters found finite, on which the choice of a recorded kernel rests
+  uint64_t scans_forgotten = 0;    // Runtime::scans_forgotten when they were last found to hold
 };
 
 struct Runtime {
@@ -71,16 +81,12 @@ struct Runtime {
   std::map<int, RecordedGraph> graphs;
   int next_graph = 1;
   std::vector<void *> retired_workspaces;  // outgrown while a graph might still name them
+  std::vector<FilterScan> capture_scans;   // filters that scan_filter called finite while recording
   // Filters that were searched for Inf / NaN: block base -> scans of ranges inside that block.
   // An entry holds the generation of the block it was made for, and leaves when the block is
   // written through this library (uploads, kernel results) or freed.
-  struct FilterScan {
-    uintptr_t ptr;
-    size_t elems;
-    uint64_t generation;
-    bool nonfinite;
-  };
   std::unordered_map<uintptr_t, std::vector<FilterScan>> filter_scans;
+  uint64_t scans_forgotten = 0;   // how many times entries have left
   int *scan_flag = nullptr;   // pinned host word the scan kernel's verdict is copied to
   int *scan_flag_dev = nullptr;
 };
@@ -106,6 +112,11 @@ size_t class_size(size_t bytes) {
 void give_back_locked(void *p, size_t cls) {
   g.free_lists[cls].push_back(p);
   g.pooled_bytes += cls;
+}
+
+// What was remembered about the filters of the block at `base` no longer holds.
+void forget_scans_locked(uintptr_t base) {
+  if (g.filter_scans.erase(base) > 0) ++g.scans_forgotten;
 }
 
 void release_pool_locked() {
@@ -244,7 +255,7 @@ void forget_filter_scans(const void *p) {
   if (it == g.live.begin()) return;
   --it;
   if (a >= it->first + it->second) return;
-  g.filter_scans.erase(it->first);
+  forget_scans_locked(it->first);
   // a replay writes the block again, with whatever its inputs hold then
   if (g.capturing) g.capture_writes.insert(it->first);
 }
@@ -266,9 +277,10 @@ int scan_filter(const float *w, int64_t elems, const char *who, bool *nonfinite)
     generation = g.generation[base];
     auto found = g.filter_scans.find(base);
     if (found != g.filter_scans.end()) {
-      for (const Runtime::FilterScan &f : found->second) {
+      for (const FilterScan &f : found->second) {
         if (f.ptr == a && f.elems == (size_t)elems && f.generation == generation) {
           *nonfinite = f.nonfinite;
+          if (g.capturing && !f.nonfinite) g.capture_scans.push_back(f);   // a replay rests on this answer
           return kOk;
         }
       }
@@ -564,6 +576,7 @@ int tfhip_shutdown(void) {
   g.capture_free.clear();
   g.capture_refs.clear();
   g.capture_writes.clear();
+  g.capture_scans.clear();
   for (void *p : g.retired_workspaces) (void)hipFree(p);
   g.retired_workspaces.clear();
   for (auto &kv : g.live) {
@@ -634,7 +647,7 @@ int tfhip_free(void *dptr) {
   g.live.erase(it);
   g.owned.erase(a);
   g.generation.erase(a);
-  g.filter_scans.erase(a);
+  forget_scans_locked(a);
   g.live_bytes -= cls;
   if (g.capturing) {
     g.capture_free[cls].push_back(dptr);   // the graph being recorded names it: the graph keeps it
@@ -665,7 +678,7 @@ int tfhip_unregister_external(void *dptr) {
   g.live.erase(it);
   g.owned.erase(a);
   g.generation.erase(a);
-  g.filter_scans.erase(a);
+  forget_scans_locked(a);
   return kOk;
 }
 
@@ -784,6 +797,7 @@ int tfhip_capture_begin(void) {
   g.capturing = true;
   g.capture_refs.clear();
   g.capture_writes.clear();
+  g.capture_scans.clear();
   return kOk;
 }
 
@@ -809,6 +823,7 @@ int tfhip_capture_end(int *graph_id, int *nodes) {
     g.capture_free.clear();
     g.capture_refs.clear();
     g.capture_writes.clear();
+    g.capture_scans.clear();
     if (e != hipSuccess) return fail(kHipError, "tfhip_capture_end: %s", hipGetErrorString(e));
     if (nodes) *nodes = (int)rec.nodes;
     return kOk;
@@ -827,8 +842,11 @@ int tfhip_capture_end(int *graph_id, int *nodes) {
       if (g.capture_writes.count(base)) rec.writes.push_back(base);
     }
   }
+  rec.scans = std::move(g.capture_scans);
+  rec.scans_forgotten = g.scans_forgotten;
   g.capture_refs.clear();
   g.capture_writes.clear();
+  g.capture_scans.clear();
   const int id = g.next_graph++;
   if (nodes) *nodes = (int)rec.nodes;
   g.graphs[id] = std::move(rec);
@@ -838,25 +856,46 @@ int tfhip_capture_end(int *graph_id, int *nodes) {
 
 int tfhip_graph_launch(int graph_id) {
   TFHIP_REQUIRE_INIT();
-  std::lock_guard<std::mutex> lock(g_mutex);
-  TFHIP_CHECK_ARG(!g.capturing, "tfhip_graph_launch: a recording is open");
-  auto it = g.graphs.find(graph_id);
-  TFHIP_CHECK_ARG(it != g.graphs.end(), "tfhip_graph_launch: no graph %d", graph_id);
-  for (auto &r : it->second.refs) {
-    // the same address, size AND hand-out: a block that was freed and handed out again
-    // at the same address belongs to someone else now
-    auto b = g.live.find(r.base);
-    auto gen = g.generation.find(r.base);
-    if (b == g.live.end() || b->second != r.size || gen == g.generation.end() || gen->second != r.generation) {
-      return fail(kOutOfRange,
-                  "tfhip_graph_launch: graph %d names the device buffer at %p (%zu bytes), which has been freed since it was recorded",
-                  graph_id, reinterpret_cast<void *>(r.base), r.size);
+  std::vector<FilterScan> scans;   // to be compared before the replay
+  uint64_t forgotten = 0;
+  for (;;) {
+    std::unique_lock<std::mutex> lock(g_mutex);
+    TFHIP_CHECK_ARG(!g.capturing, "tfhip_graph_launch: a recording is open");
+    auto it = g.graphs.find(graph_id);
+    TFHIP_CHECK_ARG(it != g.graphs.end(), "tfhip_graph_launch: no graph %d", graph_id);
+    RecordedGraph &rec = it->second;
+    for (auto &r : rec.refs) {
+      // the same address, size AND hand-out: a block that was freed and handed out again
+      // at the same address belongs to someone else now
+      auto b = g.live.find(r.base);
+      auto gen = g.generation.find(r.base);
+      if (b == g.live.end() || b->second != r.size || gen == g.generation.end() || gen->second != r.generation) {
+        return fail(kOutOfRange,
+                    "tfhip_graph_launch: graph %d names the device buffer at %p (%zu bytes), which has been freed since it was recorded",
+                    graph_id, reinterpret_cast<void *>(r.base), r.size);
+      }
+    }
+    if (!scans.empty()) rec.scans_forgotten = forgotten;   // (compared in the round before)
+    if (rec.scans.empty() || rec.scans_forgotten == g.scans_forgotten) {
+      // what the library remembered about the old contents of the blocks this replay writes
+      for (uintptr_t base : rec.writes) forget_scans_locked(base);
+      for (int r = g_repeat; r > 0; --r) TFHIP_CHECK_HIP(hipGraphLaunch(rec.exec, g.stream));
+      return kOk;
+    }
+    // Some filter, perhaps one of these, has been written since: a kernel that multiplies padding by its filter must not
+    // be replayed with an Inf or a NaN in it. What was not written is remembered, what was costs a search.
+    scans = rec.scans;
+    forgotten = g.scans_forgotten;
+    lock.unlock();
+    for (const FilterScan &f : scans) {
+      bool nonfinite = false;
+      const int rc = scan_filter(reinterpret_cast<const float *>(f.ptr), (int64_t)f.elems, "tfhip_graph_launch", &nonfinite);
+      if (rc != kOk) return rc;
+      if (nonfinite)
+        return fail(kBadArgument, "tfhip_graph_launch: the filter at %p was finite when graph %d was recorded and holds Inf or NaN now",
+                    reinterpret_cast<void *>(f.ptr), graph_id);
     }
   }
-  // what the library remembered about the old contents of the blocks this replay writes
-  for (uintptr_t base : it->second.writes) g.filter_scans.erase(base);
-  for (int r = g_repeat; r > 0; --r) TFHIP_CHECK_HIP(hipGraphLaunch(it->second.exec, g.stream));
-  return kOk;
 }
 
 int tfhip_graph_destroy(int graph_id) {

@@ -539,8 +539,10 @@ class DeviceMobileNetV2:
         if self._graph is None and self._ran and self.batch <= self._REPLAY_BATCH:
             self._record()
         if self._graph is not None:
-            self._check(self._lib.tfhip_graph_launch(self._graph))
-            return self._logits.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
+            if self._lib.tfhip_graph_launch(self._graph) == 0:
+                return self._logits.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
+            # a buffer that it names is gone, or a filter holds an Inf or a NaN: the entry points decide anew
+            self._forget_recording()
         out = self.forward()
         self._ran = True
         try:
@@ -569,11 +571,16 @@ class DeviceMobileNetV2:
             return
         self._graph, self._logits = graph.value, logits
 
-    def close(self):
+    def _forget_recording(self):
+        """The next predict() launches, the one behind it records again."""
+        self._ran = False
         if self._graph is not None:
             self._check(self._lib.tfhip_graph_destroy(self._graph))
             self._logits.free()
             self._graph = self._logits = None
+
+    def close(self):
+        self._forget_recording()
         self.input.free()
         for buf in self.transposed.values():
             buf.free()
