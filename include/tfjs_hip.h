@@ -153,10 +153,14 @@ int tfhip_graph_destroy(int graph_id);
  *   shape / never), "stream_rows" (its output rows per wavefront), "stream_blocks" (1 / 2
  *   blocks of 16 channels per wavefront), "skinny_stage" (0: the streaming GEMM never
  *   stages A in LDS). The environment variable of a knob is its name in capitals behind
- *   TFHIP_ (TFHIP_TILE, TFHIP_SPLITK, ... TFHIP_SKINNY_STAGE), read at tfhip_init(). */
+ *   TFHIP_ (TFHIP_TILE, TFHIP_SPLITK, ... TFHIP_SKINNY_STAGE), read at tfhip_init().
+ * tfhip_tuning_changes(&n): how many times a knob has been given another value. A
+ *   recording keeps the kernels that the knobs chose when it was made; a program that
+ *   sets knobs compares n to know that it is to record again. */
 int tfhip_set_launch_repeat(int n);
 int tfhip_last_kernel(char *name, size_t name_len);
 int tfhip_set_tuning(const char *name, int value);
+int tfhip_tuning_changes(int *changes);
 int tfhip_copy(void *dst, const void *src, size_t bytes);
 
 /* ---- _FusedMatMul / BatchMatMul ------------------------------------------

@@ -103,3 +103,29 @@ write(filters[5], 2.0)
 assert not predict() and predict()
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_predict_sees_exchanged_buffers_and_knobs():
+    fake_hip_util.run(MODEL + """
+def kernels():
+    '''what the last predict() launched or replayed'''
+    return [launch(i)[0] for i in range(30)]
+
+name = filters[0]
+own, shape = model.weights[name]
+other, other_input = DeviceBuffer(int(np.prod(shape)) * 4), DeviceBuffer(224 * 224 * 3 * 4)
+assert not predict() and predict() and predict()
+tiled = kernels()
+for change, undo in [(lambda: model.weights.update({name: (other, shape)}), lambda: model.weights.update({name: (own, shape)})),
+                     (lambda: setattr(model, "input", other_input), lambda: setattr(model, "input", model_input)),
+                     (lambda: check(lib.tfhip_set_tuning(b"tile", 3)), lambda: check(lib.tfhip_set_tuning(b"tile", -1)))]:
+    model_input = model.input
+    for step in (change, undo):
+        step()
+        assert not predict() and predict() and predict()
+        assert (kernels() == tiled) == (step is undo or "tuning" not in str(change.__code__.co_names))
+check(lib.tfhip_set_tuning(b"tile", -1))     # no other value: nothing to do again
+assert predict()
+other.free()
+assert errors()[0] == 0, errors()
+""")

@@ -68,3 +68,32 @@ def test_an_infinite_filter_is_not_replayed(model):
         buf.upload(old)
         assert np.array_equal(model.predict(), want) and model._graph is None
         np.testing.assert_array_equal(_replayed(model), want)
+
+
+def test_exchanged_buffers_and_knobs_are_not_ignored(model):
+    from tfjs_amd.capi import DeviceBuffer, check, load_library
+    model.predict()
+    want = _replayed(model)
+
+    def changed(change, undo):
+        change()
+        got = model.predict()
+        np.testing.assert_array_equal(got.view(np.uint32), _launched(model).view(np.uint32))
+        np.testing.assert_array_equal(_replayed(model).view(np.uint32), got.view(np.uint32))
+        undo()
+        np.testing.assert_array_equal(model.predict(), want)
+        np.testing.assert_array_equal(_replayed(model), want)
+        return got
+
+    pair = next(op for op, _ in model.plan if op["kind"] == "pwdw")
+    own, shape = model.weights[pair["w"]]
+    with DeviceBuffer.from_numpy(np.full(shape, 0.125, np.float32)) as other:
+        got = changed(lambda: model.weights.update({pair["w"]: (other, shape)}),
+                      lambda: model.weights.update({pair["w"]: (own, shape)}))
+        assert not np.array_equal(got, want)
+    own = model.input
+    with DeviceBuffer.from_numpy(np.full((2, 224, 224, 3), 0.5, np.float32)) as other:
+        got = changed(lambda: setattr(model, "input", other), lambda: setattr(model, "input", own))
+        assert not np.array_equal(got, want)
+    knob = load_library().tfhip_set_tuning
+    changed(lambda: check(knob(b"tile", 3)), lambda: check(knob(b"tile", -1)))

@@ -155,6 +155,7 @@ struct TuningTable {
   }
 };
 TuningTable g_tuning;
+int g_tuning_changes = 0;   // (a recording keeps the kernels that the knobs chose then)
 int tuning(int key) { return g_tuning.value[key]; }
 
 void read_tuning_from_environment() {
@@ -737,11 +738,19 @@ int tfhip_download(void *host, const void *src, size_t src_offset, size_t bytes)
 int tfhip_set_tuning(const char *name, int value) {
   for (int i = 0; name && i < kTuneCount; ++i) {
     if (strcmp(name, kTuningNames[i]) == 0) {
-      g_tuning.value[i] = value < 0 ? -1 : value;
+      if (value < 0) value = -1;
+      if (g_tuning.value[i] != value) ++g_tuning_changes;
+      g_tuning.value[i] = value;
       return kOk;
     }
   }
   return fail(kBadArgument, "tfhip_set_tuning: unknown knob '%s'", name ? name : "(null)");
+}
+
+int tfhip_tuning_changes(int *changes) {
+  TFHIP_CHECK_ARG(changes != nullptr, "tfhip_tuning_changes: changes is NULL");
+  *changes = g_tuning_changes;
+  return kOk;
 }
 
 int tfhip_set_launch_repeat(int n) {

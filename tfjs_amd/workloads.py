@@ -313,7 +313,7 @@ class DeviceMobileNetV2:
         self.shape, self.last_use = shape, last_use
         self.size = {name: math.prod(dims) for name, dims in shape.items()}
         # predict() runs the plan launch by launch the first time, records it the second and replays it from then on
-        self._graph = self._logits = None
+        self._graph = self._logits = self._recorded = None
         self._ran = False
         self.strides_c = i64_array([0, 0, 0, 1])
         self.zero4 = i64_array([0, 0, 0, 0])
@@ -530,18 +530,19 @@ class DeviceMobileNetV2:
 
     def predict(self):
         """forward + download of the logits, the reference's definition of one
-        timed inference (e2e/benchmarks/benchmark_util.js:246-286). The shapes, weights and
-        buffers of a model do not change, so from its second call on the launches are replayed as
-        one recorded sequence: enqueueing them one by one from Python takes 300 us, more than
+        timed inference (e2e/benchmarks/benchmark_util.js:246-286). The launches of a model are the
+        same at every call (unless a buffer is exchanged or a knob set, which is looked at), so from
+        its second call on they are replayed as one recorded sequence: enqueueing them one by one from Python takes 300 us, more than
         the GPU needs for a few pictures. Larger batches keep the host ahead anyway, and a recording
         holds activation buffers of its own: with three models in turn, batch 8 takes 304 us
         replayed and 313 launched, batch 16 392 and 368."""
         if self._graph is None and self._ran and self.batch <= self._REPLAY_BATCH:
             self._record()
         if self._graph is not None:
-            if self._lib.tfhip_graph_launch(self._graph) == 0:
+            # (the operands are compared while the GPU works)
+            if self._lib.tfhip_graph_launch(self._graph) == 0 and self._operands() == self._recorded:
                 return self._logits.download(np.float32, self.batch * 1000).reshape(self.batch, 1000)
-            # a buffer that it names is gone, or a filter holds an Inf or a NaN: the entry points decide anew
+            # other operands or knobs, a buffer that is gone, an Inf or a NaN in a filter: the entry points decide anew
             self._forget_recording()
         out = self.forward()
         self._ran = True
@@ -550,11 +551,19 @@ class DeviceMobileNetV2:
         finally:
             out.free()
 
+    def _operands(self):
+        """What the launches of an inference take from outside: a recording holds them as they were."""
+        changes = ctypes.c_int()
+        self._check(self._lib.tfhip_tuning_changes(ctypes.byref(changes)))
+        return ([self.input.ptr, changes.value] + [buf.ptr for buf, _ in self.weights.values()] +
+                [buf.ptr for buf in self.transposed.values()])
+
     def _record(self):
         """Records the launches of an inference. Where one of them is refused while a recording is open (a filter
         that has been written since the last call must be searched for Inf / NaN, which needs a wait), nothing is
         recorded: this call launches, and the next one tries again."""
         graph, nodes = ctypes.c_int(), ctypes.c_int()
+        self._recorded = self._operands()
         if self._lib.tfhip_capture_begin() != 0:
             return
         try:
