@@ -119,6 +119,9 @@ int tfhip_event_elapsed(int start_slot, int end_slot, float *ms);
  *    recorded that multiplies padding by it has been given an Inf or a NaN
  *    through this library (record again, or run the calls: they take or refuse
  *    such a filter as they always do).
+ *  - A recording takes the launches of the thread that opened it; what other
+ *    threads launch, copy or replay meanwhile runs as usual. There is one
+ *    recording at a time.
  *  - tfhip_capture_end(NULL, &nodes) discards the recording.
  * nodes: kernels in the graph. */
 int tfhip_capture_begin(void);

@@ -129,3 +129,61 @@ assert predict()
 other.free()
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_a_recording_takes_the_launches_of_its_own_thread_only():
+    """While one thread records, another's launches run, its copies work, and what it frees is kept only where the
+    recording names it."""
+    fake_hip_util.run("""
+from concurrent.futures import ThreadPoolExecutor
+pyhost.init()
+other = ThreadPoolExecutor(1)
+ones = np.ones(64, np.float32)
+
+def multiply(out):
+    check(lib.tfhip_fused_matmul(a.ptr, a.ptr, out.ptr, 1, 1, 8, 8, 8, 0, 0, None, None, 0, None, None, 0.2))
+
+def elsewhere():
+    mine = DeviceBuffer.from_numpy(ones)
+    multiply(mine)
+    where = launch()
+    mine.upload(ones)
+    assert mine.download(np.float32, 64).tolist() == ones.tolist()
+    finite = ctypes.c_int()
+    check(lib.tfhip_filter_is_finite(mine.ptr, 64, ctypes.byref(finite)))      # needs a wait for the stream
+    check(lib.tfhip_graph_launch(first.value))
+    mine.free()
+    named.free()
+    assert lib.tfhip_capture_begin() != 0 and b"already open" in lib.tfhip_last_error()
+    return where
+
+def record(body):
+    graph, nodes = ctypes.c_int(), ctypes.c_int()
+    check(lib.tfhip_capture_begin())
+    body()
+    check(lib.tfhip_capture_end(ctypes.byref(graph), ctypes.byref(nodes)))
+    return graph, nodes.value
+
+a, out, named = (DeviceBuffer.from_numpy(ones) for _ in range(3))
+first, nodes = record(lambda: multiply(out))
+assert nodes == 1
+pooled = pyhost.memory_info()["pooled_bytes"]
+
+def body():
+    multiply(named)
+    assert launch()[2]
+    name, device, recorded, words = other.submit(elsewhere).result()
+    assert not recorded
+    multiply(out)
+
+second, nodes = record(body)
+assert nodes == 2
+assert pyhost.memory_info()["pooled_bytes"] == pooled + 256      # the other thread's block; the graph keeps `named`
+before = fake.fake_hip_launches()
+check(lib.tfhip_graph_launch(second.value))
+assert fake.fake_hip_launches() - before == 2
+check(lib.tfhip_graph_destroy(second.value))
+assert pyhost.memory_info()["pooled_bytes"] == pooled + 512
+other.shutdown()
+assert errors()[0] == 0, errors()
+""")

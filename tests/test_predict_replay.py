@@ -97,3 +97,23 @@ def test_exchanged_buffers_and_knobs_are_not_ignored(model):
         assert not np.array_equal(got, want)
     knob = load_library().tfhip_set_tuning
     changed(lambda: check(knob(b"tile", 3)), lambda: check(knob(b"tile", -1)))
+
+
+def test_another_thread_launches_while_a_recording_is_open(model, monkeypatch):
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(5)
+    a, b = rng.uniform(-1, 1, (1, 33, 40)).astype(np.float32), rng.uniform(-1, 1, (1, 40, 50)).astype(np.float32)
+    want, products = pyhost.fused_matmul(a, b), []
+    want_logits = model.predict()
+    with ThreadPoolExecutor(1) as other:
+        def multiply(i, op):   # upload, launch and download, while this thread records
+            products.append(other.submit(pyhost.fused_matmul, a, b).result())
+
+        launches = model.forward
+        monkeypatch.setattr(model, "forward", lambda: launches(before=multiply))
+        model.predict()
+    monkeypatch.undo()
+    assert model._graph is not None and len(products) == len(model.plan)
+    for got in products:
+        np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(_replayed(model), want_logits)

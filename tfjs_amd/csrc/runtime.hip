@@ -2,6 +2,7 @@
 // live-block registry, host<->device copies through pinned staging, event
 // timing, and recording of a sequence of launches into a HIP graph.
 #include <ctype.h>
+#include <pthread.h>
 #include <string.h>
 
 #include <atomic>
@@ -74,7 +75,10 @@ struct Runtime {
   // allocations of the same recording, then owned by the graph), and every
   // block an operand check saw is noted in `capture_refs` (checked again at
   // each replay).
-  bool capturing = false;
+  // The launches of the thread that records go to a stream of their own, which runs nothing, so that other
+  // threads go on launching and copying meanwhile.
+  hipStream_t capture_stream = nullptr;
+  uint64_t capture_forgotten = 0;   // scans_forgotten when the recording was opened
   std::unordered_map<size_t, std::vector<void *>> capture_free;
   std::set<uintptr_t> capture_refs;
   std::set<uintptr_t> capture_writes;   // of those, the blocks some recorded call writes
@@ -94,6 +98,12 @@ struct Runtime {
 
 Runtime g;
 std::mutex g_mutex;
+std::atomic<pthread_t> g_recorder{0};   // the thread whose launches are recorded, 0: none
+bool recording() { return g_recorder.load(std::memory_order_relaxed) != 0; }
+bool recording_here() {
+  const pthread_t r = g_recorder.load(std::memory_order_relaxed);
+  return r != 0 && r == pthread_self();
+}
 std::mutex g_staging_mutex;   // the staging ring: one transfer at a time (taken before g_mutex where both are)
 thread_local char g_error[1024] = "";
 int g_repeat = 1;
@@ -172,7 +182,7 @@ void read_tuning_from_environment() {
 bool initialised() { return g.ready; }
 int init_count() { return g_init_count; }
 int device_index() { return g.device; }
-hipStream_t stream() { return g.stream; }
+hipStream_t stream() { return recording_here() ? g.capture_stream : g.stream; }
 int num_cus() { return g.prop.multiProcessorCount; }
 
 // Scratch for kernels that need device memory beyond their operands (split-K
@@ -203,7 +213,7 @@ size_t fixed_workspace_bytes() { return g_fixed_ws_bytes; }
 void *workspace(size_t bytes) {
   if (g_ws_fixed) return bytes <= g_fixed_ws_bytes ? g_fixed_ws : nullptr;
   if (bytes <= g.workspace_bytes) return g.workspace;
-  if (g.capturing || !g.graphs.empty()) {
+  if (recording() || !g.graphs.empty()) {
     // a recorded graph may name the old block: it stays allocated until shutdown
     if (g.workspace) g.retired_workspaces.push_back(g.workspace);
   } else {
@@ -232,11 +242,11 @@ bool range_is_live(const void *p, size_t bytes) {
   if (it == g.live.begin()) return false;
   --it;
   const bool inside = a >= it->first && a + bytes <= it->first + it->second && a + bytes >= a;
-  if (inside && g.capturing) g.capture_refs.insert(it->first);
+  if (inside && recording_here()) g.capture_refs.insert(it->first);
   return inside;
 }
 
-bool capturing() { return g.capturing; }
+bool capturing() { return recording_here(); }
 
 __global__ void clear_word(int *word) { *word = 0; }
 
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(256) void find_nonfinite(const unsigned *__restrict
 
 void forget_filter_scans(const void *p) {
   std::lock_guard<std::mutex> lock(g_mutex);
-  if (g.filter_scans.empty() && !g.capturing) return;
+  if (g.filter_scans.empty() && !recording_here()) return;
   const uintptr_t a = reinterpret_cast<uintptr_t>(p);
   auto it = g.live.upper_bound(a);
   if (it == g.live.begin()) return;
@@ -258,7 +268,7 @@ void forget_filter_scans(const void *p) {
   if (a >= it->first + it->second) return;
   forget_scans_locked(it->first);
   // a replay writes the block again, with whatever its inputs hold then
-  if (g.capturing) g.capture_writes.insert(it->first);
+  if (recording_here()) g.capture_writes.insert(it->first);
 }
 
 int scan_filter(const float *w, int64_t elems, const char *who, bool *nonfinite) {
@@ -281,14 +291,14 @@ int scan_filter(const float *w, int64_t elems, const char *who, bool *nonfinite)
       for (const FilterScan &f : found->second) {
         if (f.ptr == a && f.elems == (size_t)elems && f.generation == generation) {
           *nonfinite = f.nonfinite;
-          if (g.capturing && !f.nonfinite) g.capture_scans.push_back(f);   // a replay rests on this answer
+          if (recording_here() && !f.nonfinite) g.capture_scans.push_back(f);   // a replay rests on this answer
           return kOk;
         }
       }
     }
   }
   // not known yet: one small kernel and a wait for its verdict, once per filter
-  if (g.capturing)
+  if (recording_here())
     return fail(kBadArgument,
                 "%s: this filter has not been searched for Inf / NaN yet, which needs a wait for the stream; run the "
                 "call once outside the recording",
@@ -320,7 +330,7 @@ int alloc_locked(size_t bytes, void **dptr) {
   const size_t cls = class_size(bytes);
   void *p = nullptr;
   auto &fl = g.free_lists[cls];
-  if (g.capturing && !g.capture_free[cls].empty()) {
+  if (recording_here() && !g.capture_free[cls].empty()) {
     p = g.capture_free[cls].back();
     g.capture_free[cls].pop_back();
   } else if (!fl.empty()) {
@@ -331,7 +341,7 @@ int alloc_locked(size_t bytes, void **dptr) {
     hipError_t e = hipMalloc(&p, cls);
     if (e == hipErrorOutOfMemory) {
       (void)hipGetLastError();
-      if (!g.capturing) (void)hipStreamSynchronize(g.stream);   // (a recording stream cannot be waited for)
+      (void)hipStreamSynchronize(g.stream);
       release_pool_locked();
       e = hipMalloc(&p, cls);
     }
@@ -540,6 +550,7 @@ int tfhip_init(int device) {
     if (rc != kOk) return rc;
   }
   TFHIP_CHECK_HIP(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
+  TFHIP_CHECK_HIP(hipStreamCreateWithFlags(&g.capture_stream, hipStreamNonBlocking));
   TFHIP_CHECK_HIP(hipHostMalloc(reinterpret_cast<void **>(&g.staging), kSlots * kSlotBytes, hipHostMallocDefault));
   for (int i = 0; i < kSlots; ++i) {
     TFHIP_CHECK_HIP(hipEventCreateWithFlags(&g.slot_done[i], hipEventDisableTiming));
@@ -558,12 +569,12 @@ int tfhip_init(int device) {
 int tfhip_shutdown(void) {
   std::lock_guard<std::mutex> lock(g_mutex);
   if (!g.ready) return kOk;
-  if (g.capturing) {
+  if (recording()) {
     hipGraph_t abandoned = nullptr;
-    (void)hipStreamEndCapture(g.stream, &abandoned);
+    (void)hipStreamEndCapture(g.capture_stream, &abandoned);
     if (abandoned) (void)hipGraphDestroy(abandoned);
     (void)hipGetLastError();
-    g.capturing = false;
+    g_recorder = 0;
   }
   (void)hipStreamSynchronize(g.stream);
   for (auto &kv : g.graphs) {
@@ -611,7 +622,8 @@ int tfhip_shutdown(void) {
   g_workspace_allocations = 0;
   g_last_splits = 0;
   (void)hipStreamDestroy(g.stream);
-  g.stream = nullptr;
+  (void)hipStreamDestroy(g.capture_stream);
+  g.stream = g.capture_stream = nullptr;
   g.ready = false;
   return kOk;
 }
@@ -650,7 +662,8 @@ int tfhip_free(void *dptr) {
   g.generation.erase(a);
   forget_scans_locked(a);
   g.live_bytes -= cls;
-  if (g.capturing) {
+  // (another thread may free a block that the graph names as well)
+  if (recording_here() || (recording() && g.capture_refs.count(a) > 0)) {
     g.capture_free[cls].push_back(dptr);   // the graph being recorded names it: the graph keeps it
   } else {
     give_back_locked(dptr, cls);
@@ -800,10 +813,11 @@ int tfhip_event_elapsed(int start_slot, int end_slot, float *ms) {
 int tfhip_capture_begin(void) {
   TFHIP_REQUIRE_INIT();
   std::lock_guard<std::mutex> lock(g_mutex);
-  TFHIP_CHECK_ARG(!g.capturing, "tfhip_capture_begin: a recording is already open");
+  TFHIP_CHECK_ARG(!recording(), "tfhip_capture_begin: a recording is already open");
   // Relaxed mode: an allocation that misses the pool may still call hipMalloc.
-  TFHIP_CHECK_HIP(hipStreamBeginCapture(g.stream, hipStreamCaptureModeRelaxed));
-  g.capturing = true;
+  TFHIP_CHECK_HIP(hipStreamBeginCapture(g.capture_stream, hipStreamCaptureModeRelaxed));
+  g_recorder = pthread_self();
+  g.capture_forgotten = g.scans_forgotten;
   g.capture_refs.clear();
   g.capture_writes.clear();
   g.capture_scans.clear();
@@ -813,10 +827,10 @@ int tfhip_capture_begin(void) {
 int tfhip_capture_end(int *graph_id, int *nodes) {
   TFHIP_REQUIRE_INIT();
   std::lock_guard<std::mutex> lock(g_mutex);
-  TFHIP_CHECK_ARG(g.capturing, "tfhip_capture_end: no recording is open");
-  g.capturing = false;
+  TFHIP_CHECK_ARG(recording(), "tfhip_capture_end: no recording is open");
+  g_recorder = 0;
   hipGraph_t graph = nullptr;
-  hipError_t e = hipStreamEndCapture(g.stream, &graph);
+  hipError_t e = hipStreamEndCapture(g.capture_stream, &graph);
   RecordedGraph rec;
   if (e == hipSuccess) {
     (void)hipGraphGetNodes(graph, nullptr, &rec.nodes);
@@ -852,7 +866,7 @@ int tfhip_capture_end(int *graph_id, int *nodes) {
     }
   }
   rec.scans = std::move(g.capture_scans);
-  rec.scans_forgotten = g.scans_forgotten;
+  rec.scans_forgotten = g.capture_forgotten;
   g.capture_refs.clear();
   g.capture_writes.clear();
   g.capture_scans.clear();
@@ -869,7 +883,7 @@ int tfhip_graph_launch(int graph_id) {
   uint64_t forgotten = 0;
   for (;;) {
     std::unique_lock<std::mutex> lock(g_mutex);
-    TFHIP_CHECK_ARG(!g.capturing, "tfhip_graph_launch: a recording is open");
+    TFHIP_CHECK_ARG(!recording_here(), "tfhip_graph_launch: a recording is open");
     auto it = g.graphs.find(graph_id);
     TFHIP_CHECK_ARG(it != g.graphs.end(), "tfhip_graph_launch: no graph %d", graph_id);
     RecordedGraph &rec = it->second;
