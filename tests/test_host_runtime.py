@@ -187,3 +187,30 @@ assert pyhost.memory_info()["pooled_bytes"] == pooled + 512
 other.shutdown()
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_the_last_kernel_is_the_calling_threads():
+    """A label's format and arguments are left behind separately and put together when they are asked for: another
+    thread's launch must not come in between."""
+    fake_hip_util.run("""
+pyhost.init()
+a, out = DeviceBuffer(4096), DeviceBuffer(4096)
+
+def last():
+    name = ctypes.create_string_buffer(256)
+    check(lib.tfhip_last_kernel(name, 256))
+    return name.value.decode()
+
+def copy():
+    check(lib.tfhip_copy(out.ptr, a.ptr, 4096))
+    seen.append(last())
+
+seen = []
+check(lib.tfhip_fused_matmul(a.ptr, a.ptr, out.ptr, 1, 1, 8, 8, 8, 0, 0, None, None, 0, None, None, 0.2))
+mine = last()
+assert mine.startswith("few_rows<1, 1, ")
+other = threading.Thread(target=copy)
+other.start()
+other.join()
+assert seen == ["copy_f4"] and last() == mine, (seen, last())
+""")

@@ -152,14 +152,15 @@ bool capturing();
 // enqueues its kernel (see tfhip_set_launch_repeat). The label is put together
 // when somebody asks for it: a launch only leaves the format (a string literal)
 // and its arguments (whole numbers and string literals) behind, because printing
-// them costs as much host time as a fifth of the launch.
+// them costs as much host time as a fifth of the launch. Every thread has its own:
+// a format must never meet the arguments of another thread's launch.
 struct KernelLabel {
   static constexpr int kMax = 8;
   const char *fmt;
   long long arg[kMax];
   int (*print)(char *to, size_t len, const KernelLabel &label);
 };
-extern KernelLabel g_kernel_label;
+extern __thread KernelLabel g_kernel_label;
 template <size_t... I, typename... A>
 int print_kernel_label(char *to, size_t len, const KernelLabel &l, std::index_sequence<I...>, std::tuple<A...> *) {
   if constexpr (sizeof...(A) == 0) return snprintf(to, len, "%s", l.fmt);

@@ -147,7 +147,7 @@ int fail(int code, const char *fmt, ...) {
   return code;
 }
 
-KernelLabel g_kernel_label = {};
+__thread KernelLabel g_kernel_label = {};
 
 int launch_repeat() { return g_repeat; }
 
