@@ -43,10 +43,10 @@ def _stand_in():
     return _built[1]
 
 
-def run(body, timeout=60):
-    """Runs `body` behind PRELUDE and returns what it printed; fails where it fails or does not end."""
+def run(body, each=([],), timeout=60):
+    """Runs `body` behind PRELUDE, once for each list of arguments; fails where it fails or does not end."""
     code = PRELUDE % (ROOT, _stand_in()) + body
-    done = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
-                          timeout=timeout)
-    assert done.returncode == 0, done.stdout[-4000:]
-    return done.stdout
+    for args in each:
+        done = subprocess.run([sys.executable, "-c", code] + args, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                              text=True, timeout=timeout)
+        assert done.returncode == 0, done.stdout[-4000:]

@@ -214,3 +214,34 @@ other.start()
 other.join()
 assert seen == ["copy_f4"] and last() == mine, (seen, last())
 """)
+
+
+def test_copy_threads_fit_the_cpus_of_the_process():
+    """A large transfer is copied by one thread per usable CPU, four at most, and a caller that waits for the others
+    on a CPU they need sleeps."""
+    fake_hip_util.run("""
+def tasks():
+    return set(os.listdir("/proc/self/task"))
+
+def sleeps():
+    status = open("/proc/self/task/%d/status" % threading.get_native_id()).read()
+    return int(status.split("voluntary_ctxt_switches:")[1].split()[0])
+
+pyhost.init()
+cpus = sorted(os.sched_getaffinity(0))
+data = np.arange(16 << 20, dtype=np.uint32).view(np.uint8)
+buf = DeviceBuffer(data.nbytes)
+before = tasks()
+if len(sys.argv) > 1:
+    os.sched_setaffinity(0, cpus[:1])
+buf.upload(data)
+crew = tasks() - before
+assert len(crew) == min(3, len(os.sched_getaffinity(0)) - 1), crew
+for task in tasks():                    # everything on one CPU from here
+    os.sched_setaffinity(int(task), cpus[:1])
+slept = sleeps()
+buf.upload(data)
+if crew:
+    assert sleeps() > slept
+np.testing.assert_array_equal(buf.download(np.uint8, data.nbytes), data)
+""", each=([], ["one cpu"]))

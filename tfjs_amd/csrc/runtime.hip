@@ -3,6 +3,7 @@
 // timing, and recording of a sequence of launches into a HIP graph.
 #include <ctype.h>
 #include <pthread.h>
+#include <sched.h>
 #include <string.h>
 
 #include <atomic>
@@ -358,16 +359,34 @@ int alloc_locked(size_t bytes, void **dptr) {
   return kOk;
 }
 
+// One turn of a wait that is expected to end within microseconds.
+inline void relax() {
+#if defined(__x86_64__) || defined(__i386__)
+  __builtin_ia32_pause();
+#else
+  std::this_thread::yield();
+#endif
+}
+
+// CPUs that the process may use now (a container's or a batch system's set, not the machine's).
+int usable_cpus() {
+  cpu_set_t set;
+  if (sched_getaffinity(0, sizeof set, &set) != 0) return 1;
+  return CPU_COUNT(&set);
+}
+
 // memcpy by several threads, for the pieces of a transfer between the caller's memory and the staging
 // ring: one thread moves 30 GB/s of a range that no cache holds, half of what the DMA engine behind it
-// does (57 GB/s); four move 99. The workers are started by the first large transfer, sleep between
-// transfers and last as long as the process (the object is never destroyed: a worker may be asleep
-// in it when the process ends).
+// does (57 GB/s); four move 99. The workers, at most one per CPU beside the caller's, are started by the
+// first large transfer, sleep between transfers and last as long as the process (the object is never
+// destroyed: a worker may be asleep in it when the process ends). Whoever waits looks for a while
+// (kSpins turns, some 100 us) and then sleeps: where the threads outnumber the CPUs, the one that is waited
+// for needs the waiter's.
 struct CopyCrew {
-  static constexpr int kWorkers = 3;
+  static constexpr int kWorkers = 3, kSpins = 4000;
   static constexpr size_t kShare = size_t(256) << 10;   // the least that is worth waking a worker for
   std::mutex m;
-  std::condition_variable wake;
+  std::condition_variable wake, done;
   std::atomic<unsigned> round{0};   // a new value: a copy to join
   std::atomic<int> left{0};         // workers that have not finished the present one
   char *dst = nullptr;
@@ -377,7 +396,7 @@ struct CopyCrew {
 
   CopyCrew() {
     try {
-      for (int i = 1; i <= kWorkers; ++i) {
+      for (int i = 1; i <= kWorkers && i < usable_cpus(); ++i) {
         std::thread([this, i] { work(i); }).detach();
         ++workers;
       }
@@ -392,14 +411,17 @@ struct CopyCrew {
     unsigned seen = 0;
     for (;;) {
       // look for the next piece of the same transfer for a while before going to sleep
-      for (int spin = 0; spin < 4000 && round.load(std::memory_order_acquire) == seen; ++spin) __builtin_ia32_pause();
+      for (int spin = 0; spin < kSpins && round.load(std::memory_order_acquire) == seen; ++spin) relax();
       if (round.load(std::memory_order_acquire) == seen) {
         std::unique_lock<std::mutex> lock(m);
         wake.wait(lock, [&] { return round.load(std::memory_order_acquire) != seen; });
       }
       seen = round.load(std::memory_order_acquire);
       part(i);
-      left.fetch_sub(1, std::memory_order_release);
+      if (left.fetch_sub(1, std::memory_order_acq_rel) == 1) {
+        std::lock_guard<std::mutex> lock(m);
+        done.notify_one();
+      }
     }
   }
   // (one caller at a time: the staging ring's mutex is held)
@@ -415,7 +437,11 @@ struct CopyCrew {
     }
     wake.notify_all();
     part(0);
-    while (left.load(std::memory_order_acquire) > 0) __builtin_ia32_pause();
+    for (int spin = 0; spin < kSpins && left.load(std::memory_order_acquire) > 0; ++spin) relax();
+    if (left.load(std::memory_order_acquire) > 0) {
+      std::unique_lock<std::mutex> lock(m);
+      done.wait(lock, [&] { return left.load(std::memory_order_acquire) == 0; });
+    }
   }
 };
 
