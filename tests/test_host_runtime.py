@@ -245,3 +245,27 @@ if crew:
     assert sleeps() > slept
 np.testing.assert_array_equal(buf.download(np.uint8, data.nbytes), data)
 """, each=([], ["one cpu"]))
+
+
+def test_a_child_copies_without_its_parents_threads():
+    """A forked child has none of the threads that copied for its parent: it starts its own."""
+    fake_hip_util.run("""
+pyhost.init()
+data = np.arange(4 << 20, dtype=np.uint32).view(np.uint8)
+buf = DeviceBuffer(data.nbytes)
+buf.upload(data)
+child = os.fork()
+if child == 0:
+    buf.upload(data[::-1])
+    os._exit(0 if np.array_equal(buf.download(np.uint8, data.nbytes), data[::-1]) else 1)
+end = time.time() + 20
+while time.time() < end:
+    pid, status = os.waitpid(child, os.WNOHANG)
+    if pid:
+        assert status == 0, status
+        break
+    time.sleep(0.01)
+else:
+    os.kill(child, 9)
+    raise AssertionError("the child waits for ever")
+""")

@@ -5,6 +5,7 @@
 #include <pthread.h>
 #include <sched.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <atomic>
 #include <condition_variable>
@@ -451,7 +452,12 @@ void host_copy(char *d, const char *s, size_t n, bool together) {
     memcpy(d, s, n);
     return;
   }
-  static CopyCrew *crew = new CopyCrew();
+  static CopyCrew *crew = nullptr;   // (the staging ring's mutex is held)
+  static pid_t owner = 0;            // a forked child has no such threads and starts its own
+  if (owner != getpid()) {
+    crew = new CopyCrew();
+    owner = getpid();
+  }
   crew->copy(d, s, n);
 }
 
