@@ -269,3 +269,35 @@ else:
     os.kill(child, 9)
     raise AssertionError("the child waits for ever")
 """)
+
+
+def test_shutdown_waits_for_a_transfer():
+    """The staging ring is not freed under a transfer; one that waited for the ring meanwhile fails and touches
+    nothing."""
+    fake_hip_util.run("""
+from concurrent.futures import ThreadPoolExecutor
+pyhost.init()
+data = np.arange(3 << 20, dtype=np.uint32)          # 12 MB: several pieces
+buf, out = DeviceBuffer(data.nbytes), np.empty_like(data)
+buf.upload(data)
+fake.fake_hip_copy_delay(30000)
+def upload():
+    return lib.tfhip_upload(buf.ptr, 0, data.ctypes.data, data.nbytes), lib.tfhip_last_error()
+def download():
+    return lib.tfhip_download(out.ctypes.data, buf.ptr, 0, out.nbytes), lib.tfhip_last_error()
+with ThreadPoolExecutor(3) as pool:
+    first = pool.submit(upload)
+    time.sleep(0.04)
+    waiting = [pool.submit(upload), pool.submit(download)]
+    time.sleep(0.04)
+    check(lib.tfhip_shutdown())
+    assert first.result()[0] == 0
+    for w in waiting:       # (ahead of the shutdown or behind it)
+        rc, message = w.result()
+        assert rc == 0 or b"shut down" in message, (rc, message)
+fake.fake_hip_copy_delay(0)
+check(lib.tfhip_init(0))
+fresh = DeviceBuffer.from_numpy(data)
+assert np.array_equal(fresh.download(np.uint32, data.size), data)
+assert errors()[0] == 0, errors()
+""")

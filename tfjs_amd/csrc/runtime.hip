@@ -483,10 +483,19 @@ int take_slot(int *slot) {
   return kOk;
 }
 
+// Behind the wait for the ring: the library may have been shut down, and set up again, since the caller
+// checked the range.
+int still_live(const char *d, size_t bytes) {
+  if (g.ready && range_is_live(d, bytes)) return kOk;
+  return fail(kNotInitialised, "a transfer of %zu bytes: the library was shut down while it waited", bytes);
+}
+
 // Host memory -> device memory (checked by the caller), on the library's stream. 85 MB take
 // 1.7 ms, 88% of the DMA rate; with two 32 MB staging buffers filled by one thread they took 3.2 ms.
 int stage_upload(char *d, const char *h, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_staging_mutex);
+  const int alive = still_live(d, bytes);
+  if (alive != kOk) return alive;
   for (size_t done = 0; done < bytes;) {
     const size_t n = piece_bytes(done, bytes - done);
     int s = 0;
@@ -506,6 +515,8 @@ int stage_upload(char *d, const char *h, size_t bytes) {
 // its slot the DMA fills the next ones.
 int stage_download(char *h, const char *d, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_staging_mutex);
+  const int alive = still_live(d, bytes);
+  if (alive != kOk) return alive;
   constexpr size_t kKernelCopyBytes = size_t(1) << 20;
   constexpr int kAhead = 4;
   if (bytes <= kKernelCopyBytes) {
@@ -561,6 +572,7 @@ extern "C" {
 const char *tfhip_last_error(void) { return g_error; }
 
 int tfhip_init(int device) {
+  std::lock_guard<std::mutex> no_transfer(g_staging_mutex);
   std::lock_guard<std::mutex> lock(g_mutex);
   if (g.ready) {
     if (device == g.device) return kOk;
@@ -599,6 +611,7 @@ int tfhip_init(int device) {
 }
 
 int tfhip_shutdown(void) {
+  std::lock_guard<std::mutex> no_transfer(g_staging_mutex);   // (one that is under way ends first)
   std::lock_guard<std::mutex> lock(g_mutex);
   if (!g.ready) return kOk;
   if (recording()) {
