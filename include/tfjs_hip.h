@@ -379,7 +379,8 @@ int tfhip_dequant_f16(const void *q, int64_t n, float *out);
  * from byte offsets[i] of the buffer on, any alignment; scale_min holds its scale and min at 2i and 2i+1
  * (used by the affine kinds). kinds: 0 four-byte elements copied as they are (float32, int32), 1 one-byte
  * elements copied (bool), 2 / 3 uint8 affine to float32 / int32, 4 / 5 uint16 affine to float32 / int32,
- * 6 float16. The same values as tfhip_dequant_affine and tfhip_dequant_f16. The host buffer may be reused
+ * 6 float16. Large tensors of kinds 0 and 1 are uploaded where they belong; the rest passes through a
+ * temporary block of at most 256 MB (or one tensor's codes). The same values as tfhip_dequant_affine and tfhip_dequant_f16. The host buffer may be reused
  * on return; on failure no block is left behind. */
 int tfhip_decode_weights(const void *host, size_t bytes, int64_t count, const int64_t *offsets,
                          const int64_t *elems, const int *kinds, const double *scale_min, void **outs);

@@ -301,3 +301,35 @@ fresh = DeviceBuffer.from_numpy(data)
 assert np.array_equal(fresh.download(np.uint32, data.size), data)
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_plain_tensors_are_not_held_twice():
+    """What need not be decoded is uploaded into its tensor; the temporary block of the rest is bounded."""
+    fake_hip_util.run("""
+pyhost.init()
+MB = 1 << 20
+
+def load(sizes, quantized):
+    specs = [dict(name=str(i), shape=[n if quantized else n // 4], dtype="float32") for i, n in enumerate(sizes)]
+    if quantized:
+        for s in specs:
+            s["quantization"] = dict(dtype="uint8", scale=1.0, min=0.0)
+    data = np.arange(sum(sizes) // 4, dtype=np.uint32)
+    before = pyhost.memory_info()["pooled_bytes"]
+    loaded = pyhost.decode_weights_to_device(data, specs)
+    extra = pyhost.memory_info()["pooled_bytes"] - before
+    at = 0
+    for n, (buf, _) in zip(sizes, loaded.values()):
+        if not quantized and n >= 4 * MB:
+            assert np.array_equal(buf.download(np.uint32, n // 4), data[at // 4:(at + n) // 4])
+        at += n
+        buf.free()
+    lib.tfhip_shutdown()
+    check(lib.tfhip_init(0))
+    return extra
+
+assert load([24 * MB, 4 * MB, 8 * MB + 4], False) == 0
+assert load([24 * MB, 1000, 9 * MB, 4 * MB - 4, 16], False) < 5 * MB
+assert 96 * MB < load([96 * MB] * 3, True) < 288 * MB
+assert errors()[0] == 0, errors()
+""")

@@ -76,3 +76,26 @@ def test_decode_refuses_what_lies_outside_the_buffer_and_leaves_nothing_behind()
                                       (ctypes.c_int * 2)(2, kind), (ctypes.c_double * 4)(1, 0, 1, 0), outs)
         assert rc != 0 and message in lib.tfhip_last_error(), lib.tfhip_last_error()
         assert hip.memory_info()["live"] == before
+
+
+def test_decode_of_a_mixed_buffer_in_several_groups():
+    """Plain tensors around the size that is uploaded alone, codes around them, and more codes than pass through the
+    temporary block at once."""
+    hip.init()
+    rng = np.random.default_rng(1)
+    sizes = [(4 * MB, None), (70 * MB + 1, "uint8"), (4 * MB - 4, None), (90 * MB, "uint8"), (12, None), (99 * MB + 3, "uint8"),
+             (33 * MB + 1, "uint8"), (9 * MB + 4, None), (5, "uint8")]
+    raw = rng.integers(0, 256, sum(n for n, _ in sizes), dtype=np.uint8)
+    specs = [dict(name=str(i), dtype="float32", shape=[n if q else n // 4],
+                  **(dict(quantization=dict(dtype=q, scale=0.5 + i, min=-3.0)) if q else {})) for i, (n, q) in enumerate(sizes)]
+    pooled = hip.memory_info()["pooled_bytes"]
+    loaded = hip.decode_weights_to_device(raw, specs)
+    assert hip.memory_info()["pooled_bytes"] - pooled <= 288 * MB
+    at = 0
+    for i, (n, q) in enumerate(sizes):
+        buf, _ = loaded[str(i)]
+        codes = raw[at:at + n]
+        want = (codes.astype(np.float64) * (0.5 + i) - 3.0).astype(np.float32) if q else codes.copy().view(np.float32)
+        np.testing.assert_array_equal(buf.download(np.uint32, want.size), want.view(np.uint32))
+        at += n
+        buf.free()

@@ -42,9 +42,14 @@ struct FixedWorkspace {
   ~FixedWorkspace();
 };
 bool workspace_is_fixed();
-// Host memory -> [d, d + bytes) of a live block, through the pinned staging ring, on the library's stream;
-// the host range may be reused on return.
-int stage_upload(char *d, const char *h, size_t bytes);
+// Host memory -> live device memory, through the pinned staging ring, on the library's stream: the bytes at `h` go
+// to `d`, one segment behind the other. The host ranges may be reused on return.
+struct UploadSegment {
+  char *d;
+  const char *h;
+  size_t bytes;
+};
+int stage_upload(const UploadSegment *segments, size_t count);
 // Records the number of K slices a GEMM launch was cut into (tfhip_workspace_info reports the last).
 void note_splits(int splits);
 size_t fixed_workspace_bytes();

@@ -490,20 +490,65 @@ int still_live(const char *d, size_t bytes) {
   return fail(kNotInitialised, "a transfer of %zu bytes: the library was shut down while it waited", bytes);
 }
 
+// A place in a list of segments to be uploaded one behind the other.
+struct UploadPlace {
+  const UploadSegment *seg;
+  size_t off;   // in *seg
+};
+
+// Calls each(at, segment, offset in it, length) for what the next n bytes take of each segment; `at` counts from 0.
+// Returns the place behind them.
+template <typename F>
+UploadPlace for_segments(UploadPlace p, size_t n, F each) {
+  for (size_t at = 0; at < n;) {
+    if (p.off == p.seg->bytes) {
+      p = {p.seg + 1, 0};
+      continue;
+    }
+    const size_t part = p.seg->bytes - p.off < n - at ? p.seg->bytes - p.off : n - at;
+    each(at, *p.seg, p.off, part);
+    p.off += part;
+    at += part;
+  }
+  return p;
+}
+
 // Host memory -> device memory (checked by the caller), on the library's stream. 85 MB take
 // 1.7 ms, 88% of the DMA rate; with two 32 MB staging buffers filled by one thread they took 3.2 ms.
-int stage_upload(char *d, const char *h, size_t bytes) {
+int stage_upload(const UploadSegment *segments, size_t count) {
   std::lock_guard<std::mutex> lock(g_staging_mutex);
-  const int alive = still_live(d, bytes);
-  if (alive != kOk) return alive;
-  for (size_t done = 0; done < bytes;) {
-    const size_t n = piece_bytes(done, bytes - done);
+  size_t total = 0;
+  for (size_t i = 0; i < count; ++i) {
+    const int alive = still_live(segments[i].d, segments[i].bytes);
+    if (alive != kOk) return alive;
+    total += segments[i].bytes;
+  }
+  const bool together = total >= kCrewBytes;
+  UploadPlace place = {segments, 0};
+  for (size_t done = 0; done < total;) {
+    const size_t n = piece_bytes(done, total - done);
     int s = 0;
     const int rc = take_slot(&s);
     if (rc != kOk) return rc;
     char *slot = g.staging + s * kSlotBytes;
-    host_copy(slot, h + done, n, bytes >= kCrewBytes);
-    TFHIP_CHECK_HIP(hipMemcpyAsync(d + done, slot, n, hipMemcpyHostToDevice, g.stream));
+    // (segments that lie side by side in host memory, as the tensors of a shard do, are copied together)
+    const char *h = nullptr;
+    size_t from = 0, until = 0;
+    for_segments(place, n, [&](size_t at, const UploadSegment &seg, size_t off, size_t bytes) {
+      if (until > from && seg.h + off != h + (at - from)) {
+        host_copy(slot + from, h, until - from, together);
+        from = at;
+      }
+      if (at == from) h = seg.h + off;
+      until = at + bytes;
+    });
+    host_copy(slot + from, h, until - from, together);
+    // (a DMA for each: two blocks side by side on the device are still two allocations)
+    hipError_t e = hipSuccess;
+    place = for_segments(place, n, [&](size_t at, const UploadSegment &seg, size_t off, size_t bytes) {
+      if (e == hipSuccess) e = hipMemcpyAsync(seg.d + off, slot + at, bytes, hipMemcpyHostToDevice, g.stream);
+    });
+    if (e != hipSuccess) return fail(kHipError, "stage_upload: hipMemcpyAsync failed: %s", hipGetErrorString(e));
     TFHIP_CHECK_HIP(hipEventRecord(g.slot_done[s], g.stream));
     g.slot_busy[s] = true;
     done += n;
@@ -777,7 +822,8 @@ int tfhip_upload(void *dst, size_t dst_offset, const void *host, size_t bytes) {
   TFHIP_CHECK_ARG(host != nullptr, "tfhip_upload: host pointer is NULL");
   char *d = static_cast<char *>(dst) + dst_offset;
   TFHIP_CHECK_OUTPUT(d, bytes, 1, "dst");
-  return stage_upload(d, static_cast<const char *>(host), bytes);
+  const UploadSegment whole = {d, static_cast<const char *>(host), bytes};
+  return stage_upload(&whole, 1);
 }
 
 int tfhip_download(void *host, const void *src, size_t src_offset, size_t bytes) {
