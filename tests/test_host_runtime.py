@@ -333,3 +333,26 @@ assert load([24 * MB, 1000, 9 * MB, 4 * MB - 4, 16], False) < 5 * MB
 assert 96 * MB < load([96 * MB] * 3, True) < 288 * MB
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_two_threads_search_their_own_filters():
+    """A search for Inf / NaN waits for its verdict in a word that searches share: one at a time."""
+    fake_hip_util.run("""
+from concurrent.futures import ThreadPoolExecutor
+pyhost.init()
+bad = np.ones(64, np.float32)
+bad[5] = np.nan
+buffers = [DeviceBuffer.from_numpy(x) for x in (bad, np.ones(64, np.float32))]
+fake.fake_hip_copy_delay(50000)
+
+def finite(buf):
+    answer = ctypes.c_int()
+    check(lib.tfhip_filter_is_finite(buf.ptr, 64, ctypes.byref(answer)))
+    return answer.value
+
+with ThreadPoolExecutor(2) as pool:
+    first = pool.submit(finite, buffers[0])
+    time.sleep(0.01)
+    second = pool.submit(finite, buffers[1])
+    assert (first.result(), second.result()) == (0, 1)
+""")

@@ -106,6 +106,7 @@ bool recording_here() {
   const pthread_t r = g_recorder.load(std::memory_order_relaxed);
   return r != 0 && r == pthread_self();
 }
+std::mutex g_scan_mutex;      // a search of a filter for Inf / NaN (taken before g_mutex)
 std::mutex g_staging_mutex;   // the staging ring: one transfer at a time (taken before g_mutex where both are)
 thread_local char g_error[1024] = "";
 int g_repeat = 1;
@@ -299,12 +300,14 @@ int scan_filter(const float *w, int64_t elems, const char *who, bool *nonfinite)
       }
     }
   }
-  // not known yet: one small kernel and a wait for its verdict, once per filter
+  // not known yet: one small kernel and a wait for its verdict, once per filter (and one search at a time: they share
+  // the word that the verdict comes back in)
   if (recording_here())
     return fail(kBadArgument,
                 "%s: this filter has not been searched for Inf / NaN yet, which needs a wait for the stream; run the "
                 "call once outside the recording",
                 who);
+  std::lock_guard<std::mutex> searching(g_scan_mutex);
   *g.scan_flag = 0;
   clear_word<<<dim3(1), dim3(1), 0, g.stream>>>(g.scan_flag_dev);
   long long blocks = (elems + 255) / 256;
