@@ -70,6 +70,23 @@ def test_against_the_oracle(lib, m, n, k, act, shift):
         p.free()
 
 
+@pytest.mark.parametrize("m,n,k,act,shift", [
+    (20, 2309, 2053, "relu", 1), (33, 770, 2050, "linear", 0), (161, 250, 8193, "relu", 3), (16, 4097, 255, "elu", 0),
+    (32, 8200, 300, "linear", 1), (256, 255, 2049, "sigmoid", 0),
+])
+def test_strips_of_64_columns_against_the_oracle(lib, m, n, k, act, shift):
+    from oracle import pyoracle as orc
+    p = _Product(lib, m, n, k, act, shift)
+    try:
+        p.launch()
+        assert _last_kernel(lib).startswith("few_rows<%d, 4, " % (1 if m <= 16 or m > 32 else 2))
+        got = p.result()
+        want = orc.fused_matmul(p.host[0], p.host[1], bias=p.host[2], activation=act, leakyrelu_alpha=0.2)
+        assert np.max(np.abs(got - want) / np.maximum(1.0, np.abs(want))) <= 1e-4
+    finally:
+        p.free()
+
+
 def test_a_recording_gives_the_same_bits(lib):
     p = _Product(lib, 19, 200, 2000, "relu")
     try:

@@ -356,3 +356,39 @@ with ThreadPoolExecutor(2) as pool:
     second = pool.submit(finite, buffers[1])
     assert (first.result(), second.result()) == (0, 1)
 """)
+
+
+def test_which_products_the_kernel_for_few_rows_takes():
+    """Both sides of every line of its rules, by the label of the kernel that is launched."""
+    fake_hip_util.run("""
+pyhost.init()
+big = [DeviceBuffer(64 << 20) for _ in range(3)]
+
+def label():
+    name = ctypes.create_string_buffer(256)
+    check(lib.tfhip_last_kernel(name, 256))
+    return name.value.decode()
+
+def product(m, n, k):
+    check(lib.tfhip_fused_matmul(big[0].ptr, big[1].ptr, big[2].ptr, 1, 1, m, n, k, 0, 0, None, None, 0, None, None, 0.2))
+    return label()
+
+def windows(hw, c, f, out_c):
+    check(lib.tfhip_fused_conv2d(big[0].ptr, big[1].ptr, big[2].ptr, 1, hw, hw, c, f, f, out_c, 1, 1, 1, 1, f // 2, f // 2, hw,
+                                 hw, 0, None, None, 0, None, None, 0.2))
+    return label()
+
+for shape, want in {
+    (1, 4096, 2048): "few_rows<1, 1", (1, 4000, 2049): "few_rows<1, 4", (1, 4096, 1024): "few_rows<1, 1", (1, 4097, 1024): "few_rows<1, 4",
+    (16, 2048, 4096): "few_rows<1, 1", (16, 2048, 4097): "few_rows<1, 4", (17, 2304, 1536): "few_rows<2, 1",
+    (17, 2304, 2049): "few_rows<2, 4", (32, 4096, 1536): "few_rows<2, 1", (32, 4096, 1537): "few_rows<2, 4", (32, 4097, 1536): "gemm_kernel<",
+    (32, 4097, 1537): "few_rows<2, 4", (32, 8192, 1536): "gemm_kernel<", (32, 8193, 1024): "few_rows<2, 4", (33, 64, 319): "gemm_kernel<",
+    (33, 64, 320): "few_rows<1, 1", (64, 1024, 2048): "few_rows<1, 1", (64, 1024, 2049): "few_rows<1, 4", (160, 256, 8192): "few_rows<1, 4",
+    (128, 768, 1536): "few_rows<2, 1", (128, 768, 1540): "gemm_kernel<", (257, 256, 320): "few_rows<2, 1", (513, 256, 320): "gemm_kernel<",
+}.items():
+    assert product(*shape).startswith(want), (shape, product(*shape), want)
+for shape, want in {(14, 41, 3, 16): "gemm_kernel<", (14, 42, 3, 16): "few_rows<1, 1", (7, 256, 7, 256): "few_rows<1, 1",
+                    (14, 256, 7, 256): "gemm_kernel<", (10, 256, 3, 256): "few_rows<1, 1", (10, 256, 5, 256): "gemm_kernel<"}.items():
+    assert windows(*shape).startswith(want), (shape, windows(*shape), want)
+assert errors()[0] == 0, errors()
+""")

@@ -269,25 +269,73 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows_finish(FewRowsArg
   finish_tile<MB, CB>(p, blockIdx.x, bias, alpha, nullptr);
 }
 
+// How a product in tiles of 16 MB rows and 16 CB columns is cut over workgroups.
+constexpr int kFewRowsCounters = 256;
+struct FewRowsCut {
+  int row_tiles;
+  long long tiles;
+  int splits, groups_per_split;   // slices of k, and the k groups of 16 in one
+};
+inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_blocks) {
+  FewRowsCut cut;
+  cut.row_tiles = row_blocks == 1 ? (p.M + 15) / 16 : (p.M + 31) / 32;
+  cut.tiles = (long long)cut.row_tiles * (col_blocks == 1 ? (p.N + 15) / 16 : (p.N + 63) / 64);
+  const int groups = (p.K + 15) / 16;
+  // A wavefront wants about as many k groups as it fetches at once (64 or 32 groups per workgroup); more workgroups
+  // than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
+  const int wanted = row_blocks == 1 ? (groups + 63) / 64 : (groups + 31) / 32;
+  const int most = cut.tiles * 2 > kFewRowsCounters ? 1 : kFewRowsCounters / (int)cut.tiles;
+  cut.splits = wanted < most ? wanted : most;
+  cut.groups_per_split = cut.splits == 1 ? groups : (groups + cut.splits - 1) / cut.splits;
+  return cut;
+}
+
+// Strips of 64 columns, whole cache lines and a quarter of the tiles to share the slices among, where strips of 16
+// (cut as `narrow` says) find no compute unit of their own each, or where a workgroup of theirs would fetch more than twice
+// (with two row blocks three times) what it can have out at once; else strips of 16: as many workgroups as there are.
+// us, strips of 16 and 64: 1 x 2048 x 4096 8.1 and 9.0, 1 x 2304 x 4000 9.6 and 8.5; 32 x 1536 x 2304 10.1 and 10.8,
+// 32 x 3072 x 2304 17.9 and 11.6; 48 x 2304 x 768 10.4 and 8.7, 160 x 8192 x 256 28.5 and 12.8; 1 x 1024 x 4096 5.3 and
+// 7.6, 1 x 1024 x 4112 8.5 and 7.6.
+inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
+  return narrow.tiles > num_cus() || narrow.groups_per_split > (row_blocks == 1 ? 128 : 96);
+}
+
 // Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
-// tiled kernel. Up to 32 rows always. Beyond, as long as every workgroup has a compute unit of its own: the fetches of
-// a whole k range are then out at once, where the tiled kernel goes round its pipeline once per 32 k (us, tiled and
-// here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7, 128 x 1024 x 1024 with two
-// row blocks 9.1 and 7.5; windows, [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1, [1,20,20,64] 3x3 -> 16 7.9 and 5.9). A
-// short k has nothing to gain (784 x 192 x 32: 4.5 and 5.1; windows of 240 floats 5.2 and 6.1), nor has a
-// long one with two row blocks, whose wavefronts fetch half as many groups at once (128 x 3072 x 768: 14.1 and 15.5).
+// tiled kernel. As long as every workgroup has a compute unit of its own, the fetches of a whole k range are out at once,
+// where the tiled kernel goes round its pipeline once per 32 k (us, tiled and here: 49 x 960 x 160 9.2 and 5.6,
+// 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7; windows, [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1). The lines,
+// each from a grid of extents on both sides, in the same form:
+//  * more than 32 rows, K < 320: the tiled kernel is ahead up to 128 (33 x 64 x 32 3.3 and 3.9), then the two are
+//    within 10% of each other (100 x 256 x 96 4.7 and 4.2).
+//  * windows of fewer than 384 floats: behind at 144 ([1,7,7,16] 3x3 -> 32 4.4 and 4.8); ahead from 297 on
+//    ([1,14,14,33] 3x3 -> 64 7.7 and 5.9), so the line is on the safe side.
+//  * up to 32 rows always, from K = 2048 on with two row blocks: half the fetches of B, and slices enough to fill the
+//    chip (23 x 3072 x 768 9.3 with one, 7.7 with two). Except 17 to 32 rows of 4097 to 8192 columns with K <= 1536:
+//    more strips than compute units, while each of the tiled kernel's 32-wide tiles has one (32 x 512 x 8192 6.4 and
+//    8.3, 32 x 1024 x 5000 8.9 and 11.2; 32 x 2048 x 5000 14.2 and 14.2, 32 x 1024 x 12288 17.9 and 13.9).
+//  * more than 32 rows with two row blocks, K <= 1536: 128 x 1024 x 1024 9.1 and 7.5, 128 x 1536 x 768 12.8 and 10.1;
+//    128 x 3072 x 768 13.8 and 16.8. (128 x 1792 x 768, 14.4 and 11.4, is left on the wrong side.)
+//  * windows have no strips of 64: with a workgroup on a third of the compute units and more, and more than 192 groups for
+//    it, the tiled kernel is ahead ([1,10,10,256] 5x5 -> 256 14.5 and 15.4, [1,14,14,256] 7x7 -> 256 30.5 and 39.7; on
+//    64 tiles [1,7,7,256] 7x7 -> 256 21.0 and 13.8; at 144 groups [1,10,10,512] 3x3 -> 256 12.8 and 13.0).
 inline int few_rows_blocks(const GemmParams &p, bool windows) {
   if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
   if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
       tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
     return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();
-  if (p.M <= 16) return 1;
-  if (p.M > 32 && p.K < 320 && !windows) return 0;
-  if (p.M <= 32 && p.K > 2048) return 2;   // half the fetches of B, and slices enough to fill the chip
-  if ((p.M + 15) / 16 * strips <= cus) return 1;
-  if (p.M <= 32 || ((p.M + 31) / 32 * strips <= cus && p.K <= 1536)) return 2;
-  return 0;
+  int blocks = 0;
+  if (p.M <= 16) blocks = 1;
+  else if (p.M > 32 && p.K < 320 && !windows) blocks = 0;
+  else if (p.M <= 32 && p.K > 2048) blocks = 2;
+  else if ((p.M + 15) / 16 * strips <= cus) blocks = 1;
+  else if (p.M <= 32) blocks = strips > cus && strips <= 2 * cus && p.K <= 1536 ? 0 : 2;
+  else if ((p.M + 31) / 32 * strips <= cus && p.K <= 1536) blocks = 2;
+  if (windows && blocks != 0) {
+    const FewRowsCut cut = few_rows_cut(p, blocks, 1);
+    if (cut.tiles * 3 > cus && cut.groups_per_split > 192) blocks = 0;
+  }
+  return blocks;
 }
 
 // `kind`: kLoadKAny (row-major A), kLoadWindows or kLoadWindowsAny.

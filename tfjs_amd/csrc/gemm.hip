@@ -30,7 +30,6 @@ namespace {
 // copy of each array, at an address of its own; in host code the names are only stand-ins for the symbols. The
 // addresses are resolved once per device by setup_static_scratch (with that device current), and a launch takes those of
 // the device that tfhip_init was last given.
-constexpr int kFewRowsCounters = 256;
 static __device__ int few_rows_counters[kFewRowsCounters];   // one per tile that is cut, zero between launches
 // The split-K partial sums of tfhip_fused_matmul_noalloc, which tfhip_fused_matmul keeps in the library's growing workspace.
 static __device__ __align__(256) float scratch[TFHIP_NOALLOC_SCRATCH_BYTES / sizeof(float)];
@@ -50,20 +49,15 @@ int resolve(const void *symbol, const char *name, int device, void **ptr) {
 }
 
 template <int MB, int CB, int KIND>
-int launch_few_rows_shape(FewRowsArgs &q) {
-  q.row_tiles = (q.M + 16 * MB - 1) / (16 * MB);
-  const long long tiles = (long long)((q.N + 16 * CB - 1) / (16 * CB)) * q.row_tiles;
-  // A wavefront wants about as many k groups as it fetches at once (64 or 32 groups per workgroup); more workgroups
-  // than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
-  int splits = (q.groups + 64 / MB - 1) / (64 / MB);
-  if (splits > kFewRowsCounters / tiles) splits = (int)(kFewRowsCounters / tiles);
+int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
+  q.row_tiles = cut.row_tiles;
   q.splits = 1;
   q.groups_per_split = q.groups;
-  if (splits > 1) {
-    q.ws = static_cast<float *>(workspace((size_t)tiles * splits * 256 * MB * CB * sizeof(float)));
+  if (cut.splits > 1) {
+    q.ws = static_cast<float *>(workspace((size_t)cut.tiles * cut.splits * 256 * MB * CB * sizeof(float)));
     if (q.ws) {
-      q.splits = splits;
-      q.groups_per_split = (q.groups + splits - 1) / splits;
+      q.splits = cut.splits;
+      q.groups_per_split = cut.groups_per_split;
     }
   }
   note_splits(q.splits);
@@ -71,9 +65,9 @@ int launch_few_rows_shape(FewRowsArgs &q) {
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
   q.finish_apart = q.splits > 1 && capturing();
   note_kernel("few_rows<%d, %d, %d>", MB, CB, KIND);
-  const dim3 grid((unsigned)(tiles * q.splits)), block(64 * kFewRowsWaves);
+  const dim3 grid((unsigned)(cut.tiles * q.splits)), block(64 * kFewRowsWaves);
   if (q.finish_apart) {
-    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)tiles), block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)cut.tiles), block, 0, stream()>>>(q)));
   } else {
     TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q)));
   }
@@ -96,13 +90,15 @@ int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   q.b_bytes = kind == kLoadKAny ? (unsigned)((long long)p.K * p.N * 4) : p.b_bytes;
   q.groups = (p.K + 15) / 16;
   q.counters = g_device_arrays[device_index()].few_rows_counters;
-  // Strips of 64 columns, whole cache lines, once B is tens of megabytes (1 x 4096 x 4096: 14.2 us, 15.5 with strips
-  // of 16), else of 16: as many workgroups as there are.
-  const bool wide = (long long)p.K * p.N >= (8LL << 20);
-  if (kind == kLoadWindows) return row_blocks == 1 ? launch_few_rows_shape<1, 1, kLoadWindows>(q) : launch_few_rows_shape<2, 1, kLoadWindows>(q);
-  if (kind == kLoadWindowsAny) return row_blocks == 1 ? launch_few_rows_shape<1, 1, kLoadWindowsAny>(q) : launch_few_rows_shape<2, 1, kLoadWindowsAny>(q);
-  if (row_blocks == 1) return wide ? launch_few_rows_shape<1, 4, kLoadKAny>(q) : launch_few_rows_shape<1, 1, kLoadKAny>(q);
-  return wide ? launch_few_rows_shape<2, 4, kLoadKAny>(q) : launch_few_rows_shape<2, 1, kLoadKAny>(q);
+  const FewRowsCut narrow = few_rows_cut(p, row_blocks, 1);
+  const bool one = row_blocks == 1;
+  if (kind == kLoadWindows) return one ? launch_few_rows_shape<1, 1, kLoadWindows>(q, narrow) : launch_few_rows_shape<2, 1, kLoadWindows>(q, narrow);
+  if (kind == kLoadWindowsAny) return one ? launch_few_rows_shape<1, 1, kLoadWindowsAny>(q, narrow) : launch_few_rows_shape<2, 1, kLoadWindowsAny>(q, narrow);
+  if (few_rows_wide(narrow, row_blocks)) {
+    const FewRowsCut wide = few_rows_cut(p, row_blocks, 4);
+    return one ? launch_few_rows_shape<1, 4, kLoadKAny>(q, wide) : launch_few_rows_shape<2, 4, kLoadKAny>(q, wide);
+  }
+  return one ? launch_few_rows_shape<1, 1, kLoadKAny>(q, narrow) : launch_few_rows_shape<2, 1, kLoadKAny>(q, narrow);
 }
 
 int setup_static_scratch(int device) {
