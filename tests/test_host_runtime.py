@@ -392,3 +392,20 @@ for shape, want in {(14, 41, 3, 16): "gemm_kernel<", (14, 42, 3, 16): "few_rows<
     assert windows(*shape).startswith(want), (shape, windows(*shape), want)
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_filters_of_many_taps_are_gathered():
+    """An image of few channels under a filter that the matrix-core form does not hold: GEMM-shaped from 16 output
+    channels on, however few pixels there are."""
+    fake_hip_util.run("""
+pyhost.init()
+big = [DeviceBuffer(8 << 20) for _ in range(3)]
+name = ctypes.create_string_buffer(256)
+for hw, c, f, out_c, want in [(1, 3, 4, 16, "gemm_kernel<"), (16, 3, 5, 16, "gemm_kernel<"), (16, 4, 7, 64, "gemm_kernel<"),
+                              (10, 4, 11, 32, "few_rows<"), (17, 3, 5, 8, "gemm_kernel<"), (16, 3, 5, 8, "conv_few_channels<8>"),
+                              (16, 3, 3, 16, "conv_few_taps<"), (16, 3, 3, 8, "conv_few_channels<8>")]:
+    check(lib.tfhip_fused_conv2d(big[0].ptr, big[1].ptr, big[2].ptr, 1, hw, hw, c, f, f, out_c, 1, 1, 1, 1, f // 2, f // 2, hw,
+                                 hw, 0, None, None, 0, None, None, 0.2))
+    check(lib.tfhip_last_kernel(name, 256))
+    assert name.value.decode().startswith(want), (hw, c, f, out_c, name.value)
+""")

@@ -82,3 +82,14 @@ def test_neighbouring_rows_stay_apart(hip):
     x[0, 4] = np.nan
     got = hip.fused_conv2d(x, w, pad="same")
     assert np.isnan(got[0, 4]).all() and np.isfinite(np.delete(got[0], 4, 0)).all()
+
+
+@pytest.mark.parametrize("xs,fs,stride", [((1, 16, 16, 3), (5, 5, 3, 16), 1), ((1, 1, 1, 3), (4, 4, 3, 16), 1),
+                                          ((2, 11, 9, 4), (11, 11, 4, 32), 1), ((1, 30, 31, 1), (7, 7, 1, 64), 2)])
+def test_a_few_pixels_under_a_filter_of_many_taps(hip, orc, xs, fs, stride):
+    rng = np.random.default_rng(sum(xs) + sum(fs))
+    x = rng.uniform(-1, 1, xs).astype(np.float32)
+    w = rng.normal(0, 0.2, fs).astype(np.float32)
+    kw = dict(strides=stride, pad="same", bias=rng.uniform(-1, 1, (fs[3],)).astype(np.float32), activation="relu6")
+    _close(hip.fused_conv2d(x, w, **kw), orc.fused_conv2d(x, w, **kw))
+    assert not _last_kernel().startswith("conv_few_channels")

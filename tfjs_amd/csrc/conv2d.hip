@@ -411,11 +411,14 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
     p.a_sx = in_c; p.a_sk = 1;
     return launch_plain_gemm(p, false, false, vec);
   }
-  // (With more taps than the matrix-core form holds, the lane-per-pixel form is for a workgroup of pixels at most: a
-  // lane then walks K taps on its own, where the implicit GEMM gathers whole filter rows: 2 x 60 x 60 x 3, 7x7 -> 8:
-  // 26.1 and 6.8 us, 8 x 112 x 112 x 3, 7x7/2 -> 64: 39.2 and 15.1.)
+  // More taps than the matrix-core form holds: the GEMM-shaped kernels, which gather whole filter rows, where a lane that
+  // walks K taps on its own is 1.3 to 14 times slower (us, lane per pixel and gathered: [1,1,1,3] 4x4 -> 8 5.2 and 4.0,
+  // [1,7,7,3] 7x7 -> 64 33.5 and 6.1, [1,16,16,3] 5x5 -> 16 18.6 and 5.0, [2,60,60,3] 7x7 -> 8 26.1 and 6.8,
+  // [8,112,112,3] 7x7/2 -> 64 39.2 and 15.1). Eight-channel strips of at most one workgroup of pixels stay with it, slower
+  // too ([1,12,12,3] 5x5 -> 8 13.8 and 4.9): the tests hold its way with a filter of many taps there.
+  const bool lane_per_pixel = K <= kMaxTaps || (M <= 256 && out_c % 16 != 0);
   if (!nchw && in_c <= 4 && out_c % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
-      p.epi.channel_operands && activation <= TFHIP_RELU6 && (K <= kMaxTaps || M <= 256)) {
+      p.epi.channel_operands && activation <= TFHIP_RELU6 && lane_per_pixel) {
     const bool few_taps = K <= kMaxTaps && M < lim - 256 && p.a_bytes != 0;
     // 32 channels per wavefront when there are pixels enough to fill the chip that
     // way, else 16 (twice the wavefronts)
