@@ -409,3 +409,13 @@ for hw, c, f, out_c, want in [(1, 3, 4, 16, "gemm_kernel<"), (16, 3, 5, 16, "gem
     check(lib.tfhip_last_kernel(name, 256))
     assert name.value.decode().startswith(want), (hw, c, f, out_c, name.value)
 """)
+
+
+def test_predict_replays_up_to_the_batch_where_it_pays():
+    fake_hip_util.run(MODEL + """
+for batch, replays in [(8, True), (9, False)]:
+    model.close()
+    model = workloads.DeviceMobileNetV2(folder, batch)
+    model.set_input(np.zeros((batch, 224, 224, 3), np.float32))
+    assert not predict() and predict() == replays and predict() == replays
+""")

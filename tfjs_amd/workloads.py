@@ -228,7 +228,7 @@ class DeviceMobileNetV2:
     load (quantized shard uploaded once, one dequant kernel per tensor) and every
     activation stays in pooled device buffers between kernels."""
 
-    _REPLAY_BATCH = 10   # largest batch whose launches predict() replays (see there)
+    _REPLAY_BATCH = 8   # largest batch whose launches predict() replays (see there)
 
     def __init__(self, model_dir, batch, fuse_residual_add=True, fuse_expand_depthwise=True, fuse_blocks=True):
         from . import pyhost
@@ -532,10 +532,13 @@ class DeviceMobileNetV2:
         """forward + download of the logits, the reference's definition of one
         timed inference (e2e/benchmarks/benchmark_util.js:246-286). The launches of a model are the
         same at every call (unless a buffer is exchanged or a knob set, which is looked at), so from
-        its second call on they are replayed as one recorded sequence: enqueueing them one by one from Python takes 300 us, more than
-        the GPU needs for a few pictures. Larger batches keep the host ahead anyway, and a recording
-        holds activation buffers of its own: with three models in turn, batch 8 takes 304 us
-        replayed and 313 launched, batch 16 392 and 368."""
+        its second call on they are replayed as one recorded sequence: enqueueing them one by one
+        from Python takes 300 us, more than the GPU needs for a few pictures. Larger batches keep the
+        host ahead anyway, and a recording holds activation buffers of its own, which costs a program
+        with several models their cache: the line is where a replay still pays for both (us, replayed
+        and launched, one model | three in turn: batch 6 263 and 304 | 265 and 306, 8 284 and 293 |
+        290 and 303, 9 298 and 308 | 311 and 305, 10 306 and 312 | 321 and 309, 12 333 and 333 |
+        354 and 331, 16 365 and 368 | 389 and 365)."""
         if self._graph is None and self._ran and self.batch <= self._REPLAY_BATCH:
             self._record()
         if self._graph is not None:
