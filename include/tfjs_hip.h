@@ -147,8 +147,8 @@ int tfhip_graph_destroy(int graph_id);
  *   "skinny_regs" (0: the streaming GEMM always stages B in LDS), "fuse_pw_dw"
  *   (tfhip_pointwise_depthwise_pays: 1: yes for every shape the fused kernel
  *   takes, 0: never), "pw_dw_tile" (1 / 0: the channel-sliced / the row-ring
- *   pointwise + depthwise kernel where both take a shape), "tile_slice" (32 / 48 /
- *   64 channels per workgroup of the channel-sliced kernel), "tile_chunks" (its row
+ *   pointwise + depthwise kernel where both take a shape), "tile_slice" (16 / 32 /
+ *   48 / 64 channels per workgroup of the channel-sliced kernel), "tile_chunks" (its row
  *   chunks per image), "block_rows" (output rows per workgroup of the whole-block
  *   kernel), "fuse_block" (tfhip_inverted_residual_pays: 1 always, 0 never), "k_groups" (1 / 2 / 4
  *   groups of wavefronts that share a GEMM tile and split its k loop), "pw_dw_stream"
@@ -192,8 +192,9 @@ int tfhip_fused_matmul(const float *a, const float *b, float *out,
  * partial sums: not in the library's growing workspace but in a static device
  * array of TFHIP_NOALLOC_SCRATCH_BYTES that each GPU holds until the process
  * ends. The call makes no hipMalloc / hipFree. When the slices the library
- * would choose (at most 8, and 1 whenever the tiles already fill the GPU or K
- * is short) need more than the array (slices x batch x M x N x 4 bytes), it
+ * would choose (1 whenever the tiles already fill the GPU or K is short; at
+ * most 8 of the tiled kernel, and never more than 2 MiB of the kernel for few
+ * rows) need more than the array (slices x batch x M x N x 4 bytes), it
  * takes the largest number of slices that fits, down to one slice, which needs
  * no scratch: the result then has tfhip_fused_matmul's bits only where the two
  * slice counts agree, and is within the float32 bound otherwise. A slice count

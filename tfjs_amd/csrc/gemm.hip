@@ -139,10 +139,10 @@ extern "C" int tfhip_fused_matmul_noalloc(const float *a, const float *b, float 
   if (ptr == nullptr)
     return fail(kHipError, "tfhip_fused_matmul_noalloc: the static scratch array was not resolved on device %d",
                 device_index());
-  // Same kernels and the same choice of K slices as tfhip_fused_matmul; only the
-  // home of the partial sums differs, so the two agree bit for bit. Nothing needs
-  // clearing between calls: every slab element that gemm_finish reads was written
-  // by this call's gemm_kernel.
+  // Same kernels and the same choice of K slices as tfhip_fused_matmul (fewer where they do not fit); only the home of
+  // the partial sums differs. Nothing needs clearing between calls: every element that gemm_finish or the last
+  // workgroup of a few_rows tile reads was written by this call's own kernel, and the counters of few_rows are zero
+  // between launches. Its slices never take more than 2 MiB (256 tiles x slices of at most 32 x 64).
   FixedWorkspace fixed(ptr, TFHIP_NOALLOC_SCRATCH_BYTES);
   return fused_matmul_impl("tfhip_fused_matmul_noalloc", a, b, out, batch_a, batch_b, M, N, K, transpose_a,
                            transpose_b, bias, bias_strides, activation, prelu_weights, prelu_strides,
