@@ -320,6 +320,8 @@ int decode_group(DecodeGroup &group, char *temporary) {
 // `tensors` with their blocks (`out`) allocated, at `offsets` of `host`.
 int decode_all(const char *host, const std::vector<BatchEntry> &tensors, const int64_t *offsets) {
   std::vector<DecodeGroup> groups(1);
+  groups[0].entries.reserve(tensors.size());   // (nearly always the only one)
+  groups[0].code_at.reserve(tensors.size());
   for (size_t i = 0; i < tensors.size(); ++i) {
     const BatchEntry &e = tensors[i];
     const size_t bytes = uploads_alone(e) ? 0 : (size_t)e.n * code_bytes(e.kind);
