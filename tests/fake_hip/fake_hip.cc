@@ -45,7 +45,7 @@ std::vector<Launch> launches;
 thread_local int current_device = 0;
 int errors = 0;
 std::string first_error;
-std::atomic<int> copy_delay_us{0};
+std::atomic<int> copy_delay_us{0}, launch_delay_us{0};
 std::atomic<int> copies_now{0};
 std::map<hipStream_t, int> stream_device;
 thread_local struct {
@@ -136,6 +136,7 @@ int fake_hip_device_of(const void *p) {
   return inside_locked(p, 1, &b) ? b.device : -1;
 }
 void fake_hip_copy_delay(int us) { copy_delay_us = us; }
+void fake_hip_launch_delay(int us) { launch_delay_us = us; }
 
 // ---- devices, memory ----
 hipError_t hipGetDeviceCount(int *n) { *n = kDevices; return hipSuccess; }
@@ -216,6 +217,7 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t stream) {
+  if (launch_delay_us) usleep(launch_delay_us);
   std::lock_guard<std::recursive_mutex> lock(m);
   const std::string name = kernel_names[f];
   std::vector<long long> words;

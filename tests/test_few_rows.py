@@ -156,3 +156,31 @@ def test_a_cut_product_after_shutdown_and_init(lib):
         pyhost.shutdown()
         pyhost.init(0)
     np.testing.assert_array_equal(bits[0], bits[1])
+
+
+def test_two_threads_multiply_at_once(lib):
+    """Products that are cut, on this kernel (1 x 4095 x 64, 24 x 3000 x 2100) and on the tiled one with a pass that adds the
+    slices (300 x 2600 x 260): every thread gets its own, bit for bit."""
+    from concurrent.futures import ThreadPoolExecutor
+    sets = [[_Product(lib, m, n, k, "relu") for m, n, k in ((1, 64, 4095), (24, 2100, 3000), (300, 260, 2600))] for _ in range(2)]
+    want = []
+    for p in sets[0]:
+        p.launch()
+        want.append(p.result().view(np.uint32))
+
+    def serve(products):
+        got = []
+        for i in range(30):
+            p = products[i % 3]
+            p.launch()
+            got.append((i % 3, p.result().view(np.uint32)))
+        return got
+
+    try:
+        with ThreadPoolExecutor(2) as pool:
+            for done in [pool.submit(serve, products) for products in sets]:
+                for i, got in done.result():
+                    np.testing.assert_array_equal(got, want[i])
+    finally:
+        for p in sets[0] + sets[1]:
+            p.free()

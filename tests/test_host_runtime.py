@@ -419,3 +419,28 @@ for batch, replays in [(8, True), (9, False)]:
     model.set_input(np.zeros((batch, 224, 224, 3), np.float32))
     assert not predict() and predict() == replays and predict() == replays
 """)
+
+
+def test_two_threads_keep_their_partial_sums_apart():
+    """Products that are cut keep their sums in one block: from the moment a launch is given it until its last kernel
+    is enqueued no other launch uses or outgrows it."""
+    fake_hip_util.run("""
+from concurrent.futures import ThreadPoolExecutor
+pyhost.init()
+a, b, out = (DeviceBuffer(32 << 20) for _ in range(3))
+check(lib.tfhip_set_tuning(b"splitk", 4))
+fake.fake_hip_launch_delay(2000)
+
+def product(n):      # gemm_kernel, then gemm_finish; a larger block each time
+    check(lib.tfhip_fused_matmul(a.ptr, b.ptr, out.ptr, 1, 1, 1024, n, 512, 0, 0, None, None, 0, None, None, 0.2))
+
+before = fake.fake_hip_launches()
+with ThreadPoolExecutor(2) as pool:
+    for done in [pool.submit(product, n) for n in (256, 1024, 2048, 3072, 512, 4096, 1536, 768)]:
+        done.result()
+names = [launch(i)[0] for i in reversed(range(fake.fake_hip_launches() - before))]
+assert len(names) == 16
+for first, second in zip(names[::2], names[1::2]):
+    assert "gemm_kernel" in first and "gemm_finish" in second, names
+assert errors()[0] == 0, errors()
+""")

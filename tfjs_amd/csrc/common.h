@@ -7,6 +7,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <mutex>
 #include <tuple>
 #include <utility>
 
@@ -33,6 +34,9 @@ int num_cus();
 int device_index();        // the device tfhip_init was given
 // Device scratch of at least `bytes` (nullptr if it cannot be allocated); valid until the next call.
 void *workspace(size_t bytes);
+// Held from the call of workspace() until the last kernel that uses the block is enqueued: another thread's launches
+// must neither come in between, with sums of their own, nor outgrow the block.
+std::unique_lock<std::mutex> lock_workspace();
 // While a FixedWorkspace object lives, workspace() hands the thread that made it
 // the caller's block instead of the library's growing one and allocates nothing:
 // a request beyond `bytes` returns nullptr, and workspace_is_fixed() tells a

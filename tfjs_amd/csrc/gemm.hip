@@ -53,7 +53,9 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
   q.row_tiles = cut.row_tiles;
   q.splits = 1;
   q.groups_per_split = q.groups;
+  std::unique_lock<std::mutex> held;
   if (cut.splits > 1) {
+    held = lock_workspace();
     q.ws = static_cast<float *>(workspace((size_t)cut.tiles * cut.splits * 256 * MB * CB * sizeof(float)));
     if (q.ws) {
       q.splits = cut.splits;

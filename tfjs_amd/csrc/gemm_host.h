@@ -84,6 +84,7 @@ inline int launch_gemm(GemmParams &p) {
   // copy of the tile set sums a slice of k into the workspace and gemm_finish
   // adds the slices. Time model (us): fixed + k tiles on the busiest compute unit
   // x tile time, plus the second kernel.
+  std::unique_lock<std::mutex> held;
   p.splits = 1;
   p.k_per_split = p.K;
   p.ws = nullptr;
@@ -125,6 +126,7 @@ inline int launch_gemm(GemmParams &p) {
     }
     if (best > 1) {
       const size_t bytes = (size_t)best * slice_bytes;
+      held = lock_workspace();
       float *ws = bytes <= (size_t(1) << 30) ? static_cast<float *>(workspace(bytes)) : nullptr;
       if (ws) {
         p.splits = best;

@@ -213,6 +213,9 @@ FixedWorkspace::~FixedWorkspace() {
 bool workspace_is_fixed() { return g_ws_fixed; }
 size_t fixed_workspace_bytes() { return g_fixed_ws_bytes; }
 
+std::mutex g_workspace_mutex;
+std::unique_lock<std::mutex> lock_workspace() { return std::unique_lock<std::mutex>(g_workspace_mutex); }
+
 void *workspace(size_t bytes) {
   if (g_ws_fixed) return bytes <= g_fixed_ws_bytes ? g_fixed_ws : nullptr;
   if (bytes <= g.workspace_bytes) return g.workspace;
