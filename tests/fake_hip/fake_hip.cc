@@ -136,6 +136,7 @@ int fake_hip_device_of(const void *p) {
   return inside_locked(p, 1, &b) ? b.device : -1;
 }
 void fake_hip_copy_delay(int us) { copy_delay_us = us; }
+int fake_hip_copies_now(void) { return copies_now; }
 void fake_hip_launch_delay(int us) { launch_delay_us = us; }
 
 // ---- devices, memory ----

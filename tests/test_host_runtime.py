@@ -287,7 +287,8 @@ def download():
     return lib.tfhip_download(out.ctypes.data, buf.ptr, 0, out.nbytes), lib.tfhip_last_error()
 with ThreadPoolExecutor(3) as pool:
     first = pool.submit(upload)
-    time.sleep(0.04)
+    while not fake.fake_hip_copies_now():
+        time.sleep(0.001)
     waiting = [pool.submit(upload), pool.submit(download)]
     time.sleep(0.04)
     check(lib.tfhip_shutdown())
