@@ -445,7 +445,7 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
     if (units * g.units < (int64_t(1) << 32) && in_h * in_w * in_c < lim && dilation_h * in_w * in_c < lim &&
         (f_h - 1) * dilation_h * in_w * in_c + f_w * dilation_w * in_c < lim && stride_w * out_w * in_c < lim && pad_left * in_c < lim) {
       p.K = (int)(4 * units);
-      const int row_blocks = few_rows_blocks(p, true);
+      const int row_blocks = few_rows_blocks(p, true, vec);
       if (row_blocks) return launch_few_rows(p, row_blocks, vec ? kLoadWindows : kLoadWindowsAny);
       const int shape = choose_tile_shape(M, out_c, p.K, 1, num_cus());
       if (vec) return launch_gemm_shape<kLoadWindows, kLoadXVec>(shape, p);

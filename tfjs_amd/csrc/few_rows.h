@@ -301,24 +301,28 @@ inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
 }
 
 // Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
-// tiled kernel. As long as every workgroup has a compute unit of its own, the fetches of a whole k range are out at once,
-// where the tiled kernel goes round its pipeline once per 32 k (us, tiled and here: 49 x 960 x 160 9.2 and 5.6,
-// 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7; windows, [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1). The lines,
-// each from a grid of extents on both sides, in the same form:
+// tiled kernel (`vec`: that one can fetch both operands in float4s). As long as every workgroup has a compute unit of its
+// own, the fetches of a whole k range are out at once, where the tiled kernel goes round its pipeline once per 32 k (us,
+// tiled and here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7; windows,
+// [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1). The lines, each from a grid of extents on both sides, in the same form:
 //  * more than 32 rows, K < 320: the tiled kernel is ahead up to 128 (33 x 64 x 32 3.3 and 3.9), then the two are
 //    within 10% of each other (100 x 256 x 96 4.7 and 4.2).
 //  * windows of fewer than 384 floats: behind at 144 ([1,7,7,16] 3x3 -> 32 4.4 and 4.8); ahead from 297 on
 //    ([1,14,14,33] 3x3 -> 64 7.7 and 5.9), so the line is on the safe side.
 //  * up to 32 rows always, from K = 2048 on with two row blocks: half the fetches of B, and slices enough to fill the
-//    chip (23 x 3072 x 768 9.3 with one, 7.7 with two). Except 17 to 32 rows of 4097 to 8192 columns with K <= 1536:
-//    more strips than compute units, while each of the tiled kernel's 32-wide tiles has one (32 x 512 x 8192 6.4 and
-//    8.3, 32 x 1024 x 5000 8.9 and 11.2; 32 x 2048 x 5000 14.2 and 14.2, 32 x 1024 x 12288 17.9 and 13.9).
+//    chip (23 x 3072 x 768 9.3 with one, 7.7 with two). Except 17 to 32 rows of 4097 to 8192 columns with K <= 1536
+//    (where a float4 fits the rows, else 768): more strips than compute units, while each of the tiled kernel's 32-wide tiles
+//    has one (32 x 512 x 8192 6.4 and 8.3, 32 x 1024 x 5000 8.9 and 11.2; 32 x 2048 x 5000 14.2 and 14.2,
+//    32 x 1024 x 12288 17.9 and 13.9; ragged, 32 x 511 x 5001 7.3 and 8.4, 24 x 768 x 5001 9.3 and 9.5,
+//    24 x 1280 x 5001 13.4 and 10.6).
 //  * more than 32 rows with two row blocks, K <= 1536: 128 x 1024 x 1024 9.1 and 7.5, 128 x 1536 x 768 12.8 and 10.1;
 //    128 x 3072 x 768 13.8 and 16.8. (128 x 1792 x 768, 14.4 and 11.4, is left on the wrong side.)
-//  * windows have no strips of 64: with a workgroup on a third of the compute units and more, and more than 192 groups for
-//    it, the tiled kernel is ahead ([1,10,10,256] 5x5 -> 256 14.5 and 15.4, [1,14,14,256] 7x7 -> 256 30.5 and 39.7; on
-//    64 tiles [1,7,7,256] 7x7 -> 256 21.0 and 13.8; at 144 groups [1,10,10,512] 3x3 -> 256 12.8 and 13.0).
-inline int few_rows_blocks(const GemmParams &p, bool windows) {
+//  * windows have no strips of 64: with two strips and more, a workgroup on a third of the compute units and more, and
+//    more than 192 groups for it (288 where the tiled kernel's loader has units to mend), the tiled kernel is ahead
+//    ([1,10,10,256] 5x5 -> 256 14.5 and 15.4, [1,14,14,256] 7x7 -> 256 30.5 and 39.7; on 64 tiles [1,7,7,256] 7x7 -> 256
+//    21.0 and 13.8; at 144 groups [1,10,10,512] 3x3 -> 256 12.8 and 13.0; of one strip [3,34,19,260] 7x7 -> 8 30.7 and
+//    22.6; ragged, at 222 groups [3,33,22,141] 5x5/2 -> 111 22.2 and 20.3, at 399 [1,20,20,130] 7x7 -> 130 24.0 and 29.7).
+inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
   if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
   if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
       tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
@@ -329,11 +333,11 @@ inline int few_rows_blocks(const GemmParams &p, bool windows) {
   else if (p.M > 32 && p.K < 320 && !windows) blocks = 0;
   else if (p.M <= 32 && p.K > 2048) blocks = 2;
   else if ((p.M + 15) / 16 * strips <= cus) blocks = 1;
-  else if (p.M <= 32) blocks = strips > cus && strips <= 2 * cus && p.K <= 1536 ? 0 : 2;
+  else if (p.M <= 32) blocks = strips > cus && strips <= 2 * cus && p.K <= (vec ? 1536 : 768) ? 0 : 2;
   else if ((p.M + 31) / 32 * strips <= cus && p.K <= 1536) blocks = 2;
   if (windows && blocks != 0) {
     const FewRowsCut cut = few_rows_cut(p, blocks, 1);
-    if (cut.tiles * 3 > cus && cut.groups_per_split > 192) blocks = 0;
+    if (strips > 1 && cut.tiles * 3 > cus && cut.groups_per_split > (vec ? 192 : 288)) blocks = 0;
   }
   return blocks;
 }

@@ -9,7 +9,7 @@ using namespace tfhip;
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
   if (!transpose_a && !transpose_b) {
-    const int row_blocks = few_rows_blocks(p, false);
+    const int row_blocks = few_rows_blocks(p, false, vec);
     if (row_blocks) return launch_few_rows(p, row_blocks, kLoadKAny);
   }
   if (vec) {
