@@ -225,7 +225,7 @@ def mobilenet_v2_flops_per_image():
 
 class DeviceMobileNetV2:
     """MobileNetV2 resident on the GPU: weights are dequantized on the device at
-    load (quantized shard uploaded once, one dequant kernel per tensor) and every
+    load (quantized shard uploaded once, decoded by one launch) and every
     activation stays in pooled device buffers between kernels."""
 
     _REPLAY_BATCH = 8   # largest batch whose launches predict() replays (see there)
