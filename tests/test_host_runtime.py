@@ -380,12 +380,15 @@ def windows(hw, c, f, out_c):
     return label()
 
 for shape, want in {
-    (1, 4096, 2048): "few_rows<1, 1", (1, 4000, 2049): "few_rows<1, 4", (1, 4096, 1024): "few_rows<1, 1", (1, 4097, 1024): "few_rows<1, 4",
-    (16, 2048, 4096): "few_rows<1, 1", (16, 2048, 4097): "few_rows<1, 4", (17, 2304, 1536): "few_rows<2, 1",
-    (17, 2304, 2049): "few_rows<2, 4", (32, 4096, 1536): "few_rows<2, 1", (32, 4096, 1537): "few_rows<2, 4", (32, 4100, 1536): "gemm_kernel<",
-    (32, 4100, 1540): "few_rows<2, 4", (32, 4097, 768): "gemm_kernel<", (32, 4097, 769): "few_rows<2, 4", (32, 8192, 1536): "gemm_kernel<", (32, 8193, 1024): "few_rows<2, 4", (33, 64, 319): "gemm_kernel<",
-    (33, 64, 320): "few_rows<1, 1", (64, 1024, 2048): "few_rows<1, 1", (64, 1024, 2049): "few_rows<1, 4", (160, 256, 8192): "few_rows<1, 4",
-    (128, 768, 1536): "few_rows<2, 1", (128, 768, 1540): "gemm_kernel<", (257, 256, 320): "few_rows<2, 1", (513, 256, 320): "gemm_kernel<",
+    (1, 4096, 2048): "few_rows<1, 1", (1, 4000, 2049): "few_rows<1, 4", (1, 4096, 1024): "few_rows<1, 1",
+    (1, 4097, 1024): "few_rows<1, 4", (16, 2048, 4096): "few_rows<1, 1", (16, 2048, 4097): "few_rows<1, 4",
+    (17, 2304, 1536): "few_rows<2, 1", (17, 2304, 2049): "few_rows<2, 4", (32, 4096, 1536): "few_rows<2, 1",
+    (32, 4096, 1537): "few_rows<2, 4", (32, 4100, 1536): "gemm_kernel<", (32, 4100, 1540): "few_rows<2, 4",
+    (32, 4097, 768): "gemm_kernel<", (32, 4097, 769): "few_rows<2, 4", (32, 8192, 1536): "gemm_kernel<",
+    (32, 8193, 1024): "few_rows<2, 4", (33, 64, 319): "gemm_kernel<", (33, 64, 320): "few_rows<1, 1",
+    (64, 1024, 2048): "few_rows<1, 1", (64, 1024, 2049): "few_rows<1, 4", (160, 256, 8192): "few_rows<1, 4",
+    (128, 768, 1536): "few_rows<2, 1", (128, 768, 1540): "gemm_kernel<", (257, 256, 320): "few_rows<2, 1",
+    (513, 256, 320): "gemm_kernel<",
 }.items():
     assert product(*shape).startswith(want), (shape, product(*shape), want)
 for shape, want in {(14, 41, 3, 16): "gemm_kernel<", (14, 42, 3, 16): "few_rows<1, 1", (7, 256, 7, 256): "few_rows<1, 1",
