@@ -1,0 +1,136 @@
+"""The kernel that multiplies float32 operands in bf16 parts (split_gemm), on every tile it has: edges of tiles, of k tiles and
+of the groups that share k; windows of both kinds; epilogues; operands that six partial products cannot multiply."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tfjs_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = range(8)
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from tfjs_amd import pyhost
+    pyhost.init()
+    return pyhost
+
+
+@pytest.fixture(scope="module")
+def orc():
+    from oracle import pyoracle
+    return pyoracle
+
+
+@pytest.fixture
+def split():
+    """Sets the tile; unset afterwards."""
+    lib = capi.load_library()
+
+    def force(shape):
+        capi.check(lib.tfhip_set_tuning(b"split", shape))
+    yield force
+    capi.check(lib.tfhip_set_tuning(b"split", -1))
+
+
+def _took_it():
+    name = ctypes.create_string_buffer(256)
+    capi.load_library().tfhip_last_kernel(name, 256)
+    return name.value.decode().startswith("split_gemm<")
+
+
+def _bound(a, b, k):
+    """What a result may be off, per result: one rounding of the accumulator (truncated: an ulp, 2^-23) per matrix instruction
+    of 16 k and per wavefront group, eight more for the small products, the bias and the store, and 2^-25 of each product
+    for the parts left out; all relative to the sum of the products' sizes."""
+    return ((k / 16 + 12) * 2.0 ** -23 + 2.0 ** -25) * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 1e-37
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (33, 31, 33), (64, 64, 64), (65, 33, 257), (128, 128, 32), (129, 130, 131), (300, 97, 100),
+                                   (257, 193, 320), (40, 3, 65), (31, 250, 1000)])
+def test_products(hip, split, shape, m, n, k):
+    rng = np.random.default_rng(m * n + k)
+    a, b = rng.standard_normal((2, m, k)).astype(np.float32), rng.standard_normal((2, k, n)).astype(np.float32)
+    split(shape)
+    got = hip.batch_matmul(a, b)
+    assert _took_it()
+    assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= _bound(a, b, k)).all()
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("slices", [2, 3, 8])
+@pytest.mark.parametrize("m,n,k", [(70, 64, 1300), (33, 97, 2049)])
+def test_slices_of_k(hip, split, shape, slices, m, n, k):
+    rng = np.random.default_rng(slices)
+    a, b = rng.standard_normal((1, m, k)).astype(np.float32), rng.standard_normal((1, k, n)).astype(np.float32)
+    split(shape + 10 * (slices - 1))
+    got = hip.batch_matmul(a, b)
+    assert _took_it() and hip.workspace_info()["last_splits"] == slices
+    assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= _bound(a, b, k)).all()
+
+
+@pytest.mark.parametrize("act", ["linear", "relu", "relu6", "prelu", "leakyrelu", "sigmoid", "elu"])
+@pytest.mark.parametrize("n,tile", [(64, 6), (97, 6), (64, 23), (97, 23)])   # (23: in three slices)
+def test_epilogues(hip, orc, split, act, n, tile):
+    rng = np.random.default_rng(n)
+    a, b = rng.uniform(-1, 1, (1, 150, 90)).astype(np.float32), rng.uniform(-1, 1, (1, 90, n)).astype(np.float32)
+    for bias in (rng.uniform(-1, 1, (n,)).astype(np.float32), rng.uniform(-1, 1, (150, 1)).astype(np.float32), None):
+        kw = dict(bias=bias, activation=act, leakyrelu_alpha=0.3)
+        if act == "prelu":
+            kw["prelu"] = rng.uniform(-1, 1, (n,)).astype(np.float32)
+        split(tile)
+        got = hip.fused_matmul(a, b, **kw)
+        want = orc.fused_matmul(a, b, **kw)
+        assert np.max(np.abs(got - want)) <= 2e-5   # 90 products of at most 1 in another order, 2^-23 each
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("xs,fs,stride,dil,pad", [
+    ((2, 13, 11, 8), (3, 3, 8, 24), 1, 1, "same"), ((1, 20, 21, 4), (5, 5, 4, 36), 2, 1, "same"),
+    ((2, 13, 11, 5), (3, 3, 5, 7), 1, 1, "same"), ((2, 17, 3, 2), (3, 7, 2, 130), 1, 1, "same"),
+    ((1, 9, 9, 12), (3, 3, 12, 20), 1, 2, "valid"), ((1, 31, 30, 6), (5, 5, 6, 16), 1, 1, [[0, 0], [3, 0], [0, 3], [0, 0]]),
+    ((3, 40, 40, 33), (1, 1, 33, 23), 2, 1, "same"),
+])
+def test_windows(hip, orc, split, shape, xs, fs, stride, dil, pad):
+    rng = np.random.default_rng(sum(xs) + sum(fs))
+    x = rng.uniform(-1, 1, xs).astype(np.float32)
+    w = rng.uniform(-1, 1, fs).astype(np.float32)
+    kw = dict(strides=stride, dilations=dil, pad=pad, bias=rng.uniform(-1, 1, (fs[3],)).astype(np.float32), activation="relu6")
+    split(shape)
+    got = hip.fused_conv2d(x, w, **kw)
+    assert _took_it()
+    k = fs[0] * fs[1] * fs[2]
+    assert np.max(np.abs(got - orc.fused_conv2d(x, w, **kw))) <= k * (k / 16 + 12) * 2.0 ** -23 + k * 2.0 ** -24
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_what_parts_cannot_multiply(hip, split, shape):
+    m, n, k = 140, 136, 200
+    rng = np.random.default_rng(9)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    a[3, 7], a[5, 11], a[5, 12], a[8, 199] = np.inf, np.inf, -np.inf, np.nan
+    a[20, :] = 0
+    a[20, 40] = np.float32(3.4028235e38)              # rounds to Inf in bf16
+    b[9, 70], b[50, 71] = -np.inf, np.nan
+    a[30, :] *= np.float32(1e-35)                     # last parts below the smallest bf16, results too
+    b[:, 80] = np.float32(2.0)                        # with Inf in a: Inf, though the lower parts are zero
+    a[40, :] = np.float32(1e-39)                      # subnormal
+    split(shape)
+    with np.errstate(all="ignore"):
+        got = hip.batch_matmul(a[None], b[None])[0]
+        assert _took_it()
+        want = (a.astype(np.float64)[:, :, None] * b.astype(np.float64)[None]).sum(1).astype(np.float32)
+    assert (np.isnan(got) == np.isnan(want)).all()
+    inf = np.isinf(want) & (np.arange(m) != 20)[:, None]   # (row 20 may pass the largest float on the way)
+    assert (got[inf] == want[inf]).all()
+    fine = np.isfinite(want) & np.isfinite(got)
+    assert (fine == np.isfinite(want))[np.arange(m) != 20].all()
+    got, want = np.where(fine, got, 0), np.where(fine, want, 0)
+    size = np.nan_to_num(np.abs(a), posinf=0, neginf=0).astype(np.float64) @ np.nan_to_num(np.abs(b), posinf=0, neginf=0).astype(np.float64)
+    assert (np.abs(got.astype(np.float64) - want) <= (k * 2.0 ** -24 + 2.0 ** -20) * size + 2.0 ** -149 * k).all()
+    # tiny rows keep float32's precision
+    assert (np.abs(got[30] - want[30]) <= k * 2.0 ** -24 * size[30]).all()

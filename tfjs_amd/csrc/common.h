@@ -196,7 +196,7 @@ int launch_repeat();
   X(PwDwTile, "pw_dw_tile") X(TileSlice, "tile_slice") X(TileChunks, "tile_chunks")                         \
   X(FuseBlock, "fuse_block") X(KGroups, "k_groups") X(PwDwStream, "pw_dw_stream")                           \
   X(StreamRows, "stream_rows") X(StreamBlocks, "stream_blocks") X(SkinnyStage, "skinny_stage")              \
-  X(BlockRows, "block_rows")
+  X(BlockRows, "block_rows") X(Split, "split")
 enum TuningKey {
 #define TFHIP_TUNING_ENUM(id, name) kTune##id,
   TFHIP_TUNING_KNOBS(TFHIP_TUNING_ENUM)

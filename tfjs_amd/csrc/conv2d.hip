@@ -409,7 +409,9 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
                          pad_left == 0 && out_h == in_h && out_w == in_w;
   if (pointwise) {
     p.a_sx = in_c; p.a_sk = 1;
-    return launch_plain_gemm(p, false, false, vec);
+    // The kernels that fuse an expansion with the depthwise stage behind it (up to 160 input channels) multiply in float32:
+    // a model gives the same bits with and without that fusion.
+    return launch_plain_gemm(p, false, false, vec, in_c <= 160);
   }
   // More taps than the matrix-core form holds: the GEMM-shaped kernels, which gather whole filter rows, where a lane that
   // walks K taps on its own is 1.3 to 14 times slower (us, lane per pixel and gathered: [1,1,1,3] 4x4 -> 8 5.2 and 4.0,
@@ -447,6 +449,9 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
       p.K = (int)(4 * units);
       const int row_blocks = few_rows_blocks(p, true, vec);
       if (row_blocks) return launch_few_rows(p, row_blocks, vec ? kLoadWindows : kLoadWindowsAny);
+      const int a_kind = vec ? kLoadWindows : kLoadWindowsAny;
+      const SplitChoice split = split_gemm_choice(p, a_kind);
+      if (split.shape >= 0) return launch_split_gemm(split, p, a_kind);
       const int shape = choose_tile_shape(M, out_c, p.K, 1, num_cus());
       if (vec) return launch_gemm_shape<kLoadWindows, kLoadXVec>(shape, p);
       return launch_gemm_shape<kLoadWindowsAny, kLoadFilter>(shape, p);

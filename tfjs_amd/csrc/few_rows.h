@@ -325,7 +325,7 @@ inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
 inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
   if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
   if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
-      tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
+      tuning(kTuneSplit) >= 0 || tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
     return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();
   int blocks = 0;

@@ -6,11 +6,13 @@
 
 using namespace tfhip;
 
-int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec) {
+int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec, bool float_bits) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
   if (!transpose_a && !transpose_b) {
     const int row_blocks = few_rows_blocks(p, false, vec);
     if (row_blocks) return launch_few_rows(p, row_blocks, kLoadKAny);
+    const SplitChoice split = split_gemm_choice(p, kLoadKAny);
+    if (split.shape >= 0 && !float_bits) return launch_split_gemm(split, p, kLoadKAny);
   }
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());

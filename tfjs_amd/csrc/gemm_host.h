@@ -73,6 +73,31 @@ inline int choose_tile_shape(long long M, long long N, long long K, long long ba
   return best;
 }
 
+// Tile rows per panel of the tile numbering: ids resident together on one XCD are its share of the grid, at most two
+// workgroups on each of its 32 compute units, and cover a near-square block of C.
+inline int tile_rows_per_panel(long long grid, int bm, int bn, int tiles_m) {
+  const long long per_xcd = grid / 8 < 1 ? 1 : grid / 8;
+  const double together = (double)(per_xcd < 64 ? per_xcd : 64);
+  int g = (int)(sqrt(together * bn / bm) + 0.5);
+  g = g < 1 ? 1 : g;
+  return g > tiles_m ? tiles_m : g;
+}
+
+// Enqueues what completes a product that its kernel left as raw sums or slabs.
+inline void enqueue_finish(const GemmParams &p) {
+  const long long total = (long long)p.M * p.N * p.batch;
+  // (the residual lies like the output; a caller need not have aligned it like that)
+  const bool rows = p.splits > 1 && p.splits <= 8 && p.vec_store && p.epi.addressing == kChannel && p.ldc == p.N &&
+                    p.c_batch_stride == (p.batch > 1 ? (long long)p.M * p.N : p.c_batch_stride) && total < (1LL << 31) &&
+                    reinterpret_cast<uintptr_t>(p.epi.residual) % 16 == 0;
+  if (rows) {
+    gemm_finish_rows<<<dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream()>>>(p);
+    return;
+  }
+  const long long blocks = (total + 255) / 256, cap = (long long)num_cus() * 16;
+  gemm_finish<<<dim3((unsigned)(blocks < cap ? blocks : cap)), dim3(256), 0, stream()>>>(p);
+}
+
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int A_KIND, int B_KIND, int KG = 1>
 inline int launch_gemm(GemmParams &p) {
   using T = GemmTile<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>;
@@ -137,15 +162,7 @@ inline int launch_gemm(GemmParams &p) {
   }
   note_splits(p.splits);
   const long long grid = tiles * p.splits;
-  {
-    // ids resident together on one XCD: its share of the grid, at most two
-    // workgroups on each of its 32 compute units
-    const long long per_xcd = grid / 8 < 1 ? 1 : grid / 8;
-    const double together = (double)(per_xcd < 64 ? per_xcd : 64);
-    int g = (int)(sqrt(together * BN / BM) + 0.5);
-    g = g < 1 ? 1 : g;
-    p.group_m = g > p.tiles_m ? p.tiles_m : g;
-  }
+  p.group_m = tile_rows_per_panel(grid, BM, BN, p.tiles_m);
   if (grid > 0x7fffffffLL) return fail(kBadArgument, "gemm: %lld tiles exceed the grid limit", grid);
   if (T::LDS_FLOATS * sizeof(float) > 64 * 1024) {   // (also with KG groups of buffers)
     // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
@@ -166,13 +183,9 @@ inline int launch_gemm(GemmParams &p) {
     TFHIP_LAUNCH((gemm_kernel<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>
                   <<<dim3((unsigned)grid), dim3(256 * KG), T::LDS_FLOATS * sizeof(float), stream()>>>(p)));
   } else {
-    const long long total = (long long)p.M * p.N * p.batch;
-    long long blocks = (total + 255) / 256;
-    const long long cap = (long long)num_cus() * 16;
-    if (blocks > cap) blocks = cap;
     TFHIP_LAUNCH((gemm_kernel<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>
                   <<<dim3((unsigned)grid), dim3(256 * KG), T::LDS_FLOATS * sizeof(float), stream()>>>(p),
-                  gemm_finish<<<dim3((unsigned)blocks), dim3(256), 0, stream()>>>(p)));
+                  enqueue_finish(p)));
   }
   return kOk;
 }
@@ -225,10 +238,20 @@ inline int launch_gemm_shape(int shape, GemmParams &p) {
 // Plain (non-im2col) GEMM launch, defined once in gemm.hip: picks the loaders
 // for row-major / transposed operands; `vec` says both operands may be fetched
 // with float4 loads.
-int launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec);
+// `float_bits`: with float32 matrix instructions only.
+int launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec, bool float_bits = false);
 
 // The same for a row-major A (and a B of either kind) that cannot (gemm_ragged.hip).
 int launch_ragged_gemm(GemmParams &p, bool transpose_b);
+
+// The tile and the slices of k with which the kernel on the bf16 matrix cores (split_gemm.h) takes a product of a row-major B
+// and a row-major A or windows of an image; shape -1: it goes to gemm_kernel. Its launch; a_kind: kLoadKAny, kLoadWindows or
+// kLoadWindowsAny.
+struct SplitChoice {
+  int shape, slices;
+};
+SplitChoice split_gemm_choice(const GemmParams &p, int a_kind);
+int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind);
 
 // Fills the bias / prelu part of an Epilogue from caller strides over `rank`
 // output dims (3: batch,row,col; 4: n,h,w,c) after validating them. Sets

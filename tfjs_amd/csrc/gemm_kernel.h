@@ -154,6 +154,57 @@ __device__ __forceinline__ float4 as_float4(uint4_t v) {
   return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
 
+// Where window m begins: the image row, the float within it, and its byte offset in the image (a window that begins
+// before the image: exact modulo 2^32). Windows from X on get a row that no image has.
+__device__ __forceinline__ void window_row(const ConvGeom &g, int m, int X, int &ih, int &iw, unsigned &off) {
+  const int ow = m % g.out_w;
+  const int t2 = m / g.out_w;
+  const int oh = t2 % g.out_h, n = t2 / g.out_h;
+  const int first = oh * g.stride_h - g.pad_top;
+  ih = m < X ? first : -(1 << 28);
+  iw = ow * g.stride_wc - g.pad_leftc;
+  off = 4u * ((unsigned)n * (unsigned)g.image_len + (unsigned)(first * g.row_len) + (unsigned)iw);
+}
+
+// The unit of four k that begins at k, relative to where a window begins.
+struct WindowUnit {
+  int seg, in_seg;   // segment, and float within it
+  int dh, dl;        // image rows and floats of an image row further
+  unsigned at;       // bytes further
+};
+__device__ __forceinline__ WindowUnit window_unit(const ConvGeom &g, int k) {
+  WindowUnit u;
+  const int q = k >> 2;
+  u.seg = g.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)g.unit_magic) : q;
+  u.in_seg = 4 * (q - u.seg * g.units);
+  int fr = u.seg, fs = 0;
+  if (g.taps > 1) {
+    fr = u.seg / g.taps;
+    fs = u.seg - fr * g.taps;
+  }
+  u.dh = fr * g.dil_h;
+  u.dl = fs * g.seg_col + u.in_seg;
+  u.at = 4u * (unsigned)(fr * g.seg_row + u.dl);
+  return u;
+}
+
+// Fetches unit u of the window that begins at (ih, iw, off); `fix` tells fix_up what is not part of it.
+template <int KIND>
+__device__ __forceinline__ uint4_t load_window_unit(const ConvGeom &g, const WindowUnit &u, bool on, int ih, int iw, unsigned off,
+                                                    __amdgpu_buffer_rsrc_t rsrc, int &fix) {
+  const bool row_in = on && (unsigned)(ih + u.dh) < (unsigned)g.in_h;
+  const int lin = iw + u.dl;
+  if (KIND == kLoadWindows)   // in_c % 4 == 0: a unit lies inside the image row or outside
+    return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(row_in && (unsigned)lin < (unsigned)g.row_len ? off + u.at : kNoOffset), 0, 0);
+  // a unit may begin before the image row, or end behind it or its segment: fetched from the row's first float
+  // on in the one case, what does not belong goes when the unit is stored
+  const int before = lin < 0 ? -lin : 0;
+  const int real = min(g.row_len - lin, g.seg_len - u.in_seg);
+  fix = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
+  return __builtin_amdgcn_raw_buffer_load_b128(
+      rsrc, (int)(row_in && before < 4 && lin < g.row_len ? off + u.at + 4u * (unsigned)before : kNoOffset), 0, 0);
+}
+
 // Per-thread addressing state of one operand loader, fixed across k tiles.
 template <int VECS>
 struct LoaderState {
@@ -180,15 +231,7 @@ __device__ __forceinline__ void init_loader(LoaderState<VECS> &st, long long sx,
       const int x = x0 + (f / BK) * 4;   // consecutive lanes: consecutive k
       st.row_off[i] = x < X ? (unsigned)(x * 4) : kNoOffset;
     } else if (KIND == kLoadWindows || KIND == kLoadWindowsAny) {
-      const int m = x0 + f / (BK / 4);
-      const int ow = m % g.out_w;
-      const int t2 = m / g.out_w;
-      const int oh = t2 % g.out_h, n = t2 / g.out_h;
-      const int ih = oh * g.stride_h - g.pad_top;
-      st.row_ih[i] = m < X ? ih : -(1 << 28);   // (a row that no image has)
-      st.row_iw[i] = ow * g.stride_wc - g.pad_leftc;
-      // (a window that begins before the image: exact modulo 2^32)
-      st.row_off[i] = 4u * ((unsigned)n * (unsigned)g.image_len + (unsigned)(ih * g.row_len) + (unsigned)st.row_iw[i]);
+      window_row(g, x0 + f / (BK / 4), X, st.row_ih[i], st.row_iw[i], st.row_off[i]);
     } else if (KIND == kLoadIm2colScalar) {
       const int m = x0 + f / (BK / 4);
       if (m < X) {
@@ -239,32 +282,10 @@ __device__ __forceinline__ void load_tile(float4 (&reg)[VECS], int (&fix)[VECS],
     }
   } else if (KIND == kLoadWindows || KIND == kLoadWindowsAny) {
     const int k = k0 + (tid % (BK / 4)) * 4;
-    const int q = k >> 2;
-    const int seg = g.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)g.unit_magic) : q;
-    const int in_seg = 4 * (q - seg * g.units);
-    int fr = seg, fs = 0;
-    if (g.taps > 1) {
-      fr = seg / g.taps;
-      fs = seg - fr * g.taps;
-    }
-    const int dh = fr * g.dil_h, dl = fs * g.seg_col + in_seg;
-    const unsigned at = 4u * (unsigned)(fr * g.seg_row + dl);
+    const WindowUnit u = window_unit(g, k);
 #pragma unroll
     for (int i = 0; i < VECS; ++i) {
-      const bool row_in = k < K && (unsigned)(st.row_ih[i] + dh) < (unsigned)g.in_h;
-      const int lin = st.row_iw[i] + dl;
-      if (KIND == kLoadWindows) {   // in_c % 4 == 0: a unit lies inside the image row or outside
-        const unsigned off = row_in && (unsigned)lin < (unsigned)g.row_len ? st.row_off[i] + at : kNoOffset;
-        reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
-      } else {
-        // a unit may begin before the image row, or end behind it or its segment: fetched from the row's first float
-        // on in the one case, what does not belong goes when the unit is stored
-        const int before = lin < 0 ? -lin : 0;
-        const unsigned off = row_in && before < 4 && lin < g.row_len ? st.row_off[i] + at + 4u * (unsigned)before : kNoOffset;
-        reg[i] = as_float4(__builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0));
-        const int real = min(g.row_len - lin, g.seg_len - in_seg);
-        fix[i] = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
-      }
+      reg[i] = as_float4(load_window_unit<KIND>(g, u, k < K, st.row_ih[i], st.row_iw[i], st.row_off[i], rsrc, fix[i]));
     }
   } else if (KIND == kLoadFilter) {
     const int k = k0 + tid % BK;   // (256 % BK == 0: the same for every i)
@@ -769,6 +790,35 @@ static __global__ __launch_bounds__(256) void gemm_finish(GemmParams p) {
     v = finish(e, v, bz, row, col, n, oh, ow);
     p.c[at] = e.residual ? v + e.residual[at] : v;
   }
+}
+
+// The same for the slabs of a product with rows of whole float4s, per-column operands and a plain output: four columns per
+// thread, every slab's fetch out before the first sum.
+static __global__ __launch_bounds__(256) void gemm_finish_rows(GemmParams p) {
+  const Epilogue &e = p.epi;
+  const unsigned total = (unsigned)p.batch * (unsigned)p.M * (unsigned)p.N / 4u, at = blockIdx.x * 256u + threadIdx.x;
+  if (at >= total) return;
+  const float4_t *ws = reinterpret_cast<const float4_t *>(p.ws) + at;
+  float4_t part[8];   // (no more slices than that)
+#pragma unroll
+  for (int s = 0; s < 8; ++s) part[s] = s < p.splits ? ws[(long long)s * total] : (float4_t){0.f, 0.f, 0.f, 0.f};
+  const int col = (int)(at * 4u % (unsigned)p.N);
+  float4_t v = part[0];
+#pragma unroll
+  for (int s = 1; s < 8; ++s)
+    if (s < p.splits) v += part[s];
+  float out[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float bias = e.bias ? e.bias[(long long)(col + q) * e.bias_s[3]] : 0.f;
+    const float alpha = e.activation == TFHIP_PRELU ? e.prelu[(long long)(col + q) * e.prelu_s[3]] : 0.f;
+    out[q] = activate(e.bias ? v[q] + bias : v[q], e.activation, alpha, e.leaky_alpha);
+  }
+  if (e.residual) {
+    const float4 r = reinterpret_cast<const float4 *>(e.residual)[at];
+    out[0] += r.x; out[1] += r.y; out[2] += r.z; out[3] += r.w;
+  }
+  reinterpret_cast<float4 *>(p.c)[at] = make_float4(out[0], out[1], out[2], out[3]);
 }
 
 }  // namespace tfhip

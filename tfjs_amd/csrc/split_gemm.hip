@@ -1,0 +1,150 @@
+// Which products the kernel of split_gemm.h takes, with which tile, and its launch.
+#include "gemm_host.h"
+#include "split_gemm.h"
+
+namespace tfhip {
+namespace {
+
+// The tiles, and what a product takes with them: `launch` microseconds, and for every compute unit's round of workgroups
+// (one, or two side by side where they fit) `per_tile` for each k tile of 32 a group works through and `fixed` for the rest.
+// Least squares on 3700 products and 1900 convolutions of random extents, every tile timed on each (operands in the
+// caches): root mean square error 4 to 7% for products, 2% for windows, and the tile with the least estimate is on average 0.7%
+// slower than the fastest.
+struct SplitShape {
+  int gw, tn, kg;
+  double launch, per_tile, fixed, per_tile_two, fixed_two;   // (_two: two workgroups on a compute unit; 0: one fits)
+};
+constexpr SplitShape kSplitShapes[] = {
+    {4, 4, 1, 2.5, 1.09, 5.2, 2.17, 6.0}, {4, 4, 2, 0.0, 1.79, 7.6, 0, 0}, {4, 3, 1, 3.3, 0.93, 3.8, 1.71, 4.6}, {4, 3, 2, 0.7, 1.42, 6.4, 0, 0},
+    {4, 2, 1, 4.0, 0.77, 2.0, 1.30, 2.6}, {4, 2, 2, 1.3, 1.17, 4.9, 0, 0}, {2, 2, 4, 1.5, 1.37, 4.4, 0, 0},   {2, 1, 4, 1.9, 0.97, 3.4, 0, 0},
+};
+constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
+constexpr int kMaxSlices = 8;
+
+// The windows of an image cost their address arithmetic, ragged ones also what mends them.
+double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, double windows) {
+  const long long tiles = ((p.M + 32 * s.gw - 1) / (32 * s.gw)) * (long long)((p.N + 32 * s.tn - 1) / (32 * s.tn)) * p.batch * slices;
+  const int k_tiles = ((p.K + 31) / 32 + slices - 1) / slices, rounds_of_k = (k_tiles + s.kg - 1) / s.kg;
+  const long long cus = num_cus();
+  const double one = rounds_of_k * s.per_tile + s.fixed, two = rounds_of_k * s.per_tile_two + s.fixed_two;
+  double us;
+  if (s.per_tile_two == 0) {
+    us = (double)((tiles + cus - 1) / cus) * one;
+  } else {
+    const long long full = tiles / (2 * cus), rest = tiles % (2 * cus);
+    us = (double)full * two + (rest == 0 ? 0 : (rest <= cus ? one : two));
+  }
+  us = s.launch + us * windows;
+  if (slices > 1) us += 2.5 + 4.0 * p.batch * p.M * (double)p.N * (slices + 1) / (p.vec_store ? 4.0e6 : 1.3e6);   // gemm_finish_rows, gemm_finish
+  return us;
+}
+
+// What the same product takes with gemm_kernel, whatever tile and slices that chooses: the launch, the matrix instructions at
+// 77% of their rate or the way of k through the pipeline, whichever is longer, and what fills and empties the chip. Least
+// squares on 8800 products and 4300 convolutions of random extents, root mean square error 16%.
+double tiled_estimate_us(const GemmParams &p, double windows) {
+  const double blocks = (double)((p.M + 31) / 32) * ((p.N + 31) / 32) * p.batch, peak_us = blocks * 2048.0 * p.K / 155e6;
+  const double pipeline_us = 0.0044 * p.K * (blocks < 256 ? pow(blocks / 256, 0.27) : 1.0);
+  return 4.4 + windows * (pow(pow(peak_us / 0.77, 4) + pow(pipeline_us, 4), 0.25) + 1.4 * sqrt(peak_us));
+}
+
+template <int GW, int TN, int KG, int A_KIND, int B_KIND>
+int launch_shape(GemmParams &p, int slices) {
+  using T = SplitTile<GW, TN, KG>;
+  p.tiles_m = (p.M + T::BM - 1) / T::BM;
+  p.tiles_n = (p.N + T::BN - 1) / T::BN;
+  p.splits = 1;
+  p.k_per_split = p.K;
+  p.ws = nullptr;
+  std::unique_lock<std::mutex> held;
+  if (slices > 1) {
+    const size_t bytes = (size_t)slices * p.batch * p.M * p.N * sizeof(float);
+    held = lock_workspace();
+    // (nullptr where a caller's fixed scratch does not hold it: one slice)
+    p.ws = bytes <= (size_t(1) << 30) ? static_cast<float *>(workspace(bytes)) : nullptr;
+    if (p.ws) {
+      p.splits = slices;
+      p.k_per_split = ((p.K + 31) / 32 + slices - 1) / slices * 32;
+    }
+  }
+  note_splits(p.splits);
+  const long long grid = (long long)p.tiles_m * p.tiles_n * p.batch * p.splits;
+  if (grid > 0x7fffffffLL) return fail(kBadArgument, "split_gemm: %lld tiles exceed the grid limit", grid);
+  p.group_m = tile_rows_per_panel(grid, T::BM, T::BN, p.tiles_m);
+  const auto kernel = split_gemm<GW, TN, KG, A_KIND, B_KIND>;
+  if (T::LDS_BYTES > 64 * 1024) {
+    // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
+    static int raised = 0;
+    if (raised != init_count()) {
+      TFHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES));
+      raised = init_count();
+    }
+  }
+  note_kernel("split_gemm<%d, %d, %d, %d, %d>", GW, TN, KG, A_KIND, B_KIND);
+  p.inline_epilogue = p.splits == 1 && p.epi.channel_operands && p.epi.activation <= TFHIP_LEAKYRELU;
+  const dim3 blocks((unsigned)grid), threads(T::kThreads);
+  if (p.inline_epilogue) {
+    TFHIP_LAUNCH((kernel<<<blocks, threads, T::LDS_BYTES, stream()>>>(p)));
+  } else {
+    TFHIP_LAUNCH((kernel<<<blocks, threads, T::LDS_BYTES, stream()>>>(p), enqueue_finish(p)));
+  }
+  return kOk;
+}
+
+template <int A_KIND, int B_KIND>
+int launch_kind(SplitChoice c, GemmParams &p) {
+  switch (c.shape) {
+    case 0: return launch_shape<4, 4, 1, A_KIND, B_KIND>(p, c.slices);
+    case 1: return launch_shape<4, 4, 2, A_KIND, B_KIND>(p, c.slices);
+    case 2: return launch_shape<4, 3, 1, A_KIND, B_KIND>(p, c.slices);
+    case 3: return launch_shape<4, 3, 2, A_KIND, B_KIND>(p, c.slices);
+    case 4: return launch_shape<4, 2, 1, A_KIND, B_KIND>(p, c.slices);
+    case 5: return launch_shape<4, 2, 2, A_KIND, B_KIND>(p, c.slices);
+    case 6: return launch_shape<2, 2, 4, A_KIND, B_KIND>(p, c.slices);
+    default: return launch_shape<2, 1, 4, A_KIND, B_KIND>(p, c.slices);
+  }
+}
+
+}  // namespace
+
+SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
+  SplitChoice best = {-1, 1};
+  const int forced = tuning(kTuneSplit);
+  if (forced == 99 || tuning(kTuneTile) >= 0 || tuning(kTuneSplitK) >= 0 || tuning(kTuneKGroups) >= 0) return best;
+  // 32-bit offsets, also of the rows behind the last one that a k tile reaches; bias and PReLU weights per column or one for all
+  constexpr unsigned kMaxBytes = 0x7fffffffu;
+  if (p.K <= 0 || p.a_bytes == 0 || p.a_bytes > kMaxBytes || p.b_bytes == 0 || p.b_bytes > kMaxBytes || p.N > (1 << 22) || p.c_bytes == 0 ||
+      p.epi.addressing == kConv)
+    return best;
+  if (p.epi.channel_operands && (p.epi.bias_s[3] > 1 || p.epi.prelu_s[3] > 1)) return best;
+  if (forced >= 0 && forced < 80) return {forced % 10 % kNumSplitShapes, forced / 10 + 1};
+  // Below 0.3 GFLOP the fixed part decides, and gemm_kernel's is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, 0.3 to 0.45
+  // equal, 0.8 to 1.2 0.88 of the time, from 4 on 0.68; 13000 products); so it is with tiles that are mostly padding: few
+  // columns, few rows of each product of a batch. Under 448 rows only half of the products gain.
+  if (forced < 0 && (2.0 * p.batch * p.M * (double)p.N * p.K < 3e8 || p.N <= 32 || p.M < 64 || (long long)p.batch * p.M < 448)) return best;
+  const double windows = a_kind == kLoadWindows ? 1.08 : (a_kind == kLoadWindowsAny ? 1.35 : 1.0);
+  double best_us = 0;
+  for (int i = 0; i < kNumSplitShapes; ++i) {
+    for (int slices = 1; slices <= kMaxSlices; ++slices) {
+      if (slices > 1 && p.K < 32 * 4 * kSplitShapes[i].kg * slices) break;
+      const double us = split_estimate_us(kSplitShapes[i], p, slices, windows);
+      if (best.shape < 0 || us < best_us * (slices > 1 ? 0.97 : 1.0)) {
+        best_us = us;
+        best = {i, slices};
+      }
+    }
+  }
+  // The lead that makes up for the estimates' errors: of the 13000, half are taken, on average at 0.78 of the time; 2% of
+  // those are 5% slower than with gemm_kernel and more.
+  const double tiled = tiled_estimate_us(p, a_kind == kLoadWindows ? 1.24 : (a_kind == kLoadWindowsAny ? 1.82 : 1.0));
+  if (forced < 0 && best_us > 0.92 * tiled) best.shape = -1;
+  return best;
+}
+
+int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind) {
+  if (a_kind == kLoadWindows) return launch_kind<kLoadWindows, kLoadXVec>(choice, p);
+  if (a_kind == kLoadWindowsAny) return launch_kind<kLoadWindowsAny, kLoadFilter>(choice, p);
+  return launch_kind<kLoadKAny, kLoadXVec>(choice, p);
+}
+
+}  // namespace tfhip

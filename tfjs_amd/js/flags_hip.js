@@ -21,7 +21,7 @@ const {addon} = require('./binding');
 const TUNING_KNOBS = [
   'tile', 'splitk', 'dw_rows', 'dw_halo', 'no_skinny', 'skinny_regs', 'fuse_pw_dw',
   'pw_dw_tile', 'tile_slice', 'tile_chunks', 'fuse_block', 'k_groups', 'pw_dw_stream', 'stream_rows',
-  'stream_blocks', 'skinny_stage', 'block_rows'
+  'stream_blocks', 'skinny_stage', 'block_rows', 'split'
 ];
 /** Flags a graph-model planner reads as the defaults of its load options. */
 const PLAN_FLAGS = {HIP_FUSE_RESIDUAL_ADD: true, HIP_FUSE_POINTWISE_DEPTHWISE: true, HIP_RECORD_LAUNCHES: false};
