@@ -6,6 +6,9 @@
 #include <sched.h>
 #include <string.h>
 #include <unistd.h>
+#if defined(__x86_64__)
+#include <emmintrin.h>
+#endif
 
 #include <atomic>
 #include <condition_variable>
@@ -21,7 +24,7 @@
 namespace tfhip {
 namespace {
 
-// Pinned staging: a ring of slots. A transfer goes through it in pieces of at most a slot, so that
+// Pinned staging: a ring of slots. A transfer goes through it in pieces (an upload's of up to four slots), so that
 // copying a piece between the caller's memory and its slot overlaps the DMA of the pieces before it.
 constexpr size_t kSlotBytes = size_t(4) << 20;
 constexpr int kSlots = 16;
@@ -382,6 +385,33 @@ int usable_cpus() {
   return CPU_COUNT(&set);
 }
 
+// memcpy into the staging ring past the caches: the ring is not read by the host, and an ordinary store first fetches the line it
+// is to overwrite (one thread, a range that no cache holds: 31 GB/s, so 44; four 91 and 126). Small copies stay in the
+// cache, where the DMA finds them.
+void copy_past_caches(char *d, const char *s, size_t n) {
+#if defined(__x86_64__)
+  constexpr size_t kSmall = size_t(64) << 10;
+  if (n >= kSmall) {
+    const size_t head = (64 - reinterpret_cast<uintptr_t>(d) % 64) % 64;
+    memcpy(d, s, head);
+    d += head;
+    s += head;
+    n -= head;
+    for (; n >= 64; n -= 64, d += 64, s += 64) {
+      const __m128i *from = reinterpret_cast<const __m128i *>(s);
+      __m128i *to = reinterpret_cast<__m128i *>(d);
+      const __m128i a = _mm_loadu_si128(from), b = _mm_loadu_si128(from + 1), c = _mm_loadu_si128(from + 2), e = _mm_loadu_si128(from + 3);
+      _mm_stream_si128(to, a);
+      _mm_stream_si128(to + 1, b);
+      _mm_stream_si128(to + 2, c);
+      _mm_stream_si128(to + 3, e);
+    }
+    _mm_sfence();
+  }
+#endif
+  memcpy(d, s, n);
+}
+
 // memcpy by several threads, for the pieces of a transfer between the caller's memory and the staging
 // ring: one thread moves 30 GB/s of a range that no cache holds, half of what the DMA engine behind it
 // does (57 GB/s); four move 99. The workers, at most one per CPU beside the caller's, are started by the
@@ -399,6 +429,7 @@ struct CopyCrew {
   char *dst = nullptr;
   const char *src = nullptr;
   size_t bytes = 0, share = 0;
+  bool past_caches = false;
   int workers = 0;
 
   CopyCrew() {
@@ -412,7 +443,10 @@ struct CopyCrew {
   }
   void part(int i) {
     const size_t at = share * (size_t)i;
-    if (at < bytes) memcpy(dst + at, src + at, bytes - at < share ? bytes - at : share);
+    if (at >= bytes) return;
+    const size_t n = bytes - at < share ? bytes - at : share;
+    if (past_caches) copy_past_caches(dst + at, src + at, n);
+    else memcpy(dst + at, src + at, n);
   }
   void work(int i) {
     unsigned seen = 0;
@@ -432,7 +466,8 @@ struct CopyCrew {
     }
   }
   // (one caller at a time: the staging ring's mutex is held)
-  void copy(char *d, const char *s, size_t n) {
+  void copy(char *d, const char *s, size_t n, bool streamed) {
+    past_caches = streamed;
     dst = d;
     src = s;
     bytes = n;
@@ -452,10 +487,12 @@ struct CopyCrew {
   }
 };
 
-// `together`: the transfer this piece belongs to is long enough for the crew to be awake anyway
-void host_copy(char *d, const char *s, size_t n, bool together) {
+// `together`: the transfer this piece belongs to is long enough for the crew to be awake anyway; `to_ring`: the host does
+// not read d
+void host_copy(char *d, const char *s, size_t n, bool together, bool to_ring) {
   if (!together || n < 2 * CopyCrew::kShare) {
-    memcpy(d, s, n);
+    if (to_ring) copy_past_caches(d, s, n);
+    else memcpy(d, s, n);
     return;
   }
   static CopyCrew *crew = nullptr;   // (the staging ring's mutex is held)
@@ -464,30 +501,36 @@ void host_copy(char *d, const char *s, size_t n, bool together) {
     crew = new CopyCrew();
     owner = getpid();
   }
-  crew->copy(d, s, n);
+  crew->copy(d, s, n, to_ring);
 }
 
-// A transfer of at least this much is copied by the crew (waking it costs 10 - 15 us; 3.4 MB that
-// sit in a cache take one thread 44 us, all of it behind the DMA of the pieces before).
-constexpr size_t kCrewBytes = size_t(8) << 20;
+// A transfer of at least this much is copied by the crew: waking it costs 10 - 15 us, and one thread takes 78 us for the
+// 3.4 MB of a mobile network, four 27.
+constexpr size_t kCrewBytes = size_t(2) << 20;
 
-// How much of a transfer goes into one piece: small pieces first, so that the DMA starts early (the
-// first piece's copy is the one that nothing overlaps), whole slots for the bulk (each DMA costs
-// some 8 us of its own).
+// How much of a transfer goes into one piece: each as much as all before it (the threads fill the ring at more than twice the
+// DMA's rate, so the DMA never waits for the next one), from 1 MB, which nothing overlaps, to 16 MB: between two DMAs pass
+// some 9 us (85 MB in pieces of 1, 4 and 16 MB: 2225, 1690, 1533 us).
+constexpr size_t kLeastPiece = size_t(1) << 20, kMostPiece = size_t(16) << 20;
 size_t piece_bytes(size_t done, size_t left) {
-  const size_t want = done < (size_t(1) << 20) ? (size_t(512) << 10) : (done < kCrewBytes ? (size_t(1) << 20) : kSlotBytes);
-  return left < want + want / 2 && left <= kSlotBytes ? left : (left < want ? left : want);
+  const size_t want = done < kLeastPiece ? kLeastPiece : (done < kMostPiece ? done : kMostPiece);
+  return left < want + want / 2 && left <= kMostPiece ? left : (left < want ? left : want);
 }
 
-// A free slot of the ring (waits for the transfer that last used it).
-int take_slot(int *slot) {
+// `count` free slots side by side in the ring (waits for the transfers that last used them). A transfer through several is
+// noted at the first one: the ring goes round in order, so nobody takes the others before it.
+int take_slots(int count, int *slot) {
+  if (g.next_slot + count > kSlots) g.next_slot = 0;
   const int s = g.next_slot;
-  g.next_slot = (s + 1) % kSlots;
-  if (g.slot_busy[s]) TFHIP_CHECK_HIP(hipEventSynchronize(g.slot_done[s]));
-  g.slot_busy[s] = false;
+  g.next_slot = (s + count) % kSlots;
+  for (int i = s; i < s + count; ++i) {
+    if (g.slot_busy[i]) TFHIP_CHECK_HIP(hipEventSynchronize(g.slot_done[i]));
+    g.slot_busy[i] = false;
+  }
   *slot = s;
   return kOk;
 }
+int take_slot(int *slot) { return take_slots(1, slot); }
 
 // Behind the wait for the ring: the library may have been shut down, and set up again, since the caller
 // checked the range.
@@ -519,8 +562,8 @@ UploadPlace for_segments(UploadPlace p, size_t n, F each) {
   return p;
 }
 
-// Host memory -> device memory (checked by the caller), on the library's stream. 85 MB take
-// 1.7 ms, 88% of the DMA rate; with two 32 MB staging buffers filled by one thread they took 3.2 ms.
+// Host memory -> device memory (checked by the caller), on the library's stream. 89 MB that no cache holds: 1.74 ms, 89% of
+// the DMA's rate; 3.4 MB 121 us (in pieces of 1 and 4 MB, with ordinary stores into the ring, 2.04 ms and 144 us).
 int stage_upload(const UploadSegment *segments, size_t count) {
   std::lock_guard<std::mutex> lock(g_staging_mutex);
   size_t total = 0;
@@ -534,7 +577,7 @@ int stage_upload(const UploadSegment *segments, size_t count) {
   for (size_t done = 0; done < total;) {
     const size_t n = piece_bytes(done, total - done);
     int s = 0;
-    const int rc = take_slot(&s);
+    const int rc = take_slots((int)((n + kSlotBytes - 1) / kSlotBytes), &s);
     if (rc != kOk) return rc;
     char *slot = g.staging + s * kSlotBytes;
     // (segments that lie side by side in host memory, as the tensors of a shard do, are copied together)
@@ -542,13 +585,13 @@ int stage_upload(const UploadSegment *segments, size_t count) {
     size_t from = 0, until = 0;
     for_segments(place, n, [&](size_t at, const UploadSegment &seg, size_t off, size_t bytes) {
       if (until > from && seg.h + off != h + (at - from)) {
-        host_copy(slot + from, h, until - from, together);
+        host_copy(slot + from, h, until - from, together, true);
         from = at;
       }
       if (at == from) h = seg.h + off;
       until = at + bytes;
     });
-    host_copy(slot + from, h, until - from, together);
+    host_copy(slot + from, h, until - from, together, true);
     // (a DMA for each: two blocks side by side on the device are still two allocations)
     hipError_t e = hipSuccess;
     place = for_segments(place, n, [&](size_t at, const UploadSegment &seg, size_t off, size_t bytes) {
@@ -606,7 +649,7 @@ int stage_download(char *h, const char *d, size_t bytes) {
     const Piece &p = pieces[head];
     TFHIP_CHECK_HIP(hipEventSynchronize(g.slot_done[p.slot]));
     g.slot_busy[p.slot] = false;
-    host_copy(h + p.at, g.staging + p.slot * kSlotBytes, p.n, bytes >= kCrewBytes);
+    host_copy(h + p.at, g.staging + p.slot * kSlotBytes, p.n, bytes >= kCrewBytes, false);
     done += p.n;
     head = (head + 1) % kAhead;
     --waiting;
