@@ -87,6 +87,21 @@ def test_strips_of_64_columns_against_the_oracle(lib, m, n, k, act, shift):
         p.free()
 
 
+@pytest.mark.parametrize("m,n", [(1, 17), (1, 4200), (2, 16), (16, 33), (19, 18), (23, 2304), (20, 8300)])
+@pytest.mark.parametrize("k", [3, 16, 128, 129, 255, 257, 384, 395, 513, 1536, 1553, 2300])
+def test_every_length_of_the_way_along_k(lib, m, n, k):
+    """One to more than four groups of 16 per wavefront, whole and cut: each wavefront has one or two out and goes round.
+    A sum of k products and a bias, in any order, is off by at most k + 1 roundings of what it adds up."""
+    p = _Product(lib, m, n, k, "linear")
+    try:
+        p.launch()
+        assert _last_kernel(lib).startswith("few_rows<")
+        a, b, bias = (x.astype(np.float64) for x in p.host)
+        assert np.all(np.abs(p.result() - (a @ b + bias)) <= (k + 1) * 2.0 ** -24 * (np.abs(a) @ np.abs(b) + np.abs(bias)))
+    finally:
+        p.free()
+
+
 def test_a_recording_gives_the_same_bits(lib):
     p = _Product(lib, 19, 200, 2000, "relu")
     try:

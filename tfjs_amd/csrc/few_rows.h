@@ -85,11 +85,22 @@ __device__ __forceinline__ void finish_tile(const FewRowsArgs &p, int tile, floa
   }
 }
 
-template <int MB, int CB, int KIND>
+// U: k groups whose fetches a wavefront has out; when it has multiplied one, it asks for the one U further on, in the same
+// registers. Issuing a group's fetches takes about 0.1 us, so the first ones are back before four have been asked for:
+// with 8 at once, and the next 8 before the first are multiplied, that issue was most of the time. us, then and now:
+// 196 x 384 x 64 4.7 and 3.2, 49 x 960 x 320 6.0 and 4.4, 16 x 1280 x 2048 7.1 and 5.3, 23 x 768 x 2304 6.7 and 4.9,
+// 128 x 1536 x 768 10.3 and 8.5, 32 x 2304 x 8192 19.4 and 17.9; windows, [1,28,28,64] 5x5 -> 33 12.7 and 8.5. U = 1, 2, 4, 8:
+// 16 x 2048 x 2048 6.0, 5.9, 6.0, 6.3; 5 x 2048 x 4096 7.3, 6.6, 6.6, 7.3; 64 x 1280 x 768 5.1, 5.1, 5.2, 6.0;
+// with strips of 64 and two row blocks 32 x 1024 x 12288 12.5, 13.1, 14.6, -.
+// ROW: the product of one row, multiplied with vector instructions, four per lane, column and group: a matrix instruction
+// takes as long for one row as for sixteen, 128 cycles for a group. 1 x 1280 x 1000 6.4 and 3.5, 1 x 2048 x 4096 8.3 and 5.6.
+// (Of two rows the vector form is behind, 5.1 and 4.9 with U = 8: all lanes of a group fetch each row's float4.)
+template <int MB, int CB, int KIND, bool ROW>
 __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
+  constexpr int U = MB * CB == 8 ? 1 : 2;
   constexpr bool kWindows = KIND != kLoadKAny;
   constexpr int W = kFewRowsWaves;
-  constexpr int U = MB + CB <= 2 ? 8 : (MB + CB <= 4 ? 4 : 2);
+  static_assert(!ROW || (MB == 1 && !kWindows), "one row of a matrix");
   constexpr int kCols = 16 * CB, kRows = 16 * MB, kOut = kCols * kRows;
   __shared__ float lds[W * kOut];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r = lane & 15;
@@ -112,7 +123,7 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   int row_ih[MB], row_lin[MB];   // windows: image row and position in it of the first element
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
-    const int row = m0 + 16 * m + r;
+    const int row = ROW ? 0 : m0 + 16 * m + r;   // (ROW: the same for all lanes)
     if (kWindows) {
       const ConvGeom &c = p.conv;
       const int ow = row % c.out_w, t2 = row / c.out_w;
@@ -129,108 +140,132 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   const unsigned b_col = col < p.N ? 4u * (unsigned)col : kOutsideRow;
   const unsigned pitch = 4u * (unsigned)p.N;
 
-  struct Chunk {
+  struct {
     uint4_t a[U][MB];
     unsigned b[U][4][CB];
     int fix[U][MB];   // windows: what fix_up is to do
-  };
-  auto issue = [&](Chunk &c, int first) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = first + u * W, k = 16 * t + 4 * g;
+  } c;
+  // group t = first + step * W, into slot u
+  auto issue = [&](int u, int first, int step) __attribute__((always_inline)) {
+    const unsigned k_first = (unsigned)(16 * first + 4 * g);
+    const int t = first + step * W;
+    unsigned kb;                   // where row k of B begins, in this lane's columns
+    int live_rows = 4;             // of B, of the four
+    if (kWindows) {
+      const int k = 16 * t + 4 * g;
       const bool on = t < end && k < p.K;
-      int row = k, live_rows = 4;   // of B, and how many of the four there are
-      if (kWindows) {
-        const ConvGeom &cg = p.conv;
-        const int q = k >> 2;
-        const int seg = cg.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)cg.unit_magic) : q;
-        const int in_seg = 4 * (q - seg * cg.units);
-        int fr = seg, fs = 0;
-        if (cg.taps > 1) {
-          fr = seg / cg.taps;
-          fs = seg - fr * cg.taps;
-        }
-        const int dh = fr * cg.dil_h, dl = fs * cg.seg_col + in_seg;
-        const unsigned at = 4u * (unsigned)(fr * cg.seg_row + dl);
-        row = seg * cg.seg_len + in_seg;
-        live_rows = cg.seg_len - in_seg;
-#pragma unroll
-        for (int m = 0; m < MB; ++m) {
-          const bool row_in = on && (unsigned)(row_ih[m] + dh) < (unsigned)cg.in_h;
-          const int lin = row_lin[m] + dl;
-          const int before = KIND == kLoadWindowsAny && lin < 0 ? -lin : 0;
-          const bool in = row_in && (KIND == kLoadWindowsAny ? before < 4 && lin < cg.row_len : (unsigned)lin < (unsigned)cg.row_len);
-          c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(in ? a_row[m] + at + 4u * (unsigned)before : kNoOffset), 0, 0);
-          const int real = min(cg.row_len - lin, live_rows);
-          c.fix[u][m] = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
-        }
-      } else {
-        const unsigned ka = on ? 4u * (unsigned)k : kOutside;
-#pragma unroll
-        for (int m = 0; m < MB; ++m) c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(a_row[m] + ka), 0, 0);
+      const ConvGeom &cg = p.conv;
+      const int q = k >> 2;
+      const int seg = cg.unit_magic ? (int)__umulhi((unsigned)q, (unsigned)cg.unit_magic) : q;
+      const int in_seg = 4 * (q - seg * cg.units);
+      int fr = seg, fs = 0;
+      if (cg.taps > 1) {
+        fr = seg / cg.taps;
+        fs = seg - fr * cg.taps;
       }
-      const unsigned kb = on ? (unsigned)row * pitch + b_col : kOutside;
+      const int dh = fr * cg.dil_h, dl = fs * cg.seg_col + in_seg;
+      const unsigned at = 4u * (unsigned)(fr * cg.seg_row + dl);
+      live_rows = cg.seg_len - in_seg;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {   // (rows beyond the last lie beyond the descriptor)
-        const int at = (int)(KIND == kLoadWindowsAny && j >= live_rows ? kOutside : kb + (unsigned)j * pitch);
-        if constexpr (CB == 4) {
-          const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, at, 0, 0);
+      for (int m = 0; m < MB; ++m) {
+        const bool row_in = on && (unsigned)(row_ih[m] + dh) < (unsigned)cg.in_h;
+        const int lin = row_lin[m] + dl;
+        const int before = KIND == kLoadWindowsAny && lin < 0 ? -lin : 0;
+        const bool in = row_in && (KIND == kLoadWindowsAny ? before < 4 && lin < cg.row_len : (unsigned)lin < (unsigned)cg.row_len);
+        c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(in ? a_row[m] + at + 4u * (unsigned)before : kNoOffset), 0, 0);
+        const int real = min(cg.row_len - lin, live_rows);
+        c.fix[u][m] = before << 16 | (real < 0 ? 0 : (real < 4 ? real : 4));
+      }
+      kb = on ? (unsigned)(seg * cg.seg_len + in_seg) * pitch + b_col : kOutside;
+    } else {
+      // (a group that is not this slice's: outside both; what is asked for of k beyond the last lies behind B's last row)
+      const unsigned gone = t < end ? 0u : kOutside;   // the same for the whole wavefront
 #pragma unroll
-          for (int q = 0; q < 4; ++q) c.b[u][j][q % CB] = v[q];
-        } else {
-          c.b[u][j][0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, at, 0, 0);
-        }
+      for (int m = 0; m < MB; ++m)
+        c.a[u][m] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)(a_row[m] + 4u * k_first + 64u * (unsigned)(step * W) + gone), 0, 0);
+      kb = k_first * pitch + b_col + ((unsigned)(16 * step * W) * pitch + gone);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // (rows beyond the last lie beyond the descriptor)
+      const int at = (int)(KIND == kLoadWindowsAny && j >= live_rows ? kOutside : kb + (unsigned)j * pitch);
+      if constexpr (CB == 4) {
+        const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, at, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c.b[u][j][q % CB] = v[q];
+      } else {
+        c.b[u][j][0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, at, 0, 0);
       }
     }
   };
   float4_t acc[MB][CB];
+  float row_acc[CB];   // ROW: of this lane's k
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
     for (int q = 0; q < CB; ++q) acc[m][q] = (float4_t){0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](const Chunk &c, int first) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (first + u * W >= end) break;   // (the same for the whole wavefront)
-      const int k = 16 * (first + u * W) + 4 * g;
-      float a4[MB][4];
+  for (int q = 0; q < CB; ++q) row_acc[q] = 0.f;
+  auto multiply = [&](int u, int t) __attribute__((always_inline)) {
+    const int k = 16 * t + 4 * g;
+    float a4[MB][4];
 #pragma unroll
-      for (int m = 0; m < MB; ++m) {
-        // (the last float4 of a row may reach into the next one)
-        const float4 v = fix_up<KIND>(as_float4(c.a[u][m]), kWindows ? c.fix[u][m] : p.K - k);
-        a4[m][0] = v.x; a4[m][1] = v.y; a4[m][2] = v.z; a4[m][3] = v.w;
-      }
+    for (int m = 0; m < MB; ++m) {
+      float4 v = as_float4(c.a[u][m]);
+      if (kWindows) v = fix_up<KIND>(v, c.fix[u][m]);
+      else if (16 * t + 16 > p.K) v = fix_up<KIND>(v, p.K - k);   // (the last float4 of a row may reach into the next one)
+      a4[m][0] = v.x; a4[m][1] = v.y; a4[m][2] = v.z; a4[m][3] = v.w;
+    }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      if (ROW) {
+#pragma unroll
+        for (int q = 0; q < CB; ++q) row_acc[q] = fmaf(a4[0][j], __uint_as_float(c.b[u][j][q]), row_acc[q]);
+      } else {
 #pragma unroll
         for (int m = 0; m < MB; ++m)
 #pragma unroll
           for (int q = 0; q < CB; ++q)
             acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[m][j], __uint_as_float(c.b[u][j][q]), acc[m][q], 0, 0, 0);
+      }
     }
   };
 
-  Chunk cur, nxt;
-  issue(cur, begin);
+#pragma unroll
+  for (int u = 0; u < U; ++u) issue(u, begin, u);
   // what the column this thread finishes needs
   const int my_col = n0 + tid % kCols;
   const bool col_ok = my_col < p.N;
   const float bias = p.bias && col_ok ? p.bias[(long long)my_col * p.bias_stride] : 0.f;
   const float alpha = p.activation == TFHIP_PRELU && col_ok ? p.prelu[(long long)my_col * p.prelu_stride] : 0.f;
+  int t = begin;
 #pragma unroll 1
-  for (int t = begin; t < end; t += U * W) {
-    issue(nxt, t + U * W);   // (past the end: outside, nothing is read)
-    multiply(cur, t);
-    cur = nxt;
-  }
+  for (; t + U * W < end; t += U * W)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      multiply(u, t + u * W);
+      issue(u, t, u + U);
+    }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (t + u * W < end) multiply(u, t + u * W);   // (the same for the whole wavefront)
 
-  // ---- the wavefronts' sums: lane holds rows 16 m + 4 g .. +3 of columns CB r + q
+  // ---- the wavefronts' sums: lane holds rows 16 m + 4 g .. +3 of columns CB r + q (ROW: its k's share of the row)
+  if (ROW) {
 #pragma unroll
-  for (int m = 0; m < MB; ++m)
+    for (int q = 0; q < CB; ++q) {
+      float v = row_acc[q];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (g == 0) lds[wave * kOut + CB * r + q] = v;
+    }
+  } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int m = 0; m < MB; ++m)
 #pragma unroll
-      for (int q = 0; q < CB; ++q) lds[wave * kOut + (16 * m + 4 * g + e) * kCols + CB * r + q] = acc[m][q][e];
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int q = 0; q < CB; ++q) lds[wave * kOut + (16 * m + 4 * g + e) * kCols + CB * r + q] = acc[m][q][e];
+  }
   lds_barrier();
   auto wave_sum = [&](int i) __attribute__((always_inline)) {
     float v = lds[i];
@@ -281,9 +316,12 @@ inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_bloc
   cut.row_tiles = row_blocks == 1 ? (p.M + 15) / 16 : (p.M + 31) / 32;
   cut.tiles = (long long)cut.row_tiles * (col_blocks == 1 ? (p.N + 15) / 16 : (p.N + 63) / 64);
   const int groups = (p.K + 15) / 16;
-  // A wavefront wants about as many k groups as it fetches at once (64 or 32 groups per workgroup); more workgroups
-  // than compute units only add scratch traffic (1 x 768 x 3072 in 1, 2, 4 slices: 4.8, 8.0, 11.0 us).
-  const int wanted = row_blocks == 1 ? (groups + 63) / 64 : (groups + 31) / 32;
+  // Slices of 64 groups (of 32 with two row blocks) from the length on at which one slice takes longer than the way of the
+  // sums through memory, 128 groups for one row and 96 for more. us, one slice and more: 1 x 1280 x 1000 3.9 and 5.0,
+  // 1 x 2048 x 1000 4.4 and 4.9, 1 x 3072 x 1000 6.1 and 5.3; 8 x 1280 x 768 4.4 and 4.9, 32 x 1280 x 1000 5.1 and 5.4,
+  // 16 x 2048 x 2048 6.7 and 6.0. More workgroups than compute units only add to what goes through memory.
+  const int whole = p.M == 1 ? 128 : 96;
+  const int wanted = row_blocks == 1 ? (groups <= whole ? 1 : (groups + 63) / 64) : (groups + 31) / 32;
   const int most = cut.tiles * 2 > kFewRowsCounters ? 1 : kFewRowsCounters / (int)cut.tiles;
   cut.splits = wanted < most ? wanted : most;
   cut.groups_per_split = cut.splits == 1 ? groups : (groups + cut.splits - 1) / cut.splits;
@@ -324,7 +362,7 @@ inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
 //    22.6; ragged, at 222 groups [3,33,22,141] 5x5/2 -> 111 22.2 and 20.3, at 399 [1,20,20,130] 7x7 -> 130 24.0 and 29.7).
 inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
   if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
-  if (p.batch != 1 || p.K <= 0 || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
+  if (p.batch != 1 || p.K <= 0 || p.N > (1 << 24) || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
       tuning(kTuneSplit) >= 0 || tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
     return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();

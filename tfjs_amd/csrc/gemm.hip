@@ -50,7 +50,7 @@ int resolve(const void *symbol, const char *name, int device, void **ptr) {
   return fail(kHipError, "tfhip_init: hipGetSymbolAddress(%s) on device %d failed: %s", name, device, hipGetErrorString(e));
 }
 
-template <int MB, int CB, int KIND>
+template <int MB, int CB, int KIND, bool ROW = false>
 int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
   q.row_tiles = cut.row_tiles;
   q.splits = 1;
@@ -68,12 +68,13 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
   // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
   q.finish_apart = q.splits > 1 && capturing();
-  note_kernel("few_rows<%d, %d, %d>", MB, CB, KIND);
+  note_kernel("few_rows<%d, %d, %d, %d>", MB, CB, KIND, (int)ROW);
   const dim3 grid((unsigned)(cut.tiles * q.splits)), block(64 * kFewRowsWaves);
   if (q.finish_apart) {
-    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q), few_rows_finish<MB, CB><<<dim3((unsigned)cut.tiles), block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB, KIND, ROW><<<grid, block, 0, stream()>>>(q),
+                  few_rows_finish<MB, CB><<<dim3((unsigned)cut.tiles), block, 0, stream()>>>(q)));
   } else {
-    TFHIP_LAUNCH((few_rows<MB, CB, KIND><<<grid, block, 0, stream()>>>(q)));
+    TFHIP_LAUNCH((few_rows<MB, CB, KIND, ROW><<<grid, block, 0, stream()>>>(q)));
   }
   return kOk;
 }
@@ -100,8 +101,10 @@ int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   if (kind == kLoadWindowsAny) return one ? launch_few_rows_shape<1, 1, kLoadWindowsAny>(q, narrow) : launch_few_rows_shape<2, 1, kLoadWindowsAny>(q, narrow);
   if (few_rows_wide(narrow, row_blocks)) {
     const FewRowsCut wide = few_rows_cut(p, row_blocks, 4);
+    if (p.M == 1) return launch_few_rows_shape<1, 4, kLoadKAny, true>(q, wide);
     return one ? launch_few_rows_shape<1, 4, kLoadKAny>(q, wide) : launch_few_rows_shape<2, 4, kLoadKAny>(q, wide);
   }
+  if (p.M == 1) return launch_few_rows_shape<1, 1, kLoadKAny, true>(q, narrow);
   return one ? launch_few_rows_shape<1, 1, kLoadKAny>(q, narrow) : launch_few_rows_shape<2, 1, kLoadKAny>(q, narrow);
 }
 
