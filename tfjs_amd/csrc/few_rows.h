@@ -316,11 +316,10 @@ inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_bloc
   cut.row_tiles = row_blocks == 1 ? (p.M + 15) / 16 : (p.M + 31) / 32;
   cut.tiles = (long long)cut.row_tiles * (col_blocks == 1 ? (p.N + 15) / 16 : (p.N + 63) / 64);
   const int groups = (p.K + 15) / 16;
-  // Slices of 64 groups (of 32 with two row blocks) from the length on at which one slice takes longer than the way of the
-  // sums through memory, 128 groups for one row and 96 for more. us, one slice and more: 1 x 1280 x 1000 3.9 and 5.0,
-  // 1 x 2048 x 1000 4.4 and 4.9, 1 x 3072 x 1000 6.1 and 5.3; 8 x 1280 x 768 4.4 and 4.9, 32 x 1280 x 1000 5.1 and 5.4,
-  // 16 x 2048 x 2048 6.7 and 6.0. More workgroups than compute units only add to what goes through memory.
-  const int whole = p.M == 1 ? 128 : 96;
+  // Slices of 64 groups (of 32 with two row blocks). One row stays whole up to 128: its workgroups have less to add up, and
+  // one slice is ahead that far. us, one slice and more: 1 x 1280 x 1000 3.9 and 5.0, 1 x 2048 x 1000 4.4 and 4.9, 1 x 3072 x 1000
+  // 6.1 and 5.3. More workgroups than compute units only add to what goes through memory.
+  const int whole = p.M == 1 ? 128 : 64;
   const int wanted = row_blocks == 1 ? (groups <= whole ? 1 : (groups + 63) / 64) : (groups + 31) / 32;
   const int most = cut.tiles * 2 > kFewRowsCounters ? 1 : kFewRowsCounters / (int)cut.tiles;
   cut.splits = wanted < most ? wanted : most;
