@@ -448,9 +448,11 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
         (f_h - 1) * dilation_h * in_w * in_c + f_w * dilation_w * in_c < lim && stride_w * out_w * in_c < lim && pad_left * in_c < lim) {
       p.K = (int)(4 * units);
       const int row_blocks = few_rows_blocks(p, true, vec);
-      if (row_blocks) return launch_few_rows(p, row_blocks, vec ? kLoadWindows : kLoadWindowsAny);
       const int a_kind = vec ? kLoadWindows : kLoadWindowsAny;
+      if (row_blocks) return launch_few_rows(p, row_blocks, a_kind);
       const SplitChoice split = split_gemm_choice(p, a_kind);
+      const FewRowsForm few = few_rows_form(p, a_kind, vec, split);
+      if (few.row_blocks) return launch_few_rows(p, few.row_blocks, a_kind, few.col_blocks);
       if (split.shape >= 0) return launch_split_gemm(split, p, a_kind);
       const int shape = choose_tile_shape(M, out_c, p.K, 1, num_cus());
       if (vec) return launch_gemm_shape<kLoadWindows, kLoadXVec>(shape, p);

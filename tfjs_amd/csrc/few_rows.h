@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "gemm_host.h"
 #include "gemm_kernel.h"
 
 namespace tfhip {
@@ -33,8 +34,11 @@ struct FewRowsArgs {
   int M, N, K;
   unsigned a_bytes, b_bytes;
   int groups;               // of 16 k
-  int row_tiles;            // of 16 MB rows
+  // Tiles side by side in the order of the workgroups: the row tiles of a strip (of 16 MB rows), or, negative, the strips of a row
+  // tile. The two divisors' magic numbers are ceil(2^32 / d), exact for what is divided here, and 0 for 1.
+  int inner;
   int splits, groups_per_split;
+  unsigned inner_magic, splits_magic;
   int finish_apart;         // another launch adds the slices
   ConvGeom conv;            // A gathered from an image (k counted as there)
   int activation;
@@ -49,6 +53,16 @@ constexpr long long kFewRowsMaxBytes = 0x40000000LL;
 // lines (a fence at device scope would write back and drop whole caches instead).
 constexpr int kThrough = 16;   // sc1
 
+__device__ __forceinline__ int by_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
+
+// Strip and row tile of a tile. The operand of the longer side is what the XCDs fetch in parts: all of the shorter one each
+// (5967 x 1788 x 64 in 748 tiles, row tiles and strips side by side: 34.2 and 23.7 us).
+__device__ __forceinline__ void tile_place(const FewRowsArgs &p, int tile, int &strip, int &row_tile) {
+  const int outer = by_magic(tile, p.inner_magic), in = tile - outer * abs(p.inner);
+  strip = p.inner > 0 ? outer : in;
+  row_tile = p.inner > 0 ? in : outer;
+}
+
 // Sum over the slices (or, of one, over the wavefronts' sums in `lds`), bias, activation, residual and store of the
 // outputs of a tile; `bias` and `alpha` belong to the thread's column.
 template <int MB, int CB>
@@ -57,7 +71,9 @@ __device__ __forceinline__ void finish_tile(const FewRowsArgs &p, int tile, floa
   static_assert((64 * W) % kCols == 0, "a thread keeps its column");
   const __amdgpu_buffer_rsrc_t rsrc_ws = __builtin_amdgcn_make_buffer_rsrc(
       (void *)uniform_pointer(p.ws + (long long)tile * p.splits * kOut), 0, p.splits * kOut * 4, 0x00020000);
-  const int strip = tile / p.row_tiles, m0 = (tile - strip * p.row_tiles) * 16 * MB;
+  int strip, row_tile;
+  tile_place(p, tile, strip, row_tile);
+  const int m0 = row_tile * 16 * MB;
   const int col = strip * kCols + (int)threadIdx.x % kCols;
   const int live = min(kOut, (p.M - m0) * kCols);   // elements of the tile that exist (its rows come first)
 #pragma unroll 1
@@ -105,15 +121,19 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   __shared__ float lds[W * kOut];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // What the first fetches need, asked for at once (left to itself, the compiler makes two trips of it, 0.2 us each).
+  asm volatile("" : : "s"(p.a), "s"(p.b), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.a_bytes), "s"(p.b_bytes), "s"(p.groups), "s"(p.inner),
+               "s"(p.inner_magic), "s"(p.splits), "s"(p.splits_magic), "s"(p.groups_per_split), "s"((int)gridDim.x));
   int id = blockIdx.x;   // neighbouring strips share cache lines: each XCD (ids i, i + 8, ..) gets a contiguous band
   {
     const int per_xcd = gridDim.x / 8;
     if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   }
-  // the slices of a tile side by side, then the row tiles of a strip
-  const int tile = id / p.splits, split = id - tile * p.splits;
-  const int strip = tile / p.row_tiles, m0 = (tile - strip * p.row_tiles) * kRows;
-  const int n0 = strip * kCols;
+  // the slices of a tile side by side
+  const int tile = by_magic(id, p.splits_magic), split = id - tile * p.splits;
+  int strip, row_tile;
+  tile_place(p, tile, strip, row_tile);
+  const int m0 = row_tile * kRows, n0 = strip * kCols;
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)p.a, 0, (int)p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)p.b, 0, (int)p.b_bytes, 0x00020000);
   const int begin = split * p.groups_per_split + wave;
@@ -298,7 +318,9 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
 // The sums of the slices of one tile each, where few_rows leaves them (FewRowsArgs::finish_apart).
 template <int MB, int CB>
 __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows_finish(FewRowsArgs p) {
-  const int col = (int)(blockIdx.x / p.row_tiles) * (16 * CB) + (int)threadIdx.x % (16 * CB);
+  int strip, row_tile;
+  tile_place(p, blockIdx.x, strip, row_tile);
+  const int col = strip * (16 * CB) + (int)threadIdx.x % (16 * CB);
   const float bias = p.bias && col < p.N ? p.bias[(long long)col * p.bias_stride] : 0.f;
   const float alpha = p.activation == TFHIP_PRELU && col < p.N ? p.prelu[(long long)col * p.prelu_stride] : 0.f;
   finish_tile<MB, CB>(p, blockIdx.x, bias, alpha, nullptr);
@@ -307,14 +329,15 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows_finish(FewRowsArg
 // How a product in tiles of 16 MB rows and 16 CB columns is cut over workgroups.
 constexpr int kFewRowsCounters = 256;
 struct FewRowsCut {
-  int row_tiles;
+  int row_tiles, strips;
   long long tiles;
   int splits, groups_per_split;   // slices of k, and the k groups of 16 in one
 };
 inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_blocks) {
   FewRowsCut cut;
   cut.row_tiles = row_blocks == 1 ? (p.M + 15) / 16 : (p.M + 31) / 32;
-  cut.tiles = (long long)cut.row_tiles * (col_blocks == 1 ? (p.N + 15) / 16 : (p.N + 63) / 64);
+  cut.strips = col_blocks == 1 ? (p.N + 15) / 16 : (p.N + 63) / 64;
+  cut.tiles = (long long)cut.row_tiles * cut.strips;
   const int groups = (p.K + 15) / 16;
   // Slices of 64 groups (of 32 with two row blocks). One row stays whole up to 128: its workgroups have less to add up, and
   // one slice is ahead that far. us, one slice and more: 1 x 1280 x 1000 3.9 and 5.0, 1 x 2048 x 1000 4.4 and 4.9, 1 x 3072 x 1000
@@ -335,6 +358,13 @@ inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_bloc
 // 7.6, 1 x 1024 x 4112 8.5 and 7.6.
 inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
   return narrow.tiles > num_cus() || narrow.groups_per_split > (row_blocks == 1 ? 128 : 96);
+}
+
+// (32-bit offsets, no per-call choice of another kernel)
+inline bool few_rows_can(const GemmParams &p, bool windows) {
+  if (windows ? p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return false;
+  return p.batch == 1 && p.K > 0 && p.N <= (1 << 24) && p.epi.channel_operands && p.epi.addressing != kConv && tuning(kTuneTile) < 0 &&
+         tuning(kTuneSplit) < 0 && tuning(kTuneSplitK) < 0 && (long long)p.K * p.N * 4 <= kFewRowsMaxBytes;
 }
 
 // Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
@@ -360,10 +390,7 @@ inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
 //    21.0 and 13.8; at 144 groups [1,10,10,512] 3x3 -> 256 12.8 and 13.0; of one strip [3,34,19,260] 7x7 -> 8 30.7 and
 //    22.6; ragged, at 222 groups [3,33,22,141] 5x5/2 -> 111 22.2 and 20.3, at 399 [1,20,20,130] 7x7 -> 130 24.0 and 29.7).
 inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
-  if (windows ? p.K < 384 || p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return 0;
-  if (p.batch != 1 || p.K <= 0 || p.N > (1 << 24) || !p.epi.channel_operands || p.epi.addressing == kConv || tuning(kTuneTile) >= 0 ||
-      tuning(kTuneSplit) >= 0 || tuning(kTuneSplitK) >= 0 || (long long)p.K * p.N * 4 > kFewRowsMaxBytes)
-    return 0;
+  if (!few_rows_can(p, windows) || (windows && p.K < 384)) return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();
   int blocks = 0;
   if (p.M <= 16) blocks = 1;
@@ -379,7 +406,50 @@ inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
   return blocks;
 }
 
-// `kind`: kLoadKAny (row-major A), kLoadWindows or kLoadWindowsAny.
-int launch_few_rows(const GemmParams &p, int row_blocks, int kind);
+// The same where there are more tiles than compute units, which then share them: two row blocks with a strip of 16 columns, or one
+// with a strip of 64, where the estimate for either is below that for the kernel that would have it otherwise (`split`: what
+// the bf16 parts would take, if they are chosen; else gemm_kernel). An estimate is a launch, what a workgroup does round by round (16 k
+// per wavefront, 32 for gemm_kernel), and per compute unit its tiles' share of fetches and matrix work and their ends; tiles count in
+// part as they are and in part as full rounds over the chip. Least squares on 25000 products and 18000 convolutions of random extents in
+// the ranges below, root mean square error 4 to 9% here and 5 to 7% for gemm_kernel. Of what the lines above leave to gemm_kernel,
+// 85% of the convolutions are taken, on average at 0.79 of its time (0.71 where its loader has units to mend); of the products
+// two thirds at 0.91 and 0.87 (ragged), with up to 700 rows nearly all at 0.84 and 0.75. 1 to 4% of what is taken is 3% slower and more.
+// Of what the bf16 parts would have, 7500 that were taken: 0.90 of their time (products) and 0.76 (windows) at the median.
+// us, before and here: 48 x 2304 x 2304 15.8 and 10.0, 64 x 768 x 3072 8.0 and 6.3, [3,113,75,21] 5x5/2 -> 38 14.4 and 10.5,
+// [1,56,56,64] 3x3 -> 64 8.7 and 6.6. What is not taken at all: K below 384 (windows: 192), as with fewer tiles, where at most a fifth of 5 us is left; K above
+// 3000 (2048), where gemm_kernel cuts k into slices; more than 10000 rows, whose A comes from memory, and 40000 windows,
+// for which gemm_kernel has tiles of 256 rows (both in 0.85 of the time).
+struct FewRowsForm {
+  int row_blocks, col_blocks;   // 0, 0: not with this kernel
+};
+inline FewRowsForm few_rows_form(const GemmParams &p, int kind, bool vec, const SplitChoice &split) {
+  const bool windows = kind != kLoadKAny;
+  const long long cus = num_cus(), row_pairs = (p.M + 31) / 32, rows = (p.M + 15) / 16, strips = (p.N + 15) / 16;
+  if (!few_rows_can(p, windows) || p.M <= 32 || p.N < 4 || row_pairs * strips > 3000) return {0, 0};
+  if (windows ? rows * strips <= cus || p.M > 40000 || p.K < 192 || p.K > 2048 : row_pairs * strips <= cus || p.M > 10000 || p.K < 384 || p.K > 3000)
+    return {0, 0};
+  struct Estimate {
+    double launch, round, work, tile, full;   // us; full: the part of the tiles that counts in full rounds
+  };
+  const auto us = [&](const Estimate &e, long long tiles, int depth, int waves) {
+    const int steps = (p.K + depth - 1) / depth;
+    const double share = (1 - e.full) * (double)tiles / (double)cus + e.full * (double)((tiles + cus - 1) / cus);
+    return e.launch + e.round * ((steps + waves - 1) / waves) + share * (e.work * steps + e.tile);
+  };
+  // products; windows; windows whose units need mending
+  static constexpr Estimate kTwoRows[3] = {{2.83, 0.143, 0.0435, 0.40, 0.75}, {3.16, 0.146, 0.0492, 0.71, 0.75}, {2.95, 0.279, 0.0578, 0.83, 0.75}};
+  static constexpr Estimate kWide[3] = {{3.13, 0.055, 0.0610, 0.67, 0.75}, {3.22, 0.171, 0.0656, 0.77, 0.75}, {3.19, 0.216, 0.0721, 0.80, 0.75}};
+  // gemm_kernel in tiles of 32 x 32: products, and windows, each with float4 loads and without
+  static constexpr Estimate kTiled[4] = {{4.03, 0.029, 0.141, 0.20, 0.75}, {4.00, 0.111, 0.140, 0.31, 0.5}, {3.94, 0.114, 0.145, 0.38, 0.75}, {4.47, 0.237, 0.178, 0.49, 0.5}};
+  const int which = kind == kLoadKAny ? 0 : (kind == kLoadWindows ? 1 : 2);
+  const double two_rows = us(kTwoRows[which], row_pairs * strips, 16, kFewRowsWaves);
+  const double wide = us(kWide[which], rows * ((p.N + 63) / 64), 16, kFewRowsWaves);
+  const double other = split.shape >= 0 ? split.us : us(kTiled[2 * (int)windows + (int)!vec], row_pairs * ((p.N + 31) / 32), 32, 1);
+  if (fmin(two_rows, wide) > 0.93 * other) return {0, 0};
+  return two_rows < wide ? FewRowsForm{2, 1} : FewRowsForm{1, 4};
+}
+
+// `kind`: kLoadKAny (row-major A), kLoadWindows or kLoadWindowsAny. Strips of 16 `col_blocks` columns; 0: by few_rows_wide.
+int launch_few_rows(const GemmParams &p, int row_blocks, int kind, int col_blocks = 0);
 
 }  // namespace tfhip

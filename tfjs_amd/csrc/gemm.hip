@@ -11,8 +11,12 @@ int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, 
   if (!transpose_a && !transpose_b) {
     const int row_blocks = few_rows_blocks(p, false, vec);
     if (row_blocks) return launch_few_rows(p, row_blocks, kLoadKAny);
-    const SplitChoice split = split_gemm_choice(p, kLoadKAny);
-    if (split.shape >= 0 && !float_bits) return launch_split_gemm(split, p, kLoadKAny);
+    if (!float_bits) {
+      const SplitChoice split = split_gemm_choice(p, kLoadKAny);
+      const FewRowsForm few = few_rows_form(p, kLoadKAny, vec, split);
+      if (few.row_blocks) return launch_few_rows(p, few.row_blocks, kLoadKAny, few.col_blocks);
+      if (split.shape >= 0) return launch_split_gemm(split, p, kLoadKAny);
+    }
   }
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());
@@ -52,7 +56,7 @@ int resolve(const void *symbol, const char *name, int device, void **ptr) {
 
 template <int MB, int CB, int KIND, bool ROW = false>
 int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
-  q.row_tiles = cut.row_tiles;
+  q.inner = q.M <= q.N ? cut.row_tiles : -cut.strips;
   q.splits = 1;
   q.groups_per_split = q.groups;
   std::unique_lock<std::mutex> held;
@@ -64,6 +68,10 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
       q.groups_per_split = cut.groups_per_split;
     }
   }
+  // (exact: a number below 2^32 / d; d is at most about the square root of the tiles, or 256 where there are 256 workgroups)
+  const auto magic = [](int d) { return d == 1 ? 0u : (unsigned)(((1ULL << 32) + d - 1) / d); };
+  q.inner_magic = magic(abs(q.inner));
+  q.splits_magic = magic(q.splits);
   note_splits(q.splits);
   // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
@@ -81,7 +89,7 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
 
 }  // namespace
 
-int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
+int launch_few_rows(const GemmParams &p, int row_blocks, int kind, int col_blocks) {
   FewRowsArgs q = {};
   q.a = p.a; q.b = p.b; q.c = p.c;
   q.bias = p.epi.bias; q.bias_stride = p.epi.bias ? p.epi.bias_s[3] : 0;
@@ -97,9 +105,13 @@ int launch_few_rows(const GemmParams &p, int row_blocks, int kind) {
   q.counters = g_device_arrays[device_index()].few_rows_counters;
   const FewRowsCut narrow = few_rows_cut(p, row_blocks, 1);
   const bool one = row_blocks == 1;
+  if (kind != kLoadKAny && col_blocks == 4) {
+    const FewRowsCut wide = few_rows_cut(p, row_blocks, 4);
+    return kind == kLoadWindows ? launch_few_rows_shape<1, 4, kLoadWindows>(q, wide) : launch_few_rows_shape<1, 4, kLoadWindowsAny>(q, wide);
+  }
   if (kind == kLoadWindows) return one ? launch_few_rows_shape<1, 1, kLoadWindows>(q, narrow) : launch_few_rows_shape<2, 1, kLoadWindows>(q, narrow);
   if (kind == kLoadWindowsAny) return one ? launch_few_rows_shape<1, 1, kLoadWindowsAny>(q, narrow) : launch_few_rows_shape<2, 1, kLoadWindowsAny>(q, narrow);
-  if (few_rows_wide(narrow, row_blocks)) {
+  if (col_blocks ? col_blocks == 4 : few_rows_wide(narrow, row_blocks)) {
     const FewRowsCut wide = few_rows_cut(p, row_blocks, 4);
     if (p.M == 1) return launch_few_rows_shape<1, 4, kLoadKAny, true>(q, wide);
     return one ? launch_few_rows_shape<1, 4, kLoadKAny>(q, wide) : launch_few_rows_shape<2, 4, kLoadKAny>(q, wide);

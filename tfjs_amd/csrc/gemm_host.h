@@ -238,17 +238,18 @@ inline int launch_gemm_shape(int shape, GemmParams &p) {
 // Plain (non-im2col) GEMM launch, defined once in gemm.hip: picks the loaders
 // for row-major / transposed operands; `vec` says both operands may be fetched
 // with float4 loads.
-// `float_bits`: with float32 matrix instructions only.
+// `float_bits`: as gemm_kernel sums, with float32 matrix instructions and k in order.
 int launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec, bool float_bits = false);
 
 // The same for a row-major A (and a B of either kind) that cannot (gemm_ragged.hip).
 int launch_ragged_gemm(GemmParams &p, bool transpose_b);
 
 // The tile and the slices of k with which the kernel on the bf16 matrix cores (split_gemm.h) takes a product of a row-major B
-// and a row-major A or windows of an image; shape -1: it goes to gemm_kernel. Its launch; a_kind: kLoadKAny, kLoadWindows or
-// kLoadWindowsAny.
+// and a row-major A or windows of an image; shape -1: it goes to gemm_kernel. `us`: what it takes, by
+// estimate. Its launch; a_kind: kLoadKAny, kLoadWindows or kLoadWindowsAny.
 struct SplitChoice {
   int shape, slices;
+  double us;
 };
 SplitChoice split_gemm_choice(const GemmParams &p, int a_kind);
 int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind);

@@ -108,7 +108,7 @@ int launch_kind(SplitChoice c, GemmParams &p) {
 }  // namespace
 
 SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
-  SplitChoice best = {-1, 1};
+  SplitChoice best = {-1, 1, 0};
   const int forced = tuning(kTuneSplit);
   if (forced == 99 || tuning(kTuneTile) >= 0 || tuning(kTuneSplitK) >= 0 || tuning(kTuneKGroups) >= 0) return best;
   // 32-bit offsets, also of the rows behind the last one that a k tile reaches; bias and PReLU weights per column or one for all
@@ -117,7 +117,7 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
       p.epi.addressing == kConv)
     return best;
   if (p.epi.channel_operands && (p.epi.bias_s[3] > 1 || p.epi.prelu_s[3] > 1)) return best;
-  if (forced >= 0 && forced < 80) return {forced % 10 % kNumSplitShapes, forced / 10 + 1};
+  if (forced >= 0 && forced < 80) return {forced % 10 % kNumSplitShapes, forced / 10 + 1, 0};
   // Below 0.3 GFLOP the fixed part decides, and gemm_kernel's is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, 0.3 to 0.45
   // equal, 0.8 to 1.2 0.88 of the time, from 4 on 0.68; 13000 products); so it is with tiles that are mostly padding: few
   // columns, few rows of each product of a batch. Under 448 rows only half of the products gain.
@@ -130,7 +130,7 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
       const double us = split_estimate_us(kSplitShapes[i], p, slices, windows);
       if (best.shape < 0 || us < best_us * (slices > 1 ? 0.97 : 1.0)) {
         best_us = us;
-        best = {i, slices};
+        best = {i, slices, us};
       }
     }
   }
