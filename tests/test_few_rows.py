@@ -105,10 +105,12 @@ def test_every_length_of_the_way_along_k(lib, m, n, k):
 @pytest.mark.parametrize("m,n,k,form", [
     (700, 333, 501, "2, 1"), (9000, 33, 401, "2, 1"), (4097, 19, 833, "2, 1"), (2081, 130, 517, "1, 4"), (64, 4095, 384, "1, 4"),
     (33, 4096, 3000, "1, 4"), (1200, 100, 2700, "1, 4"), (1030, 515, 385, "1, 4"),
+    (33, 64, 316, "1, 1"), (200, 60, 16, "1, 1"), (785, 32, 192, "1, 1"), (300, 300, 300, "2, 1"),
 ])
-def test_more_tiles_than_compute_units(lib, m, n, k, form):
-    """Rows and columns that end inside a tile, tiles in either order, k that ends inside a group. The bound as above."""
-    p = _Product(lib, m, n, k, "linear", 1)
+def test_every_form_of_more_than_32_rows(lib, m, n, k, form):
+    """Rows and columns that end inside a tile, tiles in either order, k that ends inside a group. The bound as above. (Below
+    K = 320 only operands that float4s fit are taken.)"""
+    p = _Product(lib, m, n, k, "linear", int(k >= 320))
     try:
         p.launch()
         assert _last_kernel(lib).startswith("few_rows<%s, " % form)
@@ -119,10 +121,11 @@ def test_more_tiles_than_compute_units(lib, m, n, k, form):
 
 
 @pytest.mark.parametrize("xs,out_c,f,stride,dil,form", [
-    ((2, 70, 69, 40), 8, 3, 1, 1, "2, 1, 3"), ((1, 56, 56, 64), 64, 3, 1, 1, "1, 4, 3"), ((1, 56, 45, 32), 64, 3, 1, 2, "1, 4, 3"),
+    ((1, 14, 13, 32), 64, 3, 1, 1, "1, 1, 3"), ((2, 70, 69, 40), 8, 3, 1, 1, "2, 1, 3"),
+    ((1, 56, 56, 64), 64, 3, 1, 1, "1, 4, 3"), ((1, 56, 45, 32), 64, 3, 1, 2, "1, 4, 3"),
     ((1, 50, 47, 11), 21, 5, 1, 1, "2, 1, 5"), ((3, 113, 75, 21), 38, 5, 2, 1, "1, 4, 5"), ((2, 37, 41, 23), 70, 3, 1, 2, "2, 1, 5"),
 ])
-def test_more_windows_than_compute_units(lib, xs, out_c, f, stride, dil, form):
+def test_every_form_of_windows(lib, xs, out_c, f, stride, dil, form):
     import torch
 
     from tfjs_amd import pyhost as hip
@@ -134,8 +137,8 @@ def test_more_windows_than_compute_units(lib, xs, out_c, f, stride, dil, form):
     assert _last_kernel(lib).startswith("few_rows<%s, " % form)
 
     def conv(x, w):
-        return torch.nn.functional.conv2d(torch.from_numpy(x.astype(np.float64)).permute(0, 3, 1, 2), torch.from_numpy(w.astype(np.float64)).permute(3, 2, 0, 1),
-                                          stride=stride, padding=pad, dilation=dil).permute(0, 2, 3, 1).numpy()
+        x, w = torch.from_numpy(x.astype(np.float64)).permute(0, 3, 1, 2), torch.from_numpy(w.astype(np.float64)).permute(3, 2, 0, 1)
+        return torch.nn.functional.conv2d(x, w, stride=stride, padding=pad, dilation=dil).permute(0, 2, 3, 1).numpy()
     # f * f * in_c products in any order: no more roundings than that
     assert np.all(np.abs(got - conv(x, w)) <= f * f * xs[3] * 2.0 ** -24 * conv(np.abs(x), np.abs(w)))
 

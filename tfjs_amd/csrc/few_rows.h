@@ -372,10 +372,11 @@ inline bool few_rows_can(const GemmParams &p, bool windows) {
 // own, the fetches of a whole k range are out at once, where the tiled kernel goes round its pipeline once per 32 k (us,
 // tiled and here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7; windows,
 // [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1). The lines, each from a grid of extents on both sides, in the same form:
-//  * more than 32 rows, K < 320: the tiled kernel is ahead up to 128 (33 x 64 x 32 3.3 and 3.9), then the two are
-//    within 10% of each other (100 x 256 x 96 4.7 and 4.2).
-//  * windows of fewer than 384 floats: behind at 144 ([1,7,7,16] 3x3 -> 32 4.4 and 4.8); ahead from 297 on
-//    ([1,14,14,33] 3x3 -> 64 7.7 and 5.9), so the line is on the safe side.
+//  * more than 32 rows, K < 320: 0.85 of the time at K = 16, 0.77 at 96, 0.6 at 300 (256 x 256 x 256 5.6 and 4.2, 784 x 192 x 32
+//    4.5 and 2.9), except where the caller wants the sums of gemm_kernel (`float_bits`), and not for ragged rows, on which
+//    the same is left: the tests of the ragged loader count on it there.
+//  * windows of fewer than 256 floats (384 with units to mend): ahead from 48 on (0.84 of the time; [1,28,28,16] 3x3 -> 32 5.5 and 3.7),
+//    but left for the same reason; above, 0.7 ([1,14,14,32] 3x3 -> 64 6.7 and 4.1).
 //  * up to 32 rows always, from K = 2048 on with two row blocks: half the fetches of B, and slices enough to fill the
 //    chip (23 x 3072 x 768 9.3 with one, 7.7 with two). Except 17 to 32 rows of 4097 to 8192 columns with K <= 1536
 //    (where a float4 fits the rows, else 768): more strips than compute units, while each of the tiled kernel's 32-wide tiles
@@ -389,12 +390,12 @@ inline bool few_rows_can(const GemmParams &p, bool windows) {
 //    ([1,10,10,256] 5x5 -> 256 14.5 and 15.4, [1,14,14,256] 7x7 -> 256 30.5 and 39.7; on 64 tiles [1,7,7,256] 7x7 -> 256
 //    21.0 and 13.8; at 144 groups [1,10,10,512] 3x3 -> 256 12.8 and 13.0; of one strip [3,34,19,260] 7x7 -> 8 30.7 and
 //    22.6; ragged, at 222 groups [3,33,22,141] 5x5/2 -> 111 22.2 and 20.3, at 399 [1,20,20,130] 7x7 -> 130 24.0 and 29.7).
-inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec) {
-  if (!few_rows_can(p, windows) || (windows && p.K < 384)) return 0;
+inline int few_rows_blocks(const GemmParams &p, bool windows, bool vec, bool float_bits = false) {
+  if (!few_rows_can(p, windows) || (windows && p.K < (vec ? 256 : 384))) return 0;
   const long long strips = (p.N + 15) / 16, cus = num_cus();
   int blocks = 0;
   if (p.M <= 16) blocks = 1;
-  else if (p.M > 32 && p.K < 320 && !windows) blocks = 0;
+  else if (p.M > 32 && p.K < 320 && !windows && (!vec || float_bits || p.K < 16)) blocks = 0;
   else if (p.M <= 32 && p.K > 2048) blocks = 2;
   else if ((p.M + 15) / 16 * strips <= cus) blocks = 1;
   else if (p.M <= 32) blocks = strips > cus && strips <= 2 * cus && p.K <= (vec ? 1536 : 768) ? 0 : 2;

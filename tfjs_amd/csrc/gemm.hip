@@ -9,7 +9,7 @@ using namespace tfhip;
 int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool vec, bool float_bits) {
   if (skinny_applies(p, transpose_a, transpose_b, vec) && tuning(kTuneNoSkinny) <= 0) return launch_skinny(p);
   if (!transpose_a && !transpose_b) {
-    const int row_blocks = few_rows_blocks(p, false, vec);
+    const int row_blocks = few_rows_blocks(p, false, vec, float_bits);
     if (row_blocks) return launch_few_rows(p, row_blocks, kLoadKAny);
     if (!float_bits) {
       const SplitChoice split = split_gemm_choice(p, kLoadKAny);
