@@ -17,6 +17,9 @@ struct ExpandDwTileArgs {
   int rows, chunks_h;              // output rows per workgroup, workgroups along the rows
   int erows, ecols;                // expanded tile with halo: rows of the tallest chunk, columns
   unsigned x_bytes;
+  // magic_of the divisors in the kernel's addresses (0: of 1): columns of the tile inside the image, of the tile, of
+  // the result, and chunks_h (0 also where that is not exact for every workgroup)
+  unsigned inside_magic, ecols_magic, out_w_magic, chunks_magic;
   int stream_out;                  // the result leaves as non-temporal stores (8 MB or more in all, or an image
                                    // beyond 32-bit offsets), else written through
 };

@@ -35,7 +35,7 @@ struct FewRowsArgs {
   unsigned a_bytes, b_bytes;
   int groups;               // of 16 k
   // Tiles side by side in the order of the workgroups: the row tiles of a strip (of 16 MB rows), or, negative, the strips of a row
-  // tile. The two divisors' magic numbers are ceil(2^32 / d), exact for what is divided here, and 0 for 1.
+  // tile. The two divisors' magic numbers (magic_of).
   int inner;
   int splits, groups_per_split;
   unsigned inner_magic, splits_magic;
@@ -52,8 +52,6 @@ constexpr long long kFewRowsMaxBytes = 0x40000000LL;
 // Sums over wavefronts are written through to memory and read past the reader's L2, which does not see other XCDs'
 // lines (a fence at device scope would write back and drop whole caches instead).
 constexpr int kThrough = 16;   // sc1
-
-__device__ __forceinline__ int by_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
 
 // Strip and row tile of a tile. The operand of the longer side is what the XCDs fetch in parts: all of the shorter one each
 // (5967 x 1788 x 64 in 748 tiles, row tiles and strips side by side: 34.2 and 23.7 us).

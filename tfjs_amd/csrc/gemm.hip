@@ -69,9 +69,8 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
     }
   }
   // (exact: a number below 2^32 / d; d is at most about the square root of the tiles, or 256 where there are 256 workgroups)
-  const auto magic = [](int d) { return d == 1 ? 0u : (unsigned)(((1ULL << 32) + d - 1) / d); };
-  q.inner_magic = magic(abs(q.inner));
-  q.splits_magic = magic(q.splits);
+  q.inner_magic = magic_of(abs(q.inner));
+  q.splits_magic = magic_of(q.splits);
   note_splits(q.splits);
   // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
