@@ -58,6 +58,11 @@ struct Taps {
   float4 t0, t1, t2;
 };
 
+__device__ __forceinline__ float4 load4(__amdgpu_buffer_rsrc_t rsrc, int offset, int row) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, row, 0);
+  return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+}
+
 // S: stride of the depthwise stage. K = 16 KF + (HALF ? 8 : 0) input channels.
 // TAPS > 0: the first stage is a convolution of at most 4 TAPS taps (filter height x width x input
 // channels, a network stem) gathered element by element with the lane layout and instruction
@@ -81,6 +86,10 @@ void expand_dw_stream(ExpandDwStreamArgs g, StemTaps taps) {
   // Workgroup ids i, i + 8, i + 16, ... share an XCD and its L2: each XCD takes one contiguous band
   // of the wavefront sequence, so that the channel blocks of a strip, which read the same input
   // rows, find them in one L2 instead of fetching them into all eight.
+  // every argument in one trip (left to itself, the compiler makes four of it)
+  asm volatile("" : : "s"(g.b2), "s"(g.in_h), "s"(g.in_w), "s"(g.c), "s"(g.pad_top), "s"(g.pad_left),
+               "s"(g.strip_w), "s"(g.strips), "s"(g.rows), "s"(g.chunks_h), "s"(g.cblocks), "s"((unsigned)g.waves), "s"(g.x_bytes),
+               "s"(g.by_magic), "s"(g.cgroups_magic), "s"(g.strips_magic), "s"(g.chunks_magic), "s"((unsigned)gridDim.x));
   unsigned block = blockIdx.x;
   {
     const unsigned per_xcd = gridDim.x / 8;
@@ -89,11 +98,19 @@ void expand_dw_stream(ExpandDwStreamArgs g, StemTaps taps) {
   unsigned w = block * 4 + (unsigned)__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   if (w >= (unsigned)g.waves) return;   // (whole wavefronts: nothing below synchronises across them)
   const unsigned cgroups = (unsigned)(g.cblocks + NCB - 1) / NCB;
-  const int cb0 = (int)(w % cgroups) * NCB;         // first channel block of this wavefront
-  w /= cgroups;
-  const int strip = (int)(w % (unsigned)g.strips);
-  w /= (unsigned)g.strips;
-  const int chunk = (int)(w % (unsigned)g.chunks_h), n = (int)(w / (unsigned)g.chunks_h);
+  unsigned w1, w2;
+  int n;
+  if (__builtin_expect(g.by_magic, 1)) {
+    w1 = (unsigned)by_magic((int)w, g.cgroups_magic);
+    w2 = (unsigned)by_magic((int)w1, g.strips_magic);
+    n = by_magic((int)w2, g.chunks_magic);
+  } else {
+    w1 = w / cgroups;
+    w2 = w1 / (unsigned)g.strips;
+    n = (int)(w2 / (unsigned)g.chunks_h);
+  }
+  const int cb0 = (int)(w - w1 * cgroups) * NCB;    // first channel block of this wavefront
+  const int strip = (int)(w1 - w2 * (unsigned)g.strips), chunk = (int)w2 - n * g.chunks_h;
   const int oh0 = chunk * g.rows, ow0 = strip * g.strip_w;
   const int rows = oh0 + g.rows <= g.out_h ? g.rows : g.out_h - oh0;
   const int e0 = oh0 * S - g.pad_top;               // first expanded row this wavefront needs
@@ -105,6 +122,10 @@ void expand_dw_stream(ExpandDwStreamArgs g, StemTaps taps) {
     ch[u] = 16 * cbs[u] + 4 * grp;
   }
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)g.x, 0, (int)g.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw1 = __builtin_amdgcn_make_buffer_rsrc((void *)g.w1, 0, g.k * g.c * 4, 0x00020000);   // (of TAPS > 0)
+  const __amdgpu_buffer_rsrc_t rw2 = __builtin_amdgcn_make_buffer_rsrc((void *)g.w2, 0, 9 * g.c * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb1 = __builtin_amdgcn_make_buffer_rsrc((void *)g.b1, 0, g.b1 ? g.c * 4 : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb2 = __builtin_amdgcn_make_buffer_rsrc((void *)g.b2, 0, g.b2 ? g.c * 4 : 0, 0x00020000);
 
   int tap_dh[TAPS > 0 ? TAPS : 1], tap_dw[TAPS > 0 ? TAPS : 1];
   unsigned tap_off[TAPS > 0 ? TAPS : 1];
@@ -218,7 +239,8 @@ void expand_dw_stream(ExpandDwStreamArgs g, StemTaps taps) {
 #pragma unroll
       for (int t = 0; t < TAPS; ++t) {
         const int k = 4 * t + grp;
-        wt[u][t] = k < g.k ? g.w1[(long long)k * g.c + 16 * cbs[u] + r] : 0.f;   // taps beyond the filter multiply zeros
+        // (taps beyond the filter, which multiply zeros, lie beyond the descriptor)
+        wt[u][t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw1, (k * g.c + 16 * cbs[u] + r) * 4, 0, 0));
       }
     } else {
       const float *col = g.w1 + 16 * cbs[u] + r;
@@ -233,18 +255,13 @@ void expand_dw_stream(ExpandDwStreamArgs g, StemTaps taps) {
         wh[u] = make_float2(col[(long long)k * g.c], col[(long long)(k + 1) * g.c]);
       }
     }
-    // (a missing bias: the fetch goes to the depthwise weights instead and is dropped; a branch around a
-    // load would make the wavefront wait at its end for every fetch in flight)
-    {
-      const float4_t v = *reinterpret_cast<const float4_t *>((g.b1 ? g.b1 : g.w2) + ch[u]);
-      b1q[u] = g.b1 ? v : float4_t{0.f, 0.f, 0.f, 0.f};
-    }
+    // (a missing bias: an empty descriptor, of which zeros are read; with a branch around a load, or a choice that
+    // the compiler makes one of, the wavefront waits at its end for every fetch in flight)
+    const float4 b = load4(rb1, ch[u] * 4, 0);
+    b1q[u] = float4_t{b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int t = 0; t < 9; ++t) w2q[u][t] = *reinterpret_cast<const float4 *>(g.w2 + (long long)t * g.c + ch[u]);
-    {
-      const float4 v = *reinterpret_cast<const float4 *>((g.b2 ? g.b2 : g.w2) + ch[u]);
-      b2q[u] = g.b2 ? v : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int t = 0; t < 9; ++t) w2q[u][t] = load4(rw2, ch[u] * 4, t * g.c * 4);
+    b2q[u] = load4(rb2, ch[u] * 4, 0);
   }
 
   // expanded row e of block b, channel block u: activation applied, zero outside the map (the
@@ -504,6 +521,11 @@ bool plan_expand_dw_stream(ExpandDwStreamArgs &g) {
   g.rows = rows;
   g.chunks_h = (g.out_h + rows - 1) / rows;
   g.waves = (long long)g.batch * g.chunks_h * g.strips * cgroups;
+  const int most = g.strips > cgroups ? g.strips : cgroups;
+  g.by_magic = (double)g.waves * (g.chunks_h > most ? g.chunks_h : most) < 4294967296.0 ? 1 : 0;
+  g.cgroups_magic = magic_of(cgroups);
+  g.strips_magic = magic_of(g.strips);
+  g.chunks_magic = magic_of(g.chunks_h);
   g.through = (long long)g.out_h * g.out_w * g.c * 4 <= 0xfffffff0LL ? 1 : 0;
   return true;
 }
