@@ -361,6 +361,9 @@ int fused_conv2d(const float *x, const float *filter, float *y, int64_t batch, i
   g.in_h = (int)in_h; g.in_w = (int)in_w; g.in_c = (int)in_c; g.f_w = (int)f_w;
   g.stride_h = (int)stride_h; g.stride_w = (int)stride_w; g.dil_h = (int)dilation_h; g.dil_w = (int)dilation_w;
   g.pad_top = (int)pad_top; g.pad_left = (int)pad_left; g.out_h = (int)out_h; g.out_w = (int)out_w;
+  // (rows are counted to the end of the last tile, 256 rows at most)
+  g.by_magic = (double)(M + 256) * (double)(out_h > out_w ? out_h : out_w) < 4294967296.0 ? 1 : 0;
+  g.out_h_magic = magic_of(g.out_h); g.out_w_magic = magic_of(g.out_w);
   if (nchw) {
     g.xs_n = in_c * in_h * in_w; g.xs_c = in_h * in_w; g.xs_h = in_w; g.xs_w = 1;
   } else {

@@ -143,13 +143,7 @@ __global__ __launch_bounds__(64 * kFewRowsWaves) void few_rows(FewRowsArgs p) {
   for (int m = 0; m < MB; ++m) {
     const int row = ROW ? 0 : m0 + 16 * m + r;   // (ROW: the same for all lanes)
     if (kWindows) {
-      const ConvGeom &c = p.conv;
-      const int ow = row % c.out_w, t2 = row / c.out_w;
-      const int oh = t2 % c.out_h, n = t2 / c.out_h;
-      const int ih = oh * c.stride_h - c.pad_top;
-      row_ih[m] = row < p.M ? ih : -(1 << 28);   // (a row that no image has)
-      row_lin[m] = ow * c.stride_wc - c.pad_leftc;
-      a_row[m] = 4u * ((unsigned)n * (unsigned)c.image_len + (unsigned)(ih * c.row_len) + (unsigned)row_lin[m]);
+      window_row(p.conv, row, p.M, row_ih[m], row_lin[m], a_row[m]);
     } else {
       a_row[m] = row < p.M ? 4u * (unsigned)row * (unsigned)p.K : kOutsideRow;
     }

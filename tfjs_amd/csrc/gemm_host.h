@@ -83,6 +83,18 @@ inline int tile_rows_per_panel(long long grid, int bm, int bn, int tiles_m) {
   return g > tiles_m ? tiles_m : g;
 }
 
+// The numbering of a launch's tiles (tile_of): group_m is set.
+inline void number_tiles(GemmParams &p, long long grid) {
+  const int tiles = p.tiles_m * p.tiles_n, last = p.tiles_m % p.group_m;
+  p.by_magic = grid < 65536 ? 1 : 0;   // (the square of what is divided and of the divisors; 256 workgroups per unit hide a division)
+  if (!p.by_magic) return;
+  p.batch_magic = magic_of(tiles * p.batch);
+  p.tiles_magic = magic_of(tiles);
+  p.panel_magic = magic_of(p.group_m * p.tiles_n);
+  p.rows_magic = magic_of(p.group_m);
+  p.last_rows_magic = magic_of(last ? last : p.group_m);
+}
+
 // Enqueues what completes a product that its kernel left as raw sums or slabs.
 inline void enqueue_finish(const GemmParams &p) {
   const long long total = (long long)p.M * p.N * p.batch;
@@ -164,6 +176,7 @@ inline int launch_gemm(GemmParams &p) {
   const long long grid = tiles * p.splits;
   p.group_m = tile_rows_per_panel(grid, BM, BN, p.tiles_m);
   if (grid > 0x7fffffffLL) return fail(kBadArgument, "gemm: %lld tiles exceed the grid limit", grid);
+  number_tiles(p, grid);
   if (T::LDS_FLOATS * sizeof(float) > 64 * 1024) {   // (also with KG groups of buffers)
     // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
     static int raised = 0;

@@ -71,6 +71,8 @@ struct ConvGeom {
   int f_w;            // k = (r * f_w + s) * in_c + c
   int stride_h, stride_w, dil_h, dil_w, pad_top, pad_left;
   int out_h, out_w;
+  int by_magic;                              // the next two are exact for every row of the product
+  unsigned out_h_magic, out_w_magic;         // magic_of
   // kLoadWindows*: a filter row (columns not dilated), else a filter tap, is a segment: `seg_len` floats that lie side
   // by side in the image as in the filter, so one comparison with the image row's ends covers all its columns
   // and channels. k runs over the segments in units of four (the last of a segment may be partly empty: k counts
@@ -100,6 +102,10 @@ struct GemmParams {
   unsigned c_bytes;
   int tiles_m, tiles_n;
   int group_m;    // tile rows per panel of the tile numbering
+  // magic_of the divisors of tile_of: tiles of all products of the batch, of one, of a panel, tile rows of a panel and of
+  // the last; by_magic: they are exact for every workgroup
+  int by_magic;
+  unsigned batch_magic, tiles_magic, panel_magic, rows_magic, last_rows_magic;
   // split K: the grid holds `splits` copies of the tile set, copy s sums
   // k in [s * k_per_split, (s+1) * k_per_split) into ws[s][batch][M][N]
   int splits, k_per_split;
@@ -157,9 +163,15 @@ __device__ __forceinline__ float4 as_float4(uint4_t v) {
 // Where window m begins: the image row, the float within it, and its byte offset in the image (a window that begins
 // before the image: exact modulo 2^32). Windows from X on get a row that no image has.
 __device__ __forceinline__ void window_row(const ConvGeom &g, int m, int X, int &ih, int &iw, unsigned &off) {
-  const int ow = m % g.out_w;
-  const int t2 = m / g.out_w;
-  const int oh = t2 % g.out_h, n = t2 / g.out_h;
+  int t2, n;
+  if (__builtin_expect(g.by_magic, 1)) {   // (the same for all; a division takes 25 instructions)
+    t2 = by_magic(m, g.out_w_magic);
+    n = by_magic(t2, g.out_h_magic);
+  } else {
+    t2 = m / g.out_w;
+    n = t2 / g.out_h;
+  }
+  const int ow = m - t2 * g.out_w, oh = t2 - n * g.out_h;
   const int first = oh * g.stride_h - g.pad_top;
   ih = m < X ? first : -(1 << 28);
   iw = ow * g.stride_wc - g.pad_leftc;
@@ -394,6 +406,43 @@ __device__ __forceinline__ float quad_element(const float4 &v, int j) {
   return j == 0 ? v.x : (j == 1 ? v.y : (j == 2 ? v.z : v.w));
 }
 
+// Workgroup id -> slice of k, product of the batch, tile. Ids i, i+8, i+16, ... share an XCD; each XCD gets one contiguous
+// band of the tile sequence. Tiles are numbered in panels of group_m tile rows, column by column inside a panel, so that
+// the run of consecutive ids that is resident on one XCD covers a near-square block of C: the rows of A and columns of B it
+// needs per k tile are as few as possible and stay in that XCD's L2.
+// (The divisions as multiplications, here and in window_row: they were 150 of the 270 instructions before the first fetch, 250 with
+// windows. us, before and so: [8,56,56,64] 3x3 -> 64 18.7 and 17.8, 1568 x 320 x 1280 13.6 and 12.9, 784 x 144 x 32 4.1 and 4.0.)
+__device__ __forceinline__ void tile_of(const GemmParams &p, int &split, int &bz, int &tile_m, int &tile_n) {
+  int id = blockIdx.x;
+  {
+    const int per_xcd = gridDim.x / 8;
+    if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
+  }
+  const int tiles_per_batch = p.tiles_m * p.tiles_n, panel = p.group_m * p.tiles_n;
+  split = bz = 0;
+  if (__builtin_expect(p.by_magic, 1)) {
+    if (p.splits * p.batch > 1) {
+      split = by_magic(id, p.batch_magic);
+      id -= split * tiles_per_batch * p.batch;
+      bz = by_magic(id, p.tiles_magic);
+    }
+    const int t = id - bz * tiles_per_batch, q = by_magic(t, p.panel_magic), first_m = q * p.group_m, in_panel = t - q * panel;
+    const bool last = p.tiles_m - first_m < p.group_m;
+    tile_n = by_magic(in_panel, last ? p.last_rows_magic : p.rows_magic);
+    tile_m = first_m + in_panel - tile_n * (last ? p.tiles_m - first_m : p.group_m);
+  } else {
+    if (p.splits * p.batch > 1) {   // (most launches: one product, not split; no division for them)
+      split = id / (tiles_per_batch * p.batch);
+      id -= split * tiles_per_batch * p.batch;
+      bz = id / tiles_per_batch;
+    }
+    const int t = id - bz * tiles_per_batch, first_m = t / panel * p.group_m, in_panel = t % panel;
+    const int rows = p.tiles_m - first_m < p.group_m ? p.tiles_m - first_m : p.group_m;
+    tile_n = in_panel / rows;
+    tile_m = first_m + in_panel % rows;
+  }
+}
+
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int A_KIND, int B_KIND, int KG = 1>
 __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
   using T = GemmTile<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>;
@@ -403,28 +452,16 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
   // those fetches into three or four batches, each waiting a scalar-cache miss of its own.
   asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.c), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.batch), "s"(p.a_sx), "s"(p.a_sk),
                "s"(p.b_sx), "s"(p.b_sk), "s"(p.ldc), "s"(p.a_bytes), "s"(p.b_bytes), "s"(p.tiles_m), "s"(p.tiles_n),
-               "s"(p.group_m), "s"(p.splits), "s"(p.k_per_split), "s"(p.vec_store), "s"(p.inline_epilogue),
+               "s"(p.group_m), "s"(p.by_magic), "s"(p.panel_magic), "s"(p.rows_magic), "s"(p.last_rows_magic), "s"(p.splits),
+               "s"(p.k_per_split), "s"(p.vec_store), "s"(p.inline_epilogue),
                "s"(p.epi.bias), "s"(p.epi.bias_s[3]), "s"(p.epi.activation), "s"(p.epi.residual), "s"(p.epi.addressing));
   // this wavefront's group, and its thread index inside the group
   const int kgroup = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
   float *lds_a = lds + kgroup * T::GROUP_LDS_FLOATS;   // [3][BM][PITCH]
   float *lds_b = lds_a + 3 * T::A_BUF;                 // [3][BN][PITCH]
 
-  // Workgroup id -> (batch, tile_m, tile_n). Ids i, i+8, i+16, ... share an XCD;
-  // give each XCD one contiguous band of the tile sequence.
-  int id = blockIdx.x;
-  {
-    const int per_xcd = gridDim.x / 8;
-    if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
-  }
-  const int tiles_per_batch = p.tiles_m * p.tiles_n;
-  int split = 0, bz = 0;
-  if (p.splits * p.batch > 1) {   // (most launches: one product, not split; no division for them)
-    split = id / (tiles_per_batch * p.batch);
-    id -= split * tiles_per_batch * p.batch;
-    bz = id / tiles_per_batch;
-  }
-  const int t = id - bz * tiles_per_batch;
+  int split, bz, tile_m, tile_n;
+  tile_of(p, split, bz, tile_m, tile_n);
   int k_begin = split * p.k_per_split;
   int k_end = k_begin + p.k_per_split < p.K ? k_begin + p.k_per_split : p.K;
   // the groups cut this range into KG runs of whole k tiles, all of the same tile count (a run that
@@ -438,23 +475,14 @@ __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmParams p) {
     k_end = run_end < k_end ? run_end : k_end;
     if (k_end < k_begin) k_end = k_begin;
   }
-  // Tiles are numbered in panels of group_m tile rows, column by column inside a
-  // panel, so that the run of consecutive ids that is resident on one XCD covers
-  // a near-square block of C: the rows of A and columns of B it needs per k tile
-  // are as few as possible and stay in that XCD's L2.
-  const int width = p.group_m * p.tiles_n;
-  const int first_m = (t / width) * p.group_m;
-  const int gsz = p.tiles_m - first_m < p.group_m ? p.tiles_m - first_m : p.group_m;
-  const int in_group = t % width;
-  const int tile_m = first_m + in_group % gsz, tile_n = in_group / gsz;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   // The operand bases are the same for the whole workgroup; readfirstlane pins
   // them to scalar registers so that the buffer descriptors built from them are
   // scalar too (a descriptor the compiler believes to vary per lane makes it
   // wrap every buffer load in a loop over the distinct values).
-  const float *A = uniform_pointer(p.a + (long long)(bz % p.batch_a) * p.a_batch_stride);
-  const float *B = uniform_pointer(p.b + (long long)(bz % p.batch_b) * p.b_batch_stride);
+  const float *A = uniform_pointer(p.a + (long long)(p.batch == 1 ? 0 : bz % p.batch_a) * p.a_batch_stride);
+  const float *B = uniform_pointer(p.b + (long long)(p.batch == 1 ? 0 : bz % p.batch_b) * p.b_batch_stride);
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)p.b_bytes, 0x00020000);
 

@@ -110,31 +110,16 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
   extern __shared__ char split_lds[];
   // (the arguments of the prologue in one piece, as in gemm_kernel)
   asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.batch), "s"(p.a_sx), "s"(p.b_sk), "s"(p.a_bytes),
-               "s"(p.b_bytes), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.group_m), "s"(p.splits), "s"(p.k_per_split));
-  // workgroup id -> (slice of k, batch, tile), as in gemm_kernel
-  int id = blockIdx.x;
-  {
-    const int per_xcd = gridDim.x / 8;
-    if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
-  }
-  const int tiles_per_batch = p.tiles_m * p.tiles_n;
-  int split = 0, bz = 0;
-  if (p.splits * p.batch > 1) {
-    split = id / (tiles_per_batch * p.batch);
-    id -= split * tiles_per_batch * p.batch;
-    bz = id / tiles_per_batch;
-  }
-  const int t = id - bz * tiles_per_batch;
+               "s"(p.b_bytes), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.group_m), "s"(p.by_magic),
+               "s"(p.panel_magic), "s"(p.rows_magic), "s"(p.last_rows_magic), "s"(p.splits), "s"(p.k_per_split), "s"((int)gridDim.x));
+  int split, bz, tile_m, tile_n;
+  tile_of(p, split, bz, tile_m, tile_n);
   const int k_begin = split * p.k_per_split;
   const int k_end = k_begin + p.k_per_split < p.K ? k_begin + p.k_per_split : p.K;
-  const int panel = p.group_m * p.tiles_n;
-  const int first_m = (t / panel) * p.group_m;
-  const int gsz = p.tiles_m - first_m < p.group_m ? p.tiles_m - first_m : p.group_m;
-  const int in_panel = t % panel;
-  const int m0 = (first_m + in_panel % gsz) * T::BM, n0 = in_panel / gsz * T::BN;
+  const int m0 = tile_m * T::BM, n0 = tile_n * T::BN;
 
-  const float *A = uniform_pointer(p.a + (long long)(bz % p.batch_a) * p.a_batch_stride);
-  const float *B = uniform_pointer(p.b + (long long)(bz % p.batch_b) * p.b_batch_stride);
+  const float *A = uniform_pointer(p.a + (long long)(p.batch == 1 ? 0 : bz % p.batch_a) * p.a_batch_stride);
+  const float *B = uniform_pointer(p.b + (long long)(p.batch == 1 ? 0 : bz % p.batch_b) * p.b_batch_stride);
   const int group = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / T::kGroupThreads) : 0;
   const int tid = (int)threadIdx.x - group * T::kGroupThreads, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -71,6 +71,7 @@ int launch_shape(GemmParams &p, int slices) {
   const long long grid = (long long)p.tiles_m * p.tiles_n * p.batch * p.splits;
   if (grid > 0x7fffffffLL) return fail(kBadArgument, "split_gemm: %lld tiles exceed the grid limit", grid);
   p.group_m = tile_rows_per_panel(grid, T::BM, T::BN, p.tiles_m);
+  number_tiles(p, grid);
   const auto kernel = split_gemm<GW, TN, KG, A_KIND, B_KIND>;
   if (T::LDS_BYTES > 64 * 1024) {
     // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
