@@ -221,24 +221,44 @@ struct DwColsArgs {
   int blocks_per_row;  // workgroups along a row
   int chunks_h, rows;  // row chunks per image, output rows per chunk
   int xcd_run;         // > 0: workgroup ids are dealt to the XCDs in contiguous runs of this many
+  int by_magic;        // the next three are exact for every workgroup and lane
+  unsigned block_magic, chunk_magic, c4_magic;   // magic_of blocks_per_row, chunks_h, c4_total
   unsigned x_bytes, y_bytes;
   int streamed;        // the result is stored non-temporally (kDwStreamBytes)
 };
+
+// A lane's place: float4 f (column ow, channel quad q) of a row of image n, and the chunk of rows. The divisions as
+// multiplications by the host's reciprocals, the arguments in one trip: us, before and so, [8,57,43,120] 5x5/2 5.4 and 5.2,
+// [8,112,112,96] 3x3 13.7 and 13.4.
+__device__ __forceinline__ void cols_place(const DwParams &p, const DwColsArgs &g, int &chunk, int &n, int &f, int &ow, int &q) {
+  asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.y), "s"(p.in_h), "s"(p.in_w), "s"(p.pad_top), "s"(p.pad_left), "s"(p.out_h), "s"(p.out_w),
+               "s"(g.c4_total), "s"(g.row_quads), "s"(g.blocks_per_row), "s"(g.chunks_h), "s"(g.rows), "s"(g.xcd_run), "s"(g.by_magic),
+               "s"(g.block_magic), "s"(g.chunk_magic), "s"(g.c4_magic), "s"(g.x_bytes), "s"(g.y_bytes));
+  // workgroup ids i, i + 8, ... share an XCD: each XCD takes a contiguous run, so that the columns
+  // two neighbouring workgroups both read come from one L2
+  const int wg = g.xcd_run ? (int)(blockIdx.x % 8) * g.xcd_run + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+  int t;
+  if (__builtin_expect(g.by_magic, 1)) {
+    t = by_magic(wg, g.block_magic);
+    n = by_magic(t, g.chunk_magic);
+  } else {
+    t = wg / g.blocks_per_row;
+    n = t / g.chunks_h;
+  }
+  chunk = t - n * g.chunks_h;
+  f = (wg - t * g.blocks_per_row) * kColsThreads + (int)threadIdx.x;
+  ow = __builtin_expect(g.by_magic, 1) ? by_magic(f, g.c4_magic) : f / g.c4_total;
+  q = f - ow * g.c4_total;
+}
 
 template <int S, bool GENERAL, bool STREAM>
 __global__ __launch_bounds__(kColsThreads) void depthwise_3x3_cols(DwParams p, Epilogue e, DwColsArgs g) {
   constexpr int A = S;        // input rows in flight beyond the window in use: one output row ahead (two, three and
                               // four rows ahead measured the same: the launch is not short of loads in flight)
   constexpr int NB = 3 + A;   // ring of input rows
-  // workgroup ids i, i + 8, ... share an XCD: each XCD takes a contiguous run, so that the columns
-  // two neighbouring workgroups both read come from one L2
-  const unsigned wg = g.xcd_run ? (blockIdx.x % 8) * (unsigned)g.xcd_run + blockIdx.x / 8 : blockIdx.x;
-  const int bx = (int)(wg % (unsigned)g.blocks_per_row);
-  const unsigned t = wg / (unsigned)g.blocks_per_row;
-  const int chunk = (int)(t % (unsigned)g.chunks_h), n = (int)(t / (unsigned)g.chunks_h);
-  const int f = bx * kColsThreads + (int)threadIdx.x;
+  int chunk, n, f, ow, q;
+  cols_place(p, g, chunk, n, f, ow, q);
   if (f >= g.row_quads) return;
-  const int ow = f / g.c4_total, q = f - ow * g.c4_total;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)g.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.y, 0, (int)g.y_bytes, 0x00020000);
   const unsigned pix = (unsigned)g.c4_total * 16u;   // bytes per pixel
@@ -347,13 +367,9 @@ template <int F, int S, int VEC, bool GENERAL, bool STREAM>
 __global__ __launch_bounds__(kColsThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void depthwise_cols_sums(DwParams p, Epilogue e, DwColsArgs g) {
   constexpr int NACC = (F + S - 1) / S;   // output rows in progress
-  const unsigned wg = g.xcd_run ? (blockIdx.x % 8) * (unsigned)g.xcd_run + blockIdx.x / 8 : blockIdx.x;
-  const int bx = (int)(wg % (unsigned)g.blocks_per_row);
-  const unsigned t = wg / (unsigned)g.blocks_per_row;
-  const int chunk = (int)(t % (unsigned)g.chunks_h), n = (int)(t / (unsigned)g.chunks_h);
-  const int f = bx * kColsThreads + (int)threadIdx.x;
+  int chunk, n, f, ow, q;
+  cols_place(p, g, chunk, n, f, ow, q);
   if (f >= g.row_quads) return;
-  const int ow = f / g.c4_total, q = f - ow * g.c4_total;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)g.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.y, 0, (int)g.y_bytes, 0x00020000);
   constexpr unsigned kUnit = 4u * VEC;
@@ -461,6 +477,11 @@ bool plan_cols(DwColsArgs &g, const DwParams &p, int vec, int rows, int per_cu) 
   g.streamed = g.y_bytes >= kDwStreamBytes;
   const long long wgs = (long long)g.blocks_per_row * g.chunks_h * p.batch;
   g.xcd_run = wgs % 8 == 0 ? (int)(wgs / 8) : 0;
+  const int most = g.blocks_per_row > g.chunks_h ? g.blocks_per_row : g.chunks_h;
+  g.by_magic = (double)wgs * most < 4294967296.0 && ((double)g.row_quads + kColsThreads) * g.c4_total < 4294967296.0 ? 1 : 0;
+  g.block_magic = magic_of(g.blocks_per_row);
+  g.chunk_magic = magic_of(g.chunks_h);
+  g.c4_magic = magic_of(g.c4_total);
   return wgs <= 0x7fffffffLL;
 }
 
