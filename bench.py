@@ -43,6 +43,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 MFMA_FP32_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix, published
+MFMA_BF16_PEAK_TFLOPS = 2516.6  # dense bf16 matrix, published; a float32 product in bf16 parts takes six of them
 RIDGE = MFMA_FP32_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)
 BATCH = 32
 
@@ -57,12 +58,12 @@ def measured_traffic():
     return traffic.load(os.path.join(ROOT, "profiles", "traffic.json"))
 
 
-def roofline_entry(flops, nbytes, seconds):
+def roofline_entry(flops, nbytes, seconds, kernel=""):
     """Prices `seconds` against the roof that bounds a kernel of this intensity."""
-    if nbytes > 0 and flops / nbytes > RIDGE:
+    peak = round(MFMA_BF16_PEAK_TFLOPS / 6, 1) if kernel.startswith("split_gemm") else MFMA_FP32_PEAK_TFLOPS
+    if nbytes > 0 and flops / nbytes > RIDGE * peak / MFMA_FP32_PEAK_TFLOPS:
         achieved = flops / seconds / 1e12
-        return dict(bound="mfma", achieved=round(achieved, 3), peak=MFMA_FP32_PEAK_TFLOPS, unit="TFLOP/s",
-                    frac=round(achieved / MFMA_FP32_PEAK_TFLOPS, 4))
+        return dict(bound="mfma", achieved=round(achieved, 3), peak=peak, unit="TFLOP/s", frac=round(achieved / peak, 4))
     achieved = nbytes / seconds / 1e9
     return dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                 frac=round(achieved / HBM_PEAK_GBS, 4))
@@ -275,7 +276,7 @@ def bench_model(model_dir, steps, warmup):
         model.close()
     dominant = max(by_symbol, key=lambda k: by_symbol[k]["seconds"])
     d = by_symbol[dominant]
-    roof = roofline_entry(d["flops"], d["bytes"], d["seconds"])
+    roof = roofline_entry(d["flops"], d["bytes"], d["seconds"], dominant)
     traffic_table, traffic_stale = measured_traffic()
     roof.update(kernel=dominant, launches_per_step=d["launches"],
                 avg_launch_us=round(d["seconds"] / d["launches"] * 1e6, 2),
@@ -283,7 +284,7 @@ def bench_model(model_dir, steps, warmup):
                 algorithmic_bytes_per_launch=round(d["bytes"] / d["launches"]),
                 traffic=traffic_table.get(dominant), traffic_stale=traffic_stale)
     symbols = {k: dict(us_per_step=round(v["seconds"] * 1e6, 1), launches=v["launches"],
-                       **roofline_entry(v["flops"], v["bytes"], v["seconds"])) for k, v in by_symbol.items()}
+                       **roofline_entry(v["flops"], v["bytes"], v["seconds"], k)) for k, v in by_symbol.items()}
     return dict(ms_per_step=seconds / steps * 1e3, kernel_ms_per_step=kernel_seconds * 1e3, roofline=roof,
                 symbols=symbols, ops=ops, marker_us=marker_ms * 1e3, plan_kernels=[names[i] for i in range(n_ops)])
 
@@ -321,7 +322,7 @@ def bench_kernels(cold=True, only=None):
         """One configuration's line: `frac` (and us, achieved) are the cold-cache launch, operands from
         memory; `frac_warm` / `us_warm` the same kernel launched back to back on one operand set, which a
         working set below the 256 MB memory-side cache flatters."""
-        cold, warm = roofline_entry(flops, nbytes, cold_s), roofline_entry(flops, nbytes, warm_s)
+        cold, warm = (roofline_entry(flops, nbytes, s, last_kernel(lib)) for s in (cold_s, warm_s))
         out.append(dict(config=name, kernel=last_kernel(lib), us=round(cold_s * 1e6, 2), us_warm=round(warm_s * 1e6, 2),
                         flops=flops, bytes=nbytes, frac_warm=warm["frac"], achieved_warm=warm["achieved"],
                         operand_sets=sets_for(nbytes), **cold))
