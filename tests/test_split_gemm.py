@@ -61,6 +61,25 @@ def test_products(hip, split, shape, m, n, k):
     assert (np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= _bound(a, b, k)).all()
 
 
+@pytest.mark.parametrize("shape", [s + 10 * (n - 1) for s in SHAPES for n in (1, 3)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (33, 31, 36), (64, 64, 64), (129, 130, 132), (300, 97, 100), (70, 64, 1300), (33, 193, 2052)])
+def test_a_transposed_operand(hip, split, shape, m, n, k):
+    """Its rows end where the next begins: what a fetch holds of that is not multiplied, and an Inf or NaN there neither."""
+    rng = np.random.default_rng(m * n + k)
+    a, b = rng.standard_normal((2, m, k)).astype(np.float32), rng.standard_normal((2, n, k)).astype(np.float32)
+    split(shape)
+    got = hip.batch_matmul(a, b, transpose_b=True)
+    assert _took_it()
+    assert (np.abs(got - a.astype(np.float64) @ b.transpose(0, 2, 1).astype(np.float64)) <= _bound(a, b.transpose(0, 2, 1), k)).all()
+    b[:, n // 2] = np.nan
+    a[0, m // 2] = np.inf
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ b.transpose(0, 2, 1).astype(np.float64)
+    got = hip.batch_matmul(a, b, transpose_b=True)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("slices", [2, 3, 8])
 @pytest.mark.parametrize("m,n,k", [(70, 64, 1300), (33, 97, 2049)])

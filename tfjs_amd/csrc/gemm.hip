@@ -18,6 +18,10 @@ int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, 
       if (split.shape >= 0) return launch_split_gemm(split, p, kLoadKAny);
     }
   }
+  if (!transpose_a && transpose_b && vec && !float_bits) {
+    const SplitChoice split = split_gemm_choice(p, kLoadKAny);
+    if (split.shape >= 0) return launch_split_gemm(split, p, kLoadKAny, true);
+  }
   if (vec) {
     const int shape = choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus());
     if (!transpose_a && !transpose_b) return launch_gemm_shape<kLoadKVec, kLoadXVec>(shape, p);

@@ -258,14 +258,14 @@ int launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, bool ve
 int launch_ragged_gemm(GemmParams &p, bool transpose_b);
 
 // The tile and the slices of k with which the kernel on the bf16 matrix cores (split_gemm.h) takes a product of a row-major B
-// and a row-major A or windows of an image; shape -1: it goes to gemm_kernel. `us`: what it takes, by
+// and a row-major A or windows of an image, or of a row-major A and a transposed B where float4s fit both; shape -1: it goes to gemm_kernel. `us`: what it takes, by
 // estimate. Its launch; a_kind: kLoadKAny, kLoadWindows or kLoadWindowsAny.
 struct SplitChoice {
   int shape, slices;
   double us;
 };
 SplitChoice split_gemm_choice(const GemmParams &p, int a_kind);
-int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind);
+int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind, bool transposed_b = false);
 
 // Fills the bias / prelu part of an Epilogue from caller strides over `rank`
 // output dims (3: batch,row,col; 4: n,h,w,c) after validating them. Sets

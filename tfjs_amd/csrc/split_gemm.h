@@ -9,7 +9,8 @@
 // 5.0e-7, 9.8e-7, this kernel 0.5e-7, 0.9e-7, 1.6e-7, 3.4e-7; all-positive operands 1.2e-7 ... 8.3e-7 and 0.5e-7 ... 3.0e-7.
 //
 // us, gemm_kernel and here (rate of the product itself): 1024 x 2304 x 768 33.8 and 25.4 (142 TFLOP/s), 1024 x 3072 x 768 41.5
-// and 30.4, 3072 x 3072 x 1024 154 and 106 (183), 3072 x 4096 x 1024 189 and 131 (197), [8,56,56,64] 3x3 -> 64 27.0 and 18.5.
+// and 30.4, 3072 x 3072 x 1024 154 and 106 (183), 3072 x 4096 x 1024 189 and 131 (197), [8,56,56,64] 3x3 -> 64 27.0 and 17.8.
+// Of a transposed B, 128 x (384 x 64 x 384) 36 and 31, 128 x (512 x 64 x 512) 56 and 44, 1024 x 3072 x 768 39.9 and 30.2.
 // What bounds it: on the largest the matrix cores, three quarters of the time; the rest waits for fetches and barriers. On
 // 1024 rows, 6 us of launch, prologue (2.5: arguments, the first fetch, the first tile's splitting) and results (2.7).
 //
@@ -100,13 +101,14 @@ __device__ __forceinline__ float one_of_a(const GemmParams &p, __amdgpu_buffer_r
   return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)(in ? at : kNoOffset), 0, 0));
 }
 
-// A_KIND: kLoadKAny (row-major), kLoadWindows or kLoadWindowsAny. B_KIND: kLoadXVec (row-major), kLoadFilter. Any extents
+// A_KIND: kLoadKAny (row-major), kLoadWindows or kLoadWindowsAny. B_KIND: kLoadXVec (row-major), kLoadFilter, kLoadKVec
+// (transposed: a row per column, K a multiple of four; its lanes run along k, eight to a column). Any extents otherwise
 // and any 4-byte alignment: what lies beyond an operand reads as zero, and what the last fetch of a row of A holds of the
 // next row meets rows of B that are zero.
 template <int GW, int TN, int KG, int A_KIND, int B_KIND>
 __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
   using T = SplitTile<GW, TN, KG>;
-  constexpr bool kWindows = A_KIND != kLoadKAny;
+  constexpr bool kWindows = A_KIND != kLoadKAny, kColumns = B_KIND == kLoadKVec;
   extern __shared__ char split_lds[];
   // (the arguments of the prologue in one piece, as in gemm_kernel)
   asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.batch), "s"(p.a_sx), "s"(p.b_sk), "s"(p.a_bytes),
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
 #pragma unroll
   for (int v = 0; v < 4; ++v) a_from[v] = r * 128 + (((4 * (v >> 1) + 2 * h + (v & 1)) ^ r) & 7) * 16;
   int row_ih[4], row_iw[4];
-  unsigned a_off[4], b_off;
+  unsigned a_off[4], b_off[kColumns ? T::XW : 1];
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int row = m0 + 32 * wave + 8 * v + (lane >> 3);
@@ -142,15 +144,18 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
     else a_off[v] = row < p.M ? 4u * ((unsigned)row * (unsigned)p.a_sx + 4u * (unsigned)(lane & 7)) : kNoOffset;
   }
   // B: this thread fetches the four k from 4 kb on of columns XW xb .. XW xb + XW - 1
-  const int kb = tid >> 3 & 7, xb = (tid & 7) + (tid >> 6) * 8;
+  const int kb = kColumns ? tid & 7 : tid >> 3 & 7, xb = (kColumns ? tid >> 3 & 7 : tid & 7) + (tid >> 6) * 8;
   int b_to[T::XW], b_from[2];
 #pragma unroll
   for (int c = 0; c < T::XW; ++c) b_to[c] = plane_offset(T::XW * xb + c, kb >> 1) + (kb & 1) * 8;
 #pragma unroll
   for (int s = 0; s < 2; ++s) b_from[s] = plane_offset(r, 2 * s + h);
-  {
-    const int x = n0 + T::XW * xb;
-    b_off = x < p.N ? 4u * ((B_KIND == kLoadFilter ? 0u : 4u * (unsigned)kb * (unsigned)p.b_sk) + (unsigned)x) : kNoOffset;
+#pragma unroll
+  for (int c = 0; c < (kColumns ? T::XW : 1); ++c) {
+    const int x = n0 + T::XW * xb + c;
+    const unsigned at = kColumns ? (unsigned)x * (unsigned)p.b_sx + 4u * (unsigned)kb
+                                 : (B_KIND == kLoadFilter ? 0u : 4u * (unsigned)kb * (unsigned)p.b_sk) + (unsigned)x;
+    b_off[c] = x < p.N ? 4u * at : kNoOffset;
   }
 
   uint4_t ra[4];   // fetched, not yet in LDS
@@ -176,6 +181,16 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
   auto load_b = [&](int tile) __attribute__((always_inline)) {
     const int k0 = tile_k(tile);
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, k0 < k_end ? (int)p.b_bytes : 0, 0x00020000);
+    if constexpr (kColumns) {   // (of k beyond the end nothing, whatever A holds there)
+#pragma unroll
+      for (int c = 0; c < T::XW; ++c) {
+        const unsigned off = k0 + 4 * kb < k_end ? __builtin_elementwise_add_sat(b_off[c], 4u * (unsigned)k0) : kNoOffset;
+        const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rb[j][c] = __uint_as_float(v[j]);
+      }
+      return;
+    }
     unsigned unit = 4u * (unsigned)k0 * (unsigned)p.b_sk;
     int live = 4;
     if (B_KIND == kLoadFilter) {
@@ -185,7 +200,7 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      unsigned off = __builtin_elementwise_add_sat(b_off, unit + 4u * (unsigned)j * (unsigned)p.b_sk);
+      unsigned off = __builtin_elementwise_add_sat(b_off[0], unit + 4u * (unsigned)j * (unsigned)p.b_sk);
       if (B_KIND == kLoadFilter) off = j < live ? off : kNoOffset;
       if constexpr (T::XW == 4) {
         const uint4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off, 0, 0);
@@ -443,7 +458,7 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
         for (int j = 0; j < TN; ++j) {
           const int x = n0 + 32 * j + r;
           const float b = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-              rsrc_b, (int)(b_row >= 0 && x < p.N ? 4u * ((unsigned)b_row * (unsigned)p.b_sk + (unsigned)x) : kNoOffset), 0, 0));
+              rsrc_b, (int)(b_row >= 0 && x < p.N ? 4u * ((unsigned)b_row * (unsigned)p.b_sk + (unsigned)x * (unsigned)(kColumns ? p.b_sx : 1)) : kNoOffset), 0, 0));
           acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b, a, acc[j], 0, 0, 0);
         }
       }

@@ -142,7 +142,8 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
   return best;
 }
 
-int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind) {
+int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind, bool transposed_b) {
+  if (transposed_b) return launch_kind<kLoadKAny, kLoadKVec>(choice, p);
   if (a_kind == kLoadWindows) return launch_kind<kLoadWindows, kLoadXVec>(choice, p);
   if (a_kind == kLoadWindowsAny) return launch_kind<kLoadWindowsAny, kLoadFilter>(choice, p);
   return launch_kind<kLoadKAny, kLoadXVec>(choice, p);
