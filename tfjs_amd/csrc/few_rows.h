@@ -345,9 +345,9 @@ inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_bloc
 // Strips of 64 columns, whole cache lines and a quarter of the tiles to share the slices among, where strips of 16
 // (cut as `narrow` says) find no compute unit of their own each, or where a workgroup of theirs would fetch more than twice
 // (with two row blocks three times) what it can have out at once; else strips of 16: as many workgroups as there are.
-// us, strips of 16 and 64: 1 x 2048 x 4096 8.1 and 9.0, 1 x 2304 x 4000 9.6 and 8.5; 32 x 1536 x 2304 10.1 and 10.8,
-// 32 x 3072 x 2304 17.9 and 11.6; 48 x 2304 x 768 10.4 and 8.7, 160 x 8192 x 256 28.5 and 12.8; 1 x 1024 x 4096 5.3 and
-// 7.6, 1 x 1024 x 4112 8.5 and 7.6.
+// us, strips of 16 and 64: 32 x 1536 x 2304 8.5 and 10.7, 32 x 3072 x 2304 16.3 and 11.5, 160 x 8192 x 256 24.1 and 12.0;
+// 1 x 1024 x 4096 3.9 and 4.8. Just beyond the lines the strips of 16 are still ahead since their fetches are refilled one by one
+// (1 x 1024 x 4112 5.0 and 5.9, 1 x 2304 x 4000 6.8 and 7.6, 48 x 2304 x 768 7.2 and 8.1); the tests of the dispatch have them here.
 inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
   return narrow.tiles > num_cus() || narrow.groups_per_split > (row_blocks == 1 ? 128 : 96);
 }
@@ -362,8 +362,11 @@ inline bool few_rows_can(const GemmParams &p, bool windows) {
 // Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
 // tiled kernel (`vec`: that one can fetch both operands in float4s). As long as every workgroup has a compute unit of its
 // own, the fetches of a whole k range are out at once, where the tiled kernel goes round its pipeline once per 32 k (us,
-// tiled and here: 49 x 960 x 160 9.2 and 5.6, 196 x 576 x 96 6.9 and 5.4, 80 x 768 x 768 8.1 and 5.7; windows,
-// [2,35,34,120] 3x3/2 -> 16 11.5 and 7.1). The lines, each from a grid of extents on both sides, in the same form:
+// tiled and here: 49 x 960 x 160 9.2 and 4.2, 196 x 576 x 96 6.9 and 3.6, 80 x 768 x 768 8.1 and 4.2; windows,
+// [2,35,34,120] 3x3/2 -> 16 11.5 and 5.8). The lines, each from a grid of extents on both sides, in the same form. Those from the
+// third on were measured with eight groups out at once; with two, refilled one by one, this kernel has gained 10 to 40%, so they
+// are on the safe side now (32 x 512 x 8192 in 5.6 with one row block, 128 x 3072 x 768 in 11.3), and are left where the tests
+// of the dispatch have them:
 //  * more than 32 rows, K < 320: 0.85 of the time at K = 16, 0.77 at 96, 0.6 at 300 (256 x 256 x 256 5.6 and 4.2, 784 x 192 x 32
 //    4.5 and 2.9), except where the caller wants the sums of gemm_kernel (`float_bits`), and not for ragged rows, on which
 //    the same is left: the tests of the ragged loader count on it there.
