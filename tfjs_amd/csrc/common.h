@@ -228,7 +228,7 @@ inline int64_t strided_extent(const int64_t *dims, const int64_t *strides, int r
 }
 
 // n / d as a multiplication by ceil(2^32 / d), 0 standing for d = 1: exact for n below 2^32 / d.
-inline unsigned magic_of(int d) { return d <= 1 ? 0u : (unsigned)(((1ULL << 32) + (unsigned)d - 1) / (unsigned)d); }
+inline unsigned magic_of(int d) { return d <= 1 ? 0u : 0xffffffffu / (unsigned)d + 1; }
 __device__ __forceinline__ int by_magic(int n, unsigned magic) { return magic ? (int)__umulhi((unsigned)n, magic) : n; }
 
 }  // namespace tfhip
