@@ -153,3 +153,37 @@ def test_what_parts_cannot_multiply(hip, split, shape):
     assert (np.abs(got.astype(np.float64) - want) <= (k * 2.0 ** -24 + 2.0 ** -20) * size + 2.0 ** -149 * k).all()
     # tiny rows keep float32's precision
     assert (np.abs(got[30] - want[30]) <= k * 2.0 ** -24 * size[30]).all()
+
+
+# Exponents of the two operands: one so small that its lower parts, or all of it, lie below the smallest bf16, against an ordinary
+# or a large one; both small; sums beyond what an accumulator of scaled parts holds; an operand beyond it.
+SIZES = [(-120, 100), (-125, 100), (-130, 110), (-135, 120), (-149, 126), (-140, 35), (-149, 0), (-140, -5), (-60, -64), (50, 50), (110, -100),
+         (126, -70)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("form", ["plain", "transposed", "windows", "ragged windows"])
+def test_operands_of_every_size(hip, split, shape, form):
+    """Nothing of an operand is lost, whatever the other one is. One rounding per product, as with float32 instructions, and 24 for
+    what else a result passes through; a subnormal result is off by its last place, once per product at most."""
+    rng = np.random.default_rng(shape)
+    mantissa = 1 + 2.0 ** -14 - 2.0 ** -20   # what bf16 parts lose of it has one sign
+    split(shape)
+    for small, large in SIZES:
+        for ea, eb in ((small, large), (large, small)):
+            if form.endswith("windows"):
+                c = 8 if form == "windows" else 5
+                x = np.full((1, 12, 11, c), np.ldexp(mantissa, ea), np.float32)
+                w = np.ldexp(rng.uniform(1, 2, (3, 3, c, 21)), eb).astype(np.float32)
+                got = hip.fused_conv2d(x, w).reshape(90, 21)
+                a = np.stack([x[0, i:i + 3, j:j + 3].reshape(-1) for i in range(10) for j in range(9)])
+                b = w.reshape(9 * c, 21)
+            else:
+                a = np.full((150, 100), np.ldexp(mantissa, ea), np.float32)
+                b = np.ldexp(rng.uniform(1, 2, (100, 70)), eb).astype(np.float32)
+                transposed = form == "transposed"
+                got = hip.batch_matmul(a[None], np.ascontiguousarray(b.T if transposed else b)[None], transpose_b=transposed)[0]
+            assert _took_it()
+            want = a.astype(np.float64) @ b.astype(np.float64)   # (all positive: the sum of the products' sizes too)
+            k = a.shape[1]
+            assert (np.abs(got - want) <= (k + 24) * 2.0 ** -24 * want + k * 2.0 ** -149).all(), (ea, eb)
