@@ -187,3 +187,40 @@ def test_operands_of_every_size(hip, split, shape, form):
             want = a.astype(np.float64) @ b.astype(np.float64)   # (all positive: the sum of the products' sizes too)
             k = a.shape[1]
             assert (np.abs(got - want) <= (k + 24) * 2.0 ** -24 * want + k * 2.0 ** -149).all(), (ea, eb)
+
+
+@pytest.mark.parametrize("shape", [s + 10 * (n - 1) for s in SHAPES for n in (1, 2)])
+@pytest.mark.parametrize("form", ["plain", "transposed", "windows", "ragged windows"])
+@pytest.mark.parametrize("largest", [1.0, 1e32])   # (the largest: among sums that are kept, and of a tile that is done again)
+def test_inf_and_nan(hip, split, shape, form, largest):
+    """Results that an Inf or NaN enters are what IEEE arithmetic makes of them, all others what they are without."""
+    rng = np.random.default_rng(shape)
+    split(shape)
+    if form.endswith("windows"):
+        c = 8 if form == "windows" else 5
+        x, w = rng.standard_normal((1, 24, 15, c)).astype(np.float32), rng.standard_normal((3, 3, c, 37)).astype(np.float32)
+        x[0, 4, 4, 2], x[0, 12, 2, 1], x[0, 12, 4, 1], x[0, 20, 10, c - 1] = np.nan, np.inf, -np.inf, np.inf
+        x[0, 17, 6, 0] = largest
+        w[1, 1, 2, 5], w[0, 2, 1, 6], w[:, :, :, 7] = np.inf, 0, 1   # (1: all but its high part is zero)
+        a = np.stack([x[0, i:i + 3, j:j + 3].reshape(-1) for i in range(22) for j in range(13)])
+        b = w.reshape(9 * c, 37)
+        run = lambda: hip.fused_conv2d(x, w).reshape(a.shape[0], 37)
+    else:
+        m, n, k = 150, 70, 132 if form == "transposed" else 131
+        a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+        a[3, 0], a[9, 100], a[9, 101], a[20, 50], a[140, k - 1] = np.inf, np.inf, -np.inf, np.nan, -np.inf
+        a[30], a[31, :] = 0, 2.0 ** -149
+        a[40, 7] = largest
+        b[:, 11], b[0, 12], b[100, 13], b[5, 14], b[k - 1, 69] = 1, 0, 2.0 ** -149, np.inf, np.nan
+        args = (np.ascontiguousarray(b.T)[None], True) if form == "transposed" else (b[None], False)
+        run = lambda: hip.batch_matmul(a[None], args[0], transpose_b=args[1])[0]
+    got = run()
+    assert _took_it()
+    with np.errstate(invalid="ignore"):
+        want = (a.astype(np.float64)[:, :, None] * b.astype(np.float64)[None]).sum(1)
+        size = np.abs(a.astype(np.float64)[:, :, None] * b.astype(np.float64)[None]).sum(1)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    # one rounding per product, as with float32 instructions, and 24 for what else a result passes through
+    assert (np.abs(got[fine] - want[fine]) <= (a.shape[1] + 24) * 2.0 ** -24 * size[fine] + a.shape[1] * 2.0 ** -149).all()

@@ -20,8 +20,12 @@
 // 2^-134 everything, whatever it is multiplied by; encoder layers of [8,128] and [8,384] took 1.4% and 2.7% less, [8,56,56,64]
 // 3x3 -> 64 17.8 us (18.4 with it).
 //
-// What is left, the last stage sees in the results, and the tile is done again with float32 instructions: an Inf or NaN in an
-// operand, an operand from 2^104 on or a sum from 2^80 on makes every result it enters Inf or NaN.
+// An Inf or NaN in an operand, an operand from 2^104 on or a sum from 2^80 on makes every result it enters Inf or NaN, not
+// always the right one of the two; the last stage sees them. It then fetches the tile's operands once more for the largest
+// float of each. Where these are small enough that nothing can have overflowed, the sums of the high parts alone are right for
+// such results; else the tile is done again with float32 instructions, one float per lane and fetch. us, without an Inf or NaN,
+// with one, with one in every row: 1024 x 2304 x 768 28, 41, 42, 3072 x 3072 x 1024 107, 138, 159, [8,56,56,64] 3x3 -> 64 18.4, 30, 31
+// (gemm_kernel 34 to 38, 154 and 27.5, all the same); with an operand of 1e32 94, 225 and 78.
 //
 // One workgroup: KG groups of GW wavefronts share a tile of 32 GW x 32 TN results; every group takes every KG-th k tile of
 // 32. A wavefront owns 32 rows.
@@ -367,19 +371,18 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
   }
   lds_barrier();
   float *sums = reinterpret_cast<float *>(split_lds);   // [KG][BM][PITCH]
-  int *again = reinterpret_cast<int *>(split_lds + T::SUM_BYTES);
-  auto write_sums = [&]() __attribute__((always_inline)) {
+  unsigned *seen = reinterpret_cast<unsigned *>(split_lds + T::SUM_BYTES);   // an Inf or NaN; the largest float of A's rows, of B's columns
+  auto write_sums = [&](auto sum_of) __attribute__((always_inline)) {
     float *mine = sums + (group * T::BM + 32 * wave + r) * T::PITCH + 4 * h;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<float4_t *>(mine + 32 * j + 8 * q) = (float4_t){acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+      for (int q = 0; q < 16; q += 4)
+        *reinterpret_cast<float4_t *>(mine + 32 * j + 2 * q) =
+            (float4_t){sum_of(acc[j][q], low[j][q]), sum_of(acc[j][q + 1], low[j][q + 1]), sum_of(acc[j][q + 2], low[j][q + 2]), sum_of(acc[j][q + 3], low[j][q + 3])};
   };
-#pragma unroll
-  for (int j = 0; j < TN; ++j) acc[j] += low[j];
-  if (threadIdx.x == 0) *again = 0;
-  write_sums();
+  if (threadIdx.x < 3) seen[threadIdx.x] = 0;
+  write_sums([](float high, float small) { return high + small; });
   lds_barrier();
   const bool to_ws = p.splits > 1;
   const int ldc = to_ws ? p.N : (int)p.ldc;
@@ -392,8 +395,7 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
   const int rows = row0 >= kRowsAtOnce || col >= p.N ? 0 : (p.M - m0 < T::BM ? p.M - m0 : T::BM);
   const unsigned first = 4u * ((unsigned)(m0 + row0) * (unsigned)ldc + (unsigned)col), stride = 4u * (unsigned)(kRowsAtOnce * ldc);
   float unscale = kSplitUnscale;
-  auto finish = [&](auto act_tag) __attribute__((always_inline)) {
-    constexpr int ACT = decltype(act_tag)::value;
+  auto finish = [&](auto act) __attribute__((always_inline)) {   // (an integral_constant or an int)
 #pragma unroll 2
     for (int i = 0; i < kPasses; ++i) {
       const int row = row0 + i * kRowsAtOnce;
@@ -406,13 +408,13 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
         bool bad = false;   // (what lies beyond the last column does not matter)
 #pragma unroll
         for (int q = 0; q < 4; ++q) bad |= col + q < p.N && !(fabsf(v[q]) < INFINITY);
-        if (bad) *again = 1;
+        if (bad) seen[0] = 1;
       }
       float res[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float x = v[q] * unscale + bias[q];
-        res[q] = ACT == TFHIP_LINEAR ? x : activate(x, ACT, alpha[q], e.leaky_alpha);
+        res[q] = act == TFHIP_LINEAR ? x : activate(x, act, alpha[q], e.leaky_alpha);
       }
       const unsigned at = first + (unsigned)i * stride;
       if (residual) {
@@ -428,23 +430,54 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
       }
     }
   };
-  auto finish_all = [&]() __attribute__((always_inline)) {
-    switch (fused ? e.activation : TFHIP_LINEAR) {
-      case TFHIP_RELU: finish(std::integral_constant<int, TFHIP_RELU>()); break;
-      case TFHIP_RELU6: finish(std::integral_constant<int, TFHIP_RELU6>()); break;
-      case TFHIP_PRELU: finish(std::integral_constant<int, TFHIP_PRELU>()); break;
-      case TFHIP_LEAKYRELU: finish(std::integral_constant<int, TFHIP_LEAKYRELU>()); break;
-      default: finish(std::integral_constant<int, TFHIP_LINEAR>()); break;
-    }
-  };
+  const int activation = fused ? e.activation : TFHIP_LINEAR;
+  switch (activation) {
+    case TFHIP_RELU: finish(std::integral_constant<int, TFHIP_RELU>()); break;
+    case TFHIP_RELU6: finish(std::integral_constant<int, TFHIP_RELU6>()); break;
+    case TFHIP_PRELU: finish(std::integral_constant<int, TFHIP_PRELU>()); break;
+    case TFHIP_LEAKYRELU: finish(std::integral_constant<int, TFHIP_LEAKYRELU>()); break;
+    default: finish(std::integral_constant<int, TFHIP_LINEAR>()); break;
+  }
+  lds_barrier();
+  if (seen[0] == 0) return;   // (the same for the whole workgroup)
+
+  // The sums of the high parts are right where an Inf or NaN enters them (a high part is zero for a zero only, so Inf times
+  // anything else is Inf), and where none does the small products are finite, unless an operand or a sum is too large.
+  __builtin_assume(tiles > 0);   // (a slice without any sums up zeros)
+  unsigned most_a = 0, most_b = 0;
 #pragma unroll 1
-  for (int pass = 0;; ++pass) {
-    finish_all();
-    if (pass > 0) return;
-    lds_barrier();
-    if (*again == 0) return;   // (the same for the whole workgroup)
-    unscale = 1.f;
+  for (int tile = 0; tile < tiles; ++tile) {
+    load_a(tile);
+    load_b(tile);
+    // (behind a row of A lies the next one: an Inf there meets zeros of B, and counts as too large)
+    const int live = kWindows ? 4 : k_end - tile_k(tile) - 4 * (lane & 7);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint4_t x = A_KIND == kLoadWindowsAny ? __builtin_bit_cast(uint4_t, fix_up<A_KIND>(as_float4(ra[v]), fix[v])) : ra[v];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const unsigned size = x[j] & 0x7fffffffu;
+        if (size < 0x7f800000u || j >= live) most_a = max(most_a, size);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < T::XW; ++c) {
+        const unsigned size = __float_as_uint(rb[j][c]) & 0x7fffffffu;
+        if (size < 0x7f800000u) most_b = max(most_b, size);
+      }
+  }
+  atomicMax(seen + 1, most_a);
+  atomicMax(seen + 2, most_b);
+  lds_barrier();
+  // below 2^(exponent - 126) each, of fewer than 2^bits products: scaled and rounded up, a part and the sums stay below 2^128
+  const int exponent_a = (int)(seen[1] >> 23), exponent_b = (int)(seen[2] >> 23), bits = 32 - __builtin_clz((unsigned)(k_end - k_begin));
+  if (exponent_a <= 229 && exponent_b <= 229 && exponent_a + exponent_b + bits <= 331) {
+    write_sums([](float high, float small) { return fabsf(high) < INFINITY ? high + small : high; });
+  } else {
     // The tile once more, with float32 matrix instructions: lane (h, r) multiplies k + h of row r and of column 32 j + r.
+    unscale = 1.f;
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)p.a_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)p.b_bytes, 0x00020000);
     const int row = m0 + 32 * wave + r;
@@ -470,9 +503,10 @@ __global__ __launch_bounds__(64 * GW * KG, 2) void split_gemm(GemmParams p) {
           acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b, a, acc[j], 0, 0, 0);
         }
       }
-    write_sums();   // (nobody reads the old ones any more)
-    lds_barrier();
+    write_sums([](float sum, float) { return sum; });
   }
+  lds_barrier();
+  finish(activation);
 }
 
 }  // namespace tfhip
