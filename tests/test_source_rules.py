@@ -75,3 +75,23 @@ def test_the_checker_sees_what_it_is_meant_to_refuse():
     assert _asm_statements(_strip_comments(ok)) == [(2, "")]
     two = 'void h() { __asm__ __volatile__("s_nop 0\\n" "s_nop 1" ::: "memory"); }'
     assert _asm_statements(_strip_comments(two))[0][1] == "s_nop 0\\ns_nop 1"
+
+
+# A static of a function is shared by every thread that launches. The two that are plain are read and written with the staging
+# ring's mutex held.
+STATIC = re.compile(r"^[ \t]+static (?!constexpr\b|const\b|inline\b|std::atomic<|std::mutex\b|thread_local\b)([^;({=]*)[;{=]", re.M)
+GUARDED = ("CopyCrew *crew", "pid_t owner")
+
+
+def _shared_statics(text):
+    return [m.group(1).strip() for m in STATIC.finditer(_strip_comments(text))]
+
+
+def test_no_static_that_two_launching_threads_write():
+    seen = []
+    for path in _sources():
+        for declared in _shared_statics(open(path).read()):
+            assert declared in GUARDED, "%s: static %s: a data race; std::atomic" % (os.path.relpath(path, ROOT), declared)
+            seen.append(declared)
+    assert sorted(seen) == sorted(GUARDED)
+    assert _shared_statics("void f() {\n  static int raised = 0;\n  static std::atomic<int> fine{0};\n}") == ["int raised"]

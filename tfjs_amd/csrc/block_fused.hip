@@ -331,12 +331,9 @@ __global__ __launch_bounds__(kThreads) void inverted_residual_block(BlockArgs g)
 
 template <int S, int KF, int TEAM>
 int launch_block(const BlockArgs &g, size_t lds_bytes) {
-  static int raised = 0;
-  if (raised != init_count()) {
-    TFHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(inverted_residual_block<S, KF, TEAM>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    raised = init_count();
-  }
+  static std::atomic<int> raised{0};
+  const int rc = raise_lds_limit(raised, reinterpret_cast<const void *>(inverted_residual_block<S, KF, TEAM>), 160 * 1024);
+  if (rc != kOk) return rc;
   note_kernel("inverted_residual_block<%d, %d, %d>", S, KF, TEAM);
   TFHIP_LAUNCH((inverted_residual_block<S, KF, TEAM><<<dim3((unsigned)(g.batch * g.chunks_h)), dim3(kThreads), lds_bytes, stream()>>>(g)));
   return kOk;

@@ -7,6 +7,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
 #include <mutex>
 #include <tuple>
 #include <utility>
@@ -132,6 +133,16 @@ bool capturing();
   do {                                                            \
     if (!(cond)) return ::tfhip::fail(::tfhip::kBadArgument, __VA_ARGS__); \
   } while (0)
+
+// A launch with more dynamic LDS than the default limit needs an attribute of the kernel, once per device set-up. `raised`: the
+// set-up for which the caller's kernel has it; several threads may launch it for the first time, and each may set it.
+inline int raise_lds_limit(std::atomic<int> &raised, const void *kernel, int bytes) {
+  const int now = init_count();
+  if (raised.load(std::memory_order_acquire) == now) return kOk;
+  TFHIP_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  raised.store(now, std::memory_order_release);
+  return kOk;
+}
 
 // Operand `name` of `elems` float-sized (`esize` bytes) elements must be live.
 #define TFHIP_CHECK_RANGE(ptr, elems, esize, name)                             \

@@ -298,13 +298,9 @@ __global__ __launch_bounds__(256) void expand_dw_3x3(ExpandDwArgs g, StemTaps ta
 
 template <int S, int KF, bool HALF, int ACT, int TAPS>
 int launch_expand_dw_act(const ExpandDwArgs &g, const StemTaps &taps, size_t lds_bytes) {
-  // dynamic LDS above the default limit needs the attribute once per instantiation and device set-up
-  static int raised = 0;
-  if (raised != init_count()) {
-    TFHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(expand_dw_3x3<S, KF, HALF, ACT, TAPS>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    raised = init_count();
-  }
+  static std::atomic<int> raised{0};
+  const int rc = raise_lds_limit(raised, reinterpret_cast<const void *>(expand_dw_3x3<S, KF, HALF, ACT, TAPS>), 160 * 1024);
+  if (rc != kOk) return rc;
   const long long wgs = (long long)g.batch * g.chunks_h * g.tiles_w;
   note_kernel("expand_dw_3x3<%d, %d, %s, %d, %d>", S, KF, HALF ? "true" : "false", ACT, TAPS);
   TFHIP_LAUNCH((expand_dw_3x3<S, KF, HALF, ACT, TAPS><<<dim3((unsigned)wgs), dim3(256), lds_bytes, stream()>>>(g, taps)));

@@ -271,13 +271,9 @@ __global__ __launch_bounds__(256) void expand_dw_tile(ExpandDwTileArgs g) {
 
 template <int S, int KF, bool HALF, int NCB>
 int launch_tile(const ExpandDwTileArgs &g, size_t lds_bytes) {
-  // dynamic LDS above the default limit needs the attribute once per instantiation and device set-up
-  static int raised = 0;
-  if (raised != init_count()) {
-    TFHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(expand_dw_tile<S, KF, HALF, NCB>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    raised = init_count();
-  }
+  static std::atomic<int> raised{0};
+  const int rc = raise_lds_limit(raised, reinterpret_cast<const void *>(expand_dw_tile<S, KF, HALF, NCB>), 160 * 1024);
+  if (rc != kOk) return rc;
   note_kernel("expand_dw_tile<%d, %d, %s, %d>", S, KF, HALF ? "true" : "false", NCB);
   const dim3 grid((unsigned)(g.batch * g.chunks_h), (unsigned)g.slices);
   TFHIP_LAUNCH((expand_dw_tile<S, KF, HALF, NCB><<<grid, dim3(256), lds_bytes, stream()>>>(g)));

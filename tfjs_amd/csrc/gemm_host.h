@@ -178,14 +178,10 @@ inline int launch_gemm(GemmParams &p) {
   if (grid > 0x7fffffffLL) return fail(kBadArgument, "gemm: %lld tiles exceed the grid limit", grid);
   number_tiles(p, grid);
   if (T::LDS_FLOATS * sizeof(float) > 64 * 1024) {   // (also with KG groups of buffers)
-    // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
-    static int raised = 0;
-    if (raised != init_count()) {
-      TFHIP_CHECK_HIP(hipFuncSetAttribute(
-          reinterpret_cast<const void *>(gemm_kernel<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>),
-          hipFuncAttributeMaxDynamicSharedMemorySize, (int)(T::LDS_FLOATS * sizeof(float))));
-      raised = init_count();
-    }
+    static std::atomic<int> raised{0};
+    const int rc = raise_lds_limit(raised, reinterpret_cast<const void *>(gemm_kernel<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>),
+                                   (int)(T::LDS_FLOATS * sizeof(float)));
+    if (rc != kOk) return rc;
   }
   note_kernel("gemm_kernel<%d, %d, %d, %d, %d, %d, %d, %d>", BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG);
   // The fused epilogue covers per-column operands with a relu-family activation;

@@ -395,7 +395,9 @@ __global__ __launch_bounds__(256) void skinny_gemm_regs(SkinnyArgs g) {
 
 template <int TN, int KF, bool HALF>
 inline int launch_skinny_regs(const SkinnyArgs &g, int column_groups) {
-  static int resident = 0;   // workgroups per compute unit at this instantiation's register count
+  // workgroups per compute unit at this instantiation's register count (threads that launch it first may each ask)
+  static std::atomic<int> known{0};
+  int resident = known.load(std::memory_order_relaxed);
   if (resident == 0) {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, skinny_gemm_regs<TN, KF, HALF, false>, 256, 0) != hipSuccess || n < 1) {
@@ -403,6 +405,7 @@ inline int launch_skinny_regs(const SkinnyArgs &g, int column_groups) {
       n = 1;
     }
     resident = n;
+    known.store(n, std::memory_order_relaxed);
   }
   // all workgroups resident at once; wavefront w takes row blocks w, w + waves, ...
   const long long blocks = (g.M + 15) / 16;

@@ -74,12 +74,9 @@ int launch_shape(GemmParams &p, int slices) {
   number_tiles(p, grid);
   const auto kernel = split_gemm<GW, TN, KG, A_KIND, B_KIND>;
   if (T::LDS_BYTES > 64 * 1024) {
-    // dynamic LDS above the default limit: the attribute once per instantiation and device set-up
-    static int raised = 0;
-    if (raised != init_count()) {
-      TFHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES));
-      raised = init_count();
-    }
+    static std::atomic<int> raised{0};
+    const int rc = raise_lds_limit(raised, reinterpret_cast<const void *>(kernel), T::LDS_BYTES);
+    if (rc != kOk) return rc;
   }
   note_kernel("split_gemm<%d, %d, %d, %d, %d>", GW, TN, KG, A_KIND, B_KIND);
   p.inline_epilogue = p.splits == 1 && p.epi.channel_operands && p.epi.activation <= TFHIP_LEAKYRELU;
