@@ -199,7 +199,7 @@ int tfhip_fused_matmul(const float *a, const float *b, float *out,
  * takes the largest number of slices that fits, down to one slice, which needs
  * no scratch: the result then has tfhip_fused_matmul's bits only where the two
  * slice counts agree, and is within the float32 bound otherwise. A slice count
- * the caller forced with the "splitk" knob is not reduced: if it does not fit,
+ * the caller forced with the "splitk" or the "split" knob is not reduced: if it does not fit,
  * the call fails with a message that states both sizes, and launches nothing.
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * (other threads, other streams) race on it. The array belongs to the calling

@@ -450,3 +450,32 @@ for first, second in zip(names[::2], names[1::2]):
     assert "gemm_kernel" in first and "gemm_finish" in second, names
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_slices_of_a_product_in_bf16_parts_fit_the_fixed_scratch():
+    """A caller's fixed scratch (16 MiB): slices that the caller forced and that it does not hold are refused, the library's own
+    choice comes down to what it holds."""
+    fake_hip_util.run("""
+pyhost.init()
+a, b, out = (DeviceBuffer(128 << 20) for _ in range(3))
+
+def product(m, n, k, entry=lib.tfhip_fused_matmul_noalloc):
+    return entry(a.ptr, b.ptr, out.ptr, 1, 1, m, n, k, 0, 0, None, None, 0, None, None, 0.2)
+
+check(lib.tfhip_set_tuning(b"split", 20))                 # three slices
+check(product(1024, 1365, 512))                           # 12288 bytes short of the array
+assert "split_gemm" in launch(1)[0] and pyhost.workspace_info()["last_splits"] == 3
+launches = fake.fake_hip_launches()
+assert product(1024, 1366, 512) != 0
+message = lib.tfhip_last_error().decode()
+assert str(3 * 1024 * 1366 * 4) in message and "16777216" in message, message
+assert fake.fake_hip_launches() == launches
+check(lib.tfhip_set_tuning(b"split", -1))
+for m, n, k in ((1280, 1280, 8192), (1344, 1536, 8192), (2432, 1024, 8192)):
+    check(product(m, n, k, lib.tfhip_fused_matmul))
+    wanted, fits = pyhost.workspace_info()["last_splits"], (16 << 20) // (m * n * 4)
+    assert "split_gemm" in launch(1)[0] and wanted > fits, (wanted, fits)
+    check(product(m, n, k))
+    assert pyhost.workspace_info()["last_splits"] == fits, (m, n, k)
+assert errors()[0] == 0, errors()
+""")

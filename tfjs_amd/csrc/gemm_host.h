@@ -110,6 +110,21 @@ inline void enqueue_finish(const GemmParams &p) {
   gemm_finish<<<dim3((unsigned)(blocks < cap ? blocks : cap)), dim3(256), 0, stream()>>>(p);
 }
 
+// Slices of k whose sums a caller's fixed scratch does not hold: a count the caller forced is refused, the library's own choice
+// comes down to what fits (one slice needs no scratch at all).
+inline int fit_fixed_scratch(const GemmParams &p, int &slices, bool forced) {
+  const size_t slice_bytes = (size_t)p.batch * p.M * p.N * sizeof(float);
+  if (slices <= 1 || !workspace_is_fixed() || (size_t)slices * slice_bytes <= fixed_workspace_bytes()) return kOk;
+  if (forced)
+    return fail(kBadArgument,
+                "gemm: %d K slices of a %d x %d x %d output need %zu bytes of scratch; the static array of the "
+                "entry point that allocates nothing holds %zu",
+                slices, p.batch, p.M, p.N, (size_t)slices * slice_bytes, fixed_workspace_bytes());
+  slices = (int)(fixed_workspace_bytes() / slice_bytes);
+  if (slices < 2) slices = 1;
+  return kOk;
+}
+
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int A_KIND, int B_KIND, int KG = 1>
 inline int launch_gemm(GemmParams &p) {
   using T = GemmTile<BM, BN, BK, WAVES_M, WAVES_N, A_KIND, B_KIND, KG>;
@@ -148,19 +163,8 @@ inline int launch_gemm(GemmParams &p) {
     const bool was_forced = forced > 0 && forced <= 64 && forced <= k_tiles;
     if (was_forced) best = forced;
     const size_t slice_bytes = (size_t)p.batch * p.M * p.N * sizeof(float);
-    if (best > 1 && workspace_is_fixed() && (size_t)best * slice_bytes > fixed_workspace_bytes()) {
-      // a caller's fixed scratch: a slice count the caller forced is refused, the library's own choice
-      // comes down to what fits (one slice needs no scratch at all). The library's own choice keeps
-      // slices x tiles within the compute units and a tile within 128 x 128, so on 256 units it never
-      // asks for more than 16 MiB; this is for a device with more of them.
-      if (was_forced)
-        return fail(kBadArgument,
-                    "gemm: %d K slices of a %d x %d x %d output need %zu bytes of scratch; the static array of the "
-                    "entry point that allocates nothing holds %zu",
-                    best, p.batch, p.M, p.N, (size_t)best * slice_bytes, fixed_workspace_bytes());
-      best = (int)(fixed_workspace_bytes() / slice_bytes);
-      if (best < 2) best = 1;
-    }
+    const int fits = fit_fixed_scratch(p, best, was_forced);
+    if (fits != kOk) return fits;
     if (best > 1) {
       const size_t bytes = (size_t)best * slice_bytes;
       held = lock_workspace();

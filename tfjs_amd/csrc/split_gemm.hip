@@ -21,6 +21,9 @@ constexpr SplitShape kSplitShapes[] = {
 constexpr int kNumSplitShapes = sizeof(kSplitShapes) / sizeof(kSplitShapes[0]);
 constexpr int kMaxSlices = 8;
 
+// Whether the knob names a tile and its slices.
+bool split_forced() { return tuning(kTuneSplit) >= 0 && tuning(kTuneSplit) < 80; }
+
 // The windows of an image cost their address arithmetic, ragged ones also what mends them.
 double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, double windows) {
   const long long tiles = ((p.M + 32 * s.gw - 1) / (32 * s.gw)) * (long long)((p.N + 32 * s.tn - 1) / (32 * s.tn)) * p.batch * slices;
@@ -57,10 +60,11 @@ int launch_shape(GemmParams &p, int slices) {
   p.k_per_split = p.K;
   p.ws = nullptr;
   std::unique_lock<std::mutex> held;
+  const int fits = fit_fixed_scratch(p, slices, split_forced());
+  if (fits != kOk) return fits;
   if (slices > 1) {
     const size_t bytes = (size_t)slices * p.batch * p.M * p.N * sizeof(float);
     held = lock_workspace();
-    // (nullptr where a caller's fixed scratch does not hold it: one slice)
     p.ws = bytes <= (size_t(1) << 30) ? static_cast<float *>(workspace(bytes)) : nullptr;
     if (p.ws) {
       p.splits = slices;
@@ -115,7 +119,7 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
       p.epi.addressing == kConv)
     return best;
   if (p.epi.channel_operands && (p.epi.bias_s[3] > 1 || p.epi.prelu_s[3] > 1)) return best;
-  if (forced >= 0 && forced < 80) return {forced % 10 % kNumSplitShapes, forced / 10 + 1, 0};
+  if (split_forced()) return {forced % 10 % kNumSplitShapes, forced / 10 + 1, 0};
   // Below 0.3 GFLOP the fixed part decides, and gemm_kernel's is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, 0.3 to 0.45
   // equal, 0.8 to 1.2 0.88 of the time, from 4 on 0.68; 13000 products); so it is with tiles that are mostly padding: few
   // columns, few rows of each product of a batch. Under 448 rows only half of the products gain.
