@@ -196,7 +196,8 @@ int tfhip_fused_matmul(const float *a, const float *b, float *out,
  * would choose (1 whenever the tiles already fill the GPU or K is short; at
  * most 8 of the tiled kernel, and never more than 2 MiB of the kernel for few
  * rows) need more than the array (slices x batch x M x N x 4 bytes), it
- * takes the largest number of slices that fits, down to one slice, which needs
+ * takes the largest number of slices that fits (the kernel on the bf16 matrix
+ * cores: the best of those that fit), down to one slice, which needs
  * no scratch: the result then has tfhip_fused_matmul's bits only where the two
  * slice counts agree, and is within the float32 bound otherwise. A slice count
  * the caller forced with the "splitk" or the "split" knob is not reduced: if it does not fit,

@@ -453,8 +453,8 @@ assert errors()[0] == 0, errors()
 
 
 def test_slices_of_a_product_in_bf16_parts_fit_the_fixed_scratch():
-    """A caller's fixed scratch (16 MiB): slices that the caller forced and that it does not hold are refused, the library's own
-    choice comes down to what it holds."""
+    """A caller's fixed scratch (16 MiB): slices that the caller forced and that it does not hold are refused; the library's own
+    choice is made among what it holds, with the tile that suits that."""
     fake_hip_util.run("""
 pyhost.init()
 a, b, out = (DeviceBuffer(128 << 20) for _ in range(3))
@@ -471,11 +471,19 @@ message = lib.tfhip_last_error().decode()
 assert str(3 * 1024 * 1366 * 4) in message and "16777216" in message, message
 assert fake.fake_hip_launches() == launches
 check(lib.tfhip_set_tuning(b"split", -1))
-for m, n, k in ((1280, 1280, 8192), (1344, 1536, 8192), (2432, 1024, 8192)):
-    check(product(m, n, k, lib.tfhip_fused_matmul))
-    wanted, fits = pyhost.workspace_info()["last_splits"], (16 << 20) // (m * n * 4)
-    assert "split_gemm" in launch(1)[0] and wanted > fits, (wanted, fits)
-    check(product(m, n, k))
-    assert pyhost.workspace_info()["last_splits"] == fits, (m, n, k)
+name = ctypes.create_string_buffer(256)
+
+def choice(entry, *shape):
+    check(product(*shape, entry))
+    check(lib.tfhip_last_kernel(name, 256))
+    return name.value.decode().split(",")[:3], pyhost.workspace_info()["last_splits"]
+
+for shape, slices in (((1280, 1280, 8192), 2), ((768, 2048, 8192), 2), ((536, 1768, 13978), 3), ((1344, 1536, 8192), 1),
+                      ((2432, 1024, 8192), 1)):
+    tile, wanted = choice(lib.tfhip_fused_matmul, *shape)
+    assert tile[0] == "split_gemm<4" and wanted * shape[0] * shape[1] * 4 > 16 << 20, (shape, tile, wanted)
+    tile, taken = choice(lib.tfhip_fused_matmul_noalloc, *shape)
+    assert tile[0].startswith("split_gemm<") and taken == slices, (shape, tile, taken)
+assert tile == ["split_gemm<4", " 3", " 2"]               # (four slices: 128 x 128, one group)
 assert errors()[0] == 0, errors()
 """)
