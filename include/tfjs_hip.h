@@ -156,7 +156,7 @@ int tfhip_graph_destroy(int graph_id);
  *   shape / never), "stream_rows" (its output rows per wavefront), "stream_blocks" (1 / 2
  *   blocks of 16 channels per wavefront), "skinny_stage" (0: the streaming GEMM never
  *   stages A in LDS), "split" (the GEMM on the bf16 matrix cores: tile + 10 x (slices
- *   of k - 1), 98: wherever it can, 99: never). The environment variable of a knob is its name in capitals behind
+ *   of k - 1) below 80, else wherever it can; 99: never, all other choices as without the knob). The environment variable of a knob is its name in capitals behind
  *   TFHIP_ (TFHIP_TILE, TFHIP_SPLITK, ... TFHIP_SKINNY_STAGE), read at tfhip_init().
  * tfhip_tuning_changes(&n): how many times a knob has been given another value. A
  *   recording keeps the kernels that the knobs chose when it was made; a program that

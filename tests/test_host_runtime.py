@@ -396,6 +396,13 @@ for shape, want in {(14, 41, 3, 16): "gemm_kernel<", (14, 42, 3, 16): "few_rows<
                     (38, 256, 7, 16): "few_rows<1, 1", (28, 256, 7, 32): "gemm_kernel<", (14, 130, 5, 256): "few_rows<1, 1",
                     (20, 130, 7, 130): "gemm_kernel<"}.items():
     assert windows(*shape).startswith(want), (shape, windows(*shape), want)
+# split_gemm switched off with its knob: nothing else changes; preferred: wherever it can
+for value, small, large in ((-1, "few_rows<1, 1", "split_gemm<"), (99, "few_rows<1, 1", "gemm_kernel<"), (98, "split_gemm<", "split_gemm<"),
+                            (80, "split_gemm<", "split_gemm<"), (3, "split_gemm<4, 3, 2", "split_gemm<4, 3, 2")):
+    check(lib.tfhip_set_tuning(b"split", value))
+    assert product(1, 1000, 1280).startswith(small) and product(1024, 2304, 768).startswith(large), value
+    assert windows(7, 256, 7, 256).startswith(small), value
+check(lib.tfhip_set_tuning(b"split", -1))
 assert errors()[0] == 0, errors()
 """)
 

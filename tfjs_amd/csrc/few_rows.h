@@ -352,11 +352,12 @@ inline bool few_rows_wide(const FewRowsCut &narrow, int row_blocks) {
   return narrow.tiles > num_cus() || narrow.groups_per_split > (row_blocks == 1 ? 128 : 96);
 }
 
-// (32-bit offsets, no per-call choice of another kernel)
+// (32-bit offsets, no choice of another kernel with a knob)
 inline bool few_rows_can(const GemmParams &p, bool windows) {
+  if (tuning(kTuneSplit) >= 0 && tuning(kTuneSplit) != 99) return false;   // (99: only that split_gemm is not chosen)
   if (windows ? p.a_bytes > kFewRowsMaxBytes : (long long)p.M * p.K * 4 > kFewRowsMaxBytes) return false;
   return p.batch == 1 && p.K > 0 && p.N <= (1 << 24) && p.epi.channel_operands && p.epi.addressing != kConv && tuning(kTuneTile) < 0 &&
-         tuning(kTuneSplit) < 0 && tuning(kTuneSplitK) < 0 && (long long)p.K * p.N * 4 <= kFewRowsMaxBytes;
+         tuning(kTuneSplitK) < 0 && (long long)p.K * p.N * 4 <= kFewRowsMaxBytes;
 }
 
 // Row blocks per workgroup that this kernel takes the product of two row-major operands with, or 0: it goes to the
