@@ -494,3 +494,48 @@ for shape, slices in (((1280, 1280, 8192), 2), ((768, 2048, 8192), 2), ((536, 17
 assert tile == ["split_gemm<4", " 3", " 2"]               # (four slices: 128 x 128, one group)
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_a_label_is_the_symbol_that_is_launched():
+    """tfhip_last_kernel names the launched kernel with its template arguments, spelled as a profiler spells them: the
+    benchmark's table of measured traffic is looked up by that name."""
+    fake_hip_util.run("""
+from tfjs_amd.traffic import symbol
+pyhost.init()
+big = [DeviceBuffer(64 << 20) for _ in range(3)]
+demangle = ctypes.CDLL("libstdc++.so.6").__cxa_demangle
+demangle.restype = ctypes.c_char_p
+label = ctypes.create_string_buffer(256)
+seen = set()
+
+def same(rc):
+    check(rc)
+    check(lib.tfhip_last_kernel(label, 256))
+    status = ctypes.c_int()
+    launched = symbol(demangle(launch()[0].split(".kd")[0].encode(), None, None, ctypes.byref(status)).decode())
+    assert label.value.decode() == launched, (label.value, launched)
+    seen.add(launched.split("<")[0])
+
+def product(m, n, k, tb=0):
+    same(lib.tfhip_fused_matmul(big[0].ptr, big[1].ptr, big[2].ptr, 1, 1, m, n, k, 0, tb, None, None, 0, None, None, 0.2))
+
+def conv(hw, c, f, out_c):
+    same(lib.tfhip_fused_conv2d(big[0].ptr, big[1].ptr, big[2].ptr, 1, hw, hw, c, f, f, out_c, 1, 1, 1, 1, f // 2, f // 2, hw, hw, 0,
+                                None, None, 0, None, None, 0.2))
+
+for m, n, k in ((1, 1000, 1280), (1, 4097, 1024), (16, 512, 512), (32, 768, 2304), (32, 3072, 2304), (1024, 2304, 768), (513, 256, 320),
+                (100352, 16, 96), (100352, 32, 144)):
+    product(m, n, k)
+product(1024, 2304, 768, 1)
+for shape in ((14, 64, 3, 64), (56, 64, 3, 64), (56, 21, 5, 38), (16, 3, 3, 16), (16, 3, 3, 8), (112, 21, 5, 38)):
+    conv(*shape)
+for n, h, w, c in ((1, 7, 7, 1280), (32, 7, 7, 1280), (64, 2, 1, 32768), (1, 7, 7, 3)):
+    same(lib.tfhip_mean_hw(big[0].ptr, big[1].ptr, n, h, w, c))
+for f, s in ((3, 1), (3, 2), (5, 1), (5, 2)):
+    out = (57 + s - 1) // s
+    same(lib.tfhip_fused_depthwise_conv2d(big[0].ptr, big[1].ptr, big[2].ptr, 1, 57, 57, 96, f, f, 1, s, s, 1, 1, f // 2, f // 2, out, out,
+                                          None, None, 0, None, None, 0.2))
+assert seen >= {"few_rows", "split_gemm", "gemm_kernel", "mean_hw_vec", "mean_hw", "conv_few_taps", "depthwise_3x3_cols",
+                "depthwise_cols_sums"}, seen
+assert errors()[0] == 0, errors()
+""")

@@ -79,7 +79,7 @@ int launch_few_rows_shape(FewRowsArgs &q, const FewRowsCut &cut) {
   // In a recording the slices are added by a launch of their own: a node of a graph costs a fraction of a launch, and a
   // replay then shares no counter with whatever else the program runs. The sums and their order are the same.
   q.finish_apart = q.splits > 1 && capturing();
-  note_kernel("few_rows<%d, %d, %d, %d>", MB, CB, KIND, (int)ROW);
+  note_kernel("few_rows<%d, %d, %d, %s>", MB, CB, KIND, ROW ? "true" : "false");
   const dim3 grid((unsigned)(cut.tiles * q.splits)), block(64 * kFewRowsWaves);
   if (q.finish_apart) {
     TFHIP_LAUNCH((few_rows<MB, CB, KIND, ROW><<<grid, block, 0, stream()>>>(q),

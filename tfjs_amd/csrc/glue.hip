@@ -439,7 +439,7 @@ int tfhip_mean_hw(const float *x, float *y, int64_t batch, int64_t h, int64_t w,
     // (int: every index, also those of a loop's next round, and the magic number's exact range)
     const long long groups = blocks4 < num_cus() ? c : c / 4;
     const bool narrow = (double)batch * h * w * c < 1073741824.0 && (double)batch * groups * groups < 4294967296.0;
-    note_kernel("mean_hw_vec");
+    note_kernel("mean_hw_vec<%d, %s>", narrow && groups == c ? 1 : 4, narrow ? "int" : "long long");
     if (narrow && groups == c) {
       TFHIP_LAUNCH((mean_hw_vec<1, int><<<(unsigned)((batch * c + 31) / 32), 256, 0, stream()>>>(x, y, (int)batch, (int)(h * w), (int)c,
                                                                                                magic_of((int)groups))));
