@@ -8,11 +8,15 @@
 // bits, 2-norm relative, K = 64, 256, 768, 3072, operands N(0, 1) and N(0, 0.02): float32 matrix instructions 1.4e-7, 2.9e-7,
 // 5.0e-7, 9.8e-7, this kernel 0.5e-7, 0.9e-7, 1.6e-7, 3.4e-7; all-positive operands 1.2e-7 ... 8.3e-7 and 0.5e-7 ... 3.0e-7.
 //
-// us, gemm_kernel and here (rate of the product itself): 1024 x 2304 x 768 33.8 and 25.4 (142 TFLOP/s), 1024 x 3072 x 768 41.5
-// and 30.4, 3072 x 3072 x 1024 154 and 106 (183), 3072 x 4096 x 1024 189 and 131 (197), [8,56,56,64] 3x3 -> 64 27.0 and 17.8.
-// Of a transposed B, 128 x (384 x 64 x 384) 36 and 31, 128 x (512 x 64 x 512) 56 and 44, 1024 x 3072 x 768 39.9 and 30.2.
-// What bounds it: on the largest the matrix cores, three quarters of the time; the rest waits for fetches and barriers. On
-// 1024 rows, 6 us of launch, prologue (2.5: arguments, the first fetch, the first tile's splitting) and results (2.7).
+// us, gemm_kernel and here (rate of the product itself): 1024 x 2304 x 768 33.4 and 24.8 (146 TFLOP/s), 1024 x 3072 x 768 40.8
+// and 28.7, 3072 x 3072 x 1024 153 and 114 (170), 3072 x 4096 x 1024 189 and 139 (185), [8,56,56,64] 3x3 -> 64 26.7 and 18.2.
+// Of a transposed B, 128 x (384 x 64 x 384) 32.5 and 26.8, 128 x (512 x 64 x 512) 56 and 44, 1024 x 3072 x 768 38.8 and 28.7.
+// What bounds it: the loop, and in it the matrix cores for 64% of its cycles (128 x 128 tiles 68%), fetches and barriers for
+// the rest. A k tile of a 128 x 96 tile takes 0.71 us on 64 of the 256 units and 1.02 on all of them, where the chip's clock
+// falls from 2.34 to 1.71 GHz (busy and active cycles of launches of 1 ms, by counter). Over a launch of 3072 x 3072 x 1024 the
+// matrix cores are busy for 40% of 2.4 GHz: that clock, the waits, and 5 to 6 us of prologue and results in each of three
+// rounds are the rest. On 1024 rows, 6 us of launch, prologue (2.5: arguments, the first fetch, the first tile's splitting) and
+// results (2.7), and with 2304 or 768 columns a quarter of the units idle.
 //
 // The last bit of a float32 may be 2^-149, that of a bf16 2^-133: both operands are multiplied by 2^24 before they are split
 // (two vector instructions per pair of floats beside eleven), so that every part of every float is a normal bf16 or zero, and
