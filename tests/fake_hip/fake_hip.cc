@@ -47,6 +47,7 @@ int errors = 0;
 std::string first_error;
 std::atomic<int> copy_delay_us{0}, launch_delay_us{0};
 std::atomic<int> copies_now{0};
+std::vector<uint64_t> copy_sizes;
 std::map<hipStream_t, int> stream_device;
 thread_local struct {
   dim3 grid, block;
@@ -137,6 +138,14 @@ int fake_hip_device_of(const void *p) {
 }
 void fake_hip_copy_delay(int us) { copy_delay_us = us; }
 int fake_hip_copies_now(void) { return copies_now; }
+// The sizes of the copies since the last call, the first `most` of them; how many there were.
+int fake_hip_copy_sizes(uint64_t *sizes, int most) {
+  std::lock_guard<std::recursive_mutex> lock(m);
+  const int n = (int)copy_sizes.size();
+  for (int i = 0; i < n && i < most; ++i) sizes[i] = copy_sizes[i];
+  copy_sizes.clear();
+  return n;
+}
 void fake_hip_launch_delay(int us) { launch_delay_us = us; }
 
 // ---- devices, memory ----
@@ -169,6 +178,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t bytes, hipMemcpyKind, h
       return hipSuccess;
     }
     ++copies_now;
+    copy_sizes.push_back(bytes);
   }
   if (copy_delay_us) usleep(copy_delay_us);
   std::lock_guard<std::recursive_mutex> lock(m);

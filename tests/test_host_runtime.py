@@ -247,6 +247,24 @@ np.testing.assert_array_equal(buf.download(np.uint8, data.nbytes), data)
 """, each=([], ["one cpu"]))
 
 
+def test_the_pieces_of_an_upload():
+    """The first piece's copy overlaps nothing: half a megabyte where one thread copies, one from 2 MB on."""
+    fake_hip_util.run("""
+pyhost.init()
+K = 1024
+data = np.arange(16 << 20, dtype=np.uint32).view(np.uint8)
+buf, sizes = DeviceBuffer(data.nbytes), (ctypes.c_uint64 * 64)()
+for n, want in [(600 * K, [600]), (1024 * K, [512, 512]), (1900 * K, [512, 512, 876]), (2047 * K, [512, 512, 1023]),
+                (2048 * K, [1024, 1024]), (3400 * K, [1024, 1024, 1352]), (64 << 20, [1024, 1024, 2048, 4096, 8192, 16384, 16384, 16384])]:
+    fake.fake_hip_copy_sizes(sizes, 64)
+    check(lib.tfhip_upload(buf.ptr, 0, data.ctypes.data, n))
+    count = fake.fake_hip_copy_sizes(sizes, 64)
+    assert [s // K for s in sizes[:count]] == want, (n // K, [s // K for s in sizes[:count]])
+    np.testing.assert_array_equal(buf.download(np.uint8, n), data[:n])
+assert errors()[0] == 0, errors()
+""")
+
+
 def test_a_child_copies_without_its_parents_threads():
     """A forked child has none of the threads that copied for its parent: it starts its own."""
     fake_hip_util.run("""
