@@ -425,6 +425,34 @@ assert errors()[0] == 0, errors()
 """)
 
 
+def test_which_products_go_to_the_bf16_matrix_cores():
+    """Both sides of the line at 0.45 GFLOP, and products whose tiles are half padding, for which the others are ahead."""
+    fake_hip_util.run("""
+pyhost.init()
+big = [DeviceBuffer(64 << 20) for _ in range(3)]
+name = ctypes.create_string_buffer(256)
+
+def label():
+    check(lib.tfhip_last_kernel(name, 256))
+    return name.value.decode()
+
+for (m, n, k), want in {(1024, 1024, 210): "gemm_kernel<", (1024, 1024, 216): "split_gemm<", (1024, 2304, 768): "split_gemm<",
+                        (1024, 768, 768): "split_gemm<", (1568, 1280, 320): "split_gemm<", (933, 76, 2728): "gemm_kernel<",
+                        (461, 144, 2392): "gemm_kernel<", (4034, 93, 1250): "few_rows<"}.items():
+    check(lib.tfhip_fused_matmul(big[0].ptr, big[1].ptr, big[2].ptr, 1, 1, m, n, k, 0, 0, None, None, 0, None, None, 0.2))
+    assert label().startswith(want), (m, n, k, label())
+for (batch, h, w, c, f, out_c, stride), want in {(8, 56, 56, 64, 3, 64, 1): "split_gemm<", (8, 80, 34, 16, 3, 236, 2): "gemm_kernel<",
+                                                 (8, 80, 34, 16, 3, 237, 2): "gemm_kernel<", (1, 19, 92, 52, 3, 236, 1): "few_rows<",
+                                                 (11, 24, 44, 188, 3, 72, 2): "few_rows<"}.items():
+    out_h, out_w = -(-h // stride), -(-w // stride)
+    pad_h, pad_w = max((out_h - 1) * stride + f - h, 0) // 2, max((out_w - 1) * stride + f - w, 0) // 2
+    check(lib.tfhip_fused_conv2d(big[0].ptr, big[1].ptr, big[2].ptr, batch, h, w, c, f, f, out_c, stride, stride, 1, 1, pad_h, pad_w,
+                                 out_h, out_w, 0, None, None, 0, None, None, 0.2))
+    assert label().startswith(want), (batch, h, w, c, f, out_c, stride, label())
+assert errors()[0] == 0, errors()
+""")
+
+
 def test_filters_of_many_taps_are_gathered():
     """An image of few channels under a filter that the matrix-core form does not hold: GEMM-shaped from 16 output
     channels on, however few pixels there are."""

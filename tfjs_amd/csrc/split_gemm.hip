@@ -39,7 +39,7 @@ double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, d
   }
   us = s.launch + us * windows;
   if (slices > 1) us += 2.5 + 4.0 * p.batch * p.M * (double)p.N * (slices + 1) / (p.vec_store ? 4.0e6 : 1.3e6);   // gemm_finish_rows, gemm_finish
-  return us;
+  return 1.03 * us;   // (fitted before operands were scaled, which takes 0.5 to 4%)
 }
 
 // What the same product takes with gemm_kernel, whatever tile and slices that chooses: the launch, the matrix instructions at
@@ -120,10 +120,10 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
     return best;
   if (p.epi.channel_operands && (p.epi.bias_s[3] > 1 || p.epi.prelu_s[3] > 1)) return best;
   if (split_forced()) return {forced % 10 % kNumSplitShapes, forced / 10 + 1, 0};
-  // Below 0.3 GFLOP the fixed part decides, and gemm_kernel's is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, 0.3 to 0.45
-  // equal, 0.8 to 1.2 0.88 of the time, from 4 on 0.68; 13000 products); so it is with tiles that are mostly padding: few
+  // Below 0.45 GFLOP the fixed part decides, and that of the other kernels is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, of 39
+  // products and convolutions of 0.3 to 0.45 1.02 times; 0.8 to 1.2 0.88 of the time, from 4 on 0.7); so it is with tiles that are mostly padding: few
   // columns, few rows of each product of a batch. Under 448 rows only half of the products gain.
-  if (forced < 0 && (2.0 * p.batch * p.M * (double)p.N * p.K < 3e8 || p.N <= 32 || p.M < 64 || (long long)p.batch * p.M < 448)) return best;
+  if (forced < 0 && (2.0 * p.batch * p.M * (double)p.N * p.K < 4.5e8 || p.N <= 32 || p.M < 64 || (long long)p.batch * p.M < 448)) return best;
   const double windows = a_kind == kLoadWindows ? 1.08 : (a_kind == kLoadWindowsAny ? 1.35 : 1.0);
   double best_us = 0;
   // (Of a fixed scratch the slices that it holds, with the tile that suits those: 536 x 1768 x 13978 takes 164 us in seven, 242 in the
