@@ -58,9 +58,13 @@ def measured_traffic():
     return traffic.load(os.path.join(ROOT, "profiles", "traffic.json"))
 
 
+def mfma_peak(kernel):
+    return round(MFMA_BF16_PEAK_TFLOPS / 6, 1) if kernel.startswith("split_gemm") else MFMA_FP32_PEAK_TFLOPS
+
+
 def roofline_entry(flops, nbytes, seconds, kernel=""):
     """Prices `seconds` against the roof that bounds a kernel of this intensity."""
-    peak = round(MFMA_BF16_PEAK_TFLOPS / 6, 1) if kernel.startswith("split_gemm") else MFMA_FP32_PEAK_TFLOPS
+    peak = mfma_peak(kernel)
     if nbytes > 0 and flops / nbytes > RIDGE * peak / MFMA_FP32_PEAK_TFLOPS:
         achieved = flops / seconds / 1e12
         return dict(bound="mfma", achieved=round(achieved, 3), peak=peak, unit="TFLOP/s", frac=round(achieved / peak, 4))
@@ -271,7 +275,7 @@ def bench_model(model_dir, steps, warmup):
             src = op["src"][0] if isinstance(op["src"], tuple) else op["src"]
             ops.append(dict(op=op["kind"], x=list(model.shape[src]), y=list(model.shape[op["out"]]),
                             kernel=names[i], us=round(per_op[i] * 1e6, 2),
-                            roof_us=round(max(flops / MFMA_FP32_PEAK_TFLOPS / 1e12, nbytes / HBM_PEAK_GBS / 1e9) * 1e6, 2)))
+                            roof_us=round(max(flops / mfma_peak(names[i]) / 1e12, nbytes / HBM_PEAK_GBS / 1e9) * 1e6, 2)))
     finally:
         model.close()
     dominant = max(by_symbol, key=lambda k: by_symbol[k]["seconds"])
