@@ -29,7 +29,8 @@ double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, d
   const long long tiles = ((p.M + 32 * s.gw - 1) / (32 * s.gw)) * (long long)((p.N + 32 * s.tn - 1) / (32 * s.tn)) * p.batch * slices;
   const int k_tiles = ((p.K + 31) / 32 + slices - 1) / slices, rounds_of_k = (k_tiles + s.kg - 1) / s.kg;
   const long long cus = num_cus();
-  const double one = rounds_of_k * s.per_tile + s.fixed, two = rounds_of_k * s.per_tile_two + s.fixed_two;
+  // (fitted before operands were scaled: 1.03 of a k tile)
+  const double one = rounds_of_k * 1.03 * s.per_tile + s.fixed, two = rounds_of_k * 1.03 * s.per_tile_two + s.fixed_two;
   double us;
   if (s.per_tile_two == 0) {
     us = (double)((tiles + cus - 1) / cus) * one;
@@ -39,7 +40,7 @@ double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, d
   }
   us = s.launch + us * windows;
   if (slices > 1) us += 2.5 + 4.0 * p.batch * p.M * (double)p.N * (slices + 1) / (p.vec_store ? 4.0e6 : 1.3e6);   // gemm_finish_rows, gemm_finish
-  return 1.03 * us;   // (fitted before operands were scaled, which takes 0.5 to 4%)
+  return us;
 }
 
 // What the same product takes with gemm_kernel, whatever tile and slices that chooses: the launch, the matrix instructions at
