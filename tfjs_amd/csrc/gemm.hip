@@ -19,7 +19,7 @@ int tfhip::launch_plain_gemm(GemmParams &p, bool transpose_a, bool transpose_b, 
     }
   }
   if (!transpose_a && transpose_b && vec && !float_bits) {
-    const SplitChoice split = split_gemm_choice(p, kLoadKAny);
+    const SplitChoice split = split_gemm_choice(p, kLoadKAny, true);
     if (split.shape >= 0) return launch_split_gemm(split, p, kLoadKAny, true);
   }
   if (vec) {

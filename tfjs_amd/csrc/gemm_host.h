@@ -264,7 +264,7 @@ struct SplitChoice {
   int shape, slices;
   double us;
 };
-SplitChoice split_gemm_choice(const GemmParams &p, int a_kind);
+SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b = false);
 int launch_split_gemm(SplitChoice choice, GemmParams &p, int a_kind, bool transposed_b = false);
 
 // Fills the bias / prelu part of an Epilogue from caller strides over `rank`

@@ -110,7 +110,7 @@ int launch_kind(SplitChoice c, GemmParams &p) {
 
 }  // namespace
 
-SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
+SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b) {
   SplitChoice best = {-1, 1, 0};
   const int forced = tuning(kTuneSplit);
   if (forced == 99 || tuning(kTuneTile) >= 0 || tuning(kTuneSplitK) >= 0 || tuning(kTuneKGroups) >= 0) return best;
@@ -143,7 +143,10 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind) {
   }
   // The lead that makes up for the estimates' errors: of the 13000, half are taken, on average at 0.78 of the time; 2% of
   // those are 5% slower than with gemm_kernel and more.
-  const double tiled = tiled_estimate_us(p, a_kind == kLoadWindows ? 1.24 : (a_kind == kLoadWindowsAny ? 1.82 : 1.0));
+  // gemm_kernel is faster on a transposed B than on a row-major one (from K = 129 on 0.86 of its estimate): of 400 such products, with
+  // the estimate as it is, 28 took 3 to 27% longer here than there, with 0.9 of it nine.
+  const double tiled = tiled_estimate_us(p, a_kind == kLoadWindows ? 1.24 : (a_kind == kLoadWindowsAny ? 1.82 : 1.0)) *
+                       (transposed_b && p.K > 128 ? 0.9 : 1.0);
   if (forced < 0 && best_us > 0.92 * tiled) best.shape = -1;
   return best;
 }
