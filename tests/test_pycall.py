@@ -134,3 +134,70 @@ assert errors()[0] == 0, errors()
 
 def test_decode_weights_to_device_is_the_general_function():
     run(DECODE)
+
+
+RACE = """
+data = np.zeros(1 << 20, dtype=np.uint8)
+def manifest():
+    return [dict(name="t%d" % i, shape=[16, 8], dtype="float32", quantization=dict(dtype="uint8", scale=0.5, min=-1.0)) for i in range(400)]
+def loaded(change):
+    '''what comes back where another thread changes the manifest while the call waits for the upload'''
+    specs = manifest()
+    def other():
+        while not fake.fake_hip_copies_now():
+            time.sleep(0.0005)
+        change(specs)
+    thread = threading.Thread(target=other)
+    thread.start()
+    fake.fake_hip_copy_delay(50000)
+    got = pyhost.decode_weights_to_device(data, specs)
+    fake.fake_hip_copy_delay(0)
+    thread.join()
+    seen = [(name, buf.nbytes, shape) for name, (buf, shape) in got.items()]
+    for buf, _ in got.values():
+        buf.free()
+    return specs, seen
+"""
+
+
+@pytest.mark.parametrize("change", [
+    "specs.clear()", "specs.__delitem__(slice(10, None))", "[s.clear() for s in specs]", "[s['shape'].__setitem__(0, 1 << 30) for s in specs]",
+    "[s['shape'].clear() for s in specs]", "[s.update(name='x') for s in specs]", "specs.__setitem__(slice(None), [None] * 400)",
+])
+def test_the_manifest_is_what_it_was_when_the_call_began(change):
+    run(BODY + RACE + """
+want = [("t%d" % i, 512, [16, 8]) for i in range(400)]
+specs, got = loaded(lambda specs: """ + change + """)
+assert got == want
+assert specs != manifest(), "the other thread came too late"
+""")
+
+
+def test_a_keys_own_comparison_may_shorten_the_manifest():
+    # (a key with the hash of "name": the lookup asks it, and it takes the entries away)
+    run(BODY + RACE + """
+class Key:
+    def __hash__(self):
+        return hash("name")
+    def __eq__(self, other):
+        if armed:
+            specs.clear()
+        return False
+armed, specs = False, manifest()
+specs[0] = dict([(Key(), 1)] + list(specs[0].items()))
+armed = True
+try:
+    pyhost.decode_weights_to_device(data, specs)
+except Exception as e:
+    assert isinstance(e, (KeyError, RuntimeError, TypeError, IndexError)), e
+assert not specs
+""")
+
+
+def test_the_shape_that_comes_back_is_the_callers_own():
+    run(BODY + RACE + """
+specs = manifest()
+got = pyhost.decode_weights_to_device(data, specs)
+got["t0"][1].append(3)
+assert specs[0]["shape"] == [16, 8] and got["t1"][1] == [16, 8]
+""")

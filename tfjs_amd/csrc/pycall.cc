@@ -333,14 +333,33 @@ bool number(PyObject *o, double &to) {
   to = (double)whole;   // (rounded as ctypes does)
   return true;
 }
-// (borrowed; nullptr without an error where there is none)
-PyObject *entry_of(PyObject *dict, PyObject *key) {
+
+// An owned reference.
+class Ref {
+ public:
+  explicit Ref(PyObject *o) : o_(o) {}
+  Ref(Ref &&other) noexcept : o_(other.o_) { other.o_ = nullptr; }
+  Ref(const Ref &) = delete;
+  Ref &operator=(const Ref &) = delete;
+  ~Ref() { Py_XDECREF(o_); }
+  PyObject *get() const { return o_; }
+  explicit operator bool() const { return o_ != nullptr; }
+
+ private:
+  PyObject *o_;
+};
+
+// (none, without an error, where there is none)
+Ref entry_of(PyObject *dict, PyObject *key) {
   PyObject *const o = PyDict_GetItemWithError(dict, key);
   if (!o) PyErr_Clear();
-  return o;
+  Py_XINCREF(o);
+  return Ref(o);
 }
 
+// (all that the result is made of: other threads run during the call, and may change the manifest)
 struct Weights {
+  std::vector<Ref> names, shapes;   // (the lists are copies)
   std::vector<int64_t> offsets, elems;
   std::vector<int> kinds;
   std::vector<double> scale_min;
@@ -351,48 +370,59 @@ struct Weights {
 bool read_specs(PyObject *specs, Weights &w) {
   if (!PyList_CheckExact(specs)) return false;
   const Py_ssize_t count = PyList_GET_SIZE(specs);
+  w.names.reserve(count);
+  w.shapes.reserve(count);
   w.offsets.resize(count);
   w.elems.resize(count);
   w.kinds.resize(count);
   w.scale_min.resize(2 * count);
   for (Py_ssize_t i = 0; i < count; ++i) {
-    PyObject *const spec = PyList_GET_ITEM(specs, i);
-    if (!PyDict_CheckExact(spec)) return false;
-    PyObject *const name = entry_of(spec, g_name), *const dtype = entry_of(spec, g_dtype), *const shape = entry_of(spec, g_shape),
-                   *const q = entry_of(spec, g_quantization);
-    if (!name || !PyUnicode_CheckExact(name) || !dtype || !shape || !PyList_CheckExact(shape)) return false;
+    if (i >= PyList_GET_SIZE(specs)) return false;   // (a key's own comparison has run)
+    Py_INCREF(PyList_GET_ITEM(specs, i));
+    const Ref spec(PyList_GET_ITEM(specs, i));
+    if (!PyDict_CheckExact(spec.get())) return false;
+    Ref name = entry_of(spec.get(), g_name);
+    const Ref dtype = entry_of(spec.get(), g_dtype), extents = entry_of(spec.get(), g_shape), q = entry_of(spec.get(), g_quantization);
+    if (!name || !PyUnicode_CheckExact(name.get()) || !dtype || !extents || !PyList_CheckExact(extents.get())) return false;
+    Ref shape(PyList_GetSlice(extents.get(), 0, PyList_GET_SIZE(extents.get())));
+    if (!shape) {
+      PyErr_Clear();
+      return false;
+    }
     int64_t size = 1;
-    for (Py_ssize_t d = 0; d < PyList_GET_SIZE(shape); ++d) {
+    for (Py_ssize_t d = 0; d < PyList_GET_SIZE(shape.get()); ++d) {
       int64_t extent = 0;
-      if (!from(PyList_GET_ITEM(shape, d), extent) || extent < 0 || (extent > 0 && size > (int64_t(1) << 40) / extent)) return false;
+      if (!from(PyList_GET_ITEM(shape.get(), d), extent) || extent < 0 || (extent > 0 && size > (int64_t(1) << 40) / extent)) return false;
       size *= extent;
     }
-    const bool to_float = is_text(dtype, "float32"), to_int = is_text(dtype, "int32");
+    const bool to_float = is_text(dtype.get(), "float32"), to_int = is_text(dtype.get(), "int32");
     int kind = 0;
     size_t code = 4;
-    if (!q || q == Py_None) {
+    if (!q || q.get() == Py_None) {
       if (!to_float && !to_int) {
-        if (!is_text(dtype, "bool")) return false;
+        if (!is_text(dtype.get(), "bool")) return false;
         kind = 1;
         code = 1;
       }
     } else {
-      if (!PyDict_CheckExact(q) || (!to_float && !to_int)) return false;
-      PyObject *const coded = entry_of(q, g_dtype);
+      if (!PyDict_CheckExact(q.get()) || (!to_float && !to_int)) return false;
+      const Ref coded = entry_of(q.get(), g_dtype);
       if (!coded) return false;
-      if (is_text(coded, "float16")) {
+      if (is_text(coded.get(), "float16")) {
         if (!to_float) return false;
         kind = 6;
         code = 2;
       } else {
-        const bool bytes = is_text(coded, "uint8");
-        if (!bytes && !is_text(coded, "uint16")) return false;
+        const bool bytes = is_text(coded.get(), "uint8");
+        if (!bytes && !is_text(coded.get(), "uint16")) return false;
         kind = (bytes ? 2 : 4) + (to_int ? 1 : 0);
         code = bytes ? 1 : 2;
-        PyObject *const scale = entry_of(q, g_scale), *const min = entry_of(q, g_min);
-        if (!scale || !min || !number(scale, w.scale_min[2 * i]) || !number(min, w.scale_min[2 * i + 1])) return false;
+        const Ref scale = entry_of(q.get(), g_scale), min = entry_of(q.get(), g_min);
+        if (!scale || !min || !number(scale.get(), w.scale_min[2 * i]) || !number(min.get(), w.scale_min[2 * i + 1])) return false;
       }
     }
+    w.names.push_back(std::move(name));
+    w.shapes.push_back(std::move(shape));
     w.offsets[i] = (int64_t)w.total;
     w.elems[i] = size;
     w.kinds[i] = kind;
@@ -402,18 +432,16 @@ bool read_specs(PyObject *specs, Weights &w) {
   return true;
 }
 
-// (DeviceBuffer.adopt(block, bytes), a copy of the shape), or nullptr with an error
+// (DeviceBuffer.adopt(block, bytes), the shape), or nullptr with an error
 PyObject *adopted(PyTypeObject *type, void *block, int64_t bytes, PyObject *shape) {
   PyObject *const buf = type->tp_new(type, g_no_args, nullptr);
   PyObject *const ptr = block ? PyLong_FromVoidPtr(block) : Py_NewRef(Py_None), *const nbytes = PyLong_FromLongLong(bytes);
-  PyObject *const extents = PyList_GetSlice(shape, 0, PyList_GET_SIZE(shape));
   PyObject *pair = nullptr;
-  if (buf && ptr && nbytes && extents && PyObject_SetAttr(buf, g_nbytes, nbytes) == 0 && PyObject_SetAttr(buf, g_ptr, ptr) == 0)
-    pair = PyTuple_Pack(2, buf, extents);
+  if (buf && ptr && nbytes && PyObject_SetAttr(buf, g_nbytes, nbytes) == 0 && PyObject_SetAttr(buf, g_ptr, ptr) == 0)
+    pair = PyTuple_Pack(2, buf, shape);
   Py_XDECREF(buf);
   Py_XDECREF(ptr);
   Py_XDECREF(nbytes);
-  Py_XDECREF(extents);
   return pair;
 }
 
@@ -424,12 +452,12 @@ PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
   try {
     Weights w;
     if (!read_specs(args[1], w) || w.elems.empty()) return general();
+    std::vector<void *> outs(w.elems.size());
     Py_buffer host;
     if (PyObject_GetBuffer(args[0], &host, PyBUF_SIMPLE) != 0) {
       PyErr_Clear();
       return general();
     }
-    std::vector<void *> outs(w.elems.size());
     int status = -1;
     if (host.len > 0 && w.total <= (size_t)host.len) {
       Py_BEGIN_ALLOW_THREADS
@@ -441,16 +469,11 @@ PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
     if (status) return PyObject_CallFunction(f->check, "i", status);
     PyObject *const result = PyDict_New();
     for (size_t i = 0; result && i < outs.size(); ++i) {
-      PyObject *const spec = PyList_GET_ITEM(args[1], (Py_ssize_t)i);
-      PyObject *const name = entry_of(spec, g_name), *const shape = entry_of(spec, g_shape);
-      PyObject *const pair = name && shape && PyList_CheckExact(shape)
-                                 ? adopted(reinterpret_cast<PyTypeObject *>(f->buffer_type), outs[i], w.elems[i] * (w.kinds[i] == 1 ? 1 : 4), shape)
-                                 : nullptr;
-      const bool kept = pair && PyDict_SetItem(result, name, pair) == 0;
+      PyObject *const pair = adopted(reinterpret_cast<PyTypeObject *>(f->buffer_type), outs[i], w.elems[i] * (w.kinds[i] == 1 ? 1 : 4), w.shapes[i].get());
+      const bool kept = pair && PyDict_SetItem(result, w.names[i].get(), pair) == 0;
       Py_XDECREF(pair);
       if (!kept) {
         Py_DECREF(result);
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the manifest changed while its weights were decoded");
         return nullptr;
       }
     }
