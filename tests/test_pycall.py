@@ -201,3 +201,26 @@ got = pyhost.decode_weights_to_device(data, specs)
 got["t0"][1].append(3)
 assert specs[0]["shape"] == [16, 8] and got["t1"][1] == [16, 8]
 """)
+
+
+@pytest.mark.parametrize("wrapped", [0, 1, 399])
+def test_blocks_that_find_no_owner_are_given_back(wrapped):
+    run(BODY + RACE + """
+left = 2 * """ + str(wrapped) + """   # attributes that may still be set
+def refuse(self, name, value):
+    global left
+    if left == 0:
+        raise MemoryError("no room for " + name)
+    left -= 1
+    object.__setattr__(self, name, value)
+live = pyhost.memory_info()["live"]
+DeviceBuffer.__setattr__ = refuse
+try:
+    pyhost.decode_weights_to_device(data, manifest())
+    raise AssertionError("the buffers were wrapped")
+except MemoryError as e:
+    assert str(e) == "no room for nbytes"
+del DeviceBuffer.__setattr__
+assert pyhost.memory_info()["live"] == live
+assert errors()[0] == 0, errors()
+""")

@@ -173,6 +173,7 @@ PyTypeObject g_entry_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 // (until the library is loaded every call of the two below goes to the function in Python, which loads it)
 decltype(&tfhip_fused_matmul) g_fused_matmul = nullptr;
 decltype(&tfhip_decode_weights) g_decode_weights = nullptr;
+decltype(&tfhip_free) g_free = nullptr;
 
 // bind(name, ctypes function, its address): the same function for callers that pass plain values.
 PyObject *bind(PyObject *, PyObject *args) {
@@ -190,6 +191,7 @@ PyObject *bind(PyObject *, PyObject *args) {
     e->address = reinterpret_cast<void *>(static_cast<uintptr_t>(address));
     if (strcmp(name, "tfhip_fused_matmul") == 0) g_fused_matmul = reinterpret_cast<decltype(g_fused_matmul)>(e->address);
     if (strcmp(name, "tfhip_decode_weights") == 0) g_decode_weights = reinterpret_cast<decltype(g_decode_weights)>(e->address);
+    if (strcmp(name, "tfhip_free") == 0) g_free = reinterpret_cast<decltype(g_free)>(e->address);
     return reinterpret_cast<PyObject *>(e);
   }
   return PyErr_Format(PyExc_KeyError, "%s", name);
@@ -448,7 +450,7 @@ PyObject *adopted(PyTypeObject *type, void *block, int64_t bytes, PyObject *shap
 PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
   DecodeCall *const f = reinterpret_cast<DecodeCall *>(self);
   const auto general = [&] { return PyObject_Vectorcall(f->general, args, nargsf, kwnames); };
-  if (!g_decode_weights || PyVectorcall_NARGS(nargsf) != 2 || (kwnames && PyTuple_GET_SIZE(kwnames) > 0)) return general();
+  if (!g_decode_weights || !g_free || PyVectorcall_NARGS(nargsf) != 2 || (kwnames && PyTuple_GET_SIZE(kwnames) > 0)) return general();
   try {
     Weights w;
     if (!read_specs(args[1], w) || w.elems.empty()) return general();
@@ -467,16 +469,16 @@ PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
     PyBuffer_Release(&host);
     if (status == -1 || status == kNotInitialised) return general();
     if (status) return PyObject_CallFunction(f->check, "i", status);
-    PyObject *const result = PyDict_New();
+    PyObject *result = PyDict_New();
     for (size_t i = 0; result && i < outs.size(); ++i) {
       PyObject *const pair = adopted(reinterpret_cast<PyTypeObject *>(f->buffer_type), outs[i], w.elems[i] * (w.kinds[i] == 1 ? 1 : 4), w.shapes[i].get());
       const bool kept = pair && PyDict_SetItem(result, w.names[i].get(), pair) == 0;
       Py_XDECREF(pair);
-      if (!kept) {
-        Py_DECREF(result);
-        return nullptr;
-      }
+      if (!kept) Py_CLEAR(result);
     }
+    if (!result)   // (what was wrapped is gone, and has given nothing back)
+      for (void *block : outs)
+        if (block) g_free(block);
     return result;
   } catch (const std::bad_alloc &) {
     return PyErr_NoMemory();
