@@ -1,8 +1,14 @@
 """The compiled way into the entry points (tfjs_amd/csrc/pycall.cc) against ctypes, on a stand-in for the HIP runtime: the same
 launches for every form of the arguments, the same refusals, and the general function wherever a form is not known."""
+import os
+import subprocess
+import sys
+import sysconfig
+
 import pytest
 
-from fake_hip_util import run
+from fake_hip_util import ROOT, run
+from tfjs_amd import build, capi
 
 BODY = """
 assert capi.pycall is not None, "not built for this Python"
@@ -224,3 +230,42 @@ del DeviceBuffer.__setattr__
 assert pyhost.memory_info()["live"] == live
 assert errors()[0] == 0, errors()
 """)
+
+
+def test_the_package_does_without_an_extension_that_does_not_load(tmp_path):
+    junk = tmp_path / os.path.basename(capi.PYCALL_PATH)
+    assert capi._load_pycall(str(junk)) is None
+    junk.write_bytes(b"not a library")
+    with pytest.warns(RuntimeWarning, match="through ctypes"):
+        assert capi._load_pycall(str(junk)) is None
+    # the whole package, with such a file in the place of its own
+    code = """
+import sys, os
+sys.path.insert(0, %r)
+import importlib.util
+exists, of = os.path.exists, importlib.util.spec_from_file_location
+importlib.util.spec_from_file_location = lambda name, path, *more: of(name, %r if "_pycall" in path else path, *more)
+from tfjs_amd import capi, pyhost
+assert capi.pycall is None and pyhost.device_fused_matmul.__class__ is capi.load_library.__class__
+assert capi.load_library().tfhip_free(None) != 0
+""" % (ROOT, str(junk))
+    done = subprocess.run([sys.executable, "-W", "ignore", "-c", code], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout
+
+
+def test_the_build_does_without_an_extension_that_does_not_compile(tmp_path, monkeypatch, capsys):
+    older = tmp_path / "_pycall.so"
+    monkeypatch.setattr(build, "PYCALL", str(older))
+    for include in (str(tmp_path / "none"), str(tmp_path)):   # no Python.h; one that is of no use
+        older.write_bytes(b"of an older build")
+        monkeypatch.setattr(sysconfig, "get_paths", lambda: dict(include=include))
+        assert build.build_pycall() is None and not older.exists()
+        (tmp_path / "Python.h").write_text("#error of no use\n")
+    assert "through ctypes" in capsys.readouterr().out
+
+
+def test_the_extension_needs_nothing_newer_than_python_3_9():
+    with open(os.path.join(ROOT, "tfjs_amd", "csrc", "pycall.cc")) as f:
+        text = f.read()
+    for newer in ("Py_NewRef", "Py_XNewRef", "PyModule_AddObjectRef", "PyType_GetModule", "Py_Is("):
+        assert newer not in text

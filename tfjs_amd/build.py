@@ -74,11 +74,18 @@ def build_addon():
 
 
 def build_pycall():
+    """None where it cannot be built: the calls go through ctypes then, and an older file is not left for them to find."""
+    if os.path.exists(PYCALL):
+        os.remove(PYCALL)
     inc = sysconfig.get_paths()["include"]
     if not os.path.exists(os.path.join(inc, "Python.h")):
         return None
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", inc, "-I", os.path.join(HERE, "..", "include"),
-          os.path.join(CSRC, "pycall.cc"), "-o", PYCALL])
+    try:
+        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", inc, "-I", os.path.join(HERE, "..", "include"),
+              os.path.join(CSRC, "pycall.cc"), "-o", PYCALL])
+    except (RuntimeError, OSError) as e:
+        print("%s is not built, calls from Python go through ctypes: %s" % (os.path.basename(PYCALL), e))
+        return None
     return PYCALL
 
 

@@ -8,6 +8,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 
 import numpy as np
 
@@ -91,14 +92,18 @@ class HipBackendError(RuntimeError):
 PYCALL_PATH = os.path.join(HERE, "lib", "_pycall" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 
-def _load_pycall():
-    """The compiled argument conversions (csrc/pycall.cc), or None where they were not built for this Python: every call
-    then goes through ctypes."""
-    if not os.path.exists(PYCALL_PATH):
+def _load_pycall(path=PYCALL_PATH):
+    """The compiled argument conversions (csrc/pycall.cc), or None where they were not built for this Python or do not load:
+    every call then goes through ctypes."""
+    if not os.path.exists(path):
         return None
-    spec = importlib.util.spec_from_file_location("tfjs_amd._pycall", PYCALL_PATH)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    try:
+        spec = importlib.util.spec_from_file_location("tfjs_amd._pycall", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except Exception as e:   # (a file that is no library, or whose module cannot be set up)
+        warnings.warn("%s does not load, calls go through ctypes: %s" % (path, e), RuntimeWarning)
+        return None
     return module
 
 

@@ -437,12 +437,13 @@ bool read_specs(PyObject *specs, Weights &w) {
 // (DeviceBuffer.adopt(block, bytes), the shape), or nullptr with an error
 PyObject *adopted(PyTypeObject *type, void *block, int64_t bytes, PyObject *shape) {
   PyObject *const buf = type->tp_new(type, g_no_args, nullptr);
-  PyObject *const ptr = block ? PyLong_FromVoidPtr(block) : Py_NewRef(Py_None), *const nbytes = PyLong_FromLongLong(bytes);
+  PyObject *const address = block ? PyLong_FromVoidPtr(block) : nullptr, *const ptr = block ? address : Py_None;
+  PyObject *const nbytes = PyLong_FromLongLong(bytes);
   PyObject *pair = nullptr;
   if (buf && ptr && nbytes && PyObject_SetAttr(buf, g_nbytes, nbytes) == 0 && PyObject_SetAttr(buf, g_ptr, ptr) == 0)
     pair = PyTuple_Pack(2, buf, shape);
   Py_XDECREF(buf);
-  Py_XDECREF(ptr);
+  Py_XDECREF(address);
   Py_XDECREF(nbytes);
   return pair;
 }
@@ -506,9 +507,12 @@ PyObject *bind_decode(PyObject *, PyObject *args) {
   DecodeCall *f = PyObject_New(DecodeCall, &g_decode_type);
   if (!f) return nullptr;
   f->call = decode_vectorcall;
-  f->general = Py_NewRef(general);
-  f->buffer_type = Py_NewRef(buffer_type);
-  f->check = Py_NewRef(check);
+  f->general = general;
+  f->buffer_type = buffer_type;
+  f->check = check;
+  Py_INCREF(general);
+  Py_INCREF(buffer_type);
+  Py_INCREF(check);
   return reinterpret_cast<PyObject *>(f);
 }
 
