@@ -269,3 +269,16 @@ def test_the_extension_needs_nothing_newer_than_python_3_9():
         text = f.read()
     for newer in ("Py_NewRef", "Py_XNewRef", "PyModule_AddObjectRef", "PyType_GetModule", "Py_Is("):
         assert newer not in text
+
+
+def test_an_extension_for_other_entry_points_is_not_used(tmp_path):
+    # compiled against a header in which one entry point has an argument more
+    header = open(os.path.join(ROOT, "include", "tfjs_hip.h")).read()
+    at = header.index("int tfhip_mean_hw(") + len("int tfhip_mean_hw(")
+    (tmp_path / "tfjs_hip.h").write_text(header[:at] + "int more, " + header[at:])
+    other = tmp_path / os.path.basename(capi.PYCALL_PATH)
+    subprocess.check_call(["g++", "-O0", "-std=c++17", "-fPIC", "-shared", "-I", sysconfig.get_paths()["include"], "-I", str(tmp_path),
+                           os.path.join(ROOT, "tfjs_amd", "csrc", "pycall.cc"), "-o", str(other)])
+    with pytest.warns(RuntimeWarning, match="of another build"):
+        assert capi._load_pycall(str(other)) is None
+    assert {name: capi._codes(capi.SIGNATURES[name]) for name in capi.pycall.NAMES} == capi.pycall.NAMES

@@ -92,9 +92,14 @@ class HipBackendError(RuntimeError):
 PYCALL_PATH = os.path.join(HERE, "lib", "_pycall" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 
+def _codes(argtypes):
+    """One letter per argument: ctypes' own, for a pointer that of c_void_p."""
+    return "".join(t._type_ if isinstance(t._type_, str) else "P" for t in argtypes)
+
+
 def _load_pycall(path=PYCALL_PATH):
-    """The compiled argument conversions (csrc/pycall.cc), or None where they were not built for this Python or do not load:
-    every call then goes through ctypes."""
+    """The compiled argument conversions (csrc/pycall.cc), or None where they were not built for this Python, do not load or
+    were built for other entry points than these: every call then goes through ctypes."""
     if not os.path.exists(path):
         return None
     try:
@@ -103,6 +108,10 @@ def _load_pycall(path=PYCALL_PATH):
         spec.loader.exec_module(module)
     except Exception as e:   # (a file that is no library, or whose module cannot be set up)
         warnings.warn("%s does not load, calls go through ctypes: %s" % (path, e), RuntimeWarning)
+        return None
+    known = getattr(module, "NAMES", None)
+    if not isinstance(known, dict) or any(name not in SIGNATURES or _codes(SIGNATURES[name]) != codes for name, codes in known.items()):
+        warnings.warn("%s is of another build, calls go through ctypes" % path, RuntimeWarning)
         return None
     return module
 

@@ -145,12 +145,23 @@ PyObject *vectorcall_of(PyObject *self, PyObject *const *args, size_t nargsf, Py
   return call_entry(reinterpret_cast<Entry *>(self), args, nargsf, kwnames, Pointer(nullptr), decltype(positions(Pointer(nullptr)))());
 }
 
+// A type as ctypes codes it (pointers: c_void_p's letter).
+template <typename T>
+constexpr char code_of() {
+  return std::is_pointer<T>::value ? 'P' : (std::is_same<T, double>::value ? 'd' : (std::is_same<T, int>::value ? 'i' : (std::is_same<T, int64_t>::value ? 'l' : 'L')));
+}
+template <typename... Args>
+const char *codes_of(int (*)(Args...)) {
+  static const char codes[] = {code_of<Args>()..., 0};
+  return codes;
+}
+
 // The library is not linked: bind() brings the addresses, of whichever copy of it was loaded.
 struct Known {
-  const char *name;
+  const char *name, *codes;
   vectorcallfunc call;
 } const kKnown[] = {
-#define ENTRY(name) {#name, vectorcall_of<decltype(&name)>}
+#define ENTRY(name) {#name, codes_of(decltype(&name)(nullptr)), vectorcall_of<decltype(&name)>}
     ENTRY(tfhip_fused_matmul),          ENTRY(tfhip_fused_matmul_noalloc),      ENTRY(tfhip_fused_conv2d),
     ENTRY(tfhip_fused_conv2d_add),      ENTRY(tfhip_fused_depthwise_conv2d),    ENTRY(tfhip_fused_pointwise_depthwise),
     ENTRY(tfhip_fused_conv2d_depthwise), ENTRY(tfhip_fused_inverted_residual), ENTRY(tfhip_mean_hw),
@@ -557,12 +568,13 @@ PyMODINIT_FUNC PyInit__pycall(void) {
   if (!ready(g_decode_type, "tfjs_amd._pycall.DecodeCall", sizeof(DecodeCall), offsetof(DecodeCall, call), decode_dealloc, decode_getattro,
              decode_setattro))
     return nullptr;
-  PyObject *const module = PyModule_Create(&g_module), *const names = PyFrozenSet_New(nullptr);
+  // NAMES: the entry points and their arguments as they were when this was compiled
+  PyObject *const module = PyModule_Create(&g_module), *const names = PyDict_New();
   if (!module || !names) return nullptr;
   for (const Known &k : kKnown) {
-    PyObject *const name = PyUnicode_FromString(k.name);
-    if (!name || PySet_Add(names, name) != 0) return nullptr;
-    Py_DECREF(name);
+    PyObject *const codes = PyUnicode_FromString(k.codes);
+    if (!codes || PyDict_SetItemString(names, k.name, codes) != 0) return nullptr;
+    Py_DECREF(codes);
   }
   return PyModule_AddObject(module, "NAMES", names) == 0 ? module : nullptr;
 }
