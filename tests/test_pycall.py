@@ -282,3 +282,45 @@ def test_an_extension_for_other_entry_points_is_not_used(tmp_path):
     with pytest.warns(RuntimeWarning, match="of another build"):
         assert capi._load_pycall(str(other)) is None
     assert {name: capi._codes(capi.SIGNATURES[name]) for name in capi.pycall.NAMES} == capi.pycall.NAMES
+
+
+@pytest.mark.parametrize("name", ["device_fused_matmul", "decode_weights_to_device"])
+def test_the_compiled_functions_are_functions_to_the_rest_of_python(name):
+    run(BODY + """
+import copy, inspect, pickle, types, weakref
+f = pyhost.""" + name + """
+assert type(f) is not types.FunctionType, "not the compiled one"
+for protocol in range(pickle.HIGHEST_PROTOCOL + 1):
+    for pickler in (pickle.dumps, pickle._dumps):
+        assert pickle.loads(pickler(f, protocol)) is f
+assert copy.copy(f) is f and copy.deepcopy({"f": f})["f"] is f
+assert weakref.ref(f)() is f
+assert repr(f).startswith("<function """ + name + """ at ")
+assert inspect.isfunction(f) and f.__module__ == "tfjs_amd.pyhost" and list(inspect.signature(f).parameters)
+f.note = 3
+assert f.note == 3
+class Holder:
+    method = f
+assert Holder.method is f and Holder().method.__func__ is f
+""")
+
+
+def test_the_ctypes_functions_are_what_they_were():
+    run(BODY + """
+import pickle, weakref
+f, p = lib.tfhip_free, plain.tfhip_free
+assert type(f) is not type(p), "not the compiled one"
+assert weakref.ref(f)() is f and repr(f) == repr(f.__call__.__self__)
+assert ctypes.cast(f, ctypes.c_void_p).value == ctypes.cast(p, ctypes.c_void_p).value
+try:
+    pickle.dumps(f)
+    raise AssertionError("pickled")
+except ValueError as e:
+    assert "pointers" in str(e)
+seen = []
+lib.tfhip_mean_hw.errcheck = lambda status, fn, args: seen.append((status, args)) or 77
+assert lib.tfhip_mean_hw(a.ptr, out.ptr, 1, 7, 7, 16) == 77 and seen[0][0] == 0
+del lib.tfhip_mean_hw.errcheck
+lib.tfhip_mean_hw.restype = ctypes.c_bool
+assert lib.tfhip_mean_hw(a.ptr, out.ptr, 1, 7, 7, 16) is False
+""")

@@ -115,12 +115,12 @@ bool from(PyObject *o, const int64_t *&to) {
 struct Entry {
   PyObject_HEAD
   vectorcallfunc call;
-  PyObject *ctypes_function;
+  PyObject *weak_references, *function;   // the ctypes function
   void *address;
 };
 
 PyObject *call_ctypes(Entry *e, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
-  return PyObject_Vectorcall(e->ctypes_function, args, nargsf, kwnames);
+  return PyObject_Vectorcall(e->function, args, nargsf, kwnames);
 }
 
 template <typename... Args, size_t... I>
@@ -169,14 +169,32 @@ struct Known {
 #undef ENTRY
 };
 
+// What the callables here have of the function they stand for (all but the call itself): its attributes, its text, weak references.
+template <typename Call>
+PyObject *function_of(PyObject *self) { return reinterpret_cast<Call *>(self)->function; }
+template <typename Call>
+PyObject *text_of(PyObject *self) { return PyObject_Repr(function_of<Call>(self)); }
+
 void entry_dealloc(PyObject *self) {
-  Py_XDECREF(reinterpret_cast<Entry *>(self)->ctypes_function);
+  PyObject_ClearWeakRefs(self);
+  Py_XDECREF(function_of<Entry>(self));
   Py_TYPE(self)->tp_free(self);
 }
-// (argtypes, restype and the like are the ctypes function's)
-PyObject *entry_getattro(PyObject *self, PyObject *name) { return PyObject_GetAttr(reinterpret_cast<Entry *>(self)->ctypes_function, name); }
+PyObject *entry_getattro(PyObject *self, PyObject *name) {
+  // (ctypes' way of taking an object as an argument: cast() and the like see the ctypes function)
+  if (PyUnicode_CompareWithASCIIString(name, "_as_parameter_") == 0) {
+    Py_INCREF(function_of<Entry>(self));
+    return function_of<Entry>(self);
+  }
+  return PyObject_GetAttr(function_of<Entry>(self), name);
+}
+PyObject *entry_by_ctypes(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
+  return call_ctypes(reinterpret_cast<Entry *>(self), args, nargsf, kwnames);
+}
+// (argtypes, restype, errcheck: the ctypes function goes by them, so from then on it is what is called)
 int entry_setattro(PyObject *self, PyObject *name, PyObject *value) {
-  return PyObject_SetAttr(reinterpret_cast<Entry *>(self)->ctypes_function, name, value);
+  reinterpret_cast<Entry *>(self)->call = entry_by_ctypes;
+  return PyObject_SetAttr(function_of<Entry>(self), name, value);
 }
 
 PyTypeObject g_entry_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -197,8 +215,9 @@ PyObject *bind(PyObject *, PyObject *args) {
     Entry *e = PyObject_New(Entry, &g_entry_type);
     if (!e) return nullptr;
     e->call = k.call;
+    e->weak_references = nullptr;
     Py_INCREF(function);
-    e->ctypes_function = function;
+    e->function = function;
     e->address = reinterpret_cast<void *>(static_cast<uintptr_t>(address));
     if (strcmp(name, "tfhip_fused_matmul") == 0) g_fused_matmul = reinterpret_cast<decltype(g_fused_matmul)>(e->address);
     if (strcmp(name, "tfhip_decode_weights") == 0) g_decode_weights = reinterpret_cast<decltype(g_decode_weights)>(e->address);
@@ -215,10 +234,28 @@ const char *const kNames[kParams] = {"a", "b", "out", "batch_a", "batch_b", "m",
                                      "bias", "bias_strides", "activation", "prelu", "prelu_strides", "leakyrelu_alpha"};
 PyObject *g_names[kParams] = {}, *g_ptr = nullptr;   // (interned)
 
+// A function of the package by another body. Pickled and copied as a function is, by its name; as a class's attribute a method.
+PyObject *by_name(PyObject *self, PyObject *);
+PyMethodDef g_by_name[] = {{"__reduce__", by_name, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+template <typename Call>
+PyObject *python_getattro(PyObject *self, PyObject *name) {
+  for (const char *own : {"__reduce__", "__reduce_ex__"})
+    if (PyUnicode_CompareWithASCIIString(name, own) == 0) return PyObject_GenericGetAttr(self, name);
+  return PyObject_GetAttr(function_of<Call>(self), name);
+}
+template <typename Call>
+int python_setattro(PyObject *self, PyObject *name, PyObject *value) { return PyObject_SetAttr(function_of<Call>(self), name, value); }
+PyObject *by_name(PyObject *self, PyObject *) { return PyObject_GetAttrString(self, "__qualname__"); }
+PyObject *method_of(PyObject *self, PyObject *object, PyObject *) {
+  if (object && object != Py_None) return PyMethod_New(self, object);
+  Py_INCREF(self);
+  return self;
+}
+
 struct MatmulCall {
   PyObject_HEAD
   vectorcallfunc call;
-  PyObject *general, *activations, *check;   // the function in Python, the activations' numbers, what a status goes to
+  PyObject *weak_references, *function, *activations, *check;   // the function in Python, the activations' numbers, what a status goes to
 };
 
 bool pointer_of(PyObject *operand, void *&to) {
@@ -282,7 +319,7 @@ PyObject *matmul_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
     ok = number && from(number, activation);
     if (!ok) PyErr_Clear();
   }
-  if (!ok) return PyObject_Vectorcall(f->general, args, nargsf, kwnames);
+  if (!ok) return PyObject_Vectorcall(f->function, args, nargsf, kwnames);
   int status = 0;
   Py_BEGIN_ALLOW_THREADS
   status = g_fused_matmul(static_cast<const float *>(a), static_cast<const float *>(b), static_cast<float *>(out), size[0], size[1], size[2], size[3],
@@ -299,17 +336,12 @@ PyObject *matmul_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
 
 void matmul_dealloc(PyObject *self) {
   MatmulCall *const f = reinterpret_cast<MatmulCall *>(self);
-  Py_XDECREF(f->general);
+  PyObject_ClearWeakRefs(self);
+  Py_XDECREF(f->function);
   Py_XDECREF(f->activations);
   Py_XDECREF(f->check);
   Py_TYPE(self)->tp_free(self);
 }
-PyObject *matmul_getattro(PyObject *self, PyObject *name) { return PyObject_GetAttr(reinterpret_cast<MatmulCall *>(self)->general, name); }
-
-int matmul_setattro(PyObject *self, PyObject *name, PyObject *value) {
-  return PyObject_SetAttr(reinterpret_cast<MatmulCall *>(self)->general, name, value);
-}
-
 PyTypeObject g_matmul_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // bind_matmul(function in Python, activations, check): the same function
@@ -319,7 +351,8 @@ PyObject *bind_matmul(PyObject *, PyObject *args) {
   MatmulCall *f = PyObject_New(MatmulCall, &g_matmul_type);
   if (!f) return nullptr;
   f->call = matmul_vectorcall;
-  f->general = general;
+  f->weak_references = nullptr;
+  f->function = general;
   f->activations = activations;
   f->check = check;
   Py_INCREF(general);
@@ -333,7 +366,7 @@ PyObject *bind_matmul(PyObject *, PyObject *args) {
 struct DecodeCall {
   PyObject_HEAD
   vectorcallfunc call;
-  PyObject *general, *buffer_type, *check;   // the function in Python, DeviceBuffer, what a status goes to
+  PyObject *weak_references, *function, *buffer_type, *check;   // the function in Python, DeviceBuffer, what a status goes to
 };
 PyObject *g_name, *g_dtype, *g_shape, *g_quantization, *g_scale, *g_min, *g_nbytes, *g_no_args;
 constexpr int kNotInitialised = 1;   // (of the library's statuses: the general function sets it up)
@@ -461,7 +494,7 @@ PyObject *adopted(PyTypeObject *type, void *block, int64_t bytes, PyObject *shap
 
 PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf, PyObject *kwnames) {
   DecodeCall *const f = reinterpret_cast<DecodeCall *>(self);
-  const auto general = [&] { return PyObject_Vectorcall(f->general, args, nargsf, kwnames); };
+  const auto general = [&] { return PyObject_Vectorcall(f->function, args, nargsf, kwnames); };
   if (!g_decode_weights || !g_free || PyVectorcall_NARGS(nargsf) != 2 || (kwnames && PyTuple_GET_SIZE(kwnames) > 0)) return general();
   try {
     Weights w;
@@ -499,16 +532,12 @@ PyObject *decode_vectorcall(PyObject *self, PyObject *const *args, size_t nargsf
 
 void decode_dealloc(PyObject *self) {
   DecodeCall *const f = reinterpret_cast<DecodeCall *>(self);
-  Py_XDECREF(f->general);
+  PyObject_ClearWeakRefs(self);
+  Py_XDECREF(f->function);
   Py_XDECREF(f->buffer_type);
   Py_XDECREF(f->check);
   Py_TYPE(self)->tp_free(self);
 }
-PyObject *decode_getattro(PyObject *self, PyObject *name) { return PyObject_GetAttr(reinterpret_cast<DecodeCall *>(self)->general, name); }
-int decode_setattro(PyObject *self, PyObject *name, PyObject *value) {
-  return PyObject_SetAttr(reinterpret_cast<DecodeCall *>(self)->general, name, value);
-}
-
 PyTypeObject g_decode_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // bind_decode(function in Python, DeviceBuffer, check): the same function
@@ -518,7 +547,8 @@ PyObject *bind_decode(PyObject *, PyObject *args) {
   DecodeCall *f = PyObject_New(DecodeCall, &g_decode_type);
   if (!f) return nullptr;
   f->call = decode_vectorcall;
-  f->general = general;
+  f->weak_references = nullptr;
+  f->function = general;
   f->buffer_type = buffer_type;
   f->check = check;
   Py_INCREF(general);
@@ -531,16 +561,25 @@ PyMethodDef g_methods[] = {{"bind", bind, METH_VARARGS, nullptr}, {"bind_matmul"
                            {"bind_decode", bind_decode, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_pycall", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
-bool ready(PyTypeObject &type, const char *name, Py_ssize_t size, Py_ssize_t call_offset, destructor dealloc, getattrofunc get, setattrofunc set) {
+template <typename Call>
+bool ready(PyTypeObject &type, const char *name, destructor dealloc, getattrofunc get, setattrofunc set) {
   type.tp_name = name;
-  type.tp_basicsize = size;
-  type.tp_vectorcall_offset = call_offset;
+  type.tp_basicsize = sizeof(Call);
+  type.tp_vectorcall_offset = offsetof(Call, call);
+  type.tp_weaklistoffset = offsetof(Call, weak_references);
   type.tp_call = PyVectorcall_Call;
+  type.tp_repr = text_of<Call>;
   type.tp_dealloc = dealloc;
   type.tp_getattro = get;
   type.tp_setattro = set;
   type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
   return PyType_Ready(&type) == 0;
+}
+template <typename Call>
+bool ready_as_function(PyTypeObject &type, const char *name, destructor dealloc) {
+  type.tp_methods = g_by_name;
+  type.tp_descr_get = method_of;
+  return ready<Call>(type, name, dealloc, python_getattro<Call>, python_setattro<Call>);
 }
 
 }  // namespace
@@ -561,13 +600,9 @@ PyMODINIT_FUNC PyInit__pycall(void) {
   for (const auto &key : keys)
     if (!(*key.first = PyUnicode_InternFromString(key.second))) return nullptr;
   if (!(g_no_args = PyTuple_New(0))) return nullptr;
-  if (!ready(g_entry_type, "tfjs_amd._pycall.Entry", sizeof(Entry), offsetof(Entry, call), entry_dealloc, entry_getattro, entry_setattro)) return nullptr;
-  if (!ready(g_matmul_type, "tfjs_amd._pycall.MatmulCall", sizeof(MatmulCall), offsetof(MatmulCall, call), matmul_dealloc, matmul_getattro,
-             matmul_setattro))
-    return nullptr;
-  if (!ready(g_decode_type, "tfjs_amd._pycall.DecodeCall", sizeof(DecodeCall), offsetof(DecodeCall, call), decode_dealloc, decode_getattro,
-             decode_setattro))
-    return nullptr;
+  if (!ready<Entry>(g_entry_type, "tfjs_amd._pycall.Entry", entry_dealloc, entry_getattro, entry_setattro)) return nullptr;
+  if (!ready_as_function<MatmulCall>(g_matmul_type, "tfjs_amd._pycall.MatmulCall", matmul_dealloc)) return nullptr;
+  if (!ready_as_function<DecodeCall>(g_decode_type, "tfjs_amd._pycall.DecodeCall", decode_dealloc)) return nullptr;
   // NAMES: the entry points and their arguments as they were when this was compiled
   PyObject *const module = PyModule_Create(&g_module), *const names = PyDict_New();
   if (!module || !names) return nullptr;
