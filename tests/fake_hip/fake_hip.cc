@@ -26,7 +26,7 @@ struct Block {
 };
 struct Launch {
   std::string name;
-  std::vector<char> first;   // the leading bytes of the first argument
+  std::vector<char> first;   // the leading bytes of the first argument (of few_rows and decode_batch)
   int device;
   bool recorded;
 };
@@ -237,6 +237,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
                                  name.find("copy_to_host") != std::string::npos ? (long long)*(int *)args[2] : 0};
   Launch l = {name, {}, stream_device[stream], recording_on.count(stream) > 0};
   if (name.find("few_rows") != std::string::npos) l.first.assign((const char *)args[0], (const char *)args[0] + kNotedBytes);
+  if (name.find("decode_batch") != std::string::npos) l.first.assign((const char *)args[0], (const char *)args[0] + sizeof(void *));
   launches.push_back(l);
   if (l.recorded) {
     recording_on[stream]->kernels.push_back(name);
