@@ -466,33 +466,43 @@ int balanced_tile(int extent, int max_tile) {
 // of float4s: 2), took 1.10; 15 maps are more than 3% slower than with those, 4 more than 6%. us, before and so: [2,31,8,910] 5x5
 // 8.4 and 4.9, [4,7,38,744] 3x3 5.4 and 4.1, [1,49,107,119] 5x5/2 4.6 and 3.9, [6,16,49,784] 3x3 8.3 and 6.9, [8,57,43,120] 5x5/2 5.7 and 5.5.
 struct ColsEstimate {
-  int f, stride, vec, streamed;
   double first, step, wave, row;
 };
-constexpr ColsEstimate kColsEstimates[] = {
-    {3, 1, 1, 0, 0.00, 0.131, 0.079, 0.000}, {3, 1, 1, 1, 0.06, 0.274, 0.096, 0.024}, {3, 1, 2, 0, 0.00, 0.173, 0.186, 0.000},
-    {3, 1, 2, 1, 0.06, 0.274, 0.096, 0.024}, {3, 1, 4, 0, 0.00, 0.244, 0.249, 0.000}, {3, 1, 4, 1, 0.00, 0.262, 0.141, 0.027},
-    {3, 2, 1, 0, 0.00, 0.207, 0.109, 0.000}, {3, 2, 2, 0, 0.00, 0.369, 0.001, 0.087}, {3, 2, 4, 0, 0.00, 0.313, 0.300, 0.000},
-    {5, 1, 1, 0, 0.00, 0.197, 0.185, 0.000}, {5, 1, 1, 1, 0.00, 0.328, 0.058, 0.023}, {5, 1, 2, 0, 0.00, 0.277, 0.196, 0.045},
-    {5, 1, 2, 1, 0.00, 0.319, 0.205, 0.039}, {5, 1, 4, 0, 0.26, 0.403, 0.075, 0.089}, {5, 1, 4, 1, 0.00, 0.356, 0.144, 0.065},
-    {5, 2, 1, 0, 0.00, 0.347, 0.124, 0.028}, {5, 2, 2, 0, 0.09, 0.367, 0.275, 0.046}, {5, 2, 4, 0, 0.97, 0.453, 0.373, 0.064},
-};
+// [filter 3, 5][stride 1, 2][channels per lane 1, 2, 4][result streamed]
+constexpr ColsEstimate kColsEstimates[2][2][3][2] = {
+    {{{{0.00, 0.131, 0.079, 0.000}, {0.06, 0.274, 0.096, 0.024}}, {{0.00, 0.173, 0.186, 0.000}, {0.06, 0.274, 0.096, 0.024}},
+      {{0.00, 0.244, 0.249, 0.000}, {0.00, 0.262, 0.141, 0.027}}},
+     {{{0.00, 0.207, 0.109, 0.000}, {0.00, 0.207, 0.109, 0.000}}, {{0.00, 0.369, 0.001, 0.087}, {0.00, 0.369, 0.001, 0.087}},
+      {{0.00, 0.313, 0.300, 0.000}, {0.00, 0.313, 0.300, 0.000}}}},
+    {{{{0.00, 0.197, 0.185, 0.000}, {0.00, 0.328, 0.058, 0.023}}, {{0.00, 0.277, 0.196, 0.045}, {0.00, 0.319, 0.205, 0.039}},
+      {{0.26, 0.403, 0.075, 0.089}, {0.00, 0.356, 0.144, 0.065}}},
+     {{{0.00, 0.347, 0.124, 0.028}, {0.00, 0.347, 0.124, 0.028}}, {{0.09, 0.367, 0.275, 0.046}, {0.09, 0.367, 0.275, 0.046}},
+      {{0.97, 0.453, 0.373, 0.064}, {0.97, 0.453, 0.373, 0.064}}}}};
 constexpr int kMostRows = 28;
+struct Inverses {
+  double of[kMostRows + 1] = {};
+  constexpr Inverses() {
+    for (int i = 1; i <= kMostRows; ++i) of[i] = 1.0 / i;
+  }
+};
+constexpr Inverses kInverses;
 
-// Output rows per lane: the fewest whose estimate is within 2% of the least.
+// Output rows per lane: the fewest whose estimate is within 2% of the least. (Counts that do not divide a map evenly stand here as they
+// are: the even count with as many chunks is smaller, so its estimate is less and it is met first. Every call goes through this: with
+// integer divisions for the chunks of 28 counts it took the host 0.2 us, so 0.06.)
 int rows_per_lane(const DwParams &p, int vec, bool streamed, long long blocks_per_row) {
-  const ColsEstimate *e = nullptr;
-  for (const ColsEstimate &c : kColsEstimates)
-    if (c.f == p.f_h && c.stride == p.stride_h && c.vec == vec && (!e || c.streamed == (int)streamed)) e = &c;
+  const ColsEstimate &e = kColsEstimates[p.f_h == 5][p.stride_h - 1][vec >> 1][streamed];
   const int most = p.out_h < kMostRows ? p.out_h : kMostRows;
   const double share = (double)blocks_per_row * p.batch / num_cus();
-  double cubes[kMostRows + 1], least = 0;
+  const double wave = share * (e.wave + e.row * (p.f_h - p.stride_h)), row = share * e.row * p.stride_h;
+  double cubes[kMostRows + 1];
   for (int rows = 1; rows <= most; ++rows) {
-    const int chunk = balanced_tile(p.out_h, rows), chunks = (p.out_h + chunk - 1) / chunk;
-    const double way = e->first + e->step * chunk, work = share * chunks * (e->wave + e->row * ((chunk - 1) * p.stride_h + p.f_h));
+    const double chunks = (double)((int)((p.out_h - 0.5) * kInverses.of[rows]) + 1);   // (exact: the quotient is no nearer to a whole number than half of 1 / rows)
+    const double way = e.first + e.step * rows, work = chunks * (wave + row * rows);
     cubes[rows] = way * way * way + work * work * work;
-    if (rows == 1 || cubes[rows] < least) least = cubes[rows];
   }
+  double least = cubes[1];
+  for (int rows = 2; rows <= most; ++rows) least = cubes[rows] < least ? cubes[rows] : least;
   int rows = 1;
   while (cubes[rows] > 1.06 * least) ++rows;
   return rows;
