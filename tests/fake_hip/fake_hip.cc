@@ -29,6 +29,7 @@ struct Launch {
   std::vector<char> first;   // the leading bytes of the first argument (of few_rows and decode_batch)
   int device;
   bool recorded;
+  unsigned grid_x;
 };
 struct Recording {
   std::vector<std::string> kernels;
@@ -125,6 +126,11 @@ int fake_hip_launch(int back, char *name, size_t len, void *first, size_t first_
   memcpy(first, l.first.data(), first_len < l.first.size() ? first_len : l.first.size());
   *recorded = l.recorded;
   return l.device;
+}
+// Workgroups along x of the launch `back` launches ago.
+int fake_hip_grid(int back) {
+  std::lock_guard<std::recursive_mutex> lock(m);
+  return back < (int)launches.size() ? (int)launches[launches.size() - 1 - back].grid_x : -1;
 }
 int fake_hip_launches(void) {
   std::lock_guard<std::recursive_mutex> lock(m);
@@ -227,7 +233,7 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
   *grid = pushed.grid; *block = pushed.block; *shared = pushed.shared; *stream = pushed.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t stream) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t stream) {
   if (launch_delay_us) usleep(launch_delay_us);
   std::lock_guard<std::recursive_mutex> lock(m);
   const std::string name = kernel_names[f];
@@ -235,7 +241,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
   if (has_effect(name)) words = {*(long long *)args[0], *(long long *)(args[name.find("clear_word") == std::string::npos ? 1 : 0]),
                                  name.find("find_nonfinite") != std::string::npos ? *(long long *)args[2] :
                                  name.find("copy_to_host") != std::string::npos ? (long long)*(int *)args[2] : 0};
-  Launch l = {name, {}, stream_device[stream], recording_on.count(stream) > 0};
+  Launch l = {name, {}, stream_device[stream], recording_on.count(stream) > 0, grid.x};
   if (name.find("few_rows") != std::string::npos) l.first.assign((const char *)args[0], (const char *)args[0] + kNotedBytes);
   if (name.find("decode_batch") != std::string::npos) l.first.assign((const char *)args[0], (const char *)args[0] + sizeof(void *));
   launches.push_back(l);
@@ -273,7 +279,7 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t stream) {
   std::lock_guard<std::recursive_mutex> lock(m);
   const Recording &r = *(Recording *)e;
   for (size_t i = 0; i < r.kernels.size(); ++i) {
-    launches.push_back({r.kernels[i], {}, stream_device[stream], false});
+    launches.push_back({r.kernels[i], {}, stream_device[stream], false, 0});
     if (!r.args[i].empty()) run_kernel(r.kernels[i], r.args[i]);
   }
   return hipSuccess;

@@ -611,3 +611,23 @@ check(lib.tfhip_set_tuning(b"dw_rows", -1))
 assert "depthwise_3x3_cols" in launch()[0]
 assert best[-1] - best[14] < 0.13e-6, best
 """)
+
+
+def test_the_rows_of_a_depthwise_lane_by_size():
+    """Maps on which other counts measured 4 to 20% slower: many images, a result that is streamed at stride 2, channels that
+    fit no float4, a handful of wavefronts."""
+    fake_hip_util.run("""
+pyhost.init()
+a, w, out = DeviceBuffer(32 * 112 * 112 * 96 * 4), DeviceBuffer(1 << 17), DeviceBuffer(1 << 26)
+zeros = i64_array([0] * 4)
+for (batch, h, wd, c, stride), least, most in (((32, 112, 112, 96, 2), 4, 8), ((10, 85, 7, 80, 2), 1, 1), ((9, 44, 60, 194, 2), 3, 7), ((12, 32, 13, 929, 2), 8, 12),
+                                               ((168, 23, 33, 58, 2), 6, 6), ((3, 79, 32, 357, 1), 6, 12), ((2, 89, 18, 176, 2), 1, 1)):
+    oh, ow = -(-h // stride), -(-wd // stride)   # "same" padding
+    top, left = max((oh - 1) * stride + 3 - h, 0) // 2, max((ow - 1) * stride + 3 - wd, 0) // 2
+    check(lib.tfhip_fused_depthwise_conv2d(a.ptr, w.ptr, out.ptr, batch, h, wd, c, 3, 3, 1, stride, stride, 1, 1, top, left, oh, ow,
+                                           None, zeros, 1, None, zeros, 0.2))
+    vec = 4 if c % 4 == 0 else 2 if c % 2 == 0 else 1
+    chunks = fake.fake_hip_grid(0) // (-(-ow * (c // vec) // 64) * batch)
+    rows = -(-oh // chunks)
+    assert "_cols" in launch()[0] and least <= rows <= most, ((batch, h, wd, c, stride), rows)
+""")

@@ -458,27 +458,31 @@ int balanced_tile(int extent, int max_tile) {
   return (extent + tiles - 1) / tiles;
 }
 
-// What a launch of the column kernels takes beside what does not depend on the rows per lane, in microseconds: a lane's way down
-// its rows (`first`, and `step` per output row), and a compute unit's share of the wavefronts (`wave` each, `row` per input row);
-// the root of the cubes' sum, with the tensors' way through memory as a third. Least squares on 820 random maps of [1-16,7-112,7-112,16-960],
-// 13 row counts each, operands from memory (root mean square error 5 to 13%). The rows with the least estimate took on average 1.01
-// of the time of the best of the 13, where chunks of 14 (stride 2: 8) rows, halved until there were 8 wavefronts per compute unit (5x5
-// of float4s: 2), took 1.10; 15 maps are more than 3% slower than with those, 4 more than 6%. us, before and so: [2,31,8,910] 5x5
-// 8.4 and 4.9, [4,7,38,744] 3x3 5.4 and 4.1, [1,49,107,119] 5x5/2 4.6 and 3.9, [6,16,49,784] 3x3 8.3 and 6.9, [8,57,43,120] 5x5/2 5.7 and 5.5.
+// What a launch of the column kernels takes beside what does not depend on the rows per lane: a lane's way down its rows (`first`,
+// and `step` per output row), and a compute unit's share of the wavefronts (`wave` each, `row` per input row); the root of the
+// cubes' sum. Only which rows have the least of it matters: some entries are least squares in microseconds, the others (those with a
+// `first` and a `step` near 1 among them) were fitted to the choice itself, to the time of the rows they choose over that of the best.
+// Measured on 4378 random maps of [1-256,7-112,7-112,16-960], up to 15 row counts each, operands from memory: the rows chosen take
+// 1.006 of the time of the best of them; chunks of 14 (stride 2: 8) rows, halved until there are 8 wavefronts per compute unit (5x5 of
+// float4s: 2), 1.06. 43 maps are more than 3% slower than with those, 12 more than 6%. us, with those and so: [2,31,8,910] 5x5 8.4
+// and 4.9, [4,7,38,744] 3x3 5.4 and 4.1, [1,49,107,119] 5x5/2 4.6 and 3.9, [6,16,49,784] 3x3 8.3 and 6.9, [3,79,32,357] 3x3 9.3 and 8.7.
+// The streamed results of 3x3 at stride 2 are on a par up to 8 rows and fall behind beyond, which the estimate does not know
+// ([128,112,112,96] 4 rows 143, 8 144, 12 148, 28 156).
+constexpr int kMostRows = 28;
 struct ColsEstimate {
   double first, step, wave, row;
+  int most = kMostRows;   // rows per lane
 };
 // [filter 3, 5][stride 1, 2][channels per lane 1, 2, 4][result streamed]
 constexpr ColsEstimate kColsEstimates[2][2][3][2] = {
-    {{{{0.00, 0.131, 0.079, 0.000}, {0.06, 0.274, 0.096, 0.024}}, {{0.00, 0.173, 0.186, 0.000}, {0.06, 0.274, 0.096, 0.024}},
-      {{0.00, 0.244, 0.249, 0.000}, {0.00, 0.262, 0.141, 0.027}}},
-     {{{0.00, 0.207, 0.109, 0.000}, {0.00, 0.207, 0.109, 0.000}}, {{0.00, 0.369, 0.001, 0.087}, {0.00, 0.369, 0.001, 0.087}},
-      {{0.00, 0.313, 0.300, 0.000}, {0.00, 0.313, 0.300, 0.000}}}},
-    {{{{0.00, 0.197, 0.185, 0.000}, {0.00, 0.328, 0.058, 0.023}}, {{0.00, 0.277, 0.196, 0.045}, {0.00, 0.319, 0.205, 0.039}},
-      {{0.26, 0.403, 0.075, 0.089}, {0.00, 0.356, 0.144, 0.065}}},
-     {{{0.00, 0.347, 0.124, 0.028}, {0.00, 0.347, 0.124, 0.028}}, {{0.09, 0.367, 0.275, 0.046}, {0.09, 0.367, 0.275, 0.046}},
-      {{0.97, 0.453, 0.373, 0.064}, {0.97, 0.453, 0.373, 0.064}}}}};
-constexpr int kMostRows = 28;
+    {{{{0.98, 0.907, 0.196, 0.040}, {0.36, 0.769, 0.346, 0.038}}, {{0.01, 0.973, 0.245, 0.104}, {0.06, 0.274, 0.096, 0.024}},
+      {{0.20, 0.972, 0.834, 0.003}, {0.00, 0.262, 0.141, 0.027}}},
+     {{{0.94, 0.025, 0.051, 0.001}, {0.94, 0.488, 0.727, 0.008}}, {{0.85, 0.896, 0.262, 0.057}, {0.29, 0.915, 0.279, 0.076}},
+      {{0.98, 0.826, 0.367, 0.107}, {0.97, 0.029, 0.790, 0.020, 8}}}},
+    {{{{0.42, 0.934, 0.102, 0.078}, {0.00, 0.328, 0.058, 0.023}}, {{0.00, 0.277, 0.196, 0.045}, {0.00, 0.319, 0.205, 0.039}},
+      {{0.95, 0.028, 0.194, 0.000}, {0.73, 0.469, 0.516, 0.059}}},
+     {{{0.46, 0.858, 0.213, 0.082}, {0.00, 0.347, 0.124, 0.028}}, {{0.87, 0.236, 0.374, 0.016}, {0.09, 0.367, 0.275, 0.046}},
+      {{0.84, 0.354, 0.090, 0.078}, {0.97, 0.453, 0.373, 0.064}}}}};
 struct Inverses {
   double of[kMostRows + 1] = {};
   constexpr Inverses() {
@@ -492,7 +496,7 @@ constexpr Inverses kInverses;
 // integer divisions for the chunks of 28 counts it took the host 0.2 us, so 0.06.)
 int rows_per_lane(const DwParams &p, int vec, bool streamed, long long blocks_per_row) {
   const ColsEstimate &e = kColsEstimates[p.f_h == 5][p.stride_h - 1][vec >> 1][streamed];
-  const int most = p.out_h < kMostRows ? p.out_h : kMostRows;
+  const int most = p.out_h < e.most ? p.out_h : e.most;
   const double share = (double)blocks_per_row * p.batch / num_cus();
   const double wave = share * (e.wave + e.row * (p.f_h - p.stride_h)), row = share * e.row * p.stride_h;
   double cubes[kMostRows + 1];
