@@ -631,3 +631,27 @@ for (batch, h, wd, c, stride), least, most in (((32, 112, 112, 96, 2), 4, 8), ((
     rows = -(-oh // chunks)
     assert "_cols" in launch()[0] and least <= rows <= most, ((batch, h, wd, c, stride), rows)
 """)
+
+
+def test_products_of_a_short_k_that_suit_the_tiled_kernel():
+    """Products and windows of a few k tiles that measured 5 to 30% slower in bf16 parts (tiles of 64 x 64 or 64 x 48 that pad little,
+    results of a few MB), beside others of the same extents that are faster there."""
+    fake_hip_util.run("""
+pyhost.init()
+a, b, out = DeviceBuffer(1 << 25), DeviceBuffer(1 << 24), DeviceBuffer(1 << 27)
+zeros = i64_array([0] * 4)
+def name():
+    text = ctypes.create_string_buffer(256)
+    check(lib.tfhip_last_kernel(text, 256))
+    return text.value.decode().split("<")[0]
+for m, n, k, transposed, want in ((11616, 368, 14, 0, "gemm_kernel"), (32474, 112, 16, 0, "gemm_kernel"), (1280, 2032, 32, 0, "gemm_kernel"), (44122, 40, 32, 0, "gemm_kernel"),
+                                  (42522, 40, 21, 0, "gemm_kernel"), (28720, 41, 27, 0, "gemm_kernel"), (46998, 33, 117, 0, "gemm_kernel"), (11558, 256, 148, 1, "gemm_kernel"),
+                                  (6621, 2295, 12, 0, "split_gemm"), (1454, 4277, 23, 0, "split_gemm"), (4466, 652, 61, 0, "split_gemm"), (1613, 3645, 39, 0, "split_gemm")):
+    check(lib.tfhip_fused_matmul(a.ptr, b.ptr, out.ptr, 1, 1, m, n, k, 0, transposed, None, None, 0, None, None, 0.2))
+    assert name() == want, (m, n, k, transposed, name())
+for (batch, h, w, c, n, f), want in (((5, 172, 122, 8, 56, 3), "gemm_kernel"), ((13, 92, 83, 8, 64, 2), "gemm_kernel"), ((8, 83, 57, 16, 112, 2), "gemm_kernel"),
+                                     ((16, 67, 98, 5, 56, 2), "gemm_kernel"), ((5, 96, 85, 8, 224, 3), "split_gemm"), ((4, 92, 164, 8, 96, 2), "split_gemm"),
+                                     ((5, 127, 128, 3, 101, 3), "split_gemm")):
+    check(lib.tfhip_fused_conv2d(a.ptr, b.ptr, out.ptr, batch, h, w, c, f, f, n, 1, 1, 1, 1, (f - 1) // 2, (f - 1) // 2, h, w, 0, None, zeros, 0, None, zeros, 0.2))
+    assert name() == want, (batch, h, w, c, n, f, name())
+""")

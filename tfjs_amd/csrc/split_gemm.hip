@@ -144,10 +144,9 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b
   const bool narrow = forced < 0 && p.N <= 32;
   // Below 0.45 GFLOP the fixed part decides, and that of the other kernels is shorter (0.1 to 0.2 GFLOP 1.2 times slower here, of 39
   // products and convolutions of 0.3 to 0.45 1.02 times; 0.8 to 1.2 0.88 of the time, from 4 on 0.7), but for products of a few k tiles,
-  // whose results are most of the work: of 435 of K 8 to 128 and 0.06 to 0.45 GFLOP 104 are 3% faster and more (all together 0.94 of the time),
-  // five 3 to 5% slower, by the last line below (windows from 0.2 GFLOP on); 1454 x 4277 x 23 takes 17 us there and 11 here, 6480 x 460 x 32 9.7 and 7.5. (Of a
-  // transposed B 32 of 200 gain, 7 lose up to 28%.) So it is with tiles that are mostly padding: few columns, few rows of each product of a
-  // batch. Under 448 rows only half of the products gain.
+  // whose results are most of the work: those of K up to 128 from 0.06 GFLOP on, and windows from 0.2, go by the last lines below (1454 x 4277 x 23
+  // 17 us there and 11 here; of a transposed B 32 of 200 gain and 7 lose up to 28%). So it is with tiles that
+  // are mostly padding: few columns, few rows of each product of a batch. Under 448 rows only half of the products gain.
   const double flops = 2.0 * p.batch * p.M * (double)p.N * p.K;
   const bool small = forced < 0 && flops < 4.5e8;
   const double least = narrow ? 4.5e8
@@ -182,14 +181,25 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b
                               : tiled_estimate_us(p, a_kind == kLoadWindows ? 1.24 : (a_kind == kLoadWindowsAny ? 1.82 : 1.0)) *
                                     (transposed_b && p.K > 128 ? 0.9 : 1.0);
   if (forced >= 0 || (!small && best_us <= 0.92 * tiled)) return best;
-  // What that line leaves, by the estimate that knows of a tile's end: of 700 products of K 16 to 1024 some 140, on average at 0.78 of the time,
-  // five of them 3 to 8% slower; of 300 of K 8 to 40 230, at 0.69, one 12% slower. us, before and here: 4282 x 3818 x 32 34 and 21, 18 x
-  // (1007 x 20 x 860) of a transposed B 30 and 19, 3991 x 1333 x 71 20 and 13. (By that estimate alone, 3% of the products that the line
-  // takes were not taken any more, and up to 1.3 times slower.)
-  // Of 350 windows of K 16 to 400 that are left 43, on average at 0.86 of the time, and of 110 ragged ones 11, at 0.74 (46 of the 54 3% faster and
-  // more, six 6 to 13% slower): 130032 x 224 x 72 94 and 54, 40700 x 224 x 72 33 and 24, 81125 x 100 x 40 (ragged) 39 and 24.
-  const double lead = a_kind == kLoadKAny ? (small ? 0.92 : 0.97) : (small ? 0.87 : 0.91);
-  if (narrow || (a_kind != kLoadKAny && p.K > kEndWindows) || best_us > lead * tiled_end_us(p, a_kind, transposed_b)) best.shape = -1;
+  // What that line leaves, by the estimate that knows of a tile's end: 5300 of 7600 products of K 8 to 1024 and 0.06 to 10 GFLOP at 0.77
+  // of the time, 500 of 1500 windows of K up to 400 at 0.74, but not:
+  //  * what gemm_kernel has tiles of 64 x 64 or 64 x 48 for, which it has where they fill the chip and pad little: small products
+  //    (700, 1.0 of the time at the median) and windows (86, 1.06) there; larger products only with more of a lead (0.85).
+  //  * small products whose results are below 20 MB, but for a larger lead (0.81): 16% of them were slower, at 0.92 on average.
+  // Of what is left, 2% of the small products, 1% of the others, 1.6% of a transposed B and 1% of the windows are 3% slower and more (before
+  // these two 8, 1.4, 3.5 and 10%, up to a third: 11616 x 368 x 14 6.7 and 8.8, 32474 x 112 x 16 5.7 and 7.3, [7,96,98,3] 5x5 -> 61 17.6
+  // and 23.0). us, before and here: 4282 x 3818 x 32 34 and 21, 18 x (1007 x 20 x 860) of a transposed B 30 and 19, 3991 x 1333 x 71
+  // 20 and 13, 130032 x 224 x 72 (windows) 94 and 54, 81125 x 100 x 40 (ragged) 39 and 24. (By that estimate alone, 3% of the products that
+  // the line above takes were not taken any more, and up to 1.3 times slower.)
+  const double part = best_us / tiled_end_us(p, a_kind, transposed_b);
+  double lead = a_kind == kLoadKAny ? (small ? 0.92 : 0.97) : (small ? 0.87 : 0.91);
+  if (!narrow && (a_kind == kLoadKAny || p.K <= kEndWindows) && part <= lead) {
+    const TileShape &t = kTileShapes[choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus())];
+    if (t.bm == 64 && t.bn <= 64) lead = small || a_kind != kLoadKAny ? 0 : 0.85;
+    else if (small && a_kind == kLoadKAny && (double)p.batch * p.M * p.N < 5e6) lead = 0.81;
+    if (part <= lead) return best;
+  }
+  best.shape = -1;
   return best;
 }
 
