@@ -655,3 +655,23 @@ for (batch, h, w, c, n, f), want in (((5, 172, 122, 8, 56, 3), "gemm_kernel"), (
     check(lib.tfhip_fused_conv2d(a.ptr, b.ptr, out.ptr, batch, h, w, c, f, f, n, 1, 1, 1, 1, (f - 1) // 2, (f - 1) // 2, h, w, 0, None, zeros, 0, None, zeros, 0.2))
     assert name() == want, (batch, h, w, c, n, f, name())
 """)
+
+
+def test_choosing_the_kernel_of_a_small_product_costs_the_host_little():
+    """The estimates that a product of a few k tiles goes through, against a call that leaves them out; the least of many turns."""
+    fake_hip_util.run("""
+pyhost.init()
+a, b, out = DeviceBuffer(1 << 20), DeviceBuffer(1 << 20), DeviceBuffer(1 << 22)
+call, best = lib.tfhip_fused_matmul, {}
+args = [a.ptr, b.ptr, out.ptr, 1, 1, 1500, 600, 100, 0, 0, None, None, 0, None, None, 0.2]
+for turn in range(60):
+    for knob in (-1, 99):
+        check(lib.tfhip_set_tuning(b"split", knob))
+        start = time.perf_counter()
+        for _ in range(1000):
+            call(*args)
+        best[knob] = min(best.get(knob, 1.0), (time.perf_counter() - start) / 1000)
+check(lib.tfhip_set_tuning(b"split", -1))
+assert "gemm_kernel" in launch()[0]
+assert best[-1] - best[99] < 0.22e-6, best
+""")

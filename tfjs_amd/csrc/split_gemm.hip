@@ -42,13 +42,16 @@ double split_estimate_us(const SplitShape &s, const GemmParams &p, int slices, d
   return s.launch + us * windows + finish_us(p, slices);
 }
 
+// The fourth root of the fourth powers' sum. (With pow, 0.1 us of host time in every call that comes this far.)
+double longer_of(double a, double b) { return sqrt(sqrt(a * a * a * a + b * b * b * b)); }
+
 // What the same product takes with gemm_kernel, whatever tile and slices that chooses: the launch, the matrix instructions at
 // 77% of their rate or the way of k through the pipeline, whichever is longer, and what fills and empties the chip. Least
 // squares on 8800 products and 4300 convolutions of random extents, root mean square error 16%.
 double tiled_estimate_us(const GemmParams &p, double windows) {
   const double blocks = (double)((p.M + 31) / 32) * ((p.N + 31) / 32) * p.batch, peak_us = blocks * 2048.0 * p.K / 155e6;
   const double pipeline_us = 0.0044 * p.K * (blocks < 256 ? pow(blocks / 256, 0.27) : 1.0);
-  return 4.4 + windows * (pow(pow(peak_us / 0.77, 4) + pow(pipeline_us, 4), 0.25) + 1.4 * sqrt(peak_us));
+  return 4.4 + windows * (longer_of(peak_us / 0.77, pipeline_us) + 1.4 * sqrt(peak_us));
 }
 
 // The same with a term for each tile's end, which counts for more than k where there are a few k tiles: 1200 products of random extents,
@@ -60,7 +63,7 @@ double tiled_end_us(const GemmParams &p, int a_kind, bool transposed_b) {
   const double *t = kTerms[kind];
   const double blocks = (double)((p.M + 31) / 32) * ((p.N + 31) / 32) * p.batch, peak_us = blocks * 2048.0 * p.K / 155e6;
   const double pipeline_us = 0.0044 * p.K * (blocks < 256 ? pow(blocks / 256, 0.27) : 1.0);
-  const double us = t[0] + t[1] * pow(pow(peak_us / 0.77, 4) + pow(pipeline_us, 4), 0.25) + t[2] * sqrt(peak_us) + t[3] * blocks / 256;
+  const double us = t[0] + t[1] * longer_of(peak_us / 0.77, pipeline_us) + t[2] * sqrt(peak_us) + t[3] * blocks / 256;
   return p.K <= 32 && a_kind == kLoadKAny ? 1.2 * us : us;
 }
 
@@ -193,11 +196,11 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b
   // the line above takes were not taken any more, and up to 1.3 times slower.)
   const double part = best_us / tiled_end_us(p, a_kind, transposed_b);
   double lead = a_kind == kLoadKAny ? (small ? 0.92 : 0.97) : (small ? 0.87 : 0.91);
+  if (small && a_kind == kLoadKAny && (double)p.batch * p.M * p.N < 5e6) lead = 0.81;
   if (!narrow && (a_kind == kLoadKAny || p.K <= kEndWindows) && part <= lead) {
     const TileShape &t = kTileShapes[choose_tile_shape(p.M, p.N, p.K, p.batch, num_cus())];
-    if (t.bm == 64 && t.bn <= 64) lead = small || a_kind != kLoadKAny ? 0 : 0.85;
-    else if (small && a_kind == kLoadKAny && (double)p.batch * p.M * p.N < 5e6) lead = 0.81;
-    if (part <= lead) return best;
+    const bool suits = t.bm == 64 && t.bn <= 64;
+    if (!suits || (!small && a_kind == kLoadKAny && part <= 0.85)) return best;
   }
   best.shape = -1;
   return best;
