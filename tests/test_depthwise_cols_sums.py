@@ -76,7 +76,7 @@ def test_large_result_is_streamed(f, c):
 
 
 @pytest.mark.parametrize("f,c", [(3, 16), (5, 20), (3, 15)])
-@pytest.mark.parametrize("rows_out", [1, 7, 8, 9, 15, 17, 23, 24, 25, 63, 65])
+@pytest.mark.parametrize("rows_out", [1, 3, 5, 7, 8, 9, 10, 11, 12, 13, 14, 15, 17, 23, 24, 25, 63, 65])
 def test_every_remainder_of_workgroups_over_the_xcds(orc, f, c, rows_out):
     # one row per workgroup: what eight equal runs leave over goes as it comes
     hip.init()

@@ -42,11 +42,33 @@ def _took_it():
     return name.value.decode().startswith("split_gemm<")
 
 
+def _relative(k):
+    return (k / 16 + 12) * 2.0 ** -23 + 2.0 ** -25
+
+
+def _windows(x, w):
+    """The convolution at stride 1 with "same" padding, in 64 bits."""
+    (n, h, wd, c), (fh, fw, _, out) = x.shape, w.shape
+    padded = np.zeros((n, h + fh - 1, wd + fw - 1, c))
+    padded[:, (fh - 1) // 2:(fh - 1) // 2 + h, (fw - 1) // 2:(fw - 1) // 2 + wd] = x
+    return sum(padded[:, i:i + h, j:j + wd].reshape(-1, c) @ w[i, j].astype(np.float64) for i in range(fh) for j in range(fw)).reshape(n, h, wd, out)
+
+
+def _with_low_parts(v):
+    """Its sizes, with the last eight bits of the mantissa between 0x20 and 0x7f: less than half a unit of the second bf16 part."""
+    bits = np.abs(v).view(np.uint32)
+    return ((bits & 0xffffff00) | (0x20 + (bits & 0xff) * 0x5f // 0xff)).view(np.float32)
+
+
+def _two_parts(v):
+    return (v.view(np.uint32) & 0xffffff00).view(np.float32)
+
+
 def _bound(a, b, k):
     """What a result may be off, per result: one rounding of the accumulator (truncated: an ulp, 2^-23) per matrix instruction
     of 16 k and per wavefront group, eight more for the small products, the bias and the store, and 2^-25 of each product
     for the parts left out; all relative to the sum of the products' sizes."""
-    return ((k / 16 + 12) * 2.0 ** -23 + 2.0 ** -25) * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 1e-37
+    return _relative(k) * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 1e-37
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -96,7 +118,16 @@ def test_windows_of_a_short_k(hip, orc, xs, fs):
     got = hip.fused_conv2d(x, w, **kw)
     assert _took_it()
     k = fs[0] * fs[1] * fs[2]
-    assert np.max(np.abs(got - orc.fused_conv2d(x, w, **kw))) <= k * (k / 16 + 12) * 2.0 ** -23 + k * 2.0 ** -24
+    sums, sizes = _windows(x, w), _windows(np.abs(x), np.abs(w))
+    want = np.clip(sums + kw["bias"].astype(np.float64), 0, 6)
+    assert (np.abs(got - want) <= _relative(k) * (sizes + np.abs(kw["bias"])) + 1e-37).all()
+    # positive operands whose third parts are all positive: without those of either the sums are 2^-17 too small
+    x, w = _with_low_parts(x), _with_low_parts(w)
+    got = hip.fused_conv2d(x, w, strides=1, dilations=1, pad="same")
+    assert _took_it()
+    want = _windows(x, w)
+    assert (np.abs(got - want) <= _relative(k) * want).all()
+    assert (_windows(_two_parts(x), w) < (1 - _relative(k)) * want).mean() > 0.9   # (what the bound is there to see)
 
 
 @pytest.mark.parametrize("shape", [s + 10 * (n - 1) for s in SHAPES for n in (1, 3)])
