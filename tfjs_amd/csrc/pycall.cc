@@ -4,9 +4,9 @@
 // us for the call itself, where the launch takes 2.5 to 3.3. Here the argument types are the entry point's own, so the
 // conversions are compiled: integers, None, floats and arrays of c_int64 are taken as they are. Whatever else
 // an argument may be (c_void_p, byref(), a number out of range, a count that does not match) goes to the ctypes function, which decides
-// as it always has. us per call on the host, ctypes and here: pyhost.device_fused_matmul 4.9 and 4.0, tfhip_fused_depthwise_conv2d 4.8
-// and 4.2 (the launch itself is all of that but 0.3). Likewise the manifest of a weight buffer: 52 tensors took 24 us to read and
-// 12 to wrap.
+// as it always has. us per call on the host, ctypes and here: pyhost.device_fused_matmul 4.7 and 3.8, tfhip_fused_depthwise_conv2d 4.4
+// and 3.7 (of the latter the launch itself is all but 0.3). Likewise the manifest of a weight buffer: 52 tensors took 24 us to read
+// and 12 to wrap.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 

@@ -8,16 +8,17 @@
 // bits, 2-norm relative, K = 64, 256, 768, 3072, operands N(0, 1) and N(0, 0.02): float32 matrix instructions 1.4e-7, 2.9e-7,
 // 5.0e-7, 9.8e-7, this kernel 0.5e-7, 0.9e-7, 1.6e-7, 3.4e-7; all-positive operands 1.2e-7 ... 8.3e-7 and 0.5e-7 ... 3.0e-7.
 //
-// us, gemm_kernel and here (rate of the product itself): 1024 x 2304 x 768 33.4 and 24.0 (151 TFLOP/s), 1024 x 3072 x 768 40.8
+// us, gemm_kernel and here (rate of the product itself; extents are rows x columns x inner): 1024 x 2304 x 768 33.4 and 24.0 (151 TFLOP/s), 1024 x 3072 x 768 40.8
 // and 27.9, 3072 x 3072 x 1024 153 and 106 - 112 by machine (180), 3072 x 4096 x 1024 189 and 134 - 139 (189), [8,56,56,64] 3x3 -> 64 26.7 and 16.4.
-// Of a transposed B, 128 x (384 x 64 x 384) 32.5 and 26.8, 128 x (512 x 64 x 512) 56 and 44, 1024 x 3072 x 768 38.8 and 28.7.
+// Of a transposed B, 128 x (384 x 384 x 64) 32.5 and 26.8, 128 x (512 x 512 x 64) 56 and 44, 1024 x 3072 x 768 38.8 and 28.7.
 // What bounds it: the loop, and in it the matrix cores for 67% of its cycles (128 x 128 tiles 70%), fetches and barriers for
 // the rest. A k tile of a 128 x 96 tile takes 0.69 us on 64 of the 256 units and 0.99 on all of them, where the chip's clock
 // falls from 2.30 to 1.70 GHz (busy and active cycles of launches of 1 ms, by counter). Over a launch of 3072 x 3072 x 1024 the
 // matrix cores are busy for 43% of 2.4 GHz: that clock, the waits, and 5 to 6 us of prologue and results in each of three
-// rounds are the rest. (Half of the reads of B's fragments and half of its splitting, 64 rows per wavefront in tiles of 256 x 128, change
-// nothing: 4096^3 takes 660 us with 128 x 128 and 650, 3072 x 4096 x 1024 136 to 141 and 160. Nor do idle units: 192 tiles of 3072 x 1024 x
-// 4096 take as long as 768 of 3072 x 4096 x 1024. It is the power.) On 1024 rows, 6 us of launch, prologue (2.5: arguments, the first fetch, the first tile's splitting) and
+// rounds are the rest. (64 rows per wavefront in tiles of 256 x 128 on four wavefronts, half of the reads of B's fragments and half of its
+// splitting, change nothing: 4096^3 takes 660 us with 128 x 128 and 650, 3072 x 4096 x 1024 136 to 141 and 160. Nor do idle units: 192 tiles of
+// 3072 x 1024 x 4096 take as long as 768 of 3072 x 4096 x 1024. So the power is a part of it, not all: on eight wavefronts that tile took
+// 612 us, and the 16x16x32 instruction 2 to 4% less in large 128 x 128 tiles; both lose on smaller products.) On 1024 rows, 6 us of launch, prologue (2.5: arguments, the first fetch, the first tile's splitting) and
 // results (2.7), and with 2304 or 768 columns a quarter of the units idle. (Slices of k that the last workgroup of a tile adds, instead of a
 // launch over the whole chip: 1024 x 768 x 3072 33.2 and 37.1.)
 //

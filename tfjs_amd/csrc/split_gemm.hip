@@ -10,7 +10,7 @@ namespace {
 // Least squares on 3700 products and 1900 convolutions of random extents, every tile timed on each (operands in the
 // caches): root mean square error 4 to 7% for products, 2% for windows, and the tile with the least estimate is on average 0.7%
 // slower than the fastest. (Fitted before operands were scaled, 3% of a k tile: left as it is, since the estimate for gemm_kernel is
-// low by more than that on few k tiles, where 128 x (512 x 64 x 512) takes 56 us with it and 44 here.)
+// low by more than that on few k tiles, where 128 x (512 x 512 x 64) takes 56 us with it and 44 here.)
 struct SplitShape {
   int gw, tn, kg;
   double launch, per_tile, fixed, per_tile_two, fixed_two;   // (_two: two workgroups on a compute unit; 0: one fits)
@@ -133,6 +133,9 @@ int launch_kind(SplitChoice c, GemmParams &p) {
 
 }  // namespace
 
+// What goes here, in this order: nothing that the offsets or the epilogue cannot hold; what the knob names; nothing below `least` FLOP or of
+// few rows; of what is left the tile and slices with the least estimate, if that is 8% below the tiled kernel's (narrow: below that in tiles
+// of 32 x 32); and of a few k tiles what the estimate with a tile's end leaves.
 SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b) {
   SplitChoice best = {-1, 1, 0};
   const int forced = tuning(kTuneSplit);
@@ -191,7 +194,7 @@ SplitChoice split_gemm_choice(const GemmParams &p, int a_kind, bool transposed_b
   //  * small products whose results are below 20 MB, but for a larger lead (0.81): 16% of them were slower, at 0.92 on average.
   // Of what is left, 2% of the small products, 1% of the others, 1.6% of a transposed B and 1% of the windows are 3% slower and more (before
   // these two 8, 1.4, 3.5 and 10%, up to a third: 11616 x 368 x 14 6.7 and 8.8, 32474 x 112 x 16 5.7 and 7.3, [7,96,98,3] 5x5 -> 61 17.6
-  // and 23.0). us, before and here: 4282 x 3818 x 32 34 and 21, 18 x (1007 x 20 x 860) of a transposed B 30 and 19, 3991 x 1333 x 71
+  // and 23.0). us, before and here: 4282 x 3818 x 32 34 and 21, 18 x (1007 x 860 x 20) of a transposed B 30 and 19, 3991 x 1333 x 71
   // 20 and 13, 130032 x 224 x 72 (windows) 94 and 54, 81125 x 100 x 40 (ragged) 39 and 24. (By that estimate alone, 3% of the products that
   // the line above takes were not taken any more, and up to 1.3 times slower.)
   const double part = best_us / tiled_end_us(p, a_kind, transposed_b);
