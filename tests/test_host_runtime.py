@@ -593,7 +593,7 @@ assert errors()[0] == 0, errors()
 
 
 def test_choosing_the_rows_of_a_depthwise_lane_costs_the_host_little():
-    """The rule that every call goes through, against a count that is given; the least of many turns. (0.2 us with divisions.)"""
+    """The rule that every call goes through, against a count that is given; the least of many turns."""
     fake_hip_util.run("""
 pyhost.init()
 a, w, out = DeviceBuffer(1 << 22), DeviceBuffer(1 << 12), DeviceBuffer(1 << 22)
@@ -609,7 +609,7 @@ for turn in range(60):
         best[knob] = min(best.get(knob, 1.0), (time.perf_counter() - start) / 1000)
 check(lib.tfhip_set_tuning(b"dw_rows", -1))
 assert "depthwise_3x3_cols" in launch()[0]
-assert best[-1] - best[14] < 0.13e-6, best
+assert best[-1] < 1.2 * best[14], best   # (1.08; with divisions 1.28)
 """)
 
 
@@ -673,5 +673,5 @@ for turn in range(60):
         best[knob] = min(best.get(knob, 1.0), (time.perf_counter() - start) / 1000)
 check(lib.tfhip_set_tuning(b"split", -1))
 assert "gemm_kernel" in launch()[0]
-assert best[-1] - best[99] < 0.22e-6, best
+assert best[-1] < 1.28 * best[99], best   # (1.18; with pow 1.33)
 """)
