@@ -338,8 +338,8 @@ inline FewRowsCut few_rows_cut(const GemmParams &p, int row_blocks, int col_bloc
   // up. us, one slice and more: 1 x 1280 x 1000 3.9 and 5.0, 1 x 2048 x 1000 4.4 and 4.9, 1 x 3072 x 1000 6.1 and 5.3. Beyond, what a
   // compute unit can have out bounds the fetches (some 16 KB), so more units are ahead: with slices of 64, of 32 and the best of ten
   // counts, 16 x 2048 x 256 6.1, 5.3, 5.3, 40 x 2048 x 64 6.1, 4.8, 4.8, 16 x 4096 x 64 6.0, 5.0, 4.7, 1 x 3072 x 256 5.1, 5.0, 4.9; 140
-  // products of 1 to 64 rows, 1040 to 4096 and 64 to 1024: 1.10, 1.03 and 1 on average, none 3% slower with 32. More workgroups than
-  // compute units only add to what goes through memory.
+  // products of 1 to 64 rows, 1040 to 4096 and 64 to 1024: 1.10, 1.03 and 1 on average (of 900 others, up to 4096 columns, 14 are more than 3%
+  // slower with 32 than with 64). More workgroups than compute units only add to what goes through memory.
   const int whole = row_blocks != 1 ? 32 : (p.M == 1 ? 128 : 64);
   const int wanted = groups <= whole ? 1 : (groups + 31) / 32;
   const int most = cut.tiles * 2 > kFewRowsCounters ? 1 : kFewRowsCounters / (int)cut.tiles;
